@@ -782,38 +782,79 @@ struct PreArgs {
     size_t rstride;    // complex values between realisations of one field
 };
 
-__device__ double dev_ranff(int* idum, int* iy, int* iv)
+// ranff (accesories.f90:38-68) for one wavefront: n draws of the stream in state st
+// (idum, iy, iv(32)), each left in seq as the integer that ranff scales by 1/IM.  The
+// generator's two parts cost one lane 240 us for the 450 draws of a step; here
+//   - the linear congruence x -> 16807 x mod (2^31 - 1) jumps ahead: lane i multiplies by
+//     16807^(i+1), so 64 values come at once (exact in 64 bits, the values of the
+//     reference's Schrage steps);
+//   - the Bays-Durham shuffle is serial in iy, so its table lives in the lanes of one
+//     register (lane i holds iv(i+1)) and a draw is one readlane and one writelane.
+__device__ __forceinline__ unsigned ranff_mul(unsigned a, unsigned b)
 {
-    const int IA = 16807, IM = 2147483647, IQ = 127773, IR = 2836, NTAB_ = 32;
-    const int NDIV = 1 + (IM - 1) / NTAB_;
-    const double AM = 1.0 / IM, EPS = 1.2e-7, RNMX = 1.0 - EPS;
-    int j, k;
-    if (*idum <= 0 || *iy == 0) {
-        *idum = (-*idum > 1) ? -*idum : 1;
-        // 8 warm-up draws, then the table from iv[31] down to iv[0]: the same
-        // sequence as one loop j = 40..1 storing at j <= 32, written so that no
-        // store index is ever outside the table
-        for (j = 0; j < 8; ++j) {
-            k = *idum / IQ;
-            *idum = IA * (*idum - k * IQ) - IR * k;
-            if (*idum < 0) *idum += IM;
-        }
-        for (j = NTAB_ - 1; j >= 0; --j) {
-            k = *idum / IQ;
-            *idum = IA * (*idum - k * IQ) - IR * k;
-            if (*idum < 0) *idum += IM;
-            iv[j] = *idum;
-        }
-        *iy = iv[0];
+    const unsigned long long p = (unsigned long long)a * b;
+    unsigned r = (unsigned)(p & 0x7fffffffu) + (unsigned)(p >> 31);
+    return r >= 0x7fffffffu ? r - 0x7fffffffu : r;      // a, b < 2^31 - 1, never 0: one fold is enough
+}
+
+__device__ __forceinline__ void ranff_draws(int* st, int n, int* seq)
+{
+    const int lane = threadIdx.x & 63;
+    const int IM = 2147483647;
+    // 16807^(lane + 1) mod IM by squaring
+    unsigned pw = 1, sq = 16807u;
+    for (int e = lane + 1; e; e >>= 1) {
+        if (e & 1) pw = ranff_mul(pw, sq);
+        sq = ranff_mul(sq, sq);
     }
-    k = *idum / IQ;
-    *idum = IA * (*idum - k * IQ) - IR * k;
-    if (*idum < 0) *idum += IM;
-    j = 1 + *iy / NDIV;
-    *iy = iv[j - 1];
-    iv[j - 1] = *idum;
-    const double r = AM * (double)(*iy);
-    return r < RNMX ? r : RNMX;
+    int idum = __builtin_amdgcn_readfirstlane(st[0]), iy = __builtin_amdgcn_readfirstlane(st[1]);
+    int iv = lane < 32 ? st[2 + lane] : 0;
+    if (idum <= 0 || iy == 0) {
+        idum = (-idum > 1) ? -idum : 1;
+        // 8 warm-up values, then the table from iv(32) down to iv(1): value 9 + q of the
+        // stream is iv(32 - q)
+        const unsigned x = ranff_mul((unsigned)(idum % IM), pw);
+        iv = __shfl((int)x, 39 - (lane & 31), 64);
+        idum = __builtin_amdgcn_readlane((int)x, 39);
+        iy = __builtin_amdgcn_readlane(iv, 0);
+    }
+    for (int n0 = 0; n0 < n; n0 += 64) {
+        const int m = min(64, n - n0);
+        const int x = (int)ranff_mul((unsigned)idum, pw);
+        int out = 0;
+        for (int q = 0; q < m; ++q) {
+            const int j = iy >> 26;                     // iy / NDIV, NDIV = 1 + (IM - 1) / 32 = 2^26
+            iy = __builtin_amdgcn_readlane(iv, j);
+            iv = lane == j ? __builtin_amdgcn_readlane(x, q) : iv;
+            out = lane == q ? iy : out;
+        }
+        idum = __builtin_amdgcn_readlane(x, m - 1);
+        if (lane < m) seq[n0 + lane] = out;
+    }
+    if (lane == 0) { st[0] = idum; st[1] = iy; }
+    if (lane < 32) st[2 + lane] = iv;
+}
+
+// Index of mode (i, j, k) (1-based j, k; i = 0 real part) in a forcing table a(6,5,5)
+__device__ __forceinline__ int sth_at(int j, int k) { return 6 * ((j - 1) + 5 * (k - 1)); }
+
+// The Hermitian fix-up of the kx = 0 modes of a table (flowlib.f90:424-440, 481-510): pair q
+// of 12, whose target is never another pair's source; then the mean mode is zero
+__device__ __forceinline__ void sth_hermitian(double* t, int q)
+{
+    int src, dst;
+    if (q < 10) {
+        const int k = q / 2 + 1, j = q % 2 + 2;
+        src = sth_at(j, k);
+        dst = sth_at(7 - j, k == 1 ? 1 : 7 - k);
+    } else {
+        const int k = q - 8;                            // 2, 3
+        src = sth_at(1, k);
+        dst = sth_at(1, 7 - k);
+    }
+    t[dst] = t[src];
+    t[dst + 1] = -t[src + 1];
+    if (q == 0) { t[0] = 0.0; t[1] = 0.0; }
 }
 
 // supforDET's 225 low-mode sums (75 modes kx in 0..2, ky, kz in -2..2, times 3
@@ -867,90 +908,58 @@ __global__ void __launch_bounds__(NT) k_pre(PreArgs a)
     const int forcing = real_forcing(a.forcing, low);
     const bool own = a.forcing < 0;
     if (forcing == 2) {
-        if (tid != 0) return;
+        // supforSTH by the whole work-group: the draws by one wavefront, then one mode per
+        // thread (225 modes of white noise, 150 table entries per component).  The loops over
+        // the tables run once per step on one work-group, so latency is all they cost.
         int* st = a.sth_state + (size_t)rr * STH_STATE_STRIDE;
-        int idum = st[0], iy = st[1];
-        // shuffle table in LDS: a private array indexed by a data-dependent j is
-        // lowered to indexed register moves, which gives no protection at all
-        // against a stray index
-        __shared__ int iv[32];
-        for (int i = 0; i < 32; ++i) iv[i] = st[2 + i];
+        __shared__ int seq[450];
+        __shared__ double fr[3][150], fo[3][150];
         const double dt = a.dt, tf = own ? low[LOW_PAR + 3] : a.ou_tf, var = own ? low[LOW_PAR + 4] : a.ou_var;
         const double pi2 = a.pi2;
-        double fr[3][150];
-        for (int mc = 0; mc < 3; ++mc)                                   // flowlib.f90:405-419
-            for (int k = 0; k < 5; ++k)
-                for (int j = 0; j < 5; ++j)
-                    for (int i = 0; i < 6; i += 2) {
-                        double cont1 = dev_ranff(&idum, &iy, iv);
-                        if (cont1 < 1.e-6) cont1 = 1.e-6;
-                        const double rmag = sqrt(-4.0 * var * dt * log(cont1) / tf);
-                        const double rph = dev_ranff(&idum, &iy, iv);
-                        fr[mc][i + 6 * (j + 5 * k)] = rmag * cos(pi2 * rph);
-                        fr[mc][i + 1 + 6 * (j + 5 * k)] = rmag * sin(pi2 * rph);
-                    }
-        for (int mc = 0; mc < 3; ++mc) {                                 // 424-440
-            for (int k = 1; k <= 5; ++k) {
-                const int kk = (k == 1) ? 1 : 7 - k;
-                for (int j = 2; j <= 3; ++j) {
-                    const int jj = 7 - j;
-                    fr[mc][0 + 6 * ((jj - 1) + 5 * (kk - 1))] = fr[mc][0 + 6 * ((j - 1) + 5 * (k - 1))];
-                    fr[mc][1 + 6 * ((jj - 1) + 5 * (kk - 1))] = -fr[mc][1 + 6 * ((j - 1) + 5 * (k - 1))];
-                }
-            }
-            for (int k = 2; k <= 3; ++k) {
-                const int kk = 7 - k;
-                fr[mc][0 + 6 * (5 * (kk - 1))] = fr[mc][0 + 6 * (5 * (k - 1))];
-                fr[mc][1 + 6 * (5 * (kk - 1))] = -fr[mc][1 + 6 * (5 * (k - 1))];
-            }
-            fr[mc][0] = 0.0;
-            fr[mc][1] = 0.0;
+        if (tid < 64) ranff_draws(st, 450, seq);
+        __syncthreads();
+        if (tid < 225) {                                                 // flowlib.f90:405-419
+            const double AM = 1.0 / 2147483647, RNMX = 1.0 - 1.2e-7;
+            double cont1 = AM * (double)seq[2 * tid], rph = AM * (double)seq[2 * tid + 1];
+            cont1 = cont1 < RNMX ? cont1 : RNMX;
+            rph = rph < RNMX ? rph : RNMX;
+            if (cont1 < 1.e-6) cont1 = 1.e-6;
+            const double rmag = sqrt(-4.0 * var * dt * log(cont1) / tf);
+            const int mc = tid / 75, o = 2 * (tid % 75);
+            fr[mc][o] = rmag * cos(pi2 * rph);
+            fr[mc][o + 1] = rmag * sin(pi2 * rph);
         }
+        __syncthreads();
+        if (tid < 36) sth_hermitian(fr[tid / 12], tid % 12);             // 424-440
+        __syncthreads();
         double* b = a.sth_b + (size_t)rr * STH_B_STRIDE;
         double* fa = low + 8;
-        const double smallx = 1.0e-18, xkf = sqrt(8.0);
-        for (int k = 0; k < 5; ++k)                                      // 447-478
-            for (int j = 0; j < 5; ++j)
-                for (int i = 0; i < 6; ++i) {
-                    const int o = i + 6 * (j + 5 * k);
-                    const double kx_ = (double)(i / 2);
-                    const double ky_ = (double)(j <= 2 ? j : j - 5);
-                    const double kz_ = (double)(k <= 2 ? k : k - 5);
-                    const double radm = sqrt(kx_ * kx_ + ky_ * ky_ + kz_ * kz_);
-                    if (radm < xkf) {
-                        b[o] = b[o] * (1.0 - dt / tf) + fr[0][o];
-                        b[150 + o] = b[150 + o] * (1.0 - dt / tf) + fr[1][o];
-                        b[300 + o] = b[300 + o] * (1.0 - dt / tf) + fr[2][o];
-                        const double t1 = kx_ * b[o], t2 = ky_ * b[150 + o], t3 = kz_ * b[300 + o];
-                        double divb = (t1 + t2 + t3) / ((radm + smallx) * (radm + smallx));
-                        if (radm == 0.) divb = 0.0;
-                        fa[o] = b[o] - kx_ * divb;
-                        fa[150 + o] = b[150 + o] - ky_ * divb;
-                        fa[300 + o] = b[300 + o] - kz_ * divb;
-                    } else {
-                        fa[o] = 0.0; fa[150 + o] = 0.0; fa[300 + o] = 0.0;
-                    }
-                }
-        for (int mc = 0; mc < 3; ++mc) { fa[150 * mc] = 0.0; fa[150 * mc + 1] = 0.0; }   // 481-483
-        for (int k = 1; k <= 5; ++k) {                                   // 488-500
-            const int kk = (k == 1) ? 1 : 7 - k;
-            for (int j = 2; j <= 3; ++j) {
-                const int jj = 7 - j;
-                for (int mc = 0; mc < 3; ++mc) {
-                    fa[150 * mc + 6 * ((jj - 1) + 5 * (kk - 1))] = fa[150 * mc + 6 * ((j - 1) + 5 * (k - 1))];
-                    fa[150 * mc + 1 + 6 * ((jj - 1) + 5 * (kk - 1))] = -fa[150 * mc + 1 + 6 * ((j - 1) + 5 * (k - 1))];
-                }
+        if (tid < 150) {                                                 // 447-478
+            const double smallx = 1.0e-18, xkf = sqrt(8.0);
+            const int o = tid, i = o % 6, j = (o / 6) % 5, k = o / 30;
+            const double kx_ = (double)(i / 2);
+            const double ky_ = (double)(j <= 2 ? j : j - 5);
+            const double kz_ = (double)(k <= 2 ? k : k - 5);
+            const double radm = sqrt(kx_ * kx_ + ky_ * ky_ + kz_ * kz_);
+            double f0 = 0.0, f1 = 0.0, f2 = 0.0;
+            if (radm < xkf) {
+                const double b0 = b[o] * (1.0 - dt / tf) + fr[0][o];
+                const double b1 = b[150 + o] * (1.0 - dt / tf) + fr[1][o];
+                const double b2 = b[300 + o] * (1.0 - dt / tf) + fr[2][o];
+                b[o] = b0; b[150 + o] = b1; b[300 + o] = b2;
+                const double t1 = kx_ * b0, t2 = ky_ * b1, t3 = kz_ * b2;
+                double divb = (t1 + t2 + t3) / ((radm + smallx) * (radm + smallx));
+                if (radm == 0.) divb = 0.0;
+                f0 = b0 - kx_ * divb;
+                f1 = b1 - ky_ * divb;
+                f2 = b2 - kz_ * divb;
             }
+            fo[0][o] = f0; fo[1][o] = f1; fo[2][o] = f2;
         }
-        for (int k = 2; k <= 3; ++k) {                                   // 502-510
-            const int kk = 7 - k;
-            for (int mc = 0; mc < 3; ++mc) {
-                fa[150 * mc + 6 * (5 * (kk - 1))] = fa[150 * mc + 6 * (5 * (k - 1))];
-                fa[150 * mc + 1 + 6 * (5 * (kk - 1))] = -fa[150 * mc + 1 + 6 * (5 * (k - 1))];
-            }
-        }
-        st[0] = idum; st[1] = iy;
-        for (int i = 0; i < 32; ++i) st[2 + i] = iv[i];
+        __syncthreads();
+        if (tid < 36) sth_hermitian(fo[tid / 12], tid % 12);             // 481-510
+        __syncthreads();
+        for (int e = tid; e < 450; e += NT) fa[e] = fo[e / 150][e % 150];
         return;
     }
     if (forcing != 1) return;
