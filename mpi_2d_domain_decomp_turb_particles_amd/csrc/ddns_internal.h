@@ -265,6 +265,9 @@ int flow_init(FlowBuffers& fb, int N, int nek, int precision, int kind, int seed
 int flow_diagnostics(FlowBuffers& fb, int N, int nek, double rnu, int precision, int want, double* ek, double* dk,
                      double* tk, double* mom, hipStream_t s);
 int flow_spectrum(const FlowBuffers& fb, int N, int nek, int precision, double* ek, hipStream_t s);
+// E, D and (F given) T shell sums on the device: part 3 SPEC_BLOCKS nek, sums_dev 3 nek doubles
+int flow_shell_sums(const FlowBuffers& fb, const void* const F[3], int N, int nek, double rnu, int precision, double* part,
+                    double* sums_dev, hipStream_t s);
 // allocation-free E(k) (spectrum.hip): the partial rows in a file-scope device array whose
 // address is resolved once per device by spectrum_scratch_init
 int spectrum_scratch_init();

@@ -1069,41 +1069,49 @@ __device__ __forceinline__ double2 init_gauss(unsigned long long key, int c, int
 // reduction (kx = 0 modes at half weight), whose fixed order makes the field the same
 // bits on every run.
 template <typename T, int N>
-__global__ void k_init_modes(void* u0, void* u1, void* u2, unsigned long long key, int nek, unsigned long long* cnt2)
+__global__ void __launch_bounds__(256) k_init_modes(void* u0, void* u1, void* u2, unsigned long long key, int nek,
+                                                    unsigned long long* cnt2)
 {
     using C = cpx<T>;
     constexpr int M = N / 2;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)N * N * M) return;
-    const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
-    const int kyw = wave_index(ky, N), kzw = wave_index(kz, N);
-    const bool zero = ky == N / 2 || kz == N / 2 || (kx == 0 && ky == 0 && kz == 0);
-    double2 g[3];
+    // the counts of a work-group's modes in LDS first: one global atomic per mode made this
+    // kernel 6.5 ms at 256^3 and 131 ms at 1024^3
+    __shared__ unsigned cnt[M];
+    for (int i = threadIdx.x; i < M; i += 256) cnt[i] = 0;
+    __syncthreads();
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < (size_t)N * N * M; t += (size_t)gridDim.x * 256) {
+        const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
+        const int kyw = wave_index(ky, N), kzw = wave_index(kz, N);
+        const bool zero = ky == N / 2 || kz == N / 2 || (kx == 0 && ky == 0 && kz == 0);
+        double2 g[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        g[c] = init_gauss<N>(key, c, kz, ky, kx);
-        if (kx == 0) {
-            const double2 h = init_gauss<N>(key, c, (N - kz) & (N - 1), (N - ky) & (N - 1), 0);
-            g[c] = make_double2(0.5 * (g[c].x + h.x), 0.5 * (g[c].y - h.y));
+        for (int c = 0; c < 3; ++c) {
+            g[c] = init_gauss<N>(key, c, kz, ky, kx);
+            if (kx == 0) {
+                const double2 h = init_gauss<N>(key, c, (N - kz) & (N - 1), (N - ky) & (N - 1), 0);
+                g[c] = make_double2(0.5 * (g[c].x + h.x), 0.5 * (g[c].y - h.y));
+            }
+            if (zero) g[c] = make_double2(0.0, 0.0);
         }
-        if (zero) g[c] = make_double2(0.0, 0.0);
-    }
-    const double k[3] = {(double)kx, (double)kyw, (double)kzw};
-    double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-    if (kx == 0 && ky == 0 && kz == 0) k2 = 1.e-5;
-    const double pr = (k[0] * g[0].x + k[1] * g[1].x + k[2] * g[2].x) / k2;
-    const double pi = (k[0] * g[0].y + k[1] * g[1].y + k[2] * g[2].y) / k2;
-    void* u[3] = {u0, u1, u2};
+        const double k[3] = {(double)kx, (double)kyw, (double)kzw};
+        double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
+        if (kx == 0 && ky == 0 && kz == 0) k2 = 1.e-5;
+        const double pr = (k[0] * g[0].x + k[1] * g[1].x + k[2] * g[2].x) / k2;
+        const double pi = (k[0] * g[0].y + k[1] * g[1].y + k[2] * g[2].y) / k2;
+        void* u[3] = {u0, u1, u2};
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const double x = g[c].x - k[c] * pr, y = g[c].y - k[c] * pi;
-        ((C*)u[c])[t] = mk<C>((T)x, (T)y);
+        for (int c = 0; c < 3; ++c) {
+            const double x = g[c].x - k[c] * pr, y = g[c].y - k[c] * pi;
+            ((C*)u[c])[t] = mk<C>((T)x, (T)y);
+        }
+        const int ik2 = (int)(sqrt(k2) + 0.5);
+        // twice the shell's mode count (kx = 0 modes count one half): integer sums, the same
+        // in any order; the shell energies come from the fixed-tree E(k) reduction
+        if (ik2 >= 1 && ik2 <= nek) atomicAdd(cnt + ik2 - 1, kx == 0 ? 1u : 2u);
     }
-    const int ik2 = (int)(sqrt(k2) + 0.5);
-    if (ik2 < 1 || ik2 > nek) return;
-    // twice the shell's mode count (kx = 0 modes count one half): integer sums, the same
-    // in any order; the shell energies come from the fixed-tree E(k) reduction
-    atomicAdd(cnt2 + ik2 - 1, kx == 0 ? 1ull : 2ull);
+    __syncthreads();
+    for (int i = threadIdx.x; i < nek; i += 256)
+        if (cnt[i]) atomicAdd(cnt2 + i, (unsigned long long)cnt[i]);
 }
 
 // the shell factors (flowlib.f90:119-137), and zero above nek (139-141)
@@ -1555,7 +1563,7 @@ static int init_impl(FlowBuffers& fb, int nek, int kind, int seed, double k0, do
     DDNS_HIP(hipMalloc(&d, 2 * (size_t)nek * sizeof(double)));
     DDNS_HIP(hipMemsetAsync(d, 0, (size_t)nek * sizeof(double), s));
     const unsigned long long key = (unsigned long long)(long long)seed;
-    hipLaunchKernelGGL((k_init_modes<T, N>), dim3(g), dim3(256), 0, s, fb.U[0], fb.U[1], fb.U[2], key, nek,
+    hipLaunchKernelGGL((k_init_modes<T, N>), dim3(std::min(g, 4096u)), dim3(256), 0, s, fb.U[0], fb.U[1], fb.U[2], key, nek,
                        (unsigned long long*)d);
     DDNS_HIP(hipGetLastError());
     std::vector<unsigned long long> c2(nek);
@@ -1739,17 +1747,18 @@ __global__ void k_cross(const T* __restrict__ u0, const T* __restrict__ u1, cons
     w2[i] = ux * wy - uy * wx;
 }
 
-constexpr int DG_BLOCKS = 256;   // fixed grid of the diagnostic reductions
+constexpr int DG_BLOCKS = 256;   // fixed grid of the diagnostic reductions: one work-group per CU, of
+constexpr int DG_T = 1024;       // 16 wavefronts (with 4 the loads in flight held it to 1.7 TB/s at 256^3)
 
 // per work-group sums over a real field: mode 0: f^2, f^3, f^4 of one field;
 // mode 1: the max of |f0| + |f1| + |f2|; mode 2: sum |g|, |g|^2 and |g| f0 with
 // |g| = sqrt(f1^2 + f2^2 + f3^2) (vorticity magnitude against the divergence f0);
 // mode 3: f, f^2 of one field
 template <typename T>
-__global__ void __launch_bounds__(256) k_dg_reduce(const T* f0, const T* f1, const T* f2, const T* f3, size_t n,
+__global__ void __launch_bounds__(DG_T) k_dg_reduce(const T* f0, const T* f1, const T* f2, const T* f3, size_t n,
                                                   int mode, double* part)
 {
-    __shared__ double sh[3][256];
+    __shared__ double sh[3][DG_T];
     double a0 = 0.0, a1 = 0.0, a2 = 0.0;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         if (mode == 0) {
@@ -1769,7 +1778,7 @@ __global__ void __launch_bounds__(256) k_dg_reduce(const T* f0, const T* f1, con
     }
     sh[0][threadIdx.x] = a0; sh[1][threadIdx.x] = a1; sh[2][threadIdx.x] = a2;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
+    for (int o = DG_T / 2; o > 0; o >>= 1) {
         if (threadIdx.x < o) {
             if (mode == 1) sh[0][threadIdx.x] = fmax(sh[0][threadIdx.x], sh[0][threadIdx.x + o]);
             else {
@@ -1784,36 +1793,6 @@ __global__ void __launch_bounds__(256) k_dg_reduce(const T* f0, const T* f1, con
         part[blockIdx.x] = sh[0][0];
         part[gridDim.x + blockIdx.x] = sh[1][0];
         part[2 * gridDim.x + blockIdx.x] = sh[2][0];
-    }
-}
-
-// shell sums over |k| shells 1..nek (kx = 0 plane halved, postprocessing.f90:143-170,
-// 285-313): e = |u|^2, d = 2 nu k^2 |u|^2, tr = Re(conj(u) . F) with F the nonlinear term
-template <typename T, int N>
-__global__ void k_shells(const void* u0, const void* u1, const void* u2, const void* F0, const void* F1,
-                         const void* F2, int nek, double rnu, double* e, double* d, double* tr)
-{
-    using C = cpx<T>;
-    constexpr int M = N / 2;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)N * N * M) return;
-    const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
-    const int kyw = wave_index(ky, N), kzw = wave_index(kz, N);
-    double k2 = (double)(kx * kx + kyw * kyw + kzw * kzw);
-    if (k2 == 0.0) k2 = 1.e-5;
-    const int ik2 = (int)(sqrt(k2) + 0.5);
-    if (ik2 < 1 || ik2 > nek) return;
-    const C a = ((const C*)u0)[t], b = ((const C*)u1)[t], c = ((const C*)u2)[t];
-    const double h = kx == 0 ? 0.5 : 1.0;
-    const double ee = h * ((double)a.x * a.x + (double)a.y * a.y + (double)b.x * b.x + (double)b.y * b.y +
-                           (double)c.x * c.x + (double)c.y * c.y);
-    atomicAdd(e + ik2 - 1, ee);
-    atomicAdd(d + ik2 - 1, 2.0 * rnu * ee * k2);
-    if (F0) {
-        const C p = ((const C*)F0)[t], q = ((const C*)F1)[t], r = ((const C*)F2)[t];
-        const double tt = (double)a.x * p.x + (double)a.y * p.y + (double)b.x * q.x + (double)b.y * q.y +
-                          (double)c.x * r.x + (double)c.y * r.y;
-        atomicAdd(tr + ik2 - 1, h * tt);
     }
 }
 
@@ -1852,7 +1831,7 @@ template <typename T>
 static int dg_reduce(const T* f0, const T* f1, const T* f2, const T* f3, size_t n, int mode, double* part, double out[3],
                      hipStream_t s)
 {
-    hipLaunchKernelGGL((k_dg_reduce<T>), dim3(DG_BLOCKS), dim3(256), 0, s, f0, f1, f2, f3, n, mode, part);
+    hipLaunchKernelGGL((k_dg_reduce<T>), dim3(DG_BLOCKS), dim3(DG_T), 0, s, f0, f1, f2, f3, n, mode, part);
     DDNS_HIP(hipGetLastError());
     double h[3 * DG_BLOCKS];
     DDNS_HIP(hipMemcpyAsync(h, part, sizeof(h), hipMemcpyDeviceToHost, s));
@@ -1873,8 +1852,9 @@ static int diag_impl(FlowBuffers& fb, int nek, double rnu, int want, double* ek,
     const size_t fbytes = n3 * sizeof(T);                    // one real field = one complex field
     if (!fb.dg[0]) {
         for (int q = 0; q < 8; ++q) DDNS_HIP(hipMalloc(&fb.dg[q], fbytes));
-        // reduction partials (3 DG_BLOCKS) or the 3 nek shell sums, nek < N / 2
-        DDNS_HIP(hipMalloc(&fb.dg_part, 3 * (size_t)std::max(DG_BLOCKS, N / 2) * sizeof(double)));
+        // the 3 nek shell sums (nek < N / 2) and their partials, or the 3 DG_BLOCKS partials of
+        // a reduction over a real field
+        DDNS_HIP(hipMalloc(&fb.dg_part, 3 * (size_t)std::max(DG_BLOCKS, (SPEC_BLOCKS + 1) * (N / 2)) * sizeof(double)));
     }
     T* R[6];
     for (int q = 0; q < 6; ++q) R[q] = (T*)fb.dg[q];
@@ -1926,7 +1906,6 @@ static int diag_impl(FlowBuffers& fb, int nek, double rnu, int want, double* ek,
     }
     // spectra; the transfer needs the nonlinear term F = FFT(u x w) (turb.f90:634-650)
     double* dd = fb.dg_part;           // 3 nek shell sums
-    DDNS_HIP(hipMemsetAsync(dd, 0, 3 * (size_t)nek * sizeof(double), s));
     const void* F[3] = {nullptr, nullptr, nullptr};
     if (tk) {
         hipLaunchKernelGGL((k_cross<T>), dim3(gr), dim3(256), 0, s, R[0], R[1], R[2], R[3], R[4], R[5], n3);
@@ -1937,9 +1916,8 @@ static int diag_impl(FlowBuffers& fb, int nek, double rnu, int want, double* ek,
             F[c] = R[c];
         }
     }
-    hipLaunchKernelGGL((k_shells<T, N>), dim3(gc), dim3(256), 0, s, fb.U[0], fb.U[1], fb.U[2], F[0], F[1], F[2], nek, rnu,
-                       dd, dd + nek, dd + 2 * nek);
-    DDNS_HIP(hipGetLastError());
+    st = flow_shell_sums(fb, F, N, nek, rnu, sizeof(T) == 8 ? DDNS_FP64 : DDNS_FP32_MIXED, dd + 3 * (size_t)nek, dd, s);
+    if (st) return st;
     std::vector<double> h(3 * (size_t)nek);
     DDNS_HIP(hipMemcpyAsync(h.data(), dd, h.size() * sizeof(double), hipMemcpyDeviceToHost, s));
     DDNS_HIP(hipStreamSynchronize(s));

@@ -7,8 +7,8 @@
 // row the shell number never decreases with kx, so the 64 lanes of a row chunk form
 // runs of equal shell number; a segmented inclusive scan over the lanes sums each run,
 // and only the last lane of a run adds it to the wavefront's own LDS shell table (no
-// two lanes touch one entry).  The four wavefronts' tables are added in order into one
-// partial row per work-group, and a second kernel adds the SPEC_BLOCKS partial rows of
+// two lanes touch one entry).  The wavefronts' tables are added in order into one partial
+// row per work-group, and a second kernel adds the SPEC_BLOCKS partial rows of
 // each shell in order.  Products and sums are in double in both precision modes.
 //
 // ddns_get_spectrum runs them with the partial rows in a buffer of the handle;
@@ -19,32 +19,44 @@
 
 namespace ddns {
 
-constexpr int SPEC_T = 256;                        // threads per work-group: 4 wavefronts
-constexpr int SPEC_W = SPEC_T / 64;
+constexpr int SPEC_FT = 256;                       // threads of the final kernel: 4 shells per work-group
 
 __device__ __forceinline__ int spec_wave_index(int i, int N) { return i <= N / 2 ? i : i - N; }
 
-// Partial shell sums: part[s * SPEC_BLOCKS + b] for shell s + 1 and work-group b.
-template <typename T>
-__global__ void __launch_bounds__(SPEC_T) k_shell_partials(const void* __restrict__ u0, const void* __restrict__ u1,
-                                                           const void* __restrict__ u2, int N, int nek,
-                                                           double* __restrict__ part)
+// NV shell sums at once: E(k) alone (NV = 1), with the dissipation 2 nu k^2 E (NV = 2), and
+// with the transfer Re(conj(u) . F) of the nonlinear term F (NV = 3, postprocessing.f90:
+// 285-313).  Partial sums: part[(v * nek + s) * SPEC_BLOCKS + b] for sum v, shell s + 1 and
+// work-group b.  Each wavefront has its own shell tables in LDS (NV * nek doubles), and a
+// work-group has as many wavefronts as fit: the kernel waits on its row loads.  (Adding every
+// mode with global atomics, as the diagnostics did, took 6.46 ms at 256^3: all modes meet on
+// 126 addresses.)
+template <typename T, int NV>
+__global__ void __launch_bounds__(1024) k_shell_partials(const void* __restrict__ u0, const void* __restrict__ u1,
+                                                         const void* __restrict__ u2, const void* __restrict__ F0,
+                                                         const void* __restrict__ F1, const void* __restrict__ F2,
+                                                         int N, int nek, double rnu, double* __restrict__ part)
 {
     using C = cpx<T>;
-    __shared__ double acc[SPEC_W][SPEC_NEK_MAX];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < SPEC_W * SPEC_NEK_MAX; i += SPEC_T) (&acc[0][0])[i] = 0.0;
+    extern __shared__ double acc[];                   // [wavefront][v][shell]
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    for (int i = threadIdx.x; i < nw * NV * nek; i += blockDim.x) acc[i] = 0.0;
     __syncthreads();
+    double* mine = acc + (size_t)w * NV * nek;
     const int M = N / 2;
     const long long rows = (long long)N * N;
     const C* f[3] = {(const C*)u0, (const C*)u1, (const C*)u2};
-    for (long long r = (long long)blockIdx.x * SPEC_W + w; r < rows; r += (long long)gridDim.x * SPEC_W) {
+    const C* g[3] = {(const C*)F0, (const C*)F1, (const C*)F2};
+    for (long long r = (long long)blockIdx.x * nw + w; r < rows; r += (long long)gridDim.x * nw) {
         const int ky = (int)(r % N), kz = (int)(r / N);
         const int kyw = spec_wave_index(ky, N), kzw = spec_wave_index(kz, N);
         const int kyz2 = kyw * kyw + kzw * kzw;
         for (int c0 = 0; c0 < M; c0 += 64) {
+            // the chunk's lowest mode lies beyond the last shell: so do all that follow
+            if ((int)(sqrt((double)(c0 * c0 + kyz2)) + 0.5) > nek) break;
             const int kx = c0 + lane;
-            double e = 0.0;
+            double e[NV];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) e[v] = 0.0;
             int sh = nek + 1;                     // beyond the last shell: dropped
             if (kx < M) {
                 double k2 = (double)(kx * kx + kyz2);
@@ -54,39 +66,53 @@ __global__ void __launch_bounds__(SPEC_T) k_shell_partials(const void* __restric
 #pragma unroll
                 for (int q = 0; q < 3; ++q) {
                     const C a = f[q][t];
-                    e += (double)a.x * (double)a.x + (double)a.y * (double)a.y;
+                    e[0] += (double)a.x * (double)a.x + (double)a.y * (double)a.y;
+                    if constexpr (NV == 3) {
+                        const C p = g[q][t];
+                        e[2] += (double)a.x * (double)p.x + (double)a.y * (double)p.y;
+                    }
                 }
-                if (kx == 0) e *= 0.5;
+                if (kx == 0) {
+                    e[0] *= 0.5;
+                    if constexpr (NV == 3) e[2] *= 0.5;
+                }
+                if constexpr (NV >= 2) e[1] = 2.0 * rnu * e[0] * k2;
                 if (sh > nek) sh = nek + 1;
             }
             // segmented inclusive scan: sh is non-decreasing over the lanes
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) {
-                const double ev = __shfl_up(e, o, 64);
                 const int sv = __shfl_up(sh, o, 64);
-                if (lane >= o && sv == sh) e += ev;
+                const bool same = lane >= o && sv == sh;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    const double ev = __shfl_up(e[v], o, 64);
+                    if (same) e[v] += ev;
+                }
             }
             const int snext = __shfl_down(sh, 1, 64);
             const bool tail = lane == 63 || snext != sh;
-            if (tail && sh >= 1 && sh <= nek) acc[w][sh - 1] += e;
+            if (tail && sh >= 1 && sh <= nek) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) mine[v * nek + sh - 1] += e[v];
+            }
         }
     }
     __syncthreads();
-    for (int s = threadIdx.x; s < nek; s += SPEC_T) {
-        double v = acc[0][s];
-#pragma unroll
-        for (int q = 1; q < SPEC_W; ++q) v += acc[q][s];
+    for (int s = threadIdx.x; s < NV * nek; s += blockDim.x) {
+        double v = acc[s];
+        for (int q = 1; q < nw; ++q) v += acc[(size_t)q * NV * nek + s];
         part[(size_t)s * SPEC_BLOCKS + blockIdx.x] = v;
     }
 }
 
-// ek[s] = the SPEC_BLOCKS partials of shell s + 1, added lane-strided then by a fixed
-// wavefront tree: one wavefront per shell
-__global__ void __launch_bounds__(SPEC_T) k_shell_final(const double* __restrict__ part, int nek, double* __restrict__ ek)
+// ek[s] = the SPEC_BLOCKS partials of sum s (ns of them), added lane-strided then by a fixed
+// wavefront tree: one wavefront per sum
+__global__ void __launch_bounds__(SPEC_FT) k_shell_final(const double* __restrict__ part, int ns, double* __restrict__ ek)
 {
     const int lane = threadIdx.x & 63;
-    const int s = blockIdx.x * SPEC_W + (threadIdx.x >> 6);
-    if (s >= nek) return;
+    const int s = blockIdx.x * (SPEC_FT / 64) + (threadIdx.x >> 6);
+    if (s >= ns) return;
     double v = 0.0;
     for (int b = lane; b < SPEC_BLOCKS; b += 64) v += part[(size_t)s * SPEC_BLOCKS + b];
 #pragma unroll
@@ -94,21 +120,44 @@ __global__ void __launch_bounds__(SPEC_T) k_shell_final(const double* __restrict
     if (lane == 0) ek[s] = v;
 }
 
+template <typename T, int NV>
+static int launch_shells_t(const FlowBuffers& fb, const void* const F[3], int N, int nek, double rnu, double* part,
+                           double* sums_dev, hipStream_t s)
+{
+    // wavefronts per work-group: 16 where their tables fit in 64 KB (more work-groups of a
+    // second launch may share the CU), else 8, 4: nek <= 510 and three sums fit with 4
+    int nw = 16;
+    while (nw > 4 && (size_t)nw * NV * nek * sizeof(double) > 64 * 1024) nw /= 2;
+    hipLaunchKernelGGL((k_shell_partials<T, NV>), dim3(SPEC_BLOCKS), dim3(64 * nw), (size_t)nw * NV * nek * sizeof(double),
+                       s, (const void*)fb.U[0], (const void*)fb.U[1], (const void*)fb.U[2], F[0], F[1], F[2], N, nek, rnu,
+                       part);
+    DDNS_HIP(hipGetLastError());
+    constexpr int PER = SPEC_FT / 64;
+    hipLaunchKernelGGL(k_shell_final, dim3((unsigned)((NV * nek + PER - 1) / PER)), dim3(SPEC_FT), 0, s,
+                       (const double*)part, NV * nek, sums_dev);
+    DDNS_HIP(hipGetLastError());
+    return 0;
+}
+
 // Both kernels on stream s: part holds SPEC_BLOCKS * nek doubles, ek_dev nek doubles.
 static int launch_shells(const FlowBuffers& fb, int N, int nek, int precision, double* part, double* ek_dev,
                          hipStream_t s)
 {
+    const void* const F[3] = {nullptr, nullptr, nullptr};
+    return precision == DDNS_FP64 ? launch_shells_t<double, 1>(fb, F, N, nek, 0.0, part, ek_dev, s)
+                                  : launch_shells_t<float, 1>(fb, F, N, nek, 0.0, part, ek_dev, s);
+}
+
+// The E, D and (with F) T shell sums of the diagnostics: part holds 3 SPEC_BLOCKS nek
+// doubles, sums_dev 3 nek doubles (E, then D, then T, which is left alone without F).
+int flow_shell_sums(const FlowBuffers& fb, const void* const F[3], int N, int nek, double rnu, int precision, double* part,
+                    double* sums_dev, hipStream_t s)
+{
     if (precision == DDNS_FP64)
-        hipLaunchKernelGGL(k_shell_partials<double>, dim3(SPEC_BLOCKS), dim3(SPEC_T), 0, s, (const void*)fb.U[0],
-                           (const void*)fb.U[1], (const void*)fb.U[2], N, nek, part);
-    else
-        hipLaunchKernelGGL(k_shell_partials<float>, dim3(SPEC_BLOCKS), dim3(SPEC_T), 0, s, (const void*)fb.U[0],
-                           (const void*)fb.U[1], (const void*)fb.U[2], N, nek, part);
-    DDNS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_shell_final, dim3((unsigned)((nek + SPEC_W - 1) / SPEC_W)), dim3(SPEC_T), 0, s,
-                       (const double*)part, nek, ek_dev);
-    DDNS_HIP(hipGetLastError());
-    return 0;
+        return F[0] ? launch_shells_t<double, 3>(fb, F, N, nek, rnu, part, sums_dev, s)
+                    : launch_shells_t<double, 2>(fb, F, N, nek, rnu, part, sums_dev, s);
+    return F[0] ? launch_shells_t<float, 3>(fb, F, N, nek, rnu, part, sums_dev, s)
+                : launch_shells_t<float, 2>(fb, F, N, nek, rnu, part, sums_dev, s);
 }
 
 // ddns_get_spectrum: partial rows and the result in the handle's buffer fb.spec_part
