@@ -415,6 +415,7 @@ static void destroy_impl(ddns_handle* h)
         for (int q = 0; q < 8; ++q) if (h->fb.dg[q]) (void)hipFree(h->fb.dg[q]);
         if (h->fb.dg_part) (void)hipFree(h->fb.dg_part);
         if (h->fb.spec_part) (void)hipFree(h->fb.spec_part);
+        if (h->fb.stage) (void)hipFree(h->fb.stage);
     }
     part_free(h->pb);
     for (int i = 0; i < 16; ++i) if (h->ev[i]) (void)hipEventDestroy(h->ev[i]);
@@ -586,29 +587,10 @@ extern "C" int ddns_set_droplets(ddns_handle* h, int n, const double* yp, const 
 {
     if (!h || n < 0) return DDNS_ERR_ARG;
     if (n > h->pb.cap) return fail(h, DDNS_ERR_CAPACITY, "more droplets than capacity");
-    const int cap = h->pb.cap;
-    std::vector<double> pos(3 * (size_t)cap, 0.0), vel(3 * (size_t)cap, 0.0), rad(cap, 0.0), gid(cap, 0.0);
-    std::vector<double> fv(9 * (size_t)cap, 0.0), fd(12 * (size_t)cap, 0.0), pv(3 * (size_t)cap, 0.0);
-    for (int i = 0; i < n; ++i) {
-        for (int c = 0; c < 3; ++c) {
-            pos[(size_t)c * cap + i] = yp[8 * (size_t)i + c];
-            vel[(size_t)c * cap + i] = yp[8 * (size_t)i + 3 + c];
-            if (pertvel) pv[3 * (size_t)i + c] = pertvel[3 * (size_t)i + c];
-            for (int t = 0; t < 3; ++t) if (fvp) fv[(size_t)(3 * t + c) * cap + i] = fvp[9 * (size_t)i + 3 * t + c];
-            for (int t = 0; t < 4; ++t) if (fdp) fd[(size_t)(3 * t + c) * cap + i] = fdp[12 * (size_t)i + 3 * t + c];
-        }
-        rad[i] = yp[8 * (size_t)i + 6];
-        gid[i] = yp[8 * (size_t)i + 7];
-    }
-    DDNS_HIP(hipMemcpy(h->pb.pos, pos.data(), pos.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.vel, vel.data(), vel.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.rad, rad.data(), rad.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.gid, gid.data(), gid.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.fvp, fv.data(), fv.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.fdp, fd.data(), fd.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.pert, pv.data(), pv.size() * 8, hipMemcpyHostToDevice));
-    h->pb.hv_v = h->pb.hv_d = 0;                 // the levels were written in order
-    h->pb.v0_stale = h->pb.d0_stale = false;
+    if (n > 0 && !yp) return DDNS_ERR_ARG;
+    DDNS_HIP(hipStreamSynchronize(h->dstream));
+    const int st = part_upload(h->pb, n, yp, fvp, fdp, pertvel, h->stream);
+    if (st) return keep(h, st);
     invalidate_cells(h->pb);
     h->n = n;
     h->pc.n = n;
@@ -619,36 +601,9 @@ extern "C" int ddns_get_droplets(ddns_handle* h, int* n, double* yp, double* fvp
                                  double* vp, double* dmove)
 {
     if (!h) return DDNS_ERR_ARG;
-    DDNS_HIP(hipStreamSynchronize(h->stream));
-    const int cap = h->pb.cap, m = h->n;
-    if (n) *n = m;
-    std::vector<double> pos(3 * (size_t)cap), vel(3 * (size_t)cap), rad(cap), gid(cap);
-    std::vector<double> fv(9 * (size_t)cap), fd(12 * (size_t)cap), pv(3 * (size_t)cap), vv(3 * (size_t)cap), dm(3 * (size_t)cap);
-    DDNS_HIP(hipMemcpy(pos.data(), h->pb.pos, pos.size() * 8, hipMemcpyDeviceToHost));
-    DDNS_HIP(hipMemcpy(vel.data(), h->pb.vel, vel.size() * 8, hipMemcpyDeviceToHost));
-    DDNS_HIP(hipMemcpy(rad.data(), h->pb.rad, rad.size() * 8, hipMemcpyDeviceToHost));
-    DDNS_HIP(hipMemcpy(gid.data(), h->pb.gid, gid.size() * 8, hipMemcpyDeviceToHost));
-    DDNS_HIP(hipMemcpy(fv.data(), h->pb.fvp, fv.size() * 8, hipMemcpyDeviceToHost));
-    DDNS_HIP(hipMemcpy(fd.data(), h->pb.fdp, fd.size() * 8, hipMemcpyDeviceToHost));
-    DDNS_HIP(hipMemcpy(pv.data(), h->pb.pert, pv.size() * 8, hipMemcpyDeviceToHost));
-    DDNS_HIP(hipMemcpy(vv.data(), h->pb.vp, vv.size() * 8, hipMemcpyDeviceToHost));
-    DDNS_HIP(hipMemcpy(dm.data(), h->pb.dmove, dm.size() * 8, hipMemcpyDeviceToHost));
-    // history level t in its ring column (level 0 reads as level 1 after a shift)
-    int vc[3], dc[4];
-    for (int t = 0; t < 3; ++t) vc[t] = h->pb.vcol(t == 0 && h->pb.v0_stale ? 1 : t);
-    for (int t = 0; t < 4; ++t) dc[t] = h->pb.dcol(t == 0 && h->pb.d0_stale ? 1 : t);
-    for (int i = 0; i < m; ++i) {
-        for (int c = 0; c < 3; ++c) {
-            if (yp) { yp[8 * (size_t)i + c] = pos[(size_t)c * cap + i]; yp[8 * (size_t)i + 3 + c] = vel[(size_t)c * cap + i]; }
-            if (pertvel) pertvel[3 * (size_t)i + c] = pv[3 * (size_t)i + c];
-            if (vp) vp[3 * (size_t)i + c] = vv[(size_t)c * cap + i];
-            if (dmove) dmove[3 * (size_t)i + c] = dm[(size_t)c * cap + i];
-            for (int t = 0; t < 3; ++t) if (fvp) fvp[9 * (size_t)i + 3 * t + c] = fv[(size_t)(vc[t] + c) * cap + i];
-            for (int t = 0; t < 4; ++t) if (fdp) fdp[12 * (size_t)i + 3 * t + c] = fd[(size_t)(dc[t] + c) * cap + i];
-        }
-        if (yp) { yp[8 * (size_t)i + 6] = rad[i]; yp[8 * (size_t)i + 7] = gid[i]; }
-    }
-    return DDNS_OK;
+    if (n) *n = h->n;
+    DDNS_HIP(hipStreamSynchronize(h->dstream));
+    return keep(h, part_download(h->pb, h->n, yp, fvp, fdp, pertvel, vp, dmove, h->stream));
 }
 
 extern "C" int ddns_overlap_fix(ddns_handle* h)
@@ -1187,19 +1142,13 @@ extern "C" int ddns_collision_detect(ddns_handle* h, int n, const double* yp, co
     if (n > h->pb.cap) return fail(h, DDNS_ERR_CAPACITY, "more droplets than capacity");
     int st = ddns_set_droplets(h, n, yp, nullptr, nullptr, nullptr);
     if (st) return st;
-    const int cap = h->pb.cap;
-    std::vector<double> a(3 * (size_t)cap, 0.0), b(3 * (size_t)cap, 0.0), c(3 * (size_t)cap, 0.0), d(3 * (size_t)cap, 0.0);
-    for (int i = 0; i < n; ++i)
-        for (int k = 0; k < 3; ++k) {
-            a[(size_t)k * cap + i] = dmove[3 * (size_t)i + k];
-            b[(size_t)k * cap + i] = fvp0[3 * (size_t)i + k];
-            c[(size_t)k * cap + i] = vnew[3 * (size_t)i + k];
-            d[(size_t)k * cap + i] = vp[3 * (size_t)i + k];
-        }
-    DDNS_HIP(hipMemcpy(h->pb.dmove, a.data(), a.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.fvp, b.data(), b.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.vel, c.data(), c.size() * 8, hipMemcpyHostToDevice));
-    DDNS_HIP(hipMemcpy(h->pb.vp, d.data(), d.size() * 8, hipMemcpyHostToDevice));
+    const double* const src[4] = {dmove, fvp0, vnew, vp};
+    double* const dst[4] = {h->pb.dmove, h->pb.fvp, h->pb.vel, h->pb.vp};
+    for (int k = 0; k < 4; ++k) {
+        st = part_upload3(h->pb, n, dst[k], src[k], h->stream);
+        if (st) return keep(h, st);
+    }
+    DDNS_HIP(hipStreamSynchronize(h->stream));       // the caller's arrays are read
     h->pc.n = n;
     st = part_build_cells(h->pb, h->pc, cell_width(h), h->stream);
     if (st) return keep(h, st);

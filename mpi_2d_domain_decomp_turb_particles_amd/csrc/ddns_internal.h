@@ -206,6 +206,8 @@ struct FlowBuffers {
     void* dg[8] = {};                           // diagnostics scratch, 8 fields, allocated on first use
     double* dg_part = nullptr;                  // diagnostics reduction partials
     double* spec_part = nullptr;                // E(k): SPEC_BLOCKS partial rows of SPEC_NEK_MAX shells, then the result
+    void* stage = nullptr;                      // state transfers: a part of a field in the reference's layout
+    size_t stage_bytes = 0;                     // (allocated on first use, kept with the handle)
     int ky_tc = 0;                              // y-stage tile width chosen by flow_tune (0: the default)
     float ky_ms[3] = {0, 0, 0};                 // the tuner's time per y stage pair of each candidate (0: not valid)
     int kz_nt = 0;                              // threads of the fused z stage chosen by flow_tune (0: the default)
@@ -252,9 +254,9 @@ enum FlowPart { FLOW_INV = 0, FLOW_FWD = 1, FLOW_FWD_Y = 2, FLOW_FWD_Z = 3 };
 int flow_step(const FlowBuffers& fb, const FlowConst& fc, int precision, int part, hipStream_t s,
               hipEvent_t* ev /* FLOW_EVENTS events or nullptr */, bool capturing = false);
 constexpr int FLOW_EVENTS = 9;
-int flow_upload_state(const FlowBuffers& fb, int N, int precision, const double* const src[6], hipStream_t s);
-int flow_download_state(const FlowBuffers& fb, int N, int precision, double* const dst[6], hipStream_t s);
-int flow_download_phys(const FlowBuffers& fb, int N, int precision, double* ux, double* uy, double* uz, hipStream_t s);
+int flow_upload_state(FlowBuffers& fb, int N, int precision, const double* const src[6], hipStream_t s);
+int flow_download_state(FlowBuffers& fb, int N, int precision, double* const dst[6], hipStream_t s);
+int flow_download_phys(FlowBuffers& fb, int N, int precision, double* ux, double* uy, double* uz, hipStream_t s);
 // POSTPROC / TRANSPOSTPROC sums of the current u-hat.  want: 1 = CFL maximum and the
 // velocity-derivative moments, 2 = divergence / vorticity sums.  ek, dk, tk (nek each,
 // any may be null): energy, dissipation and transfer spectra.  mom: [0] max |u|+|v|+|w|,
@@ -272,8 +274,8 @@ int flow_shell_sums(const FlowBuffers& fb, const void* const F[3], int N, int ne
 // address is resolved once per device by spectrum_scratch_init
 int spectrum_scratch_init();
 int flow_spectrum_device(const FlowBuffers& fb, int N, int nek, int precision, int dev, double* ek_dev, hipStream_t s);
-int fft_r2c_host(const FlowBuffers& fb, int N, int precision, double* v, hipStream_t s);
-int fft_c2r_host(const FlowBuffers& fb, int N, int precision, double* v, hipStream_t s);
+int fft_r2c_host(FlowBuffers& fb, int N, int precision, double* v, hipStream_t s);
+int fft_c2r_host(FlowBuffers& fb, int N, int precision, double* v, hipStream_t s);
 int flow_profile(const FlowBuffers& fb, const FlowConst& fc, int precision, int k, double* ms, int nk, hipStream_t s);
 // times the candidate y-stage tile widths and fused z-stage work-group sizes on fb's
 // buffers (before any state is loaded) and keeps the fastest in fb.ky_tc, fb.kz_nt
@@ -370,6 +372,7 @@ struct PartBuffers {
     int* draw_off = nullptr;    // cap + 1
     int* rng_state = nullptr;   // ranff2 state: idum, iy, idum2, iv[32]
     double* red = nullptr;      // generic reduction scratch
+    double* stage = nullptr;    // 12*cap: one droplet array in the reference's layout, made on the first transfer
 };
 
 struct PartConst {
@@ -389,6 +392,14 @@ struct PartConst {
 };
 
 int part_alloc(PartBuffers& pb, int cap, int nset, int G);
+// Droplet state to and from the reference's arrays on the host (any pointer may be null; an
+// upload clears what it has no array for).  s must be ordered after the droplet block.
+int part_upload(PartBuffers& pb, int n, const double* yp, const double* fvp, const double* fdp, const double* pertvel,
+                hipStream_t s);
+int part_download(PartBuffers& pb, int n, double* yp, double* fvp, double* fdp, double* pertvel, double* vp, double* dmove,
+                  hipStream_t s);
+// one 3-vector per droplet (dst(3,n), component-major slots) from the host's a(3, n)
+int part_upload3(PartBuffers& pb, int n, double* dst, const double* a, hipStream_t s);
 // Waits for event e by polling it: after a blocking wait the host thread ran again tens
 // of microseconds after the GPU had finished, and the stream waited that long for the
 // launches that follow.

@@ -1222,6 +1222,7 @@ void flow_free(FlowBuffers& fb)
     for (int q = 0; q < 8; ++q) if (fb.dg[q]) (void)hipFree(fb.dg[q]);
     if (fb.dg_part) (void)hipFree(fb.dg_part);
     if (fb.spec_part) (void)hipFree(fb.spec_part);
+    if (fb.stage) (void)hipFree(fb.stage);
     fb = FlowBuffers{};
 }
 
@@ -1459,40 +1460,107 @@ int flow_step(const FlowBuffers& fb, const FlowConst& fc, int precision, int par
 }
 
 // ---------------------------------------------------------------- host conversion
-template <typename T>
-static int upload_spectral(void* dev, int N, const double* v, hipStream_t s)
+// State transfers.  The reference's layouts are formed on the device, in a staging buffer of
+// at most STAGE_BYTES (or one ky plane), and copied straight to or from the caller's arrays:
+// converting in host loops, through arrays that were allocated and faulted in on each call,
+// took 246 ms for the six fields of a 256^3 FP32 state against 45 ms for the copies.
+constexpr size_t STAGE_BYTES = 128u << 20;
+
+static int stage_buffer(FlowBuffers& fb, size_t bytes, double** out)
+{
+    if (fb.stage_bytes < bytes) {
+        if (fb.stage) DDNS_HIP(hipFree(fb.stage));
+        fb.stage = nullptr;
+        fb.stage_bytes = 0;
+        DDNS_HIP(hipMalloc(&fb.stage, bytes));
+        fb.stage_bytes = bytes;
+    }
+    *out = (double*)fb.stage;
+    return 0;
+}
+
+// Planes ky0 .. ky0 + gridDim.z of v(N+2, N+2, N) (kz fastest, then kx re/im, then ky) from
+// a field [kz][ky][kx], with the padding rows zero (PACK), or the field from the planes.
+// 32 x 32 tiles through LDS: kx is contiguous on one side, kz on the other.
+template <typename T, bool PACK>
+__global__ void __launch_bounds__(256) k_layout(cpx<T>* __restrict__ f, double* __restrict__ v, int N, int ky0)
 {
     using C = cpx<T>;
+    __shared__ C tile[32][33];
     const int L = N + 2, M = N / 2;
-    std::vector<C> h(field_elems(N));
-    for (int kz = 0; kz < N; ++kz)
-        for (int ky = 0; ky < N; ++ky)
-            for (int kx = 0; kx < M; ++kx) {
-                const size_t o = (size_t)kz + (size_t)L * ((size_t)(2 * kx) + (size_t)L * ky);
-                h[((size_t)kz * N + ky) * M + kx] = mk<C>((T)v[o], (T)v[o + L]);
+    const int kz0 = blockIdx.x * 32, kx0 = blockIdx.y * 32, ky = ky0 + blockIdx.z;
+    const int a = threadIdx.x & 31, b = threadIdx.x >> 5;
+    double* plane = v + (size_t)blockIdx.z * L * L;
+    if constexpr (PACK) {
+#pragma unroll
+        for (int q = 0; q < 32; q += 8) {
+            const int kz = kz0 + b + q, kx = kx0 + a;
+            tile[b + q][a] = kz < N && kx < M ? f[((size_t)kz * N + ky) * M + kx] : mk<C>((T)0, (T)0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 32; q += 8) {
+            const int kz = kz0 + a, kx = kx0 + b + q;
+            if (kz < L && kx <= M) {
+                const C c = tile[a][b + q];
+                plane[(size_t)(2 * kx) * L + kz] = (double)c.x;
+                plane[(size_t)(2 * kx + 1) * L + kz] = (double)c.y;
             }
-    DDNS_HIP(hipMemcpyAsync(dev, h.data(), h.size() * sizeof(C), hipMemcpyHostToDevice, s));
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 32; q += 8) {
+            const int kz = kz0 + a, kx = kx0 + b + q;
+            if (kz < N && kx < M)
+                tile[a][b + q] = mk<C>((T)plane[(size_t)(2 * kx) * L + kz], (T)plane[(size_t)(2 * kx + 1) * L + kz]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 32; q += 8) {
+            const int kz = kz0 + b + q, kx = kx0 + a;
+            if (kz < N && kx < M) f[((size_t)kz * N + ky) * M + kx] = tile[b + q][a];
+        }
+    }
+}
+
+// n planes of L x L doubles per chunk of the staging buffer
+static int stage_planes(int N) { return (int)std::max<size_t>(1, std::min<size_t>(N, STAGE_BYTES / sizeof(double) / (N + 2) / (N + 2))); }
+
+template <typename T>
+static int upload_spectral(FlowBuffers& fb, void* dev, int N, const double* v, hipStream_t s)
+{
+    const size_t plane = (size_t)(N + 2) * (N + 2);
+    const int np = stage_planes(N);
+    double* st = nullptr;
+    int rc = stage_buffer(fb, np * plane * sizeof(double), &st);
+    if (rc) return rc;
+    for (int ky = 0; ky < N; ky += np) {
+        const int m = std::min(np, N - ky);
+        DDNS_HIP(hipMemcpyAsync(st, v + (size_t)ky * plane, m * plane * sizeof(double), hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL((k_layout<T, false>), dim3((N + 31) / 32, (N / 2 + 31) / 32, m), dim3(256), 0, s, (cpx<T>*)dev, st,
+                           N, ky);
+        DDNS_HIP(hipGetLastError());
+    }
     DDNS_HIP(hipStreamSynchronize(s));
     return 0;
 }
 
 template <typename T>
-static int download_spectral(const void* dev, int N, double* v, hipStream_t s)
+static int download_spectral(FlowBuffers& fb, const void* dev, int N, double* v, hipStream_t s)
 {
-    using C = cpx<T>;
-    const int L = N + 2, M = N / 2;
-    std::vector<C> h(field_elems(N));
-    DDNS_HIP(hipMemcpyAsync(h.data(), dev, h.size() * sizeof(C), hipMemcpyDeviceToHost, s));
+    const size_t plane = (size_t)(N + 2) * (N + 2);
+    const int np = stage_planes(N);
+    double* st = nullptr;
+    int rc = stage_buffer(fb, np * plane * sizeof(double), &st);
+    if (rc) return rc;
+    for (int ky = 0; ky < N; ky += np) {
+        const int m = std::min(np, N - ky);
+        hipLaunchKernelGGL((k_layout<T, true>), dim3((N + 2 + 31) / 32, (N / 2 + 1 + 31) / 32, m), dim3(256), 0, s,
+                           (cpx<T>*)dev, st, N, ky);
+        DDNS_HIP(hipGetLastError());
+        DDNS_HIP(hipMemcpyAsync(v + (size_t)ky * plane, st, m * plane * sizeof(double), hipMemcpyDeviceToHost, s));
+    }
     DDNS_HIP(hipStreamSynchronize(s));
-    std::memset(v, 0, sizeof(double) * (size_t)L * L * N);
-    for (int kz = 0; kz < N; ++kz)
-        for (int ky = 0; ky < N; ++ky)
-            for (int kx = 0; kx < M; ++kx) {
-                const size_t o = (size_t)kz + (size_t)L * ((size_t)(2 * kx) + (size_t)L * ky);
-                const C c = h[((size_t)kz * N + ky) * M + kx];
-                v[o] = (double)c.x;
-                v[o + L] = (double)c.y;
-            }
     return 0;
 }
 
@@ -1505,7 +1573,7 @@ static int mark_dense(const FlowBuffers& fb)
     return 0;
 }
 
-int flow_upload_state(const FlowBuffers& fb, int N, int precision, const double* const src[6], hipStream_t s)
+int flow_upload_state(FlowBuffers& fb, int N, int precision, const double* const src[6], hipStream_t s)
 {
     DDNS_HIP(hipStreamSynchronize(s));
     const int sm = mark_dense(fb);
@@ -1513,43 +1581,59 @@ int flow_upload_state(const FlowBuffers& fb, int N, int precision, const double*
     for (int f = 0; f < 6; ++f) {
         if (!src[f]) continue;
         void* dev = f < 3 ? fb.U[f] : fb.O[f - 3];
-        const int st = precision == DDNS_FP64 ? upload_spectral<double>(dev, N, src[f], s)
-                                              : upload_spectral<float>(dev, N, src[f], s);
+        const int st = precision == DDNS_FP64 ? upload_spectral<double>(fb, dev, N, src[f], s)
+                                              : upload_spectral<float>(fb, dev, N, src[f], s);
         if (st) return st;
     }
     return 0;
 }
 
-int flow_download_state(const FlowBuffers& fb, int N, int precision, double* const dst[6], hipStream_t s)
+int flow_download_state(FlowBuffers& fb, int N, int precision, double* const dst[6], hipStream_t s)
 {
     for (int f = 0; f < 6; ++f) {
         if (!dst[f]) continue;
         const void* dev = f < 3 ? fb.U[f] : fb.O[f - 3];
-        const int st = precision == DDNS_FP64 ? download_spectral<double>(dev, N, dst[f], s)
-                                              : download_spectral<float>(dev, N, dst[f], s);
+        const int st = precision == DDNS_FP64 ? download_spectral<double>(fb, dev, N, dst[f], s)
+                                              : download_spectral<float>(fb, dev, N, dst[f], s);
         if (st) return st;
     }
     return 0;
 }
 
+// components c = 0, 1, 2 of nodes [i0, i0 + n) of the physical velocity, one after the other
 template <typename T>
-static int download_phys_t(const void* dev, int N, double* ux, double* uy, double* uz, hipStream_t s)
+__global__ void __launch_bounds__(256) k_phys_planes(const T* __restrict__ u, double* __restrict__ out, size_t i0, size_t n)
+{
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) out[c * n + i] = (double)u[3 * (i0 + i) + c];
+}
+
+template <typename T>
+static int download_phys_t(FlowBuffers& fb, int N, double* ux, double* uy, double* uz, hipStream_t s)
 {
     const size_t n3 = (size_t)N * N * N;
-    std::vector<T> h(n3 * 3);
-    DDNS_HIP(hipMemcpyAsync(h.data(), dev, h.size() * sizeof(T), hipMemcpyDeviceToHost, s));
-    DDNS_HIP(hipStreamSynchronize(s));
+    const size_t chunk = std::min(n3, STAGE_BYTES / (3 * sizeof(double)) / 256 * 256);
+    double* st = nullptr;
+    const int rc = stage_buffer(fb, 3 * chunk * sizeof(double), &st);
+    if (rc) return rc;
     double* d[3] = {ux, uy, uz};
-    for (int c = 0; c < 3; ++c)
-        if (d[c])
-            for (size_t i = 0; i < n3; ++i) d[c][i] = (double)h[3 * i + c];
+    for (size_t i = 0; i < n3; i += chunk) {
+        const size_t m = std::min(chunk, n3 - i);
+        hipLaunchKernelGGL((k_phys_planes<T>), dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, (const T*)fb.uphys, st, i, m);
+        DDNS_HIP(hipGetLastError());
+        for (int c = 0; c < 3; ++c)
+            if (d[c]) DDNS_HIP(hipMemcpyAsync(d[c] + i, st + c * m, m * sizeof(double), hipMemcpyDeviceToHost, s));
+    }
+    DDNS_HIP(hipStreamSynchronize(s));
     return 0;
 }
 
-int flow_download_phys(const FlowBuffers& fb, int N, int precision, double* ux, double* uy, double* uz, hipStream_t s)
+int flow_download_phys(FlowBuffers& fb, int N, int precision, double* ux, double* uy, double* uz, hipStream_t s)
 {
-    return precision == DDNS_FP64 ? download_phys_t<double>(fb.uphys, N, ux, uy, uz, s)
-                                  : download_phys_t<float>(fb.uphys, N, ux, uy, uz, s);
+    return precision == DDNS_FP64 ? download_phys_t<double>(fb, N, ux, uy, uz, s)
+                                  : download_phys_t<float>(fb, N, ux, uy, uz, s);
 }
 
 // ---------------------------------------------------------------- initial field
@@ -1625,7 +1709,7 @@ int flow_init(FlowBuffers& fb, int N, int nek, int precision, int kind, int seed
 
 // ---------------------------------------------------------------- stand-alone FFTs
 template <typename T, int N>
-static int r2c_impl(const FlowBuffers& fb, double* v, hipStream_t s)
+static int r2c_impl(FlowBuffers& fb, double* v, hipStream_t s)
 {
     using C = cpx<T>;
     const int L = N + 2;
@@ -1647,15 +1731,15 @@ static int r2c_impl(const FlowBuffers& fb, double* v, hipStream_t s)
     fc.N = N;
     st = launch_z<T, N>(KZ_PLAIN_FWD, fb, fc, s, fb.B[0], fb.A[1], 1.0 / N);
     if (st) return st;
-    return download_spectral<T>(fb.A[1], N, v, s);
+    return download_spectral<T>(fb, fb.A[1], N, v, s);
 }
 
 template <typename T, int N>
-static int c2r_impl(const FlowBuffers& fb, double* v, hipStream_t s)
+static int c2r_impl(FlowBuffers& fb, double* v, hipStream_t s)
 {
     const int L = N + 2;
     const size_t n3 = (size_t)N * N * N;
-    int st = upload_spectral<T>(fb.A[1], N, v, s);
+    int st = upload_spectral<T>(fb, fb.A[1], N, v, s);
     if (st) return st;
     FlowConst fc{};
     fc.N = N;
@@ -1678,7 +1762,7 @@ static int c2r_impl(const FlowBuffers& fb, double* v, hipStream_t s)
     return 0;
 }
 
-int fft_r2c_host(const FlowBuffers& fb, int N, int precision, double* v, hipStream_t s)
+int fft_r2c_host(FlowBuffers& fb, int N, int precision, double* v, hipStream_t s)
 {
     int st = 0;
     if (precision == DDNS_FP64) { DDNS_DISPATCH_N(N, st = (r2c_impl<double, NN>(fb, v, s))) }
@@ -1686,7 +1770,7 @@ int fft_r2c_host(const FlowBuffers& fb, int N, int precision, double* v, hipStre
     return st;
 }
 
-int fft_c2r_host(const FlowBuffers& fb, int N, int precision, double* v, hipStream_t s)
+int fft_c2r_host(FlowBuffers& fb, int N, int precision, double* v, hipStream_t s)
 {
     int st = 0;
     if (precision == DDNS_FP64) { DDNS_DISPATCH_N(N, st = (c2r_impl<double, NN>(fb, v, s))) }

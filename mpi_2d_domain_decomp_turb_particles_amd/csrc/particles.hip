@@ -217,7 +217,7 @@ void part_free(PartBuffers& pb)
                   pb.cell_count, pb.cell_start, pb.cell_of, pb.cell_rank, pb.sorted, pb.pk, pb.scan_tmp,
                   pb.nei_cnt, pb.nei_idx, pb.nei_m, pb.gm_Q, pb.gm_v, pb.gm_x0, pb.gm_b, pb.gm_w,
                   pb.gm_red, pb.gm_small, pb.mult, pb.cand, pb.hit, pb.flags, pb.tested, pb.nirbin, pb.bins, pb.counts,
-                  pb.pairs, pb.contact, pb.draws, pb.draw_off, pb.rng_state, pb.red};
+                  pb.pairs, pb.contact, pb.draws, pb.draw_off, pb.rng_state, pb.red, pb.stage};
     for (void* p : ps) if (p) (void)hipFree(p);
     void* sp[] = {pb.spare.cell_count, pb.spare.cell_start, pb.spare.cell_of, pb.spare.sorted, pb.spare.pk};
     for (void* p : sp) if (p) (void)hipFree(p);
@@ -226,6 +226,129 @@ void part_free(PartBuffers& pb)
     if (pb.found_host) (void)hipHostFree(pb.found_host);
     if (pb.counts_host) (void)hipHostFree(pb.counts_host);
     pb = PartBuffers{};
+}
+
+// ------------------------------------------------------------------ state transfers
+// The reference's arrays hold one droplet's K values side by side, the device one value of
+// all droplets (column c of slot i at col[c] + i).  The change of layout runs on the device, in
+// a staging buffer that is copied straight to or from the caller's array: nine columns-to-host
+// copies, nine host arrays allocated per call and a host loop took 97 ms for 1M droplets.
+struct Columns {
+    double* col[12];        // null: zeros
+};
+
+template <bool PACK>
+__global__ void __launch_bounds__(PT) k_columns(Columns a, int K, double* __restrict__ rec, int n)
+{
+    const long long e = (long long)blockIdx.x * PT + threadIdx.x;
+    if (e >= (long long)n * K) return;
+    const int i = (int)(e / K), c = (int)(e - (long long)i * K);
+    if (PACK) rec[e] = a.col[c][i];
+    else a.col[c][i] = rec[e];
+}
+
+static int stage_rows(PartBuffers& pb)
+{
+    if (!pb.stage) DDNS_HIP(hipMalloc(&pb.stage, 12 * (size_t)pb.cap * sizeof(double)));
+    return 0;
+}
+
+// host(K, n) <- columns
+static int columns_out(PartBuffers& pb, const Columns& a, int K, double* host, int n, hipStream_t s)
+{
+    if (!host || n <= 0) return 0;
+    hipLaunchKernelGGL(k_columns<true>, dim3(nblk((long long)n * K)), dim3(PT), 0, s, a, K, pb.stage, n);
+    DDNS_HIP(hipGetLastError());
+    DDNS_HIP(hipMemcpyAsync(host, pb.stage, (size_t)n * K * sizeof(double), hipMemcpyDeviceToHost, s));
+    return 0;
+}
+
+// columns <- host(K, n)
+static int columns_in(PartBuffers& pb, const Columns& a, int K, const double* host, int n, hipStream_t s)
+{
+    if (!host || n <= 0) return 0;
+    DDNS_HIP(hipMemcpyAsync(pb.stage, host, (size_t)n * K * sizeof(double), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_columns<false>, dim3(nblk((long long)n * K)), dim3(PT), 0, s, a, K, pb.stage, n);
+    DDNS_HIP(hipGetLastError());
+    return 0;
+}
+
+static Columns yp_columns(const PartBuffers& pb)
+{
+    Columns a{};
+    for (int c = 0; c < 3; ++c) {
+        a.col[c] = pb.pos + (size_t)c * pb.cap;
+        a.col[3 + c] = pb.vel + (size_t)c * pb.cap;
+    }
+    a.col[6] = pb.rad;
+    a.col[7] = pb.gid;
+    return a;
+}
+
+static Columns vec_columns(double* v, int cap)
+{
+    Columns a{};
+    for (int c = 0; c < 3; ++c) a.col[c] = v + (size_t)c * cap;
+    return a;
+}
+
+int part_upload3(PartBuffers& pb, int n, double* dst, const double* host, hipStream_t s)
+{
+    const int st = stage_rows(pb);
+    return st ? st : columns_in(pb, vec_columns(dst, pb.cap), 3, host, n, s);
+}
+
+int part_upload(PartBuffers& pb, int n, const double* yp, const double* fvp, const double* fdp, const double* pertvel,
+                hipStream_t s)
+{
+    int st = stage_rows(pb);
+    if (st) return st;
+    const size_t c = (size_t)pb.cap;
+    // slots without a droplet, and arrays that are not given, read as zeros
+    double* const base[7] = {pb.pos, pb.vel, pb.rad, pb.gid, pb.fvp, pb.fdp, pb.pert};
+    const size_t cols[7] = {3, 3, 1, 1, 9, 12, 3};
+    const bool full = (size_t)n == c;
+    const bool given[7] = {full, full, full, full, full && fvp, full && fdp, full && pertvel};
+    for (int k = 0; k < 7; ++k)
+        if (!given[k]) DDNS_HIP(hipMemsetAsync(base[k], 0, cols[k] * c * sizeof(double), s));
+    st = columns_in(pb, yp_columns(pb), 8, yp, n, s);
+    if (st) return st;
+    pb.hv_v = pb.hv_d = 0;                          // the levels are written in order
+    pb.v0_stale = pb.d0_stale = false;
+    Columns a{}, b{};
+    for (int q = 0; q < 9; ++q) a.col[q] = pb.fvp + q * c;
+    for (int q = 0; q < 12; ++q) b.col[q] = pb.fdp + q * c;
+    st = columns_in(pb, a, 9, fvp, n, s);
+    if (st) return st;
+    st = columns_in(pb, b, 12, fdp, n, s);
+    if (st) return st;
+    // pertvel is droplet-major on the device too
+    if (pertvel && n > 0) DDNS_HIP(hipMemcpyAsync(pb.pert, pertvel, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
+    DDNS_HIP(hipStreamSynchronize(s));
+    return 0;
+}
+
+int part_download(PartBuffers& pb, int n, double* yp, double* fvp, double* fdp, double* pertvel, double* vp, double* dmove,
+                  hipStream_t s)
+{
+    int st = stage_rows(pb);
+    if (st) return st;
+    const size_t c = (size_t)pb.cap;
+    // history level t in its ring column (level 0 reads as level 1 after a shift)
+    Columns a{}, b{};
+    for (int t = 0; t < 3; ++t)
+        for (int q = 0; q < 3; ++q) a.col[3 * t + q] = pb.fvp + (size_t)(pb.vcol(t == 0 && pb.v0_stale ? 1 : t) + q) * c;
+    for (int t = 0; t < 4; ++t)
+        for (int q = 0; q < 3; ++q) b.col[3 * t + q] = pb.fdp + (size_t)(pb.dcol(t == 0 && pb.d0_stale ? 1 : t) + q) * c;
+    st = columns_out(pb, yp_columns(pb), 8, yp, n, s);
+    if (!st) st = columns_out(pb, a, 9, fvp, n, s);
+    if (!st) st = columns_out(pb, b, 12, fdp, n, s);
+    if (!st) st = columns_out(pb, vec_columns(pb.vp, pb.cap), 3, vp, n, s);
+    if (!st) st = columns_out(pb, vec_columns(pb.dmove, pb.cap), 3, dmove, n, s);
+    if (st) return st;
+    if (pertvel && n > 0) DDNS_HIP(hipMemcpyAsync(pertvel, pb.pert, 3 * (size_t)n * sizeof(double), hipMemcpyDeviceToHost, s));
+    DDNS_HIP(hipStreamSynchronize(s));
+    return 0;
 }
 
 // ------------------------------------------------------------------ interpolation
