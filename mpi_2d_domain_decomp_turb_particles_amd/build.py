@@ -4,7 +4,9 @@ Usage: python -m mpi_2d_domain_decomp_turb_particles_amd.build [--no-fortran] [-
 
 Every HIP source is compiled for gfx950 only, with packed-FP32 instruction
 selection disabled.  collide.hip is compiled with -ffp-contract=off so that the
-double-precision pair tests are the same IEEE operations as the reference's.
+double-precision pair tests are the same IEEE operations as the reference's, and flow.hip
+with -ffp-contract=on: products and sums are fused inside an expression of the source only,
+so every tile shape of a kernel does the same arithmetic.
 """
 from __future__ import annotations
 
@@ -32,7 +34,7 @@ COMMON = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable", "-Wno-unused-but-set-variable",
 ]
 SOURCES = {
-    "flow.hip": [],
+    "flow.hip": ["-ffp-contract=on"],
     "particles.hip": [],
     "hdi.hip": [],
     "collide.hip": ["-ffp-contract=off"],

@@ -184,6 +184,12 @@ template <typename C> __host__ __device__ __forceinline__ C csub(C a, C b) { ret
 template <typename C> __host__ __device__ __forceinline__ C cmul(C a, C b) { return mk<C>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
 template <typename C> __host__ __device__ __forceinline__ C cconj(C a) { return mk<C>(a.x, -a.y); }
 template <typename C> __host__ __device__ __forceinline__ C cscale(C a, decltype(C{}.x) s) { return mk<C>(a.x * s, a.y * s); }
+// fused forms, one rounding per product: c + a b, c - a b, c + a s (s real)
+__host__ __device__ __forceinline__ float ffma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__host__ __device__ __forceinline__ double ffma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template <typename C> __host__ __device__ __forceinline__ C cmadd(C c, C a, C b) { return mk<C>(ffma(a.x, b.x, ffma(-a.y, b.y, c.x)), ffma(a.x, b.y, ffma(a.y, b.x, c.y))); }
+template <typename C> __host__ __device__ __forceinline__ C cmsub(C c, C a, C b) { return mk<C>(ffma(-a.x, b.x, ffma(a.y, b.y, c.x)), ffma(-a.x, b.y, ffma(-a.y, b.x, c.y))); }
+template <typename C> __host__ __device__ __forceinline__ C csmadd(C c, C a, decltype(C{}.x) s) { return mk<C>(ffma(a.x, s, c.x), ffma(a.y, s, c.y)); }
 // multiply by -i (forward) or +i (inverse)
 template <typename C, bool INV> __host__ __device__ __forceinline__ C cmul_mi(C a) { return INV ? mk<C>(-a.y, a.x) : mk<C>(a.y, -a.x); }
 

@@ -121,17 +121,17 @@ __device__ __forceinline__ void dft8(C* v)
     C o[4] = {v[1], v[3], v[5], v[7]};
     dft4<C, INV>(e);
     dft4<C, INV>(o);
-    // o[k] *= exp(-+ 2 pi i k / 8)
-    o[1] = INV ? mk<C>(h * (o[1].x - o[1].y), h * (o[1].x + o[1].y))
-               : mk<C>(h * (o[1].x + o[1].y), h * (o[1].y - o[1].x));
+    // v[k] = e[k] +- exp(-+ 2 pi i k / 8) o[k], the products fused into the sums
+    const C w1 = mk<C>(h, INV ? h : -h), w3 = mk<C>(-h, INV ? h : -h);
     o[2] = cmul_mi<C, INV>(o[2]);
-    o[3] = INV ? mk<C>(-h * (o[3].x + o[3].y), h * (o[3].x - o[3].y))
-               : mk<C>(h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        v[k] = cadd(e[k], o[k]);
-        v[k + 4] = csub(e[k], o[k]);
-    }
+    v[0] = cadd(e[0], o[0]);
+    v[4] = csub(e[0], o[0]);
+    v[1] = cmadd(e[1], o[1], w1);
+    v[5] = cmsub(e[1], o[1], w1);
+    v[2] = cadd(e[2], o[2]);
+    v[6] = csub(e[2], o[2]);
+    v[3] = cmadd(e[3], o[3], w3);
+    v[7] = cmsub(e[3], o[3], w3);
 }
 
 template <typename C, bool INV>
@@ -146,20 +146,19 @@ __device__ __forceinline__ void dft16(C* v)
     const T c1 = (T)0.92387953251128675613, s1 = (T)0.38268343236508977173;
     const T h = (T)0.70710678118654752440;
     const T sg = INV ? (T)1 : (T)-1;
-    // w_k = cos(2 pi k/16) + sg i sin(2 pi k/16)
-    const C w1 = mk<C>(c1, sg * s1), w2 = mk<C>(h, sg * h), w3 = mk<C>(s1, sg * c1);
-    const C w5 = mk<C>(-s1, sg * c1), w6 = mk<C>(-h, sg * h), w7 = mk<C>(-c1, sg * s1);
-    o[1] = cmul(o[1], w1);
-    o[2] = cmul(o[2], w2);
-    o[3] = cmul(o[3], w3);
+    // w_k = cos(2 pi k/16) + sg i sin(2 pi k/16); v[k] = e[k] +- w_k o[k], fused
+    const C w[8] = {mk<C>((T)1, (T)0), mk<C>(c1, sg * s1), mk<C>(h, sg * h), mk<C>(s1, sg * c1),
+                    mk<C>((T)0, sg), mk<C>(-s1, sg * c1), mk<C>(-h, sg * h), mk<C>(-c1, sg * s1)};
     o[4] = cmul_mi<C, INV>(o[4]);
-    o[5] = cmul(o[5], w5);
-    o[6] = cmul(o[6], w6);
-    o[7] = cmul(o[7], w7);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-        v[k] = cadd(e[k], o[k]);
-        v[k + 8] = csub(e[k], o[k]);
+        if (k == 0 || k == 4) {
+            v[k] = cadd(e[k], o[k]);
+            v[k + 8] = csub(e[k], o[k]);
+        } else {
+            v[k] = cmadd(e[k], o[k], w[k]);
+            v[k + 8] = cmsub(e[k], o[k], w[k]);
+        }
     }
 }
 
@@ -245,6 +244,82 @@ __device__ __forceinline__ void fft_tile(cpx<T>* __restrict__ lds, const cpx<T>*
     fft_pass<T, N, P::R0, 1, INV, TC, LDR, NT, K, TS>(lds, tw, tid);
     if constexpr (P::P > 1) fft_pass<T, N, P::R1, P::R0, INV, TC, LDR, NT, K, TS>(lds, tw, tid);
     if constexpr (P::P > 2) fft_pass<T, N, P::R2, P::R0 * P::R1, INV, TC, LDR, NT, K, TS>(lds, tw, tid);
+}
+
+// ---------------------------------------------------------------- columns in registers
+// The y and z stages hold a column in the registers of N / E threads: thread t of column c
+// has points t + (N / E) q, q < E, in v[q].  A Stockham pass of radix R takes points
+// j + r N / R, which are v[i + r E / R] of the thread with j = t + (N / E) i, so every pass
+// works on registers, the last pass leaves its output (points j + r N / R again) where the
+// input was, and LDS serves only the exchange between two passes: one write and one read
+// per value and exchange, where tiles kept in LDS cost a write and a read per pass and two
+// more for the transfers to HBM.  Rows go straight between HBM and the registers (TC
+// adjacent kx of one row: 128 bytes at the default widths).
+template <int N, int E> struct RPlan;
+template <> struct RPlan<32, 4>    { static constexpr int R0 = 4,  R1 = 4,  R2 = 2, R3 = 1; };
+template <> struct RPlan<64, 4>    { static constexpr int R0 = 4,  R1 = 4,  R2 = 4, R3 = 1; };
+template <> struct RPlan<32, 8>    { static constexpr int R0 = 8,  R1 = 4,  R2 = 1, R3 = 1; };
+template <> struct RPlan<64, 8>    { static constexpr int R0 = 8,  R1 = 8,  R2 = 1, R3 = 1; };
+template <> struct RPlan<128, 8>   { static constexpr int R0 = 8,  R1 = 4,  R2 = 4, R3 = 1; };
+template <> struct RPlan<128, 16>  { static constexpr int R0 = 16, R1 = 8,  R2 = 1, R3 = 1; };
+template <> struct RPlan<256, 8>   { static constexpr int R0 = 8,  R1 = 8,  R2 = 4, R3 = 1; };
+template <> struct RPlan<256, 16>  { static constexpr int R0 = 16, R1 = 16, R2 = 1, R3 = 1; };
+template <> struct RPlan<512, 8>   { static constexpr int R0 = 8,  R1 = 8,  R2 = 8, R3 = 1; };
+template <> struct RPlan<512, 16>  { static constexpr int R0 = 8,  R1 = 8,  R2 = 8, R3 = 1; };
+template <> struct RPlan<1024, 8>  { static constexpr int R0 = 8,  R1 = 8,  R2 = 4, R3 = 4; };
+template <> struct RPlan<1024, 16> { static constexpr int R0 = 16, R1 = 16, R2 = 4, R3 = 1; };
+
+// One pass of radix R and stride NS on a thread's E points; LAST leaves the result in v, the
+// other passes exchange it through lds (N rows of LDR, this column at lds[n * LDR]).  All
+// threads of the work-group call it; lds may be reused when it returns.
+template <typename T, int N, int E, int R, int NS, bool INV, int LDR, bool LAST>
+__device__ __forceinline__ void col_pass(cpx<T> (&v)[E], cpx<T>* __restrict__ lds, const cpx<T>* __restrict__ tw, int t)
+{
+    using C = cpx<T>;
+    constexpr int TT = N / E, B = E / R;
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+        const int j = t + TT * i;
+        const int m = j % NS;
+        C a[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) a[r] = v[i + r * B];
+        if constexpr (NS > 1) {
+            constexpr int STEP = N / (NS * R);
+#pragma unroll
+            for (int r = 1; r < R; ++r) {
+                C w = tw[(m * r * STEP) & (N - 1)];
+                if (INV) w.y = -w.y;
+                a[r] = cmul(a[r], w);
+            }
+        }
+        dft<R, C, INV>(a);
+        if constexpr (LAST) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[i + r * B] = a[r];
+        } else {
+            const int base = (j / NS) * NS * R + m;
+#pragma unroll
+            for (int r = 0; r < R; ++r) lds[(base + r * NS) * LDR] = a[r];
+        }
+    }
+    if constexpr (!LAST) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < E; ++q) v[q] = lds[(t + TT * q) * LDR];
+        __syncthreads();
+    }
+}
+
+// The transform of one column: in and out as v[q] = point t + (N / E) q.
+template <typename T, int N, int E, bool INV, int LDR>
+__device__ __forceinline__ void col_fft(cpx<T> (&v)[E], cpx<T>* __restrict__ lds, const cpx<T>* __restrict__ tw, int t)
+{
+    using P = RPlan<N, E>;
+    col_pass<T, N, E, P::R0, 1, INV, LDR, P::R1 == 1>(v, lds, tw, t);
+    if constexpr (P::R1 > 1) col_pass<T, N, E, P::R1, P::R0, INV, LDR, P::R2 == 1>(v, lds, tw, t);
+    if constexpr (P::R2 > 1) col_pass<T, N, E, P::R2, P::R0 * P::R1, INV, LDR, P::R3 == 1>(v, lds, tw, t);
+    if constexpr (P::R3 > 1) col_pass<T, N, E, P::R3, P::R0 * P::R1 * P::R2, INV, LDR, true>(v, lds, tw, t);
 }
 
 // the twiddle table exp(-2 pi i m / N), m < N, copied to LDS by the whole work-group

@@ -29,46 +29,41 @@ constexpr int NT = 256;
 
 enum { KZ_FULL = 0, KZ_CURL_INV = 1, KZ_PLAIN_FWD = 2, KZ_PLAIN_INV = 3 };
 
-// tile widths (kx columns per work-group) for the y and z stages
-template <typename T, int N> constexpr int ky_tc() { return (sizeof(T) == 4) ? (N >= 1024 ? 8 : 16) : (N >= 1024 ? 4 : 8); }
+// Points per thread of a column (fft_engine.h).  The plain transforms hold one value set per
+// column (16 points: at most one exchange up to N = 256).  The z stage holds three and a
+// fourth in flight: 16 points in single precision from N = 256 on (8 points cost a
+// second exchange: 300 against 258 us at 256^3), 8 where that leaves a second wavefront per
+// SIMD its registers (27 against 32 us at 128^3; all of double: 16 would need 512), 4 on the
+// grids that do not fill the chip (12 against 15 us at 32^3).
+template <typename T, int N> constexpr int col_e() { return N == 32 || N == 64 || (sizeof(T) == 8 && N == 512) ? 8 : 16; }
+template <typename T, int N> constexpr int kz_e() { return N <= 64 ? 4 : (sizeof(T) == 4 && N >= 256 ? 16 : 8); }
+// wavefronts per SIMD that the z stage's registers leave room for (double at 256^3: one, its
+// values spill at two: 484 against 542 us)
+template <typename T, int N> constexpr int kz_waves() { return sizeof(T) == 8 && N >= 256 ? 1 : 2; }
+template <int TC> constexpr int ldr_of() { return (TC >= 8) ? TC + 1 : TC; }
+
+// tile width (kx columns per work-group) of the y stage: rows of 128 bytes below N = 1024,
+// 64 there (two work-groups per CU); at least a wavefront of threads (N = 32)
+template <typename T, int N> constexpr int ky_tc() { return (sizeof(T) == 4) ? (N >= 1024 ? 8 : 16) : (N >= 1024 ? 4 : (N == 32 ? 16 : 8)); }
 // The y stage runs at one of three tile widths, chosen per grid and precision by timing
-// (flow_tune): half, once and twice the default, where the tile splits evenly over the
-// work-group's 16-byte accesses and fits LDS with the twiddles.  The width changes only
-// which columns a work-group transforms together, never the arithmetic of a column, so
-// every choice gives the same bits.
+// (flow_tune): half, once and twice the default, where a work-group has 64 to 1024 threads
+// and its exchange buffer fits LDS with the twiddles.  The width changes only which columns a
+// work-group transforms together, never the arithmetic of a column, so every choice gives
+// the same bits.
 template <typename T, int N, int TC> constexpr bool ky_fits()
 {
-    constexpr int VW = sizeof(T) == 4 ? 2 : 1;
-    return TC >= VW && TC <= N / 2 && TC % VW == 0 && (N * (TC / VW)) % 256 == 0 &&
-           (N * (TC >= 8 ? TC + 1 : TC) + N) * (int)sizeof(cpx<T>) <= 160 * 1024;
+    constexpr int nt = TC * (N / col_e<T, N>());
+    return TC >= 1 && TC <= N / 2 && nt >= 64 && nt <= 1024 && (N * ldr_of<TC>() + N) * (int)sizeof(cpx<T>) <= 160 * 1024;
 }
 template <typename T, int N> constexpr int ky_cand(int k) { return k == 0 ? ky_tc<T, N>() / 2 : (k == 1 ? ky_tc<T, N>() : 2 * ky_tc<T, N>()); }
-// z-stage tile widths for N <= 256, overridable at build time for tuning sweeps
-#ifndef DDNS_KZ_TC_F32
-#define DDNS_KZ_TC_F32 16
-#endif
-#ifndef DDNS_KZ_TC_F64
-#define DDNS_KZ_TC_F64 8
-#endif
-// persistent z stage, overridable at build time for tuning sweeps: the update
-// operands of DDNS_KZ_EPTP_BYTES / sizeof(complex) elements per thread are loaded
-// before the forward transforms, the rest of the update loop is unrolled
-// DDNS_KZ_UNROLL times, and with DDNS_KZ_NEXTB the next tile's input is loaded during
-// this tile's inverse transforms (single precision only)
-#ifndef DDNS_KZ_UNROLL
-#define DDNS_KZ_UNROLL 4
-#endif
-#ifndef DDNS_KZ_NEXTB
-#define DDNS_KZ_NEXTB 1
-#endif
-#ifndef DDNS_KZ_EPTP_BYTES
-#define DDNS_KZ_EPTP_BYTES 32
-#endif
+// tile width of the fused z stage: rows of 128 bytes, half that where the threads that would
+// take could have no more than 128 registers each (N = 1024); at least a wavefront (N = 32)
 template <typename T, int N> constexpr int kz_tc()
 {
-    if constexpr (sizeof(T) == 4) return N < 256 ? 16 : (N == 256 ? DDNS_KZ_TC_F32 : (N == 512 ? 8 : 4));
-    else return N <= 256 ? DDNS_KZ_TC_F64 : (N == 512 ? 4 : 2);
+    if constexpr (sizeof(T) == 4) return N >= 1024 ? 8 : 16;
+    else return N >= 1024 ? 4 : (N == 32 ? 16 : 8);
 }
+template <typename T, int N, int TC> constexpr int kz_threads() { return TC * (N / kz_e<T, N>()); }
 
 // Work-groups are dispatched to the 8 XCDs round-robin by linear id, and each XCD has
 // its own L2.  When a tile row is narrower than a 128-byte line, the P tiles that share
@@ -84,49 +79,24 @@ __device__ __forceinline__ int xcd_tile(int L)
         return g * (8 * P) + (r % 8) * P + r / 8;
     }
 }
-template <int TC> constexpr int ldr_of() { return (TC >= 8) ? TC + 1 : TC; }
-// One-tile (plain) z transforms for N >= 512 take rows of 128 bytes: one padded tile of
-// N rows fits in LDS at that width even where the four tiles of the fused stage do not
-template <typename T, int N> constexpr int kz_tc_plain()
-{
-    if constexpr (N < 512) return kz_tc<T, N>();
-    else return sizeof(T) == 4 ? 16 : 8;
-}
-// Where the fused z stage's tiles hold rows shorter than 128 bytes (N >= 512) the stage
-// runs as separate kernels instead: three plain forward transforms, the pointwise update,
-// the curl, six plain inverse transforms.  They move 39 fields instead of 21 but at the
-// rate of full rows (36 with the curl formed in the update): faster by 9 % (FP32) and
-// 15 % (FP64) at 512^3, 38 % at 1024^3.
-// DDNS_Z_SPLIT=1 or 0 in the environment selects one path at any N, to check them
-// against each other.
-// threads of a z work-group: the single-tile transforms of N = 1024 take 512, so that a CU,
-// which holds one such tile in LDS, has twice the loads in flight (8 % faster there; at
-// N = 512 two 256-thread tiles fit in LDS and do better)
-template <typename T, int N, int MODE> constexpr int kz_threads()
-{
-    return ((MODE == KZ_PLAIN_FWD || MODE == KZ_PLAIN_INV) && N >= 1024) ? 512 : NT;
-}
-template <typename T, int N> constexpr bool kz_split_default() { return kz_tc<T, N>() * (int)sizeof(cpx<T>) < 128; }
-template <typename T, int N> constexpr int kz_ldr()
-{
-    constexpr int TC = kz_tc<T, N>();
-    return ((4 * N * (TC + 1) + N) * (int)sizeof(cpx<T>) <= 160 * 1024) ? TC + 1 : TC;   // 4 tiles + twiddles
-}
+// tile width of the plain z transforms (the diagnostics, the split z stage): rows of 128 bytes
+template <typename T, int N> constexpr int kz_tc_plain() { return sizeof(T) == 4 || N == 32 ? 16 : 8; }
+template <typename T, int N> constexpr int kz_plain_threads() { return kz_tc_plain<T, N>() * (N / col_e<T, N>()); }
+// The z stage can also run as separate kernels: three plain forward transforms, the pointwise
+// update with the curl, six plain inverse transforms (36 fields moved instead of 21).
+// DDNS_Z_SPLIT=1 in the environment selects them, to check the two against each other.
 
 __device__ __forceinline__ int wave_index(int i, int N) { return i <= N / 2 ? i : i - N; }
 
-// Is mode (kx, ky, kz) inside the dealiasing sphere (turb.f90:405, 648-650)?  update_mode's
-// own shell index, in its precision: outside it the update sets both the new u-hat and
-// the stored nonlinear term to zero (the mean mode counts as inside: its u-hat is zero
-// but its nonlinear term is kept).
-template <typename T>
+// Is mode (kx, ky, kz) inside the dealiasing sphere, shell int(|k| + 1/2) <= nek (turb.f90:405,
+// 648-650)?  |k| < nek + 1/2 is k^2 <= nek (nek + 1) in whole numbers; the reference's rounded
+// square root gives the same (the two k^2 next to the limit are 1e-4 of a shell away from
+// it at N = 1024).  Outside it the update sets both the new u-hat and the stored nonlinear term
+// to zero (the mean mode counts as inside: its u-hat is zero but its nonlinear term is kept).
 __device__ __forceinline__ bool mode_in_sphere(int kx, int ky, int kz, int N, int nek)
 {
     const int kyw = wave_index(ky, N), kzw = wave_index(kz, N);
-    const T fx = (T)kx, fy = (T)kyw, fz = (T)kzw;
-    T k2 = fx * fx + fy * fy + fz * fz;
-    if (kx == 0 && kyw == 0 && kzw == 0) k2 = (T)1.e-5;
-    return (int)(sqrt(k2) + (T)0.5) <= nek;
+    return kx * kx + kyw * kyw + kzw * kzw <= nek * (nek + 1);
 }
 
 // Batched realisations: realisation r of a field starts r * rstride complex values after
@@ -168,6 +138,8 @@ struct KyArgs {
     double scale;
     int nf, R;         // fields per realisation, realisations: grid z runs over nf * R
     size_t rstride;
+    const double* low; // the step's stages (null: every row is read and written)
+    int nek;
 };
 
 struct KxArgs {
@@ -194,17 +166,19 @@ __device__ __forceinline__ void update_mode(int kx, int ky, int kz, int N, int n
     using C = cpx<T>;
     const int kyw = wave_index(ky, N), kzw = wave_index(kz, N);
     const T fx = (T)kx, fy = (T)kyw, fz = (T)kzw;
-    T k2 = fx * fx + fy * fy + fz * fz;
-    const bool zero_mode = (kx == 0 && kyw == 0 && kzw == 0);
-    if (zero_mode) k2 = (T)1.e-5;                                   // flowlib.f90:36-38
-    const int ik2 = (int)(sqrt(k2) + (T)0.5);                       // turb.f90:405
-    const bool keep = ik2 <= nek && !zero_mode;
+    // the shells of turb.f90:405 in whole numbers (mode_in_sphere): shell 1 holds k^2 = 1, 2,
+    // shell 2 k^2 = 3 .. 6
+    const int ki2 = kx * kx + kyw * kyw + kzw * kzw;
+    const bool zero_mode = ki2 == 0;
+    const T k2 = zero_mode ? (T)1.e-5 : (T)ki2;                     // flowlib.f90:36-38
+    const bool inside = ki2 <= nek * (nek + 1);
+    const bool keep = inside && !zero_mode;
     const T dt_h = (T)0.5 * dt, dtr = (T)1.5 * dt;                   // turb.f90:483-484
     const T ac = rnu * dt_h * k2;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        nd[c] = (ik2 <= nek) ? n[c] : mk<C>((T)0, (T)0);             // dealiasing, 648-650
-        v[c] = csub(cadd(cscale(u[c], (T)1 - ac), cscale(nd[c], dtr)), cscale(o[c], dt_h));
+        nd[c] = inside ? n[c] : mk<C>((T)0, (T)0);             // dealiasing, 648-650
+        v[c] = csmadd(csmadd(cscale(u[c], (T)1 - ac), nd[c], dtr), o[c], -dt_h);
     }
     if (forcing == 2 && kx < 3) {                                    // supforSTH add, flowlib.f90:529-559
         const int js = ky <= 2 ? ky : (ky >= N - 2 ? ky - (N - 5) : -1);
@@ -220,13 +194,13 @@ __device__ __forceinline__ void update_mode(int kx, int ky, int kz, int N, int n
         }
     }
     // projection, 669-672
-    const C t = cscale(cadd(cadd(cscale(v[0], fx), cscale(v[1], fy)), cscale(v[2], fz)), (T)1 / k2);
-    v[0] = csub(v[0], cscale(t, fx));
-    v[1] = csub(v[1], cscale(t, fy));
-    v[2] = csub(v[2], cscale(t, fz));
+    const C t = cscale(csmadd(csmadd(cscale(v[0], fx), v[1], fy), v[2], fz), (T)1 / k2);
+    v[0] = csmadd(v[0], t, -fx);
+    v[1] = csmadd(v[1], t, -fy);
+    v[2] = csmadd(v[2], t, -fz);
     const T den = (T)1 + ac;                                         // 674-676
     T f = (T)1 / den;
-    if (forcing == 1 && (ik2 == 1 || ik2 == 2)) f = f * (T)low[ik2 - 1];   // supforDET
+    if (forcing == 1 && ki2 >= 1 && ki2 <= 6) f = f * (T)low[ki2 <= 2 ? 0 : 1];   // supforDET
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         v[c] = keep ? cscale(v[c], f) : mk<C>((T)0, (T)0);
@@ -234,65 +208,30 @@ __device__ __forceinline__ void update_mode(int kx, int ky, int kz, int N, int n
 }
 
 // ------------------------------------------------------------------ z stage
-// One tile per work-group: curl and inverse z transforms of u-hat (KZ_CURL_INV, the
-// first step) or a plain forward / inverse z transform of one field.
-template <typename T, int N, int MODE>
-__global__ void __launch_bounds__((kz_threads<T, N, MODE>())) k_z(KzArgs a)
+// A plain forward / inverse z transform of one field.
+template <typename T, int N, bool INV>
+__global__ void __launch_bounds__((kz_plain_threads<T, N>())) k_z(KzArgs a)
 {
-    constexpr int NTK = kz_threads<T, N, MODE>();
     using C = cpx<T>;
-    constexpr int M = N / 2;
-    constexpr bool PLAIN = MODE == KZ_PLAIN_FWD || MODE == KZ_PLAIN_INV;
-    constexpr int TC = PLAIN ? kz_tc_plain<T, N>() : kz_tc<T, N>();
-    constexpr int LDR = PLAIN ? ldr_of<TC>() : kz_ldr<T, N>();
-    constexpr int NTILE = MODE == KZ_CURL_INV ? 4 : 1;
-    __shared__ C lds[NTILE][N * LDR];
+    constexpr int M = N / 2, E = col_e<T, N>(), TT = N / E;
+    constexpr int TC = kz_tc_plain<T, N>(), LDR = ldr_of<TC>(), NTK = kz_plain_threads<T, N>();
+    __shared__ C lds[N * LDR];
     __shared__ C tws[N];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, c = tid % TC, t = tid / TC;
     constexpr int NBX = M / TC;
-    constexpr int P = (TC * (int)sizeof(C) >= 128) ? 1 : 128 / (TC * (int)sizeof(C));
-    const int tile = xcd_tile<(NBX % P == 0) ? P : 1>(blockIdx.x);
-    const int kx0 = (tile % NBX) * TC;
-    const int ky = tile / NBX;
+    const int kx0 = (blockIdx.x % NBX) * TC, ky = blockIdx.x / NBX;
     stage_twiddles<C, N, NTK>(tws, (const C*)a.tw, tid);
-    const C* tw = tws;
-    const size_t rowstride = (size_t)N * M;
-    const size_t base = (size_t)blockIdx.y * a.rstride + (size_t)ky * M + kx0;
-
-    if constexpr (MODE == KZ_PLAIN_FWD || MODE == KZ_PLAIN_INV) {
-        const C* src = (const C*)a.B[0];
-        C* dst = (C*)a.U[0];
-        tile_load<C, N, TC, LDR, NTK>(lds[0], src + base, rowstride, tid);
-        __syncthreads();
-        fft_tile<T, N, MODE == KZ_PLAIN_INV, TC, LDR, NTK>(lds[0], tw, tid);
-        tile_store<C, N, TC, LDR, NTK>(dst + base, lds[0], rowstride, tid, (T)a.scale);
-        return;
-    } else {
+    const size_t rowstride = (size_t)N * M, base = (size_t)ky * M + kx0 + c;
+    const C* src = (const C*)a.B[0] + base;
+    C* dst = (C*)a.U[0] + base;
+    C v[E];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) tile_load<C, N, TC, LDR, NTK>(lds[q], (const C*)a.U[q] + base, rowstride, tid);
-        __syncthreads();
-        // vorticity w = i k x u (turb.f90:506-517), one component at a time in tile 3
-#pragma unroll 1
-        for (int q = 0; q < 3; ++q) {
-            for (int e = tid; e < TC * N; e += NTK) {
-                const int n = e / TC, c = e % TC;
-                const T fx = (T)(kx0 + c), fy = (T)wave_index(ky, N), fz = (T)wave_index(n, N);
-                const C ux = lds[0][n * LDR + c], uy = lds[1][n * LDR + c], uz = lds[2][n * LDR + c];
-                C w;
-                if (q == 0) w = csub(cscale(uz, fy), cscale(uy, fz));
-                else if (q == 1) w = csub(cscale(ux, fz), cscale(uz, fx));
-                else w = csub(cscale(uy, fx), cscale(ux, fy));
-                lds[3][n * LDR + c] = mk<C>(-w.y, w.x);
-            }
-            __syncthreads();
-            fft_tile<T, N, true, TC, LDR, NTK>(lds[3], tw, tid);
-            tile_store<C, N, TC, LDR, NTK>((C*)a.A[3 + q] + base, lds[3], rowstride, tid);
-            __syncthreads();
-        }
-        fft_tile<T, N, true, TC, LDR, NTK, 3, N * LDR>(lds[0], tw, tid);
+    for (int q = 0; q < E; ++q) v[q] = src[(t + TT * q) * rowstride];
+    __syncthreads();
+    col_fft<T, N, E, INV, LDR>(v, lds + c, tws, t);
+    const T sc = (T)a.scale;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) tile_store<C, N, TC, LDR, NTK>((C*)a.A[q] + base, lds[q], rowstride, tid);
-    }
+    for (int q = 0; q < E; ++q) dst[(t + TT * q) * rowstride] = cscale(v[q], sc);
 }
 
 // The split z stage's pointwise parts.  k_z_update: the update of k_z_full (dealias,
@@ -320,7 +259,7 @@ __global__ void __launch_bounds__(256) k_z_update(KzArgs a)
     if (t >= (size_t)N * N * M) return;
     const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
     // beyond the dealiasing sphere the state is zero once a step has written it
-    const bool in = a.low[LOW_ZOUT] == 0.0 || mode_in_sphere<T>(kx, ky, kz, N, a.nek);
+    const bool in = a.low[LOW_ZOUT] == 0.0 || mode_in_sphere(kx, ky, kz, N, a.nek);
     C nn[3], u3[3], o3[3], vv[3], nd[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -351,215 +290,204 @@ __global__ void __launch_bounds__(256) k_z_curl(KzArgs a)
     curl_to<T>(a, t, kx, ky, kz, N, u);
 }
 
-// The full z stage as a persistent kernel: one work-group per CU walks the tiles
-// tile = blockIdx.x, blockIdx.x + gridDim.x, ...  The LDS tiles allow only one
-// work-group per CU, so instead of a second work-group hiding HBM latency, a tile's
-// update operands (U-hat, O-hat) are loaded into registers before its forward
-// transforms, and the next tile's input B is loaded into registers during this
-// tile's curl and inverse transforms.  The curl and the inverse transforms are those
-// of k_z<KZ_CURL_INV>.
-#ifndef DDNS_KZ_NT
-#define DDNS_KZ_NT 256
-#endif
-// threads of the persistent z-stage work-group: DDNS_KZ_NT where the tile splits
-// evenly over them (16-byte moves, one update element per thread and pass), else NT
-template <typename T, int N> constexpr int kz_nt()
+// The whole z stage of a column tile in registers.  FULL: forward z transforms of N-hat, the
+// update, the curl of the new u-hat, inverse z transforms of u-hat and w-hat.  Otherwise (a
+// new state) the curl and the inverse transforms of the stored u-hat alone.
+//   - A thread holds points kz = t + (N / E) q of its column for all three components: the
+//     forward transforms end with the modes where the update and the curl need them and the
+//     inverse ones start, so the stage has no pointwise pass over LDS and only the exchange
+//     buffer of one field in it (36 KB at 256^3 FP32, four tiles took 141 KB).
+//   - It is bound by HBM: at 256^3 FP32 it moves 9C x 0.78 + 12C x 0.51 (0.87 GB).
+//   - Beyond the dealiasing sphere nothing is moved: a column with kx^2 + ky^2 beyond it
+//     (21 % of them) is neither read from B nor written to A (the y stages leave it out too),
+//     a tile of such columns ends at once, and the state's modes beyond the sphere are only
+//     written while they may still be nonzero (LOW_ZOUT).
+// The tile width (and with it the work-group's size) is timed at set-up; it changes no
+// column's arithmetic.
+template <typename T, int N, int TC> constexpr bool kz_fits()
 {
-    constexpr int tot = N * kz_tc<T, N>() * (int)sizeof(cpx<T>) / 16;
-    return (tot % DDNS_KZ_NT == 0 && (N * kz_tc<T, N>()) % DDNS_KZ_NT == 0) ? DDNS_KZ_NT : NT;
+    constexpr int nt = kz_threads<T, N, TC>();
+    return TC <= N / 2 && nt >= 64 && nt <= 512 && (N * ldr_of<TC>() + N) * (int)sizeof(cpx<T>) <= 160 * 1024;
 }
+template <typename T, int N> constexpr int kz_cand(int k) { return kz_tc<T, N>() << k; }
 
-// The persistent z stage runs with kz_nt threads or twice as many, chosen per grid and
-// precision by timing (flow_tune), where the tile splits evenly over the threads.  More
-// threads keep more of a CU's loads in flight (a CU holds one work-group: its four
-// tiles fill LDS) but leave each thread half the registers; the elements a thread
-// updates and the columns it transforms change, their arithmetic does not.  (Four times
-// as many threads leave 128 registers per thread, and the kernel spills heavily there:
-// that size is not built.)
-template <typename T, int N, int NTZ> constexpr bool kz_nt_fits()
-{
-    constexpr int tot = N * kz_tc<T, N>() * (int)sizeof(cpx<T>) / 16;
-    return NTZ <= 512 && tot % NTZ == 0 && (N * kz_tc<T, N>()) % NTZ == 0;
-}
-template <typename T, int N> constexpr int kz_nt_cand(int k) { return kz_nt<T, N>() << k; }
-
-template <typename T, int N, int NTZ>
-__global__ void __launch_bounds__(NTZ) k_z_full(KzArgs a, int ntiles)
+template <typename T, int N, int TC, bool FULL>
+__global__ void __launch_bounds__((kz_threads<T, N, TC>()), (kz_waves<T, N>())) k_z_full(KzArgs a)
 {
     using C = cpx<T>;
-    constexpr int M = N / 2;
-    constexpr int TC = kz_tc<T, N>();
-    constexpr int LDR = kz_ldr<T, N>();
-    constexpr int NBX = M / TC;
-    constexpr int EPT = TC * N / NTZ;          // update elements per thread
-    static_assert((TC * N) % NTZ == 0, "the update must split evenly over the work-group");
-    // register budget: the three-tile transforms already hold 48 complex values per
-    // lane, so only part of the update operands is loaded ahead, and the next tile's
-    // input only in single precision
-    constexpr int EPTP = DDNS_KZ_EPTP_BYTES > 0 ? std::max(1, std::min(EPT, (int)(DDNS_KZ_EPTP_BYTES / sizeof(C)))) : EPT;
-    constexpr bool NEXT_B = DDNS_KZ_NEXTB && sizeof(T) == 4;
-    __shared__ C lds[4][N * LDR];
+    constexpr int M = N / 2, E = kz_e<T, N>(), TT = N / E, NBX = M / TC, TPR = NBX * N;
+    constexpr int LDR = ldr_of<TC>();
+    constexpr int P = (TC * (int)sizeof(C) >= 128) ? 1 : 128 / (TC * (int)sizeof(C));
+    __shared__ C lds[N * LDR];
     __shared__ C tws[N];
-    const int tid = threadIdx.x;
-    stage_twiddles<C, N, NTZ>(tws, (const C*)a.tw, tid);
-    const C* tw = tws;
+    const int tid = threadIdx.x, c = tid % TC, t = tid / TC;
+    // tile = realisation * TPR + local tile (tiles that share a 128-byte line on one XCD)
+    const int tile = xcd_tile<(NBX % P == 0 && TPR % (8 * P) == 0) ? P : 1>(blockIdx.x);
+    const int rr = tile / TPR, lt = tile - rr * TPR;
+    const int kx = (lt % NBX) * TC + c, ky = lt / NBX;
     const size_t rowstride = (size_t)N * M;
-    // ntiles counts the tiles of every realisation: tile = r * TPR + local tile
-    constexpr int TPR = NBX * N;
-    auto tile_base = [&](int tl) {
-        const int r = tl / TPR, lt = tl - r * TPR;
-        return (size_t)r * a.rstride + (size_t)(lt / NBX) * M + (lt % NBX) * TC;
-    };
-    using TR = TileRegs<C, N, TC, NTZ>;
-    TR nb[3];
-    int tile = blockIdx.x;
-    if (tile < ntiles) {
-        const size_t base = tile_base(tile);
+    const size_t base = (size_t)rr * a.rstride + (size_t)ky * M + kx;
+    const double* lowr = a.low + (size_t)rr * LOW_STRIDE;
+    // beyond the dealiasing sphere the state is zero once a step has written it
+    const bool zout = lowr[LOW_ZOUT] != 0.0;
+    C u[3][E];
+    bool colin = true;
+    if constexpr (FULL) {
+        colin = mode_in_sphere(kx, ky, 0, N, a.nek);
+        if (!mode_in_sphere(kx - c, ky, 0, N, a.nek)) {          // the whole tile is beyond the sphere
+            if (!zout) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) tile_fetch<C, N, TC, NTZ>(nb[q], (const C*)a.B[q] + base, rowstride, tid);
+                for (int q = 0; q < E; ++q)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        ((C*)a.U[k])[base + (t + TT * q) * rowstride] = mk<C>((T)0, (T)0);
+                        ((C*)a.O[k])[base + (t + TT * q) * rowstride] = mk<C>((T)0, (T)0);
+                    }
+            }
+            return;
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int q = 0; q < E; ++q)
+                u[k][q] = colin ? ((const C*)a.B[k])[base + (t + TT * q) * rowstride] : mk<C>((T)0, (T)0);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int q = 0; q < E; ++q) u[k][q] = ((const C*)a.U[k])[base + (t + TT * q) * rowstride];
     }
-    for (; tile < ntiles; tile += gridDim.x) {
-        const int rr = tile / TPR, lt = tile - rr * TPR;
-        const int kx0 = (lt % NBX) * TC, ky = lt / NBX;
-        const size_t base = (size_t)rr * a.rstride + (size_t)ky * M + kx0;
-        const double* lowr = a.low + (size_t)rr * LOW_STRIDE;
+    stage_twiddles<C, N, kz_threads<T, N, TC>()>(tws, (const C*)a.tw, tid);
+    __syncthreads();
+    C* col = lds + c;
+    if constexpr (FULL) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) col_fft<T, N, E, false, LDR>(u[k], col, tws, t);
         const int forcing = real_forcing(a.forcing, lowr);
-        // beyond the dealiasing sphere the state is zero once a step has written it
-        const bool zout = lowr[LOW_ZOUT] != 0.0;
-        if (!NEXT_B && tile != (int)blockIdx.x) {
-#pragma unroll
-            for (int q = 0; q < 3; ++q) tile_fetch<C, N, TC, NTZ>(nb[q], (const C*)a.B[q] + base, rowstride, tid);
-        }
-#pragma unroll
-        for (int q = 0; q < 3; ++q) tile_put<C, N, TC, LDR, NTZ>(lds[q], nb[q], tid);
-        // the first update operands, in flight during the forward transforms
-        C uu[EPTP][3], oo[EPTP][3];
-#pragma unroll
-        for (int k = 0; k < EPTP; ++k) {
-            const int e = tid + k * NTZ, n = e / TC, c = e % TC;
-            const size_t g = base + (size_t)n * rowstride + c;
-            const bool ld = !zout || mode_in_sphere<T>(kx0 + c, ky, n, N, a.nek);
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                uu[k][q] = ld ? ((const C*)a.U[q])[g] : mk<C>((T)0, (T)0);
-                oo[k][q] = ld ? ((const C*)a.O[q])[g] : mk<C>((T)0, (T)0);
-            }
-        }
-        __syncthreads();
-        fft_tile<T, N, false, TC, LDR, NTZ, 3, N * LDR>(lds[0], tw, tid);     // the three components together
         const T inv_n = (T)1 / (T)N;
-        auto update = [&](int k, const C* u3, const C* o3) {
-            const int e = tid + k * NTZ, n = e / TC, c = e % TC;
-            const size_t g = base + (size_t)n * rowstride + c;
-            C nn[3], vv[3], nd[3];
 #pragma unroll
-            for (int q = 0; q < 3; ++q) nn[q] = cscale(lds[q][n * LDR + c], inv_n);
-            update_mode<T>(kx0 + c, ky, n, N, a.nek, forcing, (T)a.dt, (T)a.rnu, lowr, nn, u3, o3, vv, nd);
-            const bool wr = !zout || mode_in_sphere<T>(kx0 + c, ky, n, N, a.nek);
+        for (int q = 0; q < E; ++q) {
+            const int n = t + TT * q;
+            const size_t g = base + n * rowstride;
+            if (mode_in_sphere(kx, ky, n, N, a.nek)) {
+                C nn[3], u3[3], o3[3], vv[3], nd[3];
 #pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                if (wr) {
-                    ((C*)a.U[q])[g] = vv[q];
-                    ((C*)a.O[q])[g] = nd[q];
+                for (int k = 0; k < 3; ++k) {
+                    nn[k] = cscale(u[k][q], inv_n);
+                    u3[k] = ((const C*)a.U[k])[g];
+                    o3[k] = ((const C*)a.O[k])[g];
                 }
-                lds[q][n * LDR + c] = vv[q];
+                update_mode<T>(kx, ky, n, N, a.nek, forcing, (T)a.dt, (T)a.rnu, lowr, nn, u3, o3, vv, nd);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    ((C*)a.U[k])[g] = vv[k];
+                    ((C*)a.O[k])[g] = nd[k];
+                    u[k][q] = vv[k];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    u[k][q] = mk<C>((T)0, (T)0);
+                    if (!zout) {
+                        ((C*)a.U[k])[g] = u[k][q];
+                        ((C*)a.O[k])[g] = u[k][q];
+                    }
+                }
             }
-        };
-#pragma unroll
-        for (int k = 0; k < EPTP; ++k) update(k, uu[k], oo[k]);
-#pragma unroll DDNS_KZ_UNROLL
-        for (int k = EPTP; k < EPT; ++k) {
-            const int e = tid + k * NTZ, n = e / TC, c = e % TC;
-            const size_t g = base + (size_t)n * rowstride + c;
-            const bool ld = !zout || mode_in_sphere<T>(kx0 + c, ky, n, N, a.nek);
-            C u3[3], o3[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                u3[q] = ld ? ((const C*)a.U[q])[g] : mk<C>((T)0, (T)0);
-                o3[q] = ld ? ((const C*)a.O[q])[g] : mk<C>((T)0, (T)0);
-            }
-            update(k, u3, o3);
         }
-        // the next tile's input, in flight during the curl and the inverse transforms
-        // (the barrier keeps the compiler from hoisting these loads over the update)
-        asm volatile("" ::: "memory");
-        const int nt = tile + (int)gridDim.x;
-        if (NEXT_B && nt < ntiles) {
-            const size_t nbase = tile_base(nt);
+    }
+    // vorticity w = i k x u (turb.f90:506-517), one component at a time
 #pragma unroll
-            for (int q = 0; q < 3; ++q) tile_fetch<C, N, TC, NTZ>(nb[q], (const C*)a.B[q] + nbase, rowstride, tid);
-        }
-        __syncthreads();
-        // vorticity w = i k x u (turb.f90:506-517), one component at a time in tile 3
-#pragma unroll 1
-        for (int q = 0; q < 3; ++q) {
-            for (int e = tid; e < TC * N; e += NTZ) {
-                const int n = e / TC, c = e % TC;
-                const T fx = (T)(kx0 + c), fy = (T)wave_index(ky, N), fz = (T)wave_index(n, N);
-                const C ux = lds[0][n * LDR + c], uy = lds[1][n * LDR + c], uz = lds[2][n * LDR + c];
-                C w;
-                if (q == 0) w = csub(cscale(uz, fy), cscale(uy, fz));
-                else if (q == 1) w = csub(cscale(ux, fz), cscale(uz, fx));
-                else w = csub(cscale(uy, fx), cscale(ux, fy));
-                lds[3][n * LDR + c] = mk<C>(-w.y, w.x);
-            }
-            __syncthreads();
-            fft_tile<T, N, true, TC, LDR, NTZ>(lds[3], tw, tid);
-            tile_store<C, N, TC, LDR, NTZ>((C*)a.A[3 + q] + base, lds[3], rowstride, tid);
-            __syncthreads();
-        }
-        fft_tile<T, N, true, TC, LDR, NTZ, 3, N * LDR>(lds[0], tw, tid);
+    for (int k = 0; k < 3; ++k) {
+        C w[E];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) tile_store<C, N, TC, LDR, NTZ>((C*)a.A[q] + base, lds[q], rowstride, tid);
-        __syncthreads();   // the stores have read the tiles before the next tile is put
+        for (int q = 0; q < E; ++q) {
+            const T fx = (T)kx, fy = (T)wave_index(ky, N), fz = (T)wave_index(t + TT * q, N);
+            C x;
+            if (k == 0) x = csmadd(cscale(u[2][q], fy), u[1][q], -fz);
+            else if (k == 1) x = csmadd(cscale(u[0][q], fz), u[2][q], -fx);
+            else x = csmadd(cscale(u[1][q], fx), u[0][q], -fy);
+            w[q] = mk<C>(-x.y, x.x);
+        }
+        col_fft<T, N, E, true, LDR>(w, col, tws, t);
+        if (colin) {
+#pragma unroll
+            for (int q = 0; q < E; ++q) ((C*)a.A[3 + k])[base + (t + TT * q) * rowstride] = w[q];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        col_fft<T, N, E, true, LDR>(u[k], col, tws, t);
+        if (colin) {
+#pragma unroll
+            for (int q = 0; q < E; ++q) ((C*)a.A[k])[base + (t + TT * q) * rowstride] = u[k][q];
+        }
     }
 }
 
 // ------------------------------------------------------------------ y stage
+// Columns in registers as in the z stage; bound by HBM.  In a step (a.low given) the rows
+// beyond the circle kx^2 + ky^2 of the dealiasing sphere (21 % of them) are left out: the
+// inverse stage takes them as zero (unless the state was set since the last step, when the
+// z transforms of that state fill them), the forward stage does not store them.
 template <typename T, int N, bool INV, bool SYM, int TC>
-__global__ void __launch_bounds__(NT) k_y(KyArgs a)
+__global__ void __launch_bounds__((TC * (N / col_e<T, N>()))) k_y(KyArgs a)
 {
     using C = cpx<T>;
-    constexpr int M = N / 2;
+    constexpr int M = N / 2, E = col_e<T, N>(), TT = N / E, NTK = TC * TT;
     constexpr int LDR = ldr_of<TC>();
     __shared__ C lds[N * LDR];
     __shared__ C tws[N];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, c = tid % TC, t = tid / TC;
     // tiles whose rows share a 128-byte line (P of them, side by side in kx) go to linear
     // ids L, L+8, ..., i.e. to one XCD, where the second finds the line in L2
     constexpr int P = (TC * (int)sizeof(C) >= 128) ? 1 : 128 / (TC * (int)sizeof(C));
     int kxb = blockIdx.x, z = blockIdx.y, fi = blockIdx.z;
     if constexpr (P > 1) {
         if ((M / TC) % P == 0 && (gridDim.y * gridDim.z) % 8 == 0) {
-            const int t = xcd_tile<P>(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
-            kxb = t % gridDim.x;
-            z = (t / gridDim.x) % gridDim.y;
-            fi = t / (gridDim.x * gridDim.y);
+            const int l = xcd_tile<P>(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+            kxb = l % gridDim.x;
+            z = (l / gridDim.x) % gridDim.y;
+            fi = l / (gridDim.x * gridDim.y);
         }
     }
-    const int kx0 = kxb * TC;
-    stage_twiddles<C, N, NT>(tws, (const C*)a.tw, tid);
+    const int kx = kxb * TC + c;
     const int rr = fi / a.nf;
-    C* f = (C*)a.F[fi - rr * a.nf] + (size_t)rr * a.rstride;
-    const size_t base = (size_t)z * N * M + kx0;
-    tile_load<C, N, TC, LDR, NT>(lds, f + base, M, tid);
-    __syncthreads();
+    C* f = (C*)a.F[fi - rr * a.nf] + (size_t)rr * a.rstride + (size_t)z * N * M + kx;
+    const bool all = !a.low || (INV && a.low[(size_t)rr * LOW_STRIDE + LOW_ZOUT] == 0.0);
+    C v[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const int n = t + TT * q;
+        v[q] = !INV || all || mode_in_sphere(kx, n, 0, N, a.nek) ? f[(size_t)n * M] : mk<C>((T)0, (T)0);
+    }
+    stage_twiddles<C, N, NTK>(tws, (const C*)a.tw, tid);
     if constexpr (SYM) {
         // kx = 0 column: (c(ky) + conj c(-ky)) / 2, the z-transformed form of the
         // kx = 0 plane symmetrisation of flowlib.f90:264-329
-        if (kx0 == 0) {
-            for (int k = tid; k <= N / 2; k += NT) {
-                const int km = (N - k) & (N - 1);
-                const C p = lds[k * LDR], m = lds[km * LDR];
-                const C s = mk<C>((T)0.5 * (p.x + m.x), (T)0.5 * (p.y - m.y));
-                lds[k * LDR] = s;
-                lds[km * LDR] = cconj(s);
+        if (kxb == 0) {
+            if (c == 0) {
+#pragma unroll
+                for (int q = 0; q < E; ++q) lds[t + TT * q] = v[q];
             }
             __syncthreads();
+            if (c == 0) {
+#pragma unroll
+                for (int q = 0; q < E; ++q) {
+                    const C m = lds[(N - (t + TT * q)) & (N - 1)];
+                    v[q] = mk<C>((T)0.5 * (v[q].x + m.x), (T)0.5 * (v[q].y - m.y));
+                }
+            }
         }
     }
-    fft_tile<T, N, INV, TC, LDR, NT>(lds, tws, tid);
-    tile_store<C, N, TC, LDR, NT>(f + base, lds, M, tid, INV ? (T)1 : (T)a.scale);
+    __syncthreads();
+    col_fft<T, N, E, INV, LDR>(v, lds + c, tws, t);
+    const T sc = INV ? (T)1 : (T)a.scale;
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const int n = t + TT * q;
+        if (INV || all || mode_in_sphere(kx, n, 0, N, a.nek)) f[(size_t)n * M] = cscale(v[q], sc);
+    }
 }
 
 // ------------------------------------------------------------------ x stage
@@ -589,11 +517,11 @@ __device__ __forceinline__ void c2r_pack(cpx<T>* lds, const cpx<T>* tw, int tid)
             C w = tw[k];                                  // exp(-2 pi i k / N)
             w.y = -w.y;                                   // exp(+2 pi i k / N)
             const C sa = cadd(xa, cconj(xb)), da = csub(xa, cconj(xb));
-            const C za = cadd(sa, cmul(mk<C>(-w.y, w.x), da));       // + i w (xa - conj xb)
+            const C za = cmadd(sa, mk<C>(-w.y, w.x), da);            // + i w (xa - conj xb)
             if (k2 != k) {
                 const C wb = mk<C>(-w.x, w.y);            // exp(+2 pi i (M-k)/N) = -conj(w)
                 const C sb = cadd(xb, cconj(xa)), db = csub(xb, cconj(xa));
-                const C zb = cadd(sb, cmul(mk<C>(-wb.y, wb.x), db));
+                const C zb = cmadd(sb, mk<C>(-wb.y, wb.x), db);
                 lds[k2 * LDR + line] = zb;
             }
             lds[k * LDR + line] = za;
@@ -620,14 +548,12 @@ __device__ __forceinline__ void r2c_unpack_store(const cpx<T>* lds, const cpx<T>
             const C w = tw[k];                            // exp(-2 pi i k / N)
             const C e1 = cadd(za, cconj(zb)), d1 = csub(za, cconj(zb));
             // X = e1/2 - (i/2) w d1
-            const C wd = cmul(w, d1);
-            const C xa = mk<C>((T)0.5 * (e1.x + wd.y), (T)0.5 * (e1.y - wd.x));
+            const C xa = cscale(cmadd(e1, mk<C>(w.y, -w.x), d1), (T)0.5);
             out[k] = cscale(xa, scale);
             if (k2 != k) {
                 const C wb = mk<C>(-w.x, w.y);            // exp(-2 pi i (M-k)/N) = -conj(w)
                 const C e2 = cadd(zb, cconj(za)), d2 = csub(zb, cconj(za));
-                const C wd2 = cmul(wb, d2);
-                const C xb = mk<C>((T)0.5 * (e2.x + wd2.y), (T)0.5 * (e2.y - wd2.x));
+                const C xb = cscale(cmadd(e2, mk<C>(wb.y, -wb.x), d2), (T)0.5);
                 out[k2] = cscale(xb, scale);
             }
         }
@@ -1226,6 +1152,26 @@ void flow_free(FlowBuffers& fb)
     fb = FlowBuffers{};
 }
 
+// DDNS_Z_SPLIT=1: the z stage as separate kernels
+static bool z_split()
+{
+    const char* env = std::getenv("DDNS_Z_SPLIT");
+    return env && env[0] == '1';
+}
+
+// the fused z stage (or, not FULL, the curl and inverse transforms) at tile width TC
+template <typename T, int N, int TC, bool FULL>
+static bool launch_z_tc(const KzArgs& a, int R, hipStream_t s)
+{
+    if constexpr (kz_fits<T, N, TC>()) {
+        hipLaunchKernelGGL((k_z_full<T, N, TC, FULL>), dim3((unsigned)(N / 2 / TC * N * R)), dim3(kz_threads<T, N, TC>()), 0,
+                           s, a);
+        return true;
+    } else {
+        return false;
+    }
+}
+
 template <typename T, int N>
 static int launch_z(int mode, const FlowBuffers& fb, const FlowConst& fc, hipStream_t s,
                     const void* src = nullptr, void* dst = nullptr, double scale = 1.0)
@@ -1238,21 +1184,23 @@ static int launch_z(int mode, const FlowBuffers& fb, const FlowConst& fc, hipStr
     a.rstride = fb.rstride;
     const int R = fb.R;
     if (mode == KZ_PLAIN_FWD || mode == KZ_PLAIN_INV) { a.B[0] = src; a.U[0] = dst; a.rstride = 0; }
-    constexpr int TC = kz_tc<T, N>();
-    dim3 grid((N / 2 / TC) * N);
-    const char* env = (mode == KZ_FULL || mode == KZ_CURL_INV) ? std::getenv("DDNS_Z_SPLIT") : nullptr;
+    constexpr unsigned gp = (unsigned)(N / 2 / kz_tc_plain<T, N>() * N);
+    constexpr unsigned np = kz_plain_threads<T, N>();
+    if (mode == KZ_PLAIN_FWD || mode == KZ_PLAIN_INV) {
+        if (mode == KZ_PLAIN_FWD) hipLaunchKernelGGL((k_z<T, N, false>), dim3(gp), dim3(np), 0, s, a);
+        else hipLaunchKernelGGL((k_z<T, N, true>), dim3(gp), dim3(np), 0, s, a);
+        DDNS_HIP(hipGetLastError());
+        return 0;
+    }
     // a batch (R > 1) always runs the fused z stage: the split kernels take one realisation
-    const bool split = R == 1 && (env && (env[0] == '0' || env[0] == '1') ? env[0] == '1' : kz_split_default<T, N>());
-    if (split && (mode == KZ_FULL || mode == KZ_CURL_INV)) {
-        const unsigned gp = (unsigned)(N / 2 / kz_tc_plain<T, N>() * N);
+    if (R == 1 && z_split()) {
         const unsigned ge = (unsigned)(((size_t)N * N * (N / 2) + 255) / 256);
         KzArgs p = a;
-        int st;
         if (mode == KZ_FULL) {
             p.scale = 1.0 / N;
             for (int q = 0; q < 3; ++q) {                  // forward z of N-hat, in place, x 1/N
                 p.B[0] = a.B[q]; p.U[0] = (void*)a.B[q];
-                hipLaunchKernelGGL((k_z<T, N, KZ_PLAIN_FWD>), dim3(gp), dim3(kz_threads<T, N, KZ_PLAIN_FWD>()), 0, s, p);
+                hipLaunchKernelGGL((k_z<T, N, false>), dim3(gp), dim3(np), 0, s, p);
             }
             hipLaunchKernelGGL((k_z_update<T, N>), dim3(ge), dim3(256), 0, s, a);      // and the curl
         } else {
@@ -1262,46 +1210,16 @@ static int launch_z(int mode, const FlowBuffers& fb, const FlowConst& fc, hipStr
         for (int q = 0; q < 6; ++q) {                      // inverse z of u-hat and w-hat
             p.B[0] = q < 3 ? (const void*)a.U[q] : (const void*)a.A[q];
             p.U[0] = a.A[q];
-            hipLaunchKernelGGL((k_z<T, N, KZ_PLAIN_INV>), dim3(gp), dim3(kz_threads<T, N, KZ_PLAIN_INV>()), 0, s, p);
+            hipLaunchKernelGGL((k_z<T, N, true>), dim3(gp), dim3(np), 0, s, p);
         }
-        st = 0;
-        DDNS_HIP(hipGetLastError());
-        return st;
-    }
-    if (mode == KZ_PLAIN_FWD || mode == KZ_PLAIN_INV) grid = dim3((N / 2 / kz_tc_plain<T, N>()) * N);
-    if (mode == KZ_FULL) {
-        // persistent: one work-group per CU (the LDS tiles allow no more), of fb.kz_nt
-        // threads (0: the default)
-        int dev = 0, ncu = 0;
-        DDNS_HIP(hipGetDevice(&dev));
-        DDNS_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-        const int ntiles = (int)grid.x * R;
-        const dim3 g(std::max(1, std::min(ncu, ntiles)));
-        constexpr int N0 = kz_nt_cand<T, N>(0), N1 = kz_nt_cand<T, N>(1), N2 = kz_nt_cand<T, N>(2);
-        if constexpr (kz_nt_fits<T, N, N1>()) {
-            if (fb.kz_nt == N1) {
-                hipLaunchKernelGGL((k_z_full<T, N, N1>), g, dim3(N1), 0, s, a, ntiles);
-                DDNS_HIP(hipGetLastError());
-                return 0;
-            }
-        }
-        if constexpr (kz_nt_fits<T, N, N2>()) {
-            if (fb.kz_nt == N2) {
-                hipLaunchKernelGGL((k_z_full<T, N, N2>), g, dim3(N2), 0, s, a, ntiles);
-                DDNS_HIP(hipGetLastError());
-                return 0;
-            }
-        }
-        hipLaunchKernelGGL((k_z_full<T, N, N0>), g, dim3(N0), 0, s, a, ntiles);
         DDNS_HIP(hipGetLastError());
         return 0;
     }
-    if (mode == KZ_CURL_INV) grid.y = R;
-    switch (mode) {
-    case KZ_CURL_INV: hipLaunchKernelGGL((k_z<T, N, KZ_CURL_INV>), grid, dim3(NT), 0, s, a); break;
-    case KZ_PLAIN_FWD: hipLaunchKernelGGL((k_z<T, N, KZ_PLAIN_FWD>), grid, dim3(kz_threads<T, N, KZ_PLAIN_FWD>()), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_z<T, N, KZ_PLAIN_INV>), grid, dim3(kz_threads<T, N, KZ_PLAIN_INV>()), 0, s, a); break;
-    }
+    static_assert(kz_fits<T, N, kz_tc<T, N>()>(), "the default z tile must fit");
+    if (mode == KZ_FULL && fb.kz_nt == kz_threads<T, N, kz_cand<T, N>(1)>() && launch_z_tc<T, N, kz_cand<T, N>(1), true>(a, R, s))
+        ;
+    else if (mode == KZ_FULL) (void)launch_z_tc<T, N, kz_tc<T, N>(), true>(a, R, s);
+    else (void)launch_z_tc<T, N, kz_tc<T, N>(), false>(a, R, s);
     DDNS_HIP(hipGetLastError());
     return 0;
 }
@@ -1309,10 +1227,10 @@ static int launch_z(int mode, const FlowBuffers& fb, const FlowConst& fc, hipStr
 template <typename T, int N, int TC>
 static void launch_y_tc(bool inv, bool sym, const KyArgs& a, int nf, hipStream_t s)
 {
-    dim3 grid(N / 2 / TC, N, nf * a.R);
-    if (inv && sym) hipLaunchKernelGGL((k_y<T, N, true, true, TC>), grid, dim3(NT), 0, s, a);
-    else if (inv) hipLaunchKernelGGL((k_y<T, N, true, false, TC>), grid, dim3(NT), 0, s, a);
-    else hipLaunchKernelGGL((k_y<T, N, false, false, TC>), grid, dim3(NT), 0, s, a);
+    const dim3 grid(N / 2 / TC, N, nf * a.R), nt(TC * (N / col_e<T, N>()));
+    if (inv && sym) hipLaunchKernelGGL((k_y<T, N, true, true, TC>), grid, nt, 0, s, a);
+    else if (inv) hipLaunchKernelGGL((k_y<T, N, true, false, TC>), grid, nt, 0, s, a);
+    else hipLaunchKernelGGL((k_y<T, N, false, false, TC>), grid, nt, 0, s, a);
 }
 
 // candidate k of the y-stage tile widths (0 = half, 1 = default, 2 = twice the default)
@@ -1328,9 +1246,10 @@ static bool launch_y_cand(bool inv, bool sym, const KyArgs& a, int nf, hipStream
     }
 }
 
-// the y stage at the tile width fb.ky_tc (0: the default)
+// the y stage at the tile width fb.ky_tc (0: the default); nek > 0: the stage of a step, which
+// leaves out the rows beyond the dealiasing sphere
 template <typename T, int N>
-static int launch_y(bool inv, bool sym, void* const* f, int nf, const FlowBuffers& fb, hipStream_t s)
+static int launch_y(bool inv, bool sym, void* const* f, int nf, const FlowBuffers& fb, hipStream_t s, int nek = 0)
 {
     KyArgs a{};
     for (int i = 0; i < nf; ++i) a.F[i] = f[i];
@@ -1339,6 +1258,9 @@ static int launch_y(bool inv, bool sym, void* const* f, int nf, const FlowBuffer
     a.nf = nf;
     a.R = fb.R;
     a.rstride = fb.rstride;
+    a.low = nek > 0 ? fb.low : nullptr;
+    a.nek = nek;
+    static_assert(ky_fits<T, N, ky_tc<T, N>()>(), "the default y tile must fit");
     const int tc = fb.ky_tc;
     bool done = false;
     if (tc == ky_cand<T, N>(0)) done = launch_y_cand<T, N, 0>(inv, sym, a, nf, s);
@@ -1400,7 +1322,7 @@ static int step_impl(const FlowBuffers& fb, const FlowConst& fc, hipStream_t s, 
     // the timing events then become event-record nodes of the graph
     if (part == FLOW_INV) {
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[0], s, evflags));
-        int st = launch_y<T, N>(true, true, fb.A, 6, fb, s);
+        int st = launch_y<T, N>(true, true, fb.A, 6, fb, s, fc.nek);
         if (st) return st;
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[1], s, evflags));
         st = launch_x<T, N>(fb, s);
@@ -1412,7 +1334,7 @@ static int step_impl(const FlowBuffers& fb, const FlowConst& fc, hipStream_t s, 
     if (part != FLOW_FWD_Z) {
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[3], s, evflags));
         void* bb[3] = {fb.B[0], fb.B[1], fb.B[2]};
-        st = launch_y<T, N>(false, false, bb, 3, fb, s);
+        st = launch_y<T, N>(false, false, bb, 3, fb, s, fc.nek);
         if (st) return st;
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[4], s, evflags));
         st = launch_pre<T, N>(fb, fc, s);
@@ -2104,27 +2026,17 @@ static bool ky_cand_fits(int k)
 }
 
 template <typename T, int N>
-static bool kz_nt_cand_fits(int k)
+static bool kz_cand_fits(int k)
 {
-    switch (k) {
-    case 0: return kz_nt_fits<T, N, kz_nt_cand<T, N>(0)>();
-    case 1: return kz_nt_fits<T, N, kz_nt_cand<T, N>(1)>();
-    default: return kz_nt_fits<T, N, kz_nt_cand<T, N>(2)>();
-    }
+    return k == 0 || (k == 1 && kz_fits<T, N, kz_cand<T, N>(1)>());
 }
+// threads of the fused z stage's work-group at candidate k (once or twice the default width)
+template <typename T, int N> constexpr int kz_nt_cand(int k) { return kz_threads<T, N, kz_tc<T, N>()>() << k; }
 
 struct TuneRecord {
     int ky_tc, kz_nt;
     float ky_ms[3], kz_ms[3];
 };
-
-// the fused z stage is the one a step runs (not the separate kernels of the split path)
-template <typename T, int N>
-static bool z_fused_in_use()
-{
-    const char* env = std::getenv("DDNS_Z_SPLIT");
-    return env && (env[0] == '0' || env[0] == '1') ? env[0] == '0' : !kz_split_default<T, N>();
-}
 
 // times `reps` runs of launch after one untimed run (ms per run), 0 on failure
 template <typename F>
@@ -2147,7 +2059,7 @@ static int tune_impl(FlowBuffers& fb, const FlowConst& fc, hipStream_t s)
     static std::mutex mu;
     static std::map<int, TuneRecord> cache;          // key: N * 4096 + R, per precision (one map per T)
     fb.ky_tc = ky_tc<T, N>();
-    fb.kz_nt = kz_nt<T, N>();
+    fb.kz_nt = kz_nt_cand<T, N>(0);
     for (int k = 0; k < 3; ++k) fb.ky_ms[k] = fb.kz_ms[k] = 0.f;
     bool forced = false;
     if (const char* f = std::getenv("DDNS_KY_TC")) {
@@ -2159,7 +2071,7 @@ static int tune_impl(FlowBuffers& fb, const FlowConst& fc, hipStream_t s)
     if (const char* f = std::getenv("DDNS_KZ_NT")) {
         const int want = std::atoi(f);
         for (int k = 0; k < 3; ++k)
-            if (want == kz_nt_cand<T, N>(k) && kz_nt_cand_fits<T, N>(k)) fb.kz_nt = want;
+            if (want == kz_nt_cand<T, N>(k) && kz_cand_fits<T, N>(k)) fb.kz_nt = want;
         forced = true;
     }
     if (forced) return 0;
@@ -2190,24 +2102,24 @@ static int tune_impl(FlowBuffers& fb, const FlowConst& fc, hipStream_t s)
     }
     DDNS_HIP(hipMemsetAsync(fb.low, 0, (size_t)LOW_STRIDE * fb.R * sizeof(double), s));
     float best = 0.f;
-    int best_tc = ky_tc<T, N>(), best_nt = kz_nt<T, N>();
+    int best_tc = ky_tc<T, N>(), best_nt = kz_nt_cand<T, N>(0);
     int st = 0;
     for (int k = 0; k < 3 && !st; ++k) {
         if (!ky_cand_fits<T, N>(k)) continue;
         fb.ky_tc = ky_cand<T, N>(k);
         fb.ky_ms[k] = time_runs([&]() {
-            int r = launch_y<T, N>(true, true, fb.A, 6, fb, s);
-            return r ? r : launch_y<T, N>(false, false, fb.B, 3, fb, s);
+            int r = launch_y<T, N>(true, true, fb.A, 6, fb, s, fc.nek);
+            return r ? r : launch_y<T, N>(false, false, fb.B, 3, fb, s, fc.nek);
         }, 3, s, e0, e1, &st);
         if (!st && (best == 0.f || fb.ky_ms[k] < best)) {
             best = fb.ky_ms[k];
             best_tc = fb.ky_tc;
         }
     }
-    if (z_fused_in_use<T, N>()) {
+    if (!z_split()) {
         best = 0.f;
         for (int k = 0; k < 3 && !st; ++k) {
-            if (!kz_nt_cand_fits<T, N>(k)) continue;
+            if (!kz_cand_fits<T, N>(k)) continue;
             fb.kz_nt = kz_nt_cand<T, N>(k);
             fb.kz_ms[k] = time_runs([&]() { return launch_z<T, N>(KZ_FULL, fb, fc, s); }, 3, s, e0, e1, &st);
             if (!st && (best == 0.f || fb.kz_ms[k] < best)) {
@@ -2254,8 +2166,8 @@ int flow_tune(FlowBuffers& fb, const FlowConst& fc, int precision, hipStream_t s
 int flow_default_kz_nt(int N, int precision)
 {
     int nt = 0;
-    if (precision == DDNS_FP64) { DDNS_DISPATCH_N(N, nt = (kz_nt<double, NN>())) }
-    else { DDNS_DISPATCH_N(N, nt = (kz_nt<float, NN>())) }
+    if (precision == DDNS_FP64) { DDNS_DISPATCH_N(N, nt = (kz_nt_cand<double, NN>(0))) }
+    else { DDNS_DISPATCH_N(N, nt = (kz_nt_cand<float, NN>(0))) }
     return nt;
 }
 
