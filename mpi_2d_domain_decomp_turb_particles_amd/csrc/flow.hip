@@ -6,9 +6,8 @@
 // forward stage), flowlib.f90:180-562 (dealiasing, supforDET, symmetrize,
 // supforSTH).
 //
-// Layout: every complex field is [s][r][kx], kx fastest with kx < N/2, so the x
-// stage reads contiguous lines and the y and z stages read tiles of TC adjacent kx
-// columns (one 128-256 byte segment per row).  The step runs as five launches:
+// Layout: ddns_internal.h (rows of 128 bytes of kx, z columns of the state contiguous).  The
+// step runs as:
 //   Ky(inverse, 6 fields, kx = 0 column symmetrised)  ->  Kx(6 C2R, u x w, 3 R2C,
 //   physical u for the droplets)  ->  Ky(forward, 3 fields)  ->  Kpre (one block:
 //   deterministic-forcing shell energies or the OU forcing table)  ->  Kz(forward z
@@ -82,10 +81,6 @@ __device__ __forceinline__ int xcd_tile(int L)
 // tile width of the plain z transforms (the diagnostics, the split z stage): rows of 128 bytes
 template <typename T, int N> constexpr int kz_tc_plain() { return sizeof(T) == 4 || N == 32 ? 16 : 8; }
 template <typename T, int N> constexpr int kz_plain_threads() { return kz_tc_plain<T, N>() * (N / col_e<T, N>()); }
-// The z stage can also run as separate kernels: three plain forward transforms, the pointwise
-// update with the curl, six plain inverse transforms (36 fields moved instead of 21).
-// DDNS_Z_SPLIT=1 in the environment selects them, to check the two against each other.
-
 __device__ __forceinline__ int wave_index(int i, int N) { return i <= N / 2 ? i : i - N; }
 
 // Is mode (kx, ky, kz) inside the dealiasing sphere, shell int(|k| + 1/2) <= nek (turb.f90:405,
@@ -120,7 +115,7 @@ __device__ __forceinline__ int real_forcing(int forcing, const double* lowr)
 }
 
 struct KzArgs {
-    const void* B[3];
+    const void* B[3];  // N-hat: A[0..2] themselves, each point read and written by one thread
     void* U[3];
     void* O[3];
     void* A[6];
@@ -132,24 +127,27 @@ struct KzArgs {
     size_t rstride;    // complex values between realisations of one field
 };
 
+// A field as plain rows, row (z, y) of realisations in a row at p + (z N + y) rs.
+struct PlainRows {
+    void* p[6];
+    int rs[6];         // complex values from row to row
+};
+
 struct KyArgs {
-    void* F[6];
+    void* F[6];        // the fields in the intermediate layout
+    PlainRows L;       // and as plain rows
     const void* tw;
     double scale;
-    int nf, R;         // fields per realisation, realisations: grid z runs over nf * R
     size_t rstride;
     const double* low; // the step's stages (null: every row is read and written)
     int nek;
 };
 
 struct KxArgs {
-    const void* A[6];
-    void* B[3];
-    void* uphys;
+    void* B[3];        // u in, u x w out
+    void* uphys;       // w in (three rows per line), the physical velocity out
     const void* tw;    // N entries (post/pre-processing twiddles)
     const void* twh;   // N/2 entries (half-length FFT)
-    size_t rstride;    // grid y runs over the realisations
-    size_t pstride;    // reals between realisations of the physical velocity
 };
 
 // ------------------------------------------------------------------ spectral update
@@ -208,6 +206,16 @@ __device__ __forceinline__ void update_mode(int kx, int ky, int kz, int N, int n
 }
 
 // ------------------------------------------------------------------ z stage
+// How far plane t + TT q of an intermediate field lies behind plane t (t < TT, TT a divisor or
+// a multiple of the planes per block)
+template <typename T, int N, int TT>
+__device__ __forceinline__ constexpr size_t plane_step(int q)
+{
+    static_assert(TT % LZB == 0 || LZB % TT == 0, "a thread's planes must step through the blocks evenly");
+    constexpr size_t block = (size_t)N * (N / 2) * LZB;
+    return q * TT / LZB * block + q * TT % LZB * lay_w<T>();
+}
+
 // A plain forward / inverse z transform of one field.
 template <typename T, int N, bool INV>
 __global__ void __launch_bounds__((kz_plain_threads<T, N>())) k_z(KzArgs a)
@@ -221,73 +229,19 @@ __global__ void __launch_bounds__((kz_plain_threads<T, N>())) k_z(KzArgs a)
     constexpr int NBX = M / TC;
     const int kx0 = (blockIdx.x % NBX) * TC, ky = blockIdx.x / NBX;
     stage_twiddles<C, N, NTK>(tws, (const C*)a.tw, tid);
-    const size_t rowstride = (size_t)N * M, base = (size_t)ky * M + kx0 + c;
-    const C* src = (const C*)a.B[0] + base;
-    C* dst = (C*)a.U[0] + base;
+    // inverse: spectral to intermediate layout; forward: back
+    const size_t sb = spec_index<T>(N, t, ky, kx0 + c), pb = pipe_index<T>(N, t, ky, kx0 + c);
+    constexpr int SS = TT * lay_w<T>();
+    const C* src = (const C*)a.B[0] + (INV ? sb : pb);
+    C* dst = (C*)a.U[0] + (INV ? pb : sb);
     C v[E];
 #pragma unroll
-    for (int q = 0; q < E; ++q) v[q] = src[(t + TT * q) * rowstride];
+    for (int q = 0; q < E; ++q) v[q] = src[INV ? q * SS : plane_step<T, N, TT>(q)];
     __syncthreads();
     col_fft<T, N, E, INV, LDR>(v, lds + c, tws, t);
     const T sc = (T)a.scale;
 #pragma unroll
-    for (int q = 0; q < E; ++q) dst[(t + TT * q) * rowstride] = cscale(v[q], sc);
-}
-
-// The split z stage's pointwise parts.  k_z_update: the update of k_z_full (dealias,
-// AB2/CN, forcing, projection, CN divide) on the z-transformed N-hat already scaled by
-// 1/N, and the curl of the new u-hat.  k_z_curl: the curl alone, for a new state.
-// The curl is w-hat = i k x u-hat (turb.f90:506-517), into A[3..5].
-template <typename T>
-__device__ __forceinline__ void curl_to(const KzArgs& a, size_t t, int kx, int ky, int kz, int N, const cpx<T>* u)
-{
-    using C = cpx<T>;
-    const T fx = (T)kx, fy = (T)wave_index(ky, N), fz = (T)wave_index(kz, N);
-    const C w0 = csub(cscale(u[2], fy), cscale(u[1], fz));
-    const C w1 = csub(cscale(u[0], fz), cscale(u[2], fx));
-    const C w2 = csub(cscale(u[1], fx), cscale(u[0], fy));
-    ((C*)a.A[3])[t] = mk<C>(-w0.y, w0.x);
-    ((C*)a.A[4])[t] = mk<C>(-w1.y, w1.x);
-    ((C*)a.A[5])[t] = mk<C>(-w2.y, w2.x);
-}
-template <typename T, int N>
-__global__ void __launch_bounds__(256) k_z_update(KzArgs a)
-{
-    using C = cpx<T>;
-    constexpr int M = N / 2;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)N * N * M) return;
-    const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
-    // beyond the dealiasing sphere the state is zero once a step has written it
-    const bool in = a.low[LOW_ZOUT] == 0.0 || mode_in_sphere(kx, ky, kz, N, a.nek);
-    C nn[3], u3[3], o3[3], vv[3], nd[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        nn[q] = ((const C*)a.B[q])[t];
-        u3[q] = in ? ((const C*)a.U[q])[t] : mk<C>((T)0, (T)0);
-        o3[q] = in ? ((const C*)a.O[q])[t] : mk<C>((T)0, (T)0);
-    }
-    update_mode<T>(kx, ky, kz, N, a.nek, a.forcing, (T)a.dt, (T)a.rnu, a.low, nn, u3, o3, vv, nd);
-    if (in) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            ((C*)a.U[q])[t] = vv[q];
-            ((C*)a.O[q])[t] = nd[q];
-        }
-    }
-    curl_to<T>(a, t, kx, ky, kz, N, vv);
-}
-
-template <typename T, int N>
-__global__ void __launch_bounds__(256) k_z_curl(KzArgs a)
-{
-    using C = cpx<T>;
-    constexpr int M = N / 2;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)N * N * M) return;
-    const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
-    const C u[3] = {((const C*)a.U[0])[t], ((const C*)a.U[1])[t], ((const C*)a.U[2])[t]};
-    curl_to<T>(a, t, kx, ky, kz, N, u);
+    for (int q = 0; q < E; ++q) dst[INV ? plane_step<T, N, TT>(q) : q * SS] = cscale(v[q], sc);
 }
 
 // The whole z stage of a column tile in registers.  FULL: forward z transforms of N-hat, the
@@ -325,8 +279,10 @@ __global__ void __launch_bounds__((kz_threads<T, N, TC>()), (kz_waves<T, N>())) 
     const int tile = xcd_tile<(NBX % P == 0 && TPR % (8 * P) == 0) ? P : 1>(blockIdx.x);
     const int rr = tile / TPR, lt = tile - rr * TPR;
     const int kx = (lt % NBX) * TC + c, ky = lt / NBX;
-    const size_t rowstride = (size_t)N * M;
-    const size_t base = (size_t)rr * a.rstride + (size_t)ky * M + kx;
+    const size_t roff = (size_t)rr * a.rstride;
+    // point t of the column in the state (steps of SS) and between the transforms
+    const size_t sbase = roff + spec_index<T>(N, t, ky, kx), pbase = roff + pipe_index<T>(N, t, ky, kx);
+    constexpr int SS = TT * lay_w<T>();
     const double* lowr = a.low + (size_t)rr * LOW_STRIDE;
     // beyond the dealiasing sphere the state is zero once a step has written it
     const bool zout = lowr[LOW_ZOUT] != 0.0;
@@ -340,8 +296,8 @@ __global__ void __launch_bounds__((kz_threads<T, N, TC>()), (kz_waves<T, N>())) 
                 for (int q = 0; q < E; ++q)
 #pragma unroll
                     for (int k = 0; k < 3; ++k) {
-                        ((C*)a.U[k])[base + (t + TT * q) * rowstride] = mk<C>((T)0, (T)0);
-                        ((C*)a.O[k])[base + (t + TT * q) * rowstride] = mk<C>((T)0, (T)0);
+                        ((C*)a.U[k])[sbase + q * SS] = mk<C>((T)0, (T)0);
+                        ((C*)a.O[k])[sbase + q * SS] = mk<C>((T)0, (T)0);
                     }
             }
             return;
@@ -350,12 +306,12 @@ __global__ void __launch_bounds__((kz_threads<T, N, TC>()), (kz_waves<T, N>())) 
         for (int k = 0; k < 3; ++k)
 #pragma unroll
             for (int q = 0; q < E; ++q)
-                u[k][q] = colin ? ((const C*)a.B[k])[base + (t + TT * q) * rowstride] : mk<C>((T)0, (T)0);
+                u[k][q] = colin ? ((const C*)a.B[k])[pbase + plane_step<T, N, TT>(q)] : mk<C>((T)0, (T)0);
     } else {
 #pragma unroll
         for (int k = 0; k < 3; ++k)
 #pragma unroll
-            for (int q = 0; q < E; ++q) u[k][q] = ((const C*)a.U[k])[base + (t + TT * q) * rowstride];
+            for (int q = 0; q < E; ++q) u[k][q] = ((const C*)a.U[k])[sbase + q * SS];
     }
     stage_twiddles<C, N, kz_threads<T, N, TC>()>(tws, (const C*)a.tw, tid);
     __syncthreads();
@@ -368,7 +324,7 @@ __global__ void __launch_bounds__((kz_threads<T, N, TC>()), (kz_waves<T, N>())) 
 #pragma unroll
         for (int q = 0; q < E; ++q) {
             const int n = t + TT * q;
-            const size_t g = base + n * rowstride;
+            const size_t g = sbase + q * SS;
             if (mode_in_sphere(kx, ky, n, N, a.nek)) {
                 C nn[3], u3[3], o3[3], vv[3], nd[3];
 #pragma unroll
@@ -412,7 +368,7 @@ __global__ void __launch_bounds__((kz_threads<T, N, TC>()), (kz_waves<T, N>())) 
         col_fft<T, N, E, true, LDR>(w, col, tws, t);
         if (colin) {
 #pragma unroll
-            for (int q = 0; q < E; ++q) ((C*)a.A[3 + k])[base + (t + TT * q) * rowstride] = w[q];
+            for (int q = 0; q < E; ++q) ((C*)a.A[3 + k])[pbase + plane_step<T, N, TT>(q)] = w[q];
         }
     }
 #pragma unroll
@@ -420,16 +376,18 @@ __global__ void __launch_bounds__((kz_threads<T, N, TC>()), (kz_waves<T, N>())) 
         col_fft<T, N, E, true, LDR>(u[k], col, tws, t);
         if (colin) {
 #pragma unroll
-            for (int q = 0; q < E; ++q) ((C*)a.A[k])[base + (t + TT * q) * rowstride] = u[k][q];
+            for (int q = 0; q < E; ++q) ((C*)a.A[k])[pbase + plane_step<T, N, TT>(q)] = u[k][q];
         }
     }
 }
 
 // ------------------------------------------------------------------ y stage
-// Columns in registers as in the z stage; bound by HBM.  In a step (a.low given) the rows
-// beyond the circle kx^2 + ky^2 of the dealiasing sphere (21 % of them) are left out: the
-// inverse stage takes them as zero (unless the state was set since the last step, when the
-// z transforms of that state fill them), the forward stage does not store them.
+// Columns in registers as in the z stage; bound by memory.  The inverse stage takes a plane
+// from the intermediate layout to plain [y][kx] rows, where the x stage finds its lines; the
+// forward stage goes the other way.  In a step (a.low given) the rows beyond the circle
+// kx^2 + ky^2 of the dealiasing sphere (21 % of them) are left out: the inverse stage takes
+// them as zero (unless the state was set since the last step, when the z transforms of that
+// state fill them), the forward stage does not store them.
 template <typename T, int N, bool INV, bool SYM, int TC>
 __global__ void __launch_bounds__((TC * (N / col_e<T, N>()))) k_y(KyArgs a)
 {
@@ -442,24 +400,29 @@ __global__ void __launch_bounds__((TC * (N / col_e<T, N>()))) k_y(KyArgs a)
     // tiles whose rows share a 128-byte line (P of them, side by side in kx) go to linear
     // ids L, L+8, ..., i.e. to one XCD, where the second finds the line in L2
     constexpr int P = (TC * (int)sizeof(C) >= 128) ? 1 : 128 / (TC * (int)sizeof(C));
-    int kxb = blockIdx.x, z = blockIdx.y, fi = blockIdx.z;
+    int kxb = blockIdx.x, lp = blockIdx.y, fi = blockIdx.z;
     if constexpr (P > 1) {
         if ((M / TC) % P == 0 && (gridDim.y * gridDim.z) % 8 == 0) {
             const int l = xcd_tile<P>(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
             kxb = l % gridDim.x;
-            z = (l / gridDim.x) % gridDim.y;
+            lp = (l / gridDim.x) % gridDim.y;
             fi = l / (gridDim.x * gridDim.y);
         }
     }
     const int kx = kxb * TC + c;
-    const int rr = fi / a.nf;
-    C* f = (C*)a.F[fi - rr * a.nf] + (size_t)rr * a.rstride + (size_t)z * N * M + kx;
+    const int rr = lp / N, z = lp % N;
+    // row n of this plane's column: n * PS behind pf in the intermediate layout, n * ls behind lf
+    // as plain rows
+    C* pf = (C*)a.F[fi] + (size_t)rr * a.rstride + pipe_index<T>(N, z, 0, kx);
+    const int ls = a.L.rs[fi];
+    C* lf = (C*)a.L.p[fi] + (size_t)lp * N * ls + kx;
+    constexpr int PS = LZB * lay_w<T>();
     const bool all = !a.low || (INV && a.low[(size_t)rr * LOW_STRIDE + LOW_ZOUT] == 0.0);
     C v[E];
 #pragma unroll
     for (int q = 0; q < E; ++q) {
         const int n = t + TT * q;
-        v[q] = !INV || all || mode_in_sphere(kx, n, 0, N, a.nek) ? f[(size_t)n * M] : mk<C>((T)0, (T)0);
+        v[q] = !INV || all || mode_in_sphere(kx, n, 0, N, a.nek) ? (INV ? pf[(size_t)n * PS] : lf[(size_t)n * ls]) : mk<C>((T)0, (T)0);
     }
     stage_twiddles<C, N, NTK>(tws, (const C*)a.tw, tid);
     if constexpr (SYM) {
@@ -482,11 +445,12 @@ __global__ void __launch_bounds__((TC * (N / col_e<T, N>()))) k_y(KyArgs a)
     }
     __syncthreads();
     col_fft<T, N, E, INV, LDR>(v, lds + c, tws, t);
-    const T sc = INV ? (T)1 : (T)a.scale;
+    const T sc = (T)a.scale;
 #pragma unroll
     for (int q = 0; q < E; ++q) {
         const int n = t + TT * q;
-        if (INV || all || mode_in_sphere(kx, n, 0, N, a.nek)) f[(size_t)n * M] = cscale(v[q], sc);
+        if (INV) lf[(size_t)n * ls] = v[q];
+        else if (all || mode_in_sphere(kx, n, 0, N, a.nek)) pf[(size_t)n * PS] = cscale(v[q], sc);
     }
 }
 
@@ -594,22 +558,26 @@ __global__ void __launch_bounds__(NT) k_x_fused(KxArgs a)
     __shared__ C tws[N], twhs[M];
     const int tid = threadIdx.x;
     const size_t line0 = (size_t)blockIdx.x * TL;
-    const size_t roff = (size_t)blockIdx.y * a.rstride;     // this realisation's fields
     stage_twiddles<C, N, NT>(tws, (const C*)a.tw, tid);
     stage_twiddles<C, M, NT>(twhs, (const C*)a.twh, tid);
     const C* tw = tws;
     const C* twh = twhs;
     C ph[6][QP];
     TileRegs<C, TL, M, NT> next0, next1;
-    tile_fetch<C, TL, M, NT>(next0, (const C*)a.A[0] + roff + line0 * M, M, tid);
-    tile_fetch<C, TL, M, NT>(next1, (const C*)a.A[1] + roff + line0 * M, M, tid);
+    // field f of this work-group's lines; every line is read before it is written
+    auto fetch = [&](TileRegs<C, TL, M, NT>& r, int f) {
+        if (f < 3) tile_fetch<C, TL, M, NT>(r, (const C*)a.B[f] + line0 * M, M, tid);
+        else tile_fetch<C, TL, M, NT>(r, (const C*)a.uphys + (3 * line0 + f - 3) * M, 3 * M, tid);
+    };
+    fetch(next0, 0);
+    fetch(next1, 1);
 #pragma unroll
     for (int f = 0; f < 6; f += 2) {
         tile_put<C, TL, M, LDR, NT, true>(lds, next0, tid);
         tile_put<C, TL, M, LDR, NT, true>(lds + TS, next1, tid);
         if (f < 4) {
-            tile_fetch<C, TL, M, NT>(next0, (const C*)a.A[f + 2] + roff + line0 * M, M, tid);
-            tile_fetch<C, TL, M, NT>(next1, (const C*)a.A[f + 3] + roff + line0 * M, M, tid);
+            fetch(next0, f + 2);
+            fetch(next1, f + 3);
         }
         __syncthreads();
         c2r_pack<T, N, TL, LDR>(lds, tw, tid);
@@ -628,7 +596,7 @@ __global__ void __launch_bounds__(NT) k_x_fused(KxArgs a)
     // physical velocity for the droplet gather: [line][x][3], the two nodes of a complex
     // value in three vector stores
     {
-        T* up = (T*)a.uphys + (size_t)blockIdx.y * a.pstride + line0 * (size_t)N * 3;
+        T* up = (T*)a.uphys + line0 * (size_t)N * 3;
 #pragma unroll
         for (int q = 0; q < QP; ++q) {
             const int e = tid + NT * q;
@@ -653,7 +621,7 @@ __global__ void __launch_bounds__(NT) k_x_fused(KxArgs a)
     fft_tile<T, M, false, TL, LDR, NT, 3, TS>(lds, twh, tid);
     const T scale = (T)1 / (T)N;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) r2c_unpack_store<T, N, TL, LDR>(lds + c * TS, tw, (C*)a.B[c] + roff, line0, scale, tid);
+    for (int c = 0; c < 3; ++c) r2c_unpack_store<T, N, TL, LDR>(lds + c * TS, tw, (C*)a.B[c], line0, scale, tid);
 }
 
 // Stand-alone x transforms of one field (kernel-level parity of mpifft3DRC/CR).
@@ -801,7 +769,7 @@ __global__ void __launch_bounds__(NT) k_pre_dft(PreArgs a)
     const C* tw = (const C*)a.tw;
     double sr = 0.0, si = 0.0;
     for (int z = threadIdx.x; z < N; z += NT) {
-        const C v = b[((size_t)z * N + ky) * M + kx];
+        const C v = b[pipe_index<T>(N, z, ky, kx)];
         const C w = tw[(kzi * z) & (N - 1)];
         sr += (double)v.x * (double)w.x - (double)v.y * (double)w.y;
         si += (double)v.x * (double)w.y + (double)v.y * (double)w.x;
@@ -900,7 +868,7 @@ __global__ void __launch_bounds__(NT) k_pre(PreArgs a)
     if (tid < 75) {
         const int kx = tid % 3, kyw = (tid / 3) % 5 - 2, kzw = tid / 15 - 2;
         const int ky = (kyw + N) % N, kz = (kzw + N) % N;
-        const size_t g = ((size_t)kz * N + ky) * M + kx;
+        const size_t g = spec_index<T>(N, kz, ky, kx);
         C nn[3], uu[3], oo[3], vv[3], nd[3];
         for (int q = 0; q < 3; ++q) {
             nn[q] = mk<C>((T)nre[q * 75 + tid], (T)nim[q * 75 + tid]);
@@ -944,14 +912,14 @@ __global__ void k_sym(void* u0, void* u1, void* u2, size_t rstride, double* low)
     constexpr int M = N / 2;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= N * N) return;
-    const int kz = t / N, ky = t % N;
+    const int ky = t / N, kz = t % N;
     const int mz = (N - kz) & (N - 1), my = (N - ky) & (N - 1);
-    if (mz * N + my < t) return;           // the partner with the smaller index does the pair
+    if (my * N + mz < t) return;           // the partner with the smaller index does the pair
     void* fs[3] = {u0, u1, u2};
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         C* f = (C*)fs[q] + (size_t)blockIdx.y * rstride;     // realisation blockIdx.y
-        const size_t gp = ((size_t)kz * N + ky) * M, gm = ((size_t)mz * N + my) * M;
+        const size_t gp = spec_index<T>(N, kz, ky, 0), gm = spec_index<T>(N, mz, my, 0);
         const C p = f[gp], m = f[gm];
         const C s = mk<C>((T)0.5 * (p.x + m.x), (T)0.5 * (p.y - m.y));
         f[gp] = s;
@@ -1006,7 +974,8 @@ __global__ void __launch_bounds__(256) k_init_modes(void* u0, void* u1, void* u2
     for (int i = threadIdx.x; i < M; i += 256) cnt[i] = 0;
     __syncthreads();
     for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < (size_t)N * N * M; t += (size_t)gridDim.x * 256) {
-        const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
+        int kx, ky, kz;
+    spec_mode<T>(N, t, kz, ky, kx);
         const int kyw = wave_index(ky, N), kzw = wave_index(kz, N);
         const bool zero = ky == N / 2 || kz == N / 2 || (kx == 0 && ky == 0 && kz == 0);
         double2 g[3];
@@ -1048,7 +1017,9 @@ __global__ void k_init_scale(void* u0, void* u1, void* u2, int nek, const double
     constexpr int M = N / 2;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (size_t)N * N * M) return;
-    const int kx = (int)(t % M), kyw = wave_index((int)((t / M) % N), N), kzw = wave_index((int)(t / ((size_t)N * M)), N);
+    int kx, ky, kz;
+    spec_mode<T>(N, t, kz, ky, kx);
+    const int kyw = wave_index(ky, N), kzw = wave_index(kz, N);
     double k2 = (double)(kx * kx + kyw * kyw + kzw * kzw);
     if (k2 == 0.0) k2 = 1.e-5;
     const int ik2 = (int)(sqrt(k2) + 0.5);
@@ -1152,13 +1123,6 @@ void flow_free(FlowBuffers& fb)
     fb = FlowBuffers{};
 }
 
-// DDNS_Z_SPLIT=1: the z stage as separate kernels
-static bool z_split()
-{
-    const char* env = std::getenv("DDNS_Z_SPLIT");
-    return env && env[0] == '1';
-}
-
 // the fused z stage (or, not FULL, the curl and inverse transforms) at tile width TC
 template <typename T, int N, int TC, bool FULL>
 static bool launch_z_tc(const KzArgs& a, int R, hipStream_t s)
@@ -1177,7 +1141,7 @@ static int launch_z(int mode, const FlowBuffers& fb, const FlowConst& fc, hipStr
                     const void* src = nullptr, void* dst = nullptr, double scale = 1.0)
 {
     KzArgs a{};
-    for (int i = 0; i < 3; ++i) { a.B[i] = fb.B[i]; a.U[i] = fb.U[i]; a.O[i] = fb.O[i]; }
+    for (int i = 0; i < 3; ++i) { a.B[i] = fb.A[i]; a.U[i] = fb.U[i]; a.O[i] = fb.O[i]; }
     for (int i = 0; i < 6; ++i) a.A[i] = fb.A[i];
     a.tw = fb.tw; a.low = fb.low; a.dt = fc.dt; a.rnu = fc.rnu; a.nek = fc.nek; a.forcing = fc.forcing;
     a.scale = scale;
@@ -1192,29 +1156,6 @@ static int launch_z(int mode, const FlowBuffers& fb, const FlowConst& fc, hipStr
         DDNS_HIP(hipGetLastError());
         return 0;
     }
-    // a batch (R > 1) always runs the fused z stage: the split kernels take one realisation
-    if (R == 1 && z_split()) {
-        const unsigned ge = (unsigned)(((size_t)N * N * (N / 2) + 255) / 256);
-        KzArgs p = a;
-        if (mode == KZ_FULL) {
-            p.scale = 1.0 / N;
-            for (int q = 0; q < 3; ++q) {                  // forward z of N-hat, in place, x 1/N
-                p.B[0] = a.B[q]; p.U[0] = (void*)a.B[q];
-                hipLaunchKernelGGL((k_z<T, N, false>), dim3(gp), dim3(np), 0, s, p);
-            }
-            hipLaunchKernelGGL((k_z_update<T, N>), dim3(ge), dim3(256), 0, s, a);      // and the curl
-        } else {
-            hipLaunchKernelGGL((k_z_curl<T, N>), dim3(ge), dim3(256), 0, s, a);
-        }
-        p.scale = 1.0;
-        for (int q = 0; q < 6; ++q) {                      // inverse z of u-hat and w-hat
-            p.B[0] = q < 3 ? (const void*)a.U[q] : (const void*)a.A[q];
-            p.U[0] = a.A[q];
-            hipLaunchKernelGGL((k_z<T, N, true>), dim3(gp), dim3(np), 0, s, p);
-        }
-        DDNS_HIP(hipGetLastError());
-        return 0;
-    }
     static_assert(kz_fits<T, N, kz_tc<T, N>()>(), "the default z tile must fit");
     if (mode == KZ_FULL && fb.kz_nt == kz_threads<T, N, kz_cand<T, N>(1)>() && launch_z_tc<T, N, kz_cand<T, N>(1), true>(a, R, s))
         ;
@@ -1225,9 +1166,9 @@ static int launch_z(int mode, const FlowBuffers& fb, const FlowConst& fc, hipStr
 }
 
 template <typename T, int N, int TC>
-static void launch_y_tc(bool inv, bool sym, const KyArgs& a, int nf, hipStream_t s)
+static void launch_y_tc(bool inv, bool sym, const KyArgs& a, int nf, int planes, hipStream_t s)
 {
-    const dim3 grid(N / 2 / TC, N, nf * a.R), nt(TC * (N / col_e<T, N>()));
+    const dim3 grid(N / 2 / TC, planes, nf), nt(TC * (N / col_e<T, N>()));
     if (inv && sym) hipLaunchKernelGGL((k_y<T, N, true, true, TC>), grid, nt, 0, s, a);
     else if (inv) hipLaunchKernelGGL((k_y<T, N, true, false, TC>), grid, nt, 0, s, a);
     else hipLaunchKernelGGL((k_y<T, N, false, false, TC>), grid, nt, 0, s, a);
@@ -1235,50 +1176,73 @@ static void launch_y_tc(bool inv, bool sym, const KyArgs& a, int nf, hipStream_t
 
 // candidate k of the y-stage tile widths (0 = half, 1 = default, 2 = twice the default)
 template <typename T, int N, int K>
-static bool launch_y_cand(bool inv, bool sym, const KyArgs& a, int nf, hipStream_t s)
+static bool launch_y_cand(bool inv, bool sym, const KyArgs& a, int nf, int planes, hipStream_t s)
 {
     constexpr int TC = ky_cand<T, N>(K);
     if constexpr (ky_fits<T, N, TC>()) {
-        launch_y_tc<T, N, TC>(inv, sym, a, nf, s);
+        launch_y_tc<T, N, TC>(inv, sym, a, nf, planes, s);
         return true;
     } else {
         return false;
     }
 }
 
-// the y stage at the tile width fb.ky_tc (0: the default); nek > 0: the stage of a step, which
-// leaves out the rows beyond the dealiasing sphere
+// the y stage of nf fields of planes planes at the tile width fb.ky_tc (0: the default); nek > 0:
+// the stage of a step, which leaves out the rows beyond the dealiasing sphere
 template <typename T, int N>
-static int launch_y(bool inv, bool sym, void* const* f, int nf, const FlowBuffers& fb, hipStream_t s, int nek = 0)
+static int launch_y(bool inv, bool sym, void* const* f, const PlainRows& rows, int nf, const FlowBuffers& fb, int planes,
+                    hipStream_t s, int nek = 0)
 {
     KyArgs a{};
     for (int i = 0; i < nf; ++i) a.F[i] = f[i];
+    a.L = rows;
     a.tw = fb.tw;
     a.scale = 1.0 / N;
-    a.nf = nf;
-    a.R = fb.R;
     a.rstride = fb.rstride;
     a.low = nek > 0 ? fb.low : nullptr;
     a.nek = nek;
     static_assert(ky_fits<T, N, ky_tc<T, N>()>(), "the default y tile must fit");
     const int tc = fb.ky_tc;
     bool done = false;
-    if (tc == ky_cand<T, N>(0)) done = launch_y_cand<T, N, 0>(inv, sym, a, nf, s);
-    else if (tc == ky_cand<T, N>(2)) done = launch_y_cand<T, N, 2>(inv, sym, a, nf, s);
-    if (!done) launch_y_tc<T, N, ky_tc<T, N>()>(inv, sym, a, nf, s);
+    if (tc == ky_cand<T, N>(0)) done = launch_y_cand<T, N, 0>(inv, sym, a, nf, planes, s);
+    else if (tc == ky_cand<T, N>(2)) done = launch_y_cand<T, N, 2>(inv, sym, a, nf, planes, s);
+    if (!done) launch_y_tc<T, N, ky_tc<T, N>()>(inv, sym, a, nf, planes, s);
     DDNS_HIP(hipGetLastError());
     return 0;
+}
+
+// One field as plain rows.
+template <int N> static PlainRows plain_field(void* p)
+{
+    PlainRows r{};
+    r.p[0] = p;
+    r.rs[0] = N / 2;
+    return r;
+}
+
+// The step's fields between the y and x stages: u (and, after the x stage, u x w) in B, one
+// after the other; w in the physical velocity's memory, the rows of its three components
+// side by side, which are the line's three real components once the x stage has read them.
+template <typename T, int N>
+static PlainRows plain_rows(const FlowBuffers& fb)
+{
+    PlainRows r{};
+    for (int i = 0; i < 3; ++i) {
+        r.p[i] = fb.B[i];
+        r.rs[i] = N / 2;
+        r.p[3 + i] = (cpx<T>*)fb.uphys + i * (N / 2);
+        r.rs[3 + i] = 3 * (N / 2);
+    }
+    return r;
 }
 
 template <typename T, int N>
 static int launch_x(const FlowBuffers& fb, hipStream_t s)
 {
     KxArgs a{};
-    for (int i = 0; i < 6; ++i) a.A[i] = fb.A[i];
     for (int i = 0; i < 3; ++i) a.B[i] = fb.B[i];
     a.uphys = fb.uphys; a.tw = fb.tw; a.twh = fb.twh;
-    a.rstride = fb.rstride; a.pstride = fb.pstride;
-    dim3 grid((unsigned)((size_t)N * N / kxf_lines<N>()), fb.R);
+    const dim3 grid((unsigned)((size_t)fb.R * N * N / kxf_lines<N>()));
     hipLaunchKernelGGL((k_x_fused<T, N>), grid, dim3(NT), 0, s, a);
     DDNS_HIP(hipGetLastError());
     return 0;
@@ -1289,7 +1253,7 @@ static int launch_pre(const FlowBuffers& fb, const FlowConst& fc, hipStream_t s)
 {
     if (fc.forcing != 1 && fc.forcing != 2 && fc.forcing >= 0) return 0;
     PreArgs a{};
-    for (int i = 0; i < 3; ++i) { a.B[i] = fb.B[i]; a.U[i] = fb.U[i]; a.O[i] = fb.O[i]; }
+    for (int i = 0; i < 3; ++i) { a.B[i] = fb.A[i]; a.U[i] = fb.U[i]; a.O[i] = fb.O[i]; }
     a.tw = fb.tw; a.low = fb.low; a.sth_state = fb.sth_state; a.sth_b = fb.sth_b;
     a.dt = fc.dt; a.rnu = fc.rnu; a.force0 = fc.force0; a.force1 = fc.force1;
     a.ou_tf = fc.ou_tf; a.ou_var = fc.ou_var; a.pi2 = fc.pi2; a.nek = fc.nek; a.forcing = fc.forcing;
@@ -1322,7 +1286,7 @@ static int step_impl(const FlowBuffers& fb, const FlowConst& fc, hipStream_t s, 
     // the timing events then become event-record nodes of the graph
     if (part == FLOW_INV) {
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[0], s, evflags));
-        int st = launch_y<T, N>(true, true, fb.A, 6, fb, s, fc.nek);
+        int st = launch_y<T, N>(true, true, fb.A, plain_rows<T, N>(fb), 6, fb, fb.R * N, s, fc.nek);
         if (st) return st;
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[1], s, evflags));
         st = launch_x<T, N>(fb, s);
@@ -1333,8 +1297,7 @@ static int step_impl(const FlowBuffers& fb, const FlowConst& fc, hipStream_t s, 
     int st = 0;
     if (part != FLOW_FWD_Z) {
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[3], s, evflags));
-        void* bb[3] = {fb.B[0], fb.B[1], fb.B[2]};
-        st = launch_y<T, N>(false, false, bb, 3, fb, s, fc.nek);
+        st = launch_y<T, N>(false, false, fb.A, plain_rows<T, N>(fb), 3, fb, fb.R * N, s, fc.nek);
         if (st) return st;
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[4], s, evflags));
         st = launch_pre<T, N>(fb, fc, s);
@@ -1402,7 +1365,7 @@ static int stage_buffer(FlowBuffers& fb, size_t bytes, double** out)
 }
 
 // Planes ky0 .. ky0 + gridDim.z of v(N+2, N+2, N) (kz fastest, then kx re/im, then ky) from
-// a field [kz][ky][kx], with the padding rows zero (PACK), or the field from the planes.
+// a spectral field, with the padding rows zero (PACK), or the field from the planes.
 // 32 x 32 tiles through LDS: kx is contiguous on one side, kz on the other.
 template <typename T, bool PACK>
 __global__ void __launch_bounds__(256) k_layout(cpx<T>* __restrict__ f, double* __restrict__ v, int N, int ky0)
@@ -1417,7 +1380,7 @@ __global__ void __launch_bounds__(256) k_layout(cpx<T>* __restrict__ f, double* 
 #pragma unroll
         for (int q = 0; q < 32; q += 8) {
             const int kz = kz0 + b + q, kx = kx0 + a;
-            tile[b + q][a] = kz < N && kx < M ? f[((size_t)kz * N + ky) * M + kx] : mk<C>((T)0, (T)0);
+            tile[b + q][a] = kz < N && kx < M ? f[spec_index<T>(N, kz, ky, kx)] : mk<C>((T)0, (T)0);
         }
         __syncthreads();
 #pragma unroll
@@ -1440,7 +1403,7 @@ __global__ void __launch_bounds__(256) k_layout(cpx<T>* __restrict__ f, double* 
 #pragma unroll
         for (int q = 0; q < 32; q += 8) {
             const int kz = kz0 + b + q, kx = kx0 + a;
-            if (kz < N && kx < M) f[((size_t)kz * N + ky) * M + kx] = tile[b + q][a];
+            if (kz < N && kx < M) f[spec_index<T>(N, kz, ky, kx)] = tile[b + q][a];
         }
     }
 }
@@ -1630,6 +1593,38 @@ int flow_init(FlowBuffers& fb, int N, int nek, int precision, int kind, int seed
 }
 
 // ---------------------------------------------------------------- stand-alone FFTs
+// One field src (spectral) to real lines dst ([z][y][x]) through tmp (intermediate layout);
+// dst may be src.
+template <typename T, int N>
+static int c2r_dev(const FlowBuffers& fb, const void* src, void* tmp, void* dst, hipStream_t s)
+{
+    FlowConst fc{};
+    fc.N = N;
+    int st = launch_z<T, N>(KZ_PLAIN_INV, fb, fc, s, src, tmp, 1.0);
+    if (st) return st;
+    st = launch_y<T, N>(true, false, &tmp, plain_field<N>(dst), 1, fb, N, s);
+    if (st) return st;
+    hipLaunchKernelGGL((k_x_plain<T, N, true>), dim3((unsigned)((size_t)N * N / kx_lines<N>())), dim3(NT), 0, s,
+                       (const void*)dst, dst, fb.tw, fb.twh);
+    DDNS_HIP(hipGetLastError());
+    return 0;
+}
+
+// Real lines src to the spectral field dst through tmp (plain rows) and mid (intermediate
+// layout); dst may be src or tmp.
+template <typename T, int N>
+static int r2c_dev(const FlowBuffers& fb, const void* src, void* tmp, void* mid, void* dst, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_x_plain<T, N, false>), dim3((unsigned)((size_t)N * N / kx_lines<N>())), dim3(NT), 0, s, src, tmp,
+                       fb.tw, fb.twh);
+    DDNS_HIP(hipGetLastError());
+    int st = launch_y<T, N>(false, false, &mid, plain_field<N>(tmp), 1, fb, N, s);
+    if (st) return st;
+    FlowConst fc{};
+    fc.N = N;
+    return launch_z<T, N>(KZ_PLAIN_FWD, fb, fc, s, mid, dst, 1.0 / N);
+}
+
 template <typename T, int N>
 static int r2c_impl(FlowBuffers& fb, double* v, hipStream_t s)
 {
@@ -1641,19 +1636,11 @@ static int r2c_impl(FlowBuffers& fb, double* v, hipStream_t s)
         for (int y = 0; y < N; ++y)
             for (int x = 0; x < N; ++x)
                 h[((size_t)z * N + y) * N + x] = (T)v[(size_t)x + (size_t)L * ((size_t)y + (size_t)L * z)];
-    // A[0] holds the real input (same byte size as one complex field), B[0] the output
+    // A[0] holds the real input (same byte size as one complex field), A[2] the output
     DDNS_HIP(hipMemcpyAsync(fb.A[0], h.data(), n3 * sizeof(T), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL((k_x_plain<T, N, false>), dim3((unsigned)((size_t)N * N / kx_lines<N>())), dim3(NT), 0, s,
-                       fb.A[0], fb.B[0], fb.tw, fb.twh);
-    DDNS_HIP(hipGetLastError());
-    void* f[1] = {fb.B[0]};
-    int st = launch_y<T, N>(false, false, f, 1, fb, s);
+    const int st = r2c_dev<T, N>(fb, fb.A[0], fb.B[0], fb.A[1], fb.A[2], s);
     if (st) return st;
-    FlowConst fc{};
-    fc.N = N;
-    st = launch_z<T, N>(KZ_PLAIN_FWD, fb, fc, s, fb.B[0], fb.A[1], 1.0 / N);
-    if (st) return st;
-    return download_spectral<T>(fb, fb.A[1], N, v, s);
+    return download_spectral<T>(fb, fb.A[2], N, v, s);
 }
 
 template <typename T, int N>
@@ -1663,16 +1650,8 @@ static int c2r_impl(FlowBuffers& fb, double* v, hipStream_t s)
     const size_t n3 = (size_t)N * N * N;
     int st = upload_spectral<T>(fb, fb.A[1], N, v, s);
     if (st) return st;
-    FlowConst fc{};
-    fc.N = N;
-    st = launch_z<T, N>(KZ_PLAIN_INV, fb, fc, s, fb.A[1], fb.B[0], 1.0);
+    st = c2r_dev<T, N>(fb, fb.A[1], fb.B[0], fb.A[0], s);
     if (st) return st;
-    void* f[1] = {fb.B[0]};
-    st = launch_y<T, N>(true, false, f, 1, fb, s);
-    if (st) return st;
-    hipLaunchKernelGGL((k_x_plain<T, N, true>), dim3((unsigned)((size_t)N * N / kx_lines<N>())), dim3(NT), 0, s,
-                       fb.B[0], fb.A[0], fb.tw, fb.twh);
-    DDNS_HIP(hipGetLastError());
     std::vector<T> h(n3);
     DDNS_HIP(hipMemcpyAsync(h.data(), fb.A[0], n3 * sizeof(T), hipMemcpyDeviceToHost, s));
     DDNS_HIP(hipStreamSynchronize(s));
@@ -1714,7 +1693,8 @@ __global__ void k_mul_ik(const void* src, void* dst, int c)
     constexpr int M = N / 2;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (size_t)N * N * M) return;
-    const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
+    int kx, ky, kz;
+    spec_mode<T>(N, t, kz, ky, kx);
     const T k = (T)(c == 0 ? kx : (c == 1 ? wave_index(ky, N) : wave_index(kz, N)));
     const C v = ((const C*)src)[t];
     ((C*)dst)[t] = mk<C>(-(k * v.y), k * v.x);
@@ -1729,7 +1709,8 @@ __global__ void k_curl_div(const void* u0, const void* u1, const void* u2, void*
     constexpr int M = N / 2;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (size_t)N * N * M) return;
-    const int kx = (int)(t % M), ky = (int)((t / M) % N), kz = (int)(t / ((size_t)N * M));
+    int kx, ky, kz;
+    spec_mode<T>(N, t, kz, ky, kx);
     const T fx = (T)kx, fy = (T)wave_index(ky, N), fz = (T)wave_index(kz, N);
     const C a = ((const C*)u0)[t], b = ((const C*)u1)[t], d = ((const C*)u2)[t];
     C w;
@@ -1800,36 +1781,6 @@ __global__ void __launch_bounds__(DG_T) k_dg_reduce(const T* f0, const T* f1, co
         part[gridDim.x + blockIdx.x] = sh[1][0];
         part[2 * gridDim.x + blockIdx.x] = sh[2][0];
     }
-}
-
-template <typename T, int N>
-static int c2r_dev(const FlowBuffers& fb, const void* src, void* tmp, void* dst, hipStream_t s)
-{
-    FlowConst fc{};
-    fc.N = N;
-    int st = launch_z<T, N>(KZ_PLAIN_INV, fb, fc, s, src, tmp, 1.0);
-    if (st) return st;
-    void* f[1] = {tmp};
-    st = launch_y<T, N>(true, false, f, 1, fb, s);
-    if (st) return st;
-    hipLaunchKernelGGL((k_x_plain<T, N, true>), dim3((unsigned)((size_t)N * N / kx_lines<N>())), dim3(NT), 0, s, tmp, dst,
-                       fb.tw, fb.twh);
-    DDNS_HIP(hipGetLastError());
-    return 0;
-}
-
-template <typename T, int N>
-static int r2c_dev(const FlowBuffers& fb, const void* src, void* tmp, void* dst, hipStream_t s)
-{
-    hipLaunchKernelGGL((k_x_plain<T, N, false>), dim3((unsigned)((size_t)N * N / kx_lines<N>())), dim3(NT), 0, s, src, tmp,
-                       fb.tw, fb.twh);
-    DDNS_HIP(hipGetLastError());
-    void* f[1] = {tmp};
-    int st = launch_y<T, N>(false, false, f, 1, fb, s);
-    if (st) return st;
-    FlowConst fc{};
-    fc.N = N;
-    return launch_z<T, N>(KZ_PLAIN_FWD, fb, fc, s, tmp, dst, 1.0 / N);
 }
 
 // partials of a k_dg_reduce launch summed (or maxed) on the host in block order
@@ -1917,9 +1868,9 @@ static int diag_impl(FlowBuffers& fb, int nek, double rnu, int want, double* ek,
         hipLaunchKernelGGL((k_cross<T>), dim3(gr), dim3(256), 0, s, R[0], R[1], R[2], R[3], R[4], R[5], n3);
         DDNS_HIP(hipGetLastError());
         for (int c = 0; c < 3; ++c) {
-            st = r2c_dev<T, N>(fb, R[3 + c], ctmp, R[c], s);        // F_c over u_c, no longer needed
+            st = r2c_dev<T, N>(fb, R[3 + c], ctmp, R[c], R[3 + c], s);     // through u_c, no longer needed
             if (st) return st;
-            F[c] = R[c];
+            F[c] = R[3 + c];
         }
     }
     st = flow_shell_sums(fb, F, N, nek, rnu, sizeof(T) == 8 ? DDNS_FP64 : DDNS_FP32_MIXED, dd + 3 * (size_t)nek, dd, s);
@@ -2108,15 +2059,16 @@ static int tune_impl(FlowBuffers& fb, const FlowConst& fc, hipStream_t s)
         if (!ky_cand_fits<T, N>(k)) continue;
         fb.ky_tc = ky_cand<T, N>(k);
         fb.ky_ms[k] = time_runs([&]() {
-            int r = launch_y<T, N>(true, true, fb.A, 6, fb, s, fc.nek);
-            return r ? r : launch_y<T, N>(false, false, fb.B, 3, fb, s, fc.nek);
+            const PlainRows rows = plain_rows<T, N>(fb);
+            const int r = launch_y<T, N>(true, true, fb.A, rows, 6, fb, fb.R * N, s, fc.nek);
+            return r ? r : launch_y<T, N>(false, false, fb.A, rows, 3, fb, fb.R * N, s, fc.nek);
         }, 3, s, e0, e1, &st);
         if (!st && (best == 0.f || fb.ky_ms[k] < best)) {
             best = fb.ky_ms[k];
             best_tc = fb.ky_tc;
         }
     }
-    if (!z_split()) {
+    {
         best = 0.f;
         for (int k = 0; k < 3 && !st; ++k) {
             if (!kz_cand_fits<T, N>(k)) continue;

@@ -47,7 +47,7 @@ __global__ void __launch_bounds__(1024) k_shell_partials(const void* __restrict_
     const C* f[3] = {(const C*)u0, (const C*)u1, (const C*)u2};
     const C* g[3] = {(const C*)F0, (const C*)F1, (const C*)F2};
     for (long long r = (long long)blockIdx.x * nw + w; r < rows; r += (long long)gridDim.x * nw) {
-        const int ky = (int)(r % N), kz = (int)(r / N);
+        const int ky = (int)(r / N), kz = (int)(r % N);      // neighbouring rows lie side by side
         const int kyw = spec_wave_index(ky, N), kzw = spec_wave_index(kz, N);
         const int kyz2 = kyw * kyw + kzw * kzw;
         for (int c0 = 0; c0 < M; c0 += 64) {
@@ -62,7 +62,7 @@ __global__ void __launch_bounds__(1024) k_shell_partials(const void* __restrict_
                 double k2 = (double)(kx * kx + kyz2);
                 if (k2 == 0.0) k2 = 1.e-5;
                 sh = (int)(sqrt(k2) + 0.5);
-                const size_t t = (size_t)r * M + kx;
+                const size_t t = spec_index<T>(N, kz, ky, kx);
 #pragma unroll
                 for (int q = 0; q < 3; ++q) {
                     const C a = f[q][t];
