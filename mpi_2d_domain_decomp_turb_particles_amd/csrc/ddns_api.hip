@@ -75,6 +75,8 @@ struct ddns_handle {
     // set (step parity), captured by the first step that runs them; graph_mode 0 launches
     // the kernels one by one (DDNS_GRAPH=0 in the environment at ddns_create)
     hipGraphExec_t gflow[4][2] = {};
+    // whole steps without droplets: one step, and STEP_CHUNK steps, without timing events
+    hipGraphExec_t gsteps[2] = {};
     int graph_mode = 1;
     int par = 0;                 // parity of the step in progress
     bool want_next = false;      // a further step follows in this call
@@ -423,6 +425,7 @@ static void destroy_impl(ddns_handle* h)
         for (int i = 0; i < FLOW_EVENTS; ++i) if (h->fev[q][i]) (void)hipEventDestroy(h->fev[q][i]);
         for (int i = 0; i < 4; ++i) if (h->flev[q][i]) (void)hipEventDestroy(h->flev[q][i]);
         for (int a = 0; a < 4; ++a) if (h->gflow[a][q]) (void)hipGraphExecDestroy(h->gflow[a][q]);
+        if (h->gsteps[q]) (void)hipGraphExecDestroy(h->gsteps[q]);
     }
     if (h->dstream) (void)hipStreamDestroy(h->dstream);
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -697,6 +700,35 @@ static double cell_width(const ddns_handle* h)
     return w;
 }
 
+// What body queues on s, captured into an instantiated graph; null when a call fails.
+template <typename F>
+static hipGraphExec_t capture_graph(hipStream_t s, F&& body)
+{
+    hipGraph_t g = nullptr;
+    hipGraphExec_t gx = nullptr;
+    int st = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess ? 0 : DDNS_ERR_HIP;
+    if (!st) {
+        st = body();
+        const hipError_t e = hipStreamEndCapture(s, &g);
+        if (!st && e != hipSuccess) st = DDNS_ERR_HIP;
+    }
+    if (!st && hipGraphInstantiate(&gx, g, nullptr, nullptr, 0) != hipSuccess) gx = nullptr;
+    if (g) (void)hipGraphDestroy(g);
+    if (!gx) (void)hipGetLastError();
+    return gx;
+}
+
+// graph mode off for the handle (a capture failed): the kernels run one by one from now on
+static void graphs_off(ddns_handle* h)
+{
+    h->graph_mode = 0;
+    for (int b = 0; b < 2; ++b) {
+        for (int a = 0; a < 4; ++a)
+            if (h->gflow[a][b]) { (void)hipGraphExecDestroy(h->gflow[a][b]); h->gflow[a][b] = nullptr; }
+        if (h->gsteps[b]) { (void)hipGraphExecDestroy(h->gsteps[b]); h->gsteps[b] = nullptr; }
+    }
+}
+
 // Part `part` of the flow step (FlowPart: the inverse stages, the forward stages and
 // update, or one of the two pieces of the latter) with the timing events of parity q.
 // In graph mode the part is captured once into a graph (its kernels and their events)
@@ -708,33 +740,48 @@ static int run_flow_half(ddns_handle* h, int part, int q)
     hipStream_t s = h->stream;
     if (h->graph_mode) {
         hipGraphExec_t& gx = h->gflow[part][q];
-        if (!gx) {
-            hipGraph_t g = nullptr;
-            int st = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess ? 0 : DDNS_ERR_HIP;
-            if (!st) {
-                st = flow_step(h->fb, h->fc, h->prec, part, s, h->fev[q], true);
-                const hipError_t e = hipStreamEndCapture(s, &g);
-                if (!st && e != hipSuccess) st = DDNS_ERR_HIP;
-            }
-            if (!st && hipGraphInstantiate(&gx, g, nullptr, nullptr, 0) != hipSuccess) {
-                gx = nullptr;
-                st = DDNS_ERR_HIP;
-            }
-            if (g) (void)hipGraphDestroy(g);
-            if (st) {
-                (void)hipGetLastError();
-                h->graph_mode = 0;
-                for (int a = 0; a < 4; ++a)
-                    for (int b = 0; b < 2; ++b)
-                        if (h->gflow[a][b]) { (void)hipGraphExecDestroy(h->gflow[a][b]); h->gflow[a][b] = nullptr; }
-            }
-        }
-        if (gx) {
+        if (!gx) gx = capture_graph(s, [&]() { return flow_step(h->fb, h->fc, h->prec, part, s, h->fev[q], true); });
+        if (!gx) graphs_off(h);
+        else {
             DDNS_HIP(hipGraphLaunch(gx, s));
             return 0;
         }
     }
     return flow_step(h->fb, h->fc, h->prec, part, s, h->fev[q]);
+}
+
+// Steps without droplets: nothing runs beside them and their events are not read, so a whole
+// step, and STEP_CHUNK steps, are one graph without event nodes (at 32^3 FP64 two graphs
+// with nine event nodes and four event records a step took 112 us, the kernels 45).
+constexpr int STEP_CHUNK = 8;
+
+static int run_flow_steps(ddns_handle* h, int nsteps)
+{
+    hipStream_t s = h->stream;
+    for (int left = nsteps; left > 0;) {
+        const int n = left >= STEP_CHUNK ? STEP_CHUNK : 1;
+        auto body = [&]() {
+            int st = 0;
+            for (int k = 0; k < n && !st; ++k) {
+                st = flow_step(h->fb, h->fc, h->prec, FLOW_INV, s, nullptr);
+                if (!st) st = flow_step(h->fb, h->fc, h->prec, FLOW_FWD, s, nullptr);
+            }
+            return st;
+        };
+        hipGraphExec_t& gx = h->gsteps[n == 1 ? 0 : 1];
+        if (h->graph_mode && !gx) {
+            gx = capture_graph(s, body);
+            if (!gx) graphs_off(h);
+        }
+        if (h->graph_mode) {
+            DDNS_HIP(hipGraphLaunch(gx, s));
+        } else {
+            const int st = body();
+            if (st) return st;
+        }
+        left -= n;
+    }
+    return 0;
 }
 
 // The first half of a step's flow (the curl and inverse z transforms when the state
@@ -1009,7 +1056,19 @@ extern "C" int ddns_step(ddns_handle* h, int nsteps)
     DDNS_HIP(hipEventRecord(h->ev[15], s));
     h->next_queued = false;
     const bool flow_only_graph = h->graph_mode && !(h->p.npart > 0 && h->n > 0);
-    for (int k = 0; k < nsteps; ++k) {
+    if (flow_only_graph && nsteps > 0) {
+        if (!h->a_valid) {
+            st = flow_prologue(h->fb, h->fc, h->prec, s);
+            if (st) return step_fail(h, st);
+            h->a_valid = true;
+        }
+        st = run_flow_steps(h, nsteps);
+        if (st) return step_fail(h, st);
+        h->phys_valid = true;
+        h->istep += nsteps;                                                   // turb.f90:492
+        for (int k = 0; k < nsteps; ++k) h->time += h->p.dt;                  // 693
+    }
+    for (int k = flow_only_graph ? nsteps : 0; k < nsteps; ++k) {
         h->istep += 1;                                                        // turb.f90:492
         // inverse y, x stage (the first half may have been queued during the last step)
         if (!h->next_queued) {
@@ -1033,26 +1092,22 @@ extern "C" int ddns_step(ddns_handle* h, int nsteps)
         st = queue_flow_rest(h, nullptr);
         if (st) return step_fail(h, st);
         const int q = h->par;
-        // A flow-only step replayed from graphs is not waited for: the call waits once, at
-        // its end, and reports its whole time as flow time, without the per-kernel split.
-        if (!flow_only_graph) {
-            DDNS_HIP(hipEventSynchronize(h->flev[q][3]));
-            const int pairs[6][2] = {{0, 1}, {1, 2}, {3, 4}, {4, 5}, {8, 6}, {6, 7}};
-            for (int i = 0; i < 6; ++i) {
-                float t;
-                DDNS_HIP(hipEventElapsedTime(&t, h->fev[q][pairs[i][0]], h->fev[q][pairs[i][1]]));
-                kms[i] += t;
-            }
-            float t1, t2;
-            DDNS_HIP(hipEventElapsedTime(&t1, h->flev[q][0], h->flev[q][1]));
-            DDNS_HIP(hipEventElapsedTime(&t2, h->flev[q][2], h->flev[q][3]));
-            flow_ms += t1 + t2;
+        DDNS_HIP(hipEventSynchronize(h->flev[q][3]));
+        const int pairs[6][2] = {{0, 1}, {1, 2}, {3, 4}, {4, 5}, {8, 6}, {6, 7}};
+        for (int i = 0; i < 6; ++i) {
+            float t;
+            DDNS_HIP(hipEventElapsedTime(&t, h->fev[q][pairs[i][0]], h->fev[q][pairs[i][1]]));
+            kms[i] += t;
         }
+        float t1, t2;
+        DDNS_HIP(hipEventElapsedTime(&t1, h->flev[q][0], h->flev[q][1]));
+        DDNS_HIP(hipEventElapsedTime(&t2, h->flev[q][2], h->flev[q][3]));
+        flow_ms += t1 + t2;
         h->par = 1 - q;
         h->time += h->p.dt;                                                   // 693
     }
     DDNS_HIP(hipEventRecord(h->ev[7], s));
-    DDNS_HIP(hipEventSynchronize(h->ev[7]));
+    DDNS_HIP(spin_wait(h->ev[7]));
     float tot = 0;
     DDNS_HIP(hipEventElapsedTime(&tot, h->ev[15], h->ev[7]));
     h->timing = ddns_timing{};
@@ -1316,24 +1371,10 @@ static int batch_flow_half(ddns_batch* b, int part)
     const int gi = part == FLOW_INV ? 0 : 1;
     if (b->graph_mode) {
         hipGraphExec_t& gx = b->gflow[gi];
+        if (!gx) gx = capture_graph(s, [&]() { return flow_step(b->fb, b->fc, b->prec, part, s, b->fev, true); });
         if (!gx) {
-            hipGraph_t g = nullptr;
-            int st = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess ? 0 : DDNS_ERR_HIP;
-            if (!st) {
-                st = flow_step(b->fb, b->fc, b->prec, part, s, b->fev, true);
-                const hipError_t e = hipStreamEndCapture(s, &g);
-                if (!st && e != hipSuccess) st = DDNS_ERR_HIP;
-            }
-            if (!st && hipGraphInstantiate(&gx, g, nullptr, nullptr, 0) != hipSuccess) {
-                gx = nullptr;
-                st = DDNS_ERR_HIP;
-            }
-            if (g) (void)hipGraphDestroy(g);
-            if (st) {
-                (void)hipGetLastError();
-                b->graph_mode = 0;
-                for (auto& x : b->gflow) if (x) { (void)hipGraphExecDestroy(x); x = nullptr; }
-            }
+            b->graph_mode = 0;
+            for (auto& x : b->gflow) if (x) { (void)hipGraphExecDestroy(x); x = nullptr; }
         }
         if (gx) {
             DDNS_HIP(hipGraphLaunch(gx, s));
