@@ -135,7 +135,8 @@ typedef struct ddns_collision_counts {
 
 /* Kernel-level timing of the last ddns_step call, from HIP events (milliseconds). */
 typedef struct ddns_timing {
-    double flow_ms;           /* spectral step: FFT stages + fused update              */
+    double flow_ms;           /* spectral step: FFT stages + fused update (with droplets:
+                                 the call's last step, times nsteps)                   */
     double interp_ms;         /* Lagrange gather                                       */
     double cells_ms;          /* cell binning (keys + sort)                            */
     double hdi_ms;            /* HI neighbour build + GMRES                            */

@@ -131,7 +131,10 @@ struct CollArgs {
     long long* pairs;      // DDNS_PAIR_REC per pair, see k_collide
     int pair_cap;
     int* mult;
-    const unsigned long long* dmax;   // bits of the largest |dmove| of this step, and of the largest radius
+    int* rlist;            // droplets with a removal-list entry, each once, in no order
+    int* nlist;
+    int* found;            // host memory: the search's counts, for the host's check
+    const unsigned long long* ext;    // Extents of this step
     int2* cand;            // pairs handed from the search to k_collide_pairs
     int cand_cap;
     int* ncand;
@@ -142,9 +145,8 @@ struct CollArgs {
     int* far;              // set when a droplet's reach exceeds the cell width (the walk would miss partners)
 };
 
-// The largest displacement length |dmove| of the step (out[0], when dmove is given) and
-// the largest droplet radius (out[1]), as the bits of non-negative doubles (whose order
-// is the numeric order): the exact pre-filter of the collision time window and the
+// The largest displacement length |dmove| of the step (when dmove is given) and the
+// largest droplet radius into out (raise_extents): the exact pre-filter of the collision time window and the
 // reach of the candidate walks.  The radius is the droplets' own, which coalescence
 // can grow beyond the largest size class.
 __global__ void __launch_bounds__(256) k_extent_max(const double* __restrict__ dmove, const double* __restrict__ rad,
@@ -172,12 +174,9 @@ __global__ void __launch_bounds__(256) k_extent_max(const double* __restrict__ d
         wm[1][threadIdx.x >> 6] = mr;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        m = fmax(fmax(wm[0][0], wm[0][1]), fmax(wm[0][2], wm[0][3]));
-        mr = fmax(fmax(wm[1][0], wm[1][1]), fmax(wm[1][2], wm[1][3]));
-        if (m > 0.0) atomicMax(out, (unsigned long long)__double_as_longlong(m));
-        if (mr > 0.0) atomicMax(out + 1, (unsigned long long)__double_as_longlong(mr));
-    }
+    if (threadIdx.x == 0)
+        raise_extents(out, fmax(fmax(wm[0][0], wm[0][1]), fmax(wm[0][2], wm[0][3])),
+                      fmax(fmax(wm[1][0], wm[1][1]), fmax(wm[1][2], wm[1][3])));
 }
 
 // The reference's work on one pair (ih1 = droplet ia, ih2 = droplet ib or one of its
@@ -339,7 +338,7 @@ __device__ __forceinline__ void collide_pair(const CollArgs& a, int ia, const do
     int i1, i2;
     findindex(a.radius, ns, ra, rb, &i1, &i2);
     atomicAdd(a.counts + 8 + (i1 - 1) + DDNS_MAXSET * (i2 - 1), 1);
-    atomicAdd(a.mult + ib, 1);
+    if (atomicAdd(a.mult + ib, 1) == 0) a.rlist[atomicAdd(a.nlist, 1)] = ib;
     const int slot = atomicAdd(a.counts + 256, 1);
     if (slot < a.pair_cap) {
         // the collist record (1555-1562) plus where the reference meets
@@ -399,7 +398,7 @@ __device__ __forceinline__ void stage_flush(const CollArgs& a, const CandStage& 
 }
 
 __device__ __forceinline__ void collide_search(const CollArgs& a, int t, int lane, int& tested, int& touching,
-                                               const CandStage& st)
+                                               const CandStage& st, double dmax, double rbig)
 {
     const int ia = a.sorted[t];
     const size_t C = (size_t)a.cap;
@@ -422,11 +421,9 @@ __device__ __forceinline__ void collide_search(const CollArgs& a, int t, int lan
     }
     // rcoll + dmove_a + dmove_b <= rcoll + dmove_a + dmax: a pair farther apart than the
     // right side cannot pass the collision time-window test
-    const double dmax = __longlong_as_double((long long)a.dmax[0]);
     // a partner farther than 10 (ra + rbig) is outside the statistics and farther than
     // ra + rbig + dmove_a + dmax outside the collision window, rbig the largest radius:
     // only the cells within the larger of the two are walked
-    const double rbig = __longlong_as_double((long long)a.dmax[1]);
     const double reach = fmax(10. * (ra + rbig), ra + rbig + dmove_a + dmax);
     const double reach2 = reach * reach * (1. + 1e-9);
     // the walk covers the neighbour cells only: a reach beyond the cell width is reported,
@@ -488,7 +485,8 @@ __global__ void __launch_bounds__(CT) k_collide(CollArgs a)
     if (lane == 0) *st.cnt = 0;
     __builtin_amdgcn_wave_barrier();
     int tested = 0, touching = 0;
-    if (t < a.n) collide_search(a, t, lane, tested, touching, st);
+    const double dmax = read_extent(a.ext, 0), rbig = read_extent(a.ext, 1);
+    if (t < a.n) collide_search(a, t, lane, tested, touching, st, dmax, rbig);
     // the whole wavefront is back together: hand on what its stage still holds
     {
         const int c = *st.cnt;
@@ -532,6 +530,7 @@ __global__ void __launch_bounds__(256) k_collide_pairs(CollArgs a)
         __syncthreads();
     }
     const int ncand = min(*a.ncand, a.cand_cap);
+    if (blockIdx.x == 0 && threadIdx.x < 3) a.found[threadIdx.x] = a.ncand[threadIdx.x];    // ncand, ncontact, far
     long long instat = 0;
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < ncand; r += gridDim.x * blockDim.x) {
         const int2 rec = a.cand[r];
@@ -570,7 +569,7 @@ __global__ void __launch_bounds__(256) k_collide_pairs(CollArgs a)
                          bins, nirbin);
             // ih1 counts once among the droplets that collided (1578-1583)
             if (ncollip1 != 0 && atomicExch(a.hit + ia, 1) == 0) {
-                atomicAdd(a.mult + ia, 1);
+                if (atomicAdd(a.mult + ia, 1) == 0) a.rlist[atomicAdd(a.nlist, 1)] = ia;
                 atomicAdd(a.counts + 257, 1);
             }
         }
@@ -602,14 +601,16 @@ struct OverArgs {
     const int *cell_start, *sorted;
     int n, cap;
     PairGeom g;
-    const unsigned long long* rbig;   // bits of the largest radius: a partner closer than ra + rbig can overlap
+    const unsigned long long* ext;    // the largest radius rbig: a partner closer than ra + rbig can overlap
     int* cnt;
-    int* total;
+    int* rlist;            // droplets with an overlapping partner, in no order
+    int* nlist;
 };
 
 __global__ void __launch_bounds__(CT) k_overlap(OverArgs a)
 {
     const int t = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const double rbig = read_extent(a.ext, 1);
     if (t >= a.n) return;
     const int ia = a.sorted[t];
     const PairGeom& g = a.g;
@@ -627,7 +628,7 @@ __global__ void __launch_bounds__(CT) k_overlap(OverArgs a)
     // a light kernel: the row-wise walk needs no LDS, which keeps its occupancy high;
     // only the cells within ra + rbig of the droplet can hold an overlapping partner,
     // and the visiting rules are replayed for the partners within that distance only
-    const double reach = ra + __longlong_as_double((long long)*a.rbig);
+    const double reach = ra + rbig;
     const double reach2 = reach * reach * (1. + 1e-9);
     for_each_candidate(a.cell_start, g.G, cc, a.pk, a.sorted, [&](int p, int kc, const double4& cb, int ib) {
         if (p == t) return;
@@ -648,7 +649,7 @@ __global__ void __launch_bounds__(CT) k_overlap(OverArgs a)
         if (dnij <= rcoll) ++cnt;
     }, reach_span(xs, cc, g.hc, reach));
     a.cnt[ia] = cnt;
-    if (cnt) atomicAdd(a.total, cnt);
+    if (cnt) a.rlist[atomicAdd(a.nlist, 1)] = ia;
 }
 
 // ------------------------------------------------------------------ host side
@@ -668,19 +669,31 @@ static PairGeom make_geom(const PartBuffers& pb, const PartConst& pc, double dst
     return g;
 }
 
-// Several device spans (4-byte multiples) cleared by one launch instead of one fill
-// per span: the collision statistics start from zero every step.
-struct ZeroSpans {
-    unsigned* p[8];
-    size_t words[8];
-    int n;
-};
-
 __global__ void __launch_bounds__(256) k_zero_spans(ZeroSpans z)
 {
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (int k = 0; k < z.n; ++k)
-        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < z.words[k]; i += stride) z.p[k][i] = 0u;
+    zero_spans(z, (size_t)blockIdx.x * blockDim.x + threadIdx.x, (size_t)gridDim.x * blockDim.x);
+}
+
+// What a step's searches start from: the statistics bins, the counters, the removal
+// multiplicities, the per-droplet hit marks, the extents, and the flags of the HI lists
+// ([0..7]), the search ([40..42]), the draws ([48]) and the removal lists ([50..52])
+int part_step_spans(PartBuffers& pb, const PartConst& pc, ZeroSpans& z)
+{
+    const size_t nb = (size_t)pc.nset * pc.nset * DDNS_NBIN;
+    if (!pb.hit) DDNS_HIP(hipMalloc(&pb.hit, (size_t)pb.cap * sizeof(int)));
+    z = ZeroSpans{};
+    auto add = [&](void* p, size_t bytes) { z.p[z.n] = (unsigned*)p; z.words[z.n] = bytes / 4; ++z.n; };
+    add(pb.nirbin, nb * sizeof(int));
+    add(pb.bins, 7 * nb * sizeof(double));
+    add(pb.counts, 512 * sizeof(int));
+    add(pb.tested, 4 * sizeof(long long));
+    add(pb.mult, (size_t)(pc.n + 1) * sizeof(int));
+    add(pb.hit, (size_t)pc.n * sizeof(int));
+    add(pb.flags, 8 * sizeof(int));
+    add(pb.flags + 40, 3 * sizeof(int));
+    add(pb.ext, EXT_WORDS * sizeof(unsigned long long));
+    add(pb.flags + 48, 5 * sizeof(int));
+    return 0;
 }
 
 // The collision search and the pair kernel behind it are queued by part_collide_search
@@ -693,6 +706,7 @@ int part_collide_finish(PartBuffers& pb, const PartConst& pc, hipStream_t s);
 
 int part_collide(PartBuffers& pb, const PartConst& pc, hipStream_t s)
 {
+    pb.step_cleared = false;             // no step's history or advance came before
     const int st = part_collide_search(pb, pc, s);
     return st ? st : part_collide_finish(pb, pc, s);
 }
@@ -709,8 +723,11 @@ static CollArgs collide_args(PartBuffers& pb, const PartConst& pc)
     a.g = make_geom(pb, pc, dstat, pc.hdi ? pc.d_hdi : pc.d_coll, pc.nx_coll);
     a.nirbin = pb.nirbin; a.bins = pb.bins; a.counts = pb.counts; a.tested = pb.tested;
     a.pairs = pb.pairs; a.pair_cap = pb.pair_cap; a.mult = pb.mult;
-    a.dmax = (unsigned long long*)(pb.flags + 32);
+    a.ext = pb.ext;
     a.hit = pb.hit;
+    a.rlist = pb.rlist;
+    a.nlist = pb.flags + 51;
+    a.found = pb.found_host;
     a.ncand = pb.flags + 40;
     a.ncontact = pb.flags + 41;
     a.far = pb.flags + 42;
@@ -724,20 +741,14 @@ static CollArgs collide_args(PartBuffers& pb, const PartConst& pc)
 int part_collide_search(PartBuffers& pb, const PartConst& pc, hipStream_t s)
 {
     const size_t nb = (size_t)pc.nset * pc.nset * DDNS_NBIN;
-    if (!pb.hit) DDNS_HIP(hipMalloc(&pb.hit, (size_t)pb.cap * sizeof(int)));
-    {
-        // bins, counters, the removal multiplicities, the per-droplet hit marks and the
-        // search's flags ([32..35] extents, [40..41] pair counts)
+    // a step has cleared these with its history step, and its advance has left the extents;
+    // a search run again (a longer list, wider cells) or on a given state starts here
+    const bool cleared = pb.step_cleared;
+    pb.step_cleared = false;
+    if (!cleared) {
         ZeroSpans z{};
-        auto add = [&](void* p, size_t bytes) { z.p[z.n] = (unsigned*)p; z.words[z.n] = bytes / 4; ++z.n; };
-        add(pb.nirbin, nb * sizeof(int));
-        add(pb.bins, 7 * nb * sizeof(double));
-        add(pb.counts, 512 * sizeof(int));
-        add(pb.tested, 4 * sizeof(long long));
-        add(pb.mult, (size_t)(pc.n + 1) * sizeof(int));
-        add(pb.hit, (size_t)pc.n * sizeof(int));
-        add(pb.flags + 32, 11 * sizeof(int));
-        add(pb.flags + 48, sizeof(int));               // relocation-draw overflow of this step
+        const int st = part_step_spans(pb, pc, z);
+        if (st) return st;
         hipLaunchKernelGGL(k_zero_spans, dim3(512), dim3(256), 0, s, z);
         DDNS_HIP(hipGetLastError());
     }
@@ -752,12 +763,12 @@ int part_collide_search(PartBuffers& pb, const PartConst& pc, hipStream_t s)
         DDNS_HIP(hipMalloc(&pb.contact, (size_t)pb.contact_cap * DDNS_CONTACT_REC * sizeof(double)));
     }
     CollArgs a = collide_args(pb, pc);
-    hipLaunchKernelGGL(k_extent_max, dim3(std::min(256, (pc.n + 255) / 256)), dim3(256), 0, s, (const double*)pb.dmove,
-                       (const double*)pb.rad, pc.n, pb.cap, (unsigned long long*)(pb.flags + 32));
+    if (!cleared)
+        hipLaunchKernelGGL(k_extent_max, dim3(std::min(256, (pc.n + 255) / 256)), dim3(256), 0, s, (const double*)pb.dmove,
+                           (const double*)pb.rad, pc.n, pb.cap, pb.ext);
     hipLaunchKernelGGL(k_collide, dim3((pc.n + CT - 1) / CT), dim3(CT), 0, s, a);
-    // handed-on pairs and pairs in contact, read by part_collide_finish
-    DDNS_HIP(hipMemcpyAsync(pb.found_host, a.ncand, 3 * sizeof(int), hipMemcpyDeviceToHost, s));
-    // the pair kernel, sized by the last step's count (a grid-stride loop covers more)
+    // the pair kernel (which also leaves the search's counts in found_host), sized by the last
+    // step's count (a grid-stride loop covers more)
     const int nwg = std::max(256, std::min(4096, (int)((pb.last_ncand + pb.last_ncand / 4 + 255) / 256)));
     if ((int)nb <= LB_MAXBIN)
         // bins in LDS: two work-groups per CU, each folding its sums into the global bins once
@@ -822,34 +833,36 @@ int part_read_contacts(const PartBuffers& pb, double* rec, int cap, int* n, hipS
     return 0;
 }
 
-// the largest radius into rbig[1] (relocation moves droplets, it does not resize them)
+// the largest radius into the second extents (relocation moves droplets, it does not resize them)
 static int overlap_setup(PartBuffers& pb, const PartConst& pc, hipStream_t s)
 {
-    unsigned long long* rbig = (unsigned long long*)(pb.flags + 36);
-    DDNS_HIP(hipMemsetAsync(rbig, 0, 2 * sizeof(unsigned long long), s));
+    unsigned long long* ext = pb.ext + EXT_WORDS;
+    DDNS_HIP(hipMemsetAsync(ext, 0, EXT_WORDS * sizeof(unsigned long long), s));
     hipLaunchKernelGGL(k_extent_max, dim3(std::min(256, (pc.n + 255) / 256)), dim3(256), 0, s, (const double*)nullptr,
-                       (const double*)pb.rad, pc.n, pb.cap, rbig);
+                       (const double*)pb.rad, pc.n, pb.cap, ext);
+    DDNS_HIP(hipGetLastError());
     return 0;
 }
 
-// One sweep's search: the overlap grid, and the per-droplet overlap counts in mult
-static int overlap_search(PartBuffers& pb, const PartConst& pc, hipStream_t s)
+// cells of the overlap search: two droplets in adjacent reference cells (the window of
+// partlib.f90:2091) are less than 2 dx apart per component, so cells of width >= 2 dx keep every
+// such pair within the 27-cell neighbourhood
+static double overlap_width(const PartConst& pc) { return std::max(2.0 * pc.radmax, 2.0 * pc.pi2 / pc.N); }   // 2063
+
+// One sweep's search on the current grid: the per-droplet overlap counts in mult, the droplets
+// that have any in rlist.  ext: the largest radius.
+static int overlap_search(PartBuffers& pb, const PartConst& pc, const unsigned long long* ext, hipStream_t s)
 {
-    const double d_overl = 2.0 * pc.radmax;                                // 2063
-    // two droplets in adjacent reference cells (the window of partlib.f90:2091) are
-    // less than 2 dx apart per component, so cells of width >= 2 dx keep every such
-    // pair within the 27-cell neighbourhood
-    int st = part_build_cells(pb, pc, std::max(d_overl, 2.0 * pc.pi2 / pc.N), s);
-    if (st) return st;
+    const double d_overl = 2.0 * pc.radmax;
     OverArgs a{};
     a.pos = pb.pos; a.rad = pb.rad; a.pk = pb.pk; a.cell_start = pb.cell_start; a.sorted = pb.sorted;
     a.n = pc.n; a.cap = pb.cap;
     const int jmax = 1 + (int)(d_overl * (double)pc.N / pc.pi2);
     a.g = make_geom(pb, pc, d_overl, d_overl, jmax);
-    a.rbig = (unsigned long long*)(pb.flags + 36) + 1;
+    a.ext = ext;
     a.cnt = pb.mult;
-    a.total = pb.flags + 1;
-    DDNS_HIP(hipMemsetAsync(pb.flags + 1, 0, sizeof(int), s));
+    a.rlist = pb.rlist;
+    a.nlist = pb.flags + 52;
     hipLaunchKernelGGL(k_overlap, dim3((pc.n + CT - 1) / CT), dim3(CT), 0, s, a);
     DDNS_HIP(hipGetLastError());
     return 0;
@@ -859,7 +872,10 @@ static int overlap_search(PartBuffers& pb, const PartConst& pc, hipStream_t s)
 static int overlap_loop(PartBuffers& pb, const PartConst& pc, int* sweeps, int* relocated, hipStream_t s)
 {
     for (int it = *sweeps; it < 10000; ++it) {
-        int st = overlap_search(pb, pc, s);
+        int st = part_build_cells(pb, pc, overlap_width(pc), s);
+        if (st) return st;
+        DDNS_HIP(hipMemsetAsync(pb.flags + 52, 0, sizeof(int), s));
+        st = overlap_search(pb, pc, pb.ext + EXT_WORDS, s);
         if (st) return st;
         int total = 0;
         st = relocate_by_mult(pb, pc, &total, s);
@@ -886,28 +902,28 @@ int part_overlap(PartBuffers& pb, const PartConst& pc, int* sweeps, int* relocat
 // case): the first sweep and its relocation are queued, the draws made for whatever the
 // count is (as in the collision step's relocation: none for a count of 0), and the count
 // is copied to pinned memory for the step's final wait.
-int part_overlap_queue(PartBuffers& pb, const PartConst& pc, hipStream_t s, double next_width)
+int part_overlap_queue(PartBuffers& pb, const PartConst& pc, hipStream_t s, double next_width, bool grown)
 {
     pb.overlap_queued = false;
     if (pc.n == 0) return 0;
-    int st = overlap_setup(pb, pc, s);
-    if (st) return st;
-    st = overlap_search(pb, pc, s);
-    if (st) return st;
-    // the next step's grid on the same positions, while the flow's z stage runs (a
-    // relocation by this sweep invalidates it with the sweep's own grid)
-    if (next_width > 0.0) {
-        st = part_build_cells(pb, pc, next_width, s);
-        if (st) return st;
+    // the largest radius: the advance has left it, unless coalescence has grown droplets since
+    const unsigned long long* ext = pb.ext;
+    int st = 0;
+    if (grown) {
+        st = overlap_setup(pb, pc, s);
+        ext = pb.ext + EXT_WORDS;
     }
+    // the sweep's grid and the next step's, on the same positions, in the same launches (a
+    // relocation by this sweep invalidates both)
+    if (!st) st = next_width > 0.0 ? part_build_two(pb, pc, overlap_width(pc), next_width, s)
+                                   : part_build_cells(pb, pc, overlap_width(pc), s);
+    if (!st) st = overlap_search(pb, pc, ext, s);
+    if (st) return st;
     const bool kept = pb.cells_valid, spare_kept = pb.spare.valid;
-    st = relocate_async(pb, pc, s);          // invalidates the grids: positions may move
+    st = relocate_list(pb, pc, 52, false, s);          // invalidates the grids: positions may move
     if (st) return st;
     pb.overlap_cells_kept = kept;
     pb.overlap_spare_kept = spare_kept;
-    if (!pb.counts_host)
-        DDNS_HIP(hipHostMalloc((void**)&pb.counts_host, (512 + 8 + 4) * sizeof(int), hipHostMallocDefault));
-    DDNS_HIP(hipMemcpyAsync(pb.counts_host + 521, pb.draw_off + pc.n, sizeof(int), hipMemcpyDeviceToHost, s));
     pb.overlap_queued = true;
     return 0;
 }
@@ -928,7 +944,9 @@ int part_overlap_finish(PartBuffers& pb, const PartConst& pc, int* sweeps, int* 
     }
     *sweeps = 1;
     *relocated = total;
-    return overlap_loop(pb, pc, sweeps, relocated, s);
+    // the further sweeps' radius bound (the second extents)
+    const int st = overlap_setup(pb, pc, s);
+    return st ? st : overlap_loop(pb, pc, sweeps, relocated, s);
 }
 
 // canonical pair list: sort the packed keys (min gid, max gid, type)
@@ -1169,13 +1187,24 @@ int part_read_counts(const PartBuffers& pb, const PartConst& pc, ddns_collision_
 // The counts of part_read_counts through pinned memory: queued on the stream, read once
 // the caller has waited for it (no extra round trip).  A relocation that ran out of draws
 // (flags[48]) is reported here as a capacity error.
+__global__ void __launch_bounds__(512) k_report(const int* __restrict__ counts, const long long* __restrict__ tested,
+                                                const int* __restrict__ flags, int* host)
+{
+    const int t = threadIdx.x;
+    host[t] = counts[t];
+    if (t < 4) ((long long*)(host + 512))[t] = tested[t];
+    if (t == 0) host[520] = flags[48];
+    if (t == 1) host[521] = flags[50];
+}
+
 int part_queue_counts(PartBuffers& pb, hipStream_t s)
 {
     if (!pb.counts_host)
         DDNS_HIP(hipHostMalloc((void**)&pb.counts_host, (512 + 8 + 4) * sizeof(int), hipHostMallocDefault));
-    DDNS_HIP(hipMemcpyAsync(pb.counts_host, pb.counts, 512 * sizeof(int), hipMemcpyDeviceToHost, s));
-    DDNS_HIP(hipMemcpyAsync(pb.counts_host + 512, pb.tested, 4 * sizeof(long long), hipMemcpyDeviceToHost, s));
-    DDNS_HIP(hipMemcpyAsync(pb.counts_host + 520, pb.flags + 48, sizeof(int), hipMemcpyDeviceToHost, s));
+    // one kernel writes them all to host memory (four copies took 4 us of the host's time each)
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(512), 0, s, (const int*)pb.counts, (const long long*)pb.tested,
+                       (const int*)pb.flags, pb.counts_host);
+    DDNS_HIP(hipGetLastError());
     return 0;
 }
 

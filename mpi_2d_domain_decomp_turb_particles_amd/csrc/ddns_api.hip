@@ -71,10 +71,15 @@ struct ddns_handle {
     // be queued before this step's times are read
     hipEvent_t flev[2][4] = {};
     hipEvent_t fev[2][FLOW_EVENTS] = {};
-    // the parts of the flow step (FlowPart) as instantiated graphs, one per part and event
-    // set (step parity), captured by the first step that runs them; graph_mode 0 launches
-    // the kernels one by one (DDNS_GRAPH=0 in the environment at ddns_create)
-    hipGraphExec_t gflow[4][2] = {};
+    // the parts of the flow step (FlowPart) as instantiated graphs, one per part with the
+    // timing events of either set (step parity) and one without, captured by the first step
+    // that runs them; graph_mode 0 launches the kernels one by one (DDNS_GRAPH=0 in the
+    // environment at ddns_create)
+    hipGraphExec_t gflow[4][3] = {};
+    // the step in progress, and the one after it, record their kernels' times: a call's last
+    // step does.  Nine event nodes a step kept the flow stream of a 64^3 run busier than its
+    // kernels did (112 against 60 us).
+    bool timed = true, timed_next = true;
     // whole steps without droplets: one step, and STEP_CHUNK steps, without timing events
     hipGraphExec_t gsteps[2] = {};
     int graph_mode = 1;
@@ -424,9 +429,10 @@ static void destroy_impl(ddns_handle* h)
     for (int q = 0; q < 2; ++q) {
         for (int i = 0; i < FLOW_EVENTS; ++i) if (h->fev[q][i]) (void)hipEventDestroy(h->fev[q][i]);
         for (int i = 0; i < 4; ++i) if (h->flev[q][i]) (void)hipEventDestroy(h->flev[q][i]);
-        for (int a = 0; a < 4; ++a) if (h->gflow[a][q]) (void)hipGraphExecDestroy(h->gflow[a][q]);
         if (h->gsteps[q]) (void)hipGraphExecDestroy(h->gsteps[q]);
     }
+    for (auto& part : h->gflow)
+        for (auto& g : part) if (g) (void)hipGraphExecDestroy(g);
     if (h->dstream) (void)hipStreamDestroy(h->dstream);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -722,32 +728,32 @@ static hipGraphExec_t capture_graph(hipStream_t s, F&& body)
 static void graphs_off(ddns_handle* h)
 {
     h->graph_mode = 0;
-    for (int b = 0; b < 2; ++b) {
-        for (int a = 0; a < 4; ++a)
-            if (h->gflow[a][b]) { (void)hipGraphExecDestroy(h->gflow[a][b]); h->gflow[a][b] = nullptr; }
-        if (h->gsteps[b]) { (void)hipGraphExecDestroy(h->gsteps[b]); h->gsteps[b] = nullptr; }
-    }
+    for (auto& part : h->gflow)
+        for (auto& g : part) if (g) { (void)hipGraphExecDestroy(g); g = nullptr; }
+    for (auto& g : h->gsteps) if (g) { (void)hipGraphExecDestroy(g); g = nullptr; }
 }
 
 // Part `part` of the flow step (FlowPart: the inverse stages, the forward stages and
-// update, or one of the two pieces of the latter) with the timing events of parity q.
+// update, or one of the two pieces of the latter), with the timing events of parity q when
+// timed.
 // In graph mode the part is captured once into a graph (its kernels and their events)
 // and replayed with one launch: the flow step takes no decision on the host and its
 // buffers never move, so every step replays the same graph.  A failed capture turns
 // graph mode off for the handle and the kernels run one by one.
-static int run_flow_half(ddns_handle* h, int part, int q)
+static int run_flow_half(ddns_handle* h, int part, int q, bool timed)
 {
     hipStream_t s = h->stream;
+    hipEvent_t* ev = timed ? h->fev[q] : nullptr;
     if (h->graph_mode) {
-        hipGraphExec_t& gx = h->gflow[part][q];
-        if (!gx) gx = capture_graph(s, [&]() { return flow_step(h->fb, h->fc, h->prec, part, s, h->fev[q], true); });
+        hipGraphExec_t& gx = h->gflow[part][timed ? q : 2];
+        if (!gx) gx = capture_graph(s, [&]() { return flow_step(h->fb, h->fc, h->prec, part, s, ev, true); });
         if (!gx) graphs_off(h);
         else {
             DDNS_HIP(hipGraphLaunch(gx, s));
             return 0;
         }
     }
-    return flow_step(h->fb, h->fc, h->prec, part, s, h->fev[q]);
+    return flow_step(h->fb, h->fc, h->prec, part, s, ev);
 }
 
 // Steps without droplets: nothing runs beside them and their events are not read, so a whole
@@ -787,16 +793,16 @@ static int run_flow_steps(ddns_handle* h, int nsteps)
 // The first half of a step's flow (the curl and inverse z transforms when the state
 // is new, turb.f90:506-526; the inverse y and x stages and the physical velocity,
 // 527-539) on the flow stream, with the event set of parity q.
-static int queue_flow_first(ddns_handle* h, int q)
+static int queue_flow_first(ddns_handle* h, int q, bool timed)
 {
     hipStream_t s = h->stream;
-    DDNS_HIP(hipEventRecord(h->flev[q][0], s));
+    if (timed) DDNS_HIP(hipEventRecord(h->flev[q][0], s));
     if (!h->a_valid) {
         const int st = flow_prologue(h->fb, h->fc, h->prec, s);
         if (st) return st;
         h->a_valid = true;
     }
-    const int st = run_flow_half(h, FLOW_INV, q);
+    const int st = run_flow_half(h, FLOW_INV, q, timed);
     if (st) return st;
     DDNS_HIP(hipEventRecord(h->flev[q][1], s));
     return 0;
@@ -818,15 +824,15 @@ static int queue_flow_rest(ddns_handle* h, hipEvent_t after)
     hipStream_t s = h->stream;
     const int q = h->par;
     if (after) DDNS_HIP(hipStreamWaitEvent(s, after, 0));
-    DDNS_HIP(hipEventRecord(h->flev[q][2], s));
+    if (h->timed) DDNS_HIP(hipEventRecord(h->flev[q][2], s));
     h->flow_rest_queued = true;
     if (h->z_gate && after) {
         h->z_pending = true;
-        return run_flow_half(h, FLOW_FWD_Y, q);
+        return run_flow_half(h, FLOW_FWD_Y, q, h->timed);
     }
-    int st = run_flow_half(h, FLOW_FWD, q);
+    int st = run_flow_half(h, FLOW_FWD, q, h->timed);
     if (st) return st;
-    DDNS_HIP(hipEventRecord(h->flev[q][3], s));
+    if (h->timed) DDNS_HIP(hipEventRecord(h->flev[q][3], s));
     return queue_flow_next(h, after);
 }
 
@@ -842,9 +848,9 @@ static int queue_flow_z(ddns_handle* h, hipEvent_t after)
     hipStream_t s = h->stream;
     const int q = h->par;
     if (after) DDNS_HIP(hipStreamWaitEvent(s, after, 0));
-    int st = run_flow_half(h, FLOW_FWD_Z, q);
+    int st = run_flow_half(h, FLOW_FWD_Z, q, h->timed);
     if (st) return st;
-    DDNS_HIP(hipEventRecord(h->flev[q][3], s));
+    if (h->timed) DDNS_HIP(hipEventRecord(h->flev[q][3], s));
     h->z_pending = false;
     return 0;
 }
@@ -855,7 +861,7 @@ static int queue_flow_z(ddns_handle* h, hipEvent_t after)
 static int queue_flow_next(ddns_handle* h, hipEvent_t after)
 {
     if (h->want_next && after) {
-        const int st = queue_flow_first(h, 1 - h->par);
+        const int st = queue_flow_first(h, 1 - h->par, h->timed_next);
         if (st) return st;
         h->next_queued = true;
     }
@@ -982,7 +988,7 @@ static int droplet_rest(ddns_handle* h, float* ms)
     // OVERLAP_DET (610): the first sweep is queued; its count is read with the step's
     // counts, and only a sweep that relocated droplets is followed by more
     if (h->p.nonoverlap) {
-        st = part_overlap_queue(h->pb, pc, s, cell_width(h));
+        st = part_overlap_queue(h->pb, pc, s, cell_width(h), h->istep >= h->p.nstep_grow);
         if (st) return st;
     }
     st = part_queue_counts(h->pb, s);
@@ -1071,8 +1077,10 @@ extern "C" int ddns_step(ddns_handle* h, int nsteps)
     for (int k = flow_only_graph ? nsteps : 0; k < nsteps; ++k) {
         h->istep += 1;                                                        // turb.f90:492
         // inverse y, x stage (the first half may have been queued during the last step)
+        h->timed = k + 1 == nsteps;
+        h->timed_next = k + 2 == nsteps;
         if (!h->next_queued) {
-            st = queue_flow_first(h, h->par);
+            st = queue_flow_first(h, h->par, h->timed);
             if (st) return step_fail(h, st);
         }
         h->next_queued = false;
@@ -1092,17 +1100,19 @@ extern "C" int ddns_step(ddns_handle* h, int nsteps)
         st = queue_flow_rest(h, nullptr);
         if (st) return step_fail(h, st);
         const int q = h->par;
-        DDNS_HIP(hipEventSynchronize(h->flev[q][3]));
-        const int pairs[6][2] = {{0, 1}, {1, 2}, {3, 4}, {4, 5}, {8, 6}, {6, 7}};
-        for (int i = 0; i < 6; ++i) {
-            float t;
-            DDNS_HIP(hipEventElapsedTime(&t, h->fev[q][pairs[i][0]], h->fev[q][pairs[i][1]]));
-            kms[i] += t;
+        if (h->timed) {                   // the call's last step stands for all of them
+            DDNS_HIP(spin_wait(h->flev[q][3]));
+            const int pairs[6][2] = {{0, 1}, {1, 2}, {3, 4}, {4, 5}, {8, 6}, {6, 7}};
+            for (int i = 0; i < 6; ++i) {
+                float t;
+                DDNS_HIP(hipEventElapsedTime(&t, h->fev[q][pairs[i][0]], h->fev[q][pairs[i][1]]));
+                kms[i] = (double)t * nsteps;
+            }
+            float t1, t2;
+            DDNS_HIP(hipEventElapsedTime(&t1, h->flev[q][0], h->flev[q][1]));
+            DDNS_HIP(hipEventElapsedTime(&t2, h->flev[q][2], h->flev[q][3]));
+            flow_ms = ((double)t1 + t2) * nsteps;
         }
-        float t1, t2;
-        DDNS_HIP(hipEventElapsedTime(&t1, h->flev[q][0], h->flev[q][1]));
-        DDNS_HIP(hipEventElapsedTime(&t2, h->flev[q][2], h->flev[q][3]));
-        flow_ms += t1 + t2;
         h->par = 1 - q;
         h->time += h->p.dt;                                                   // 693
     }

@@ -344,6 +344,7 @@ struct PartBuffers {
     int* sorted = nullptr;      // cap
     double4* pk = nullptr;      // cap: (x, y, z, radius) of sorted[p], refreshed with the cells
     int* cell_rank = nullptr;   // cap: place of a droplet among those of its cell (build scratch)
+    int* cell_rank2 = nullptr;  // cap: the same for a second grid built in the same launches
     bool cells_valid = false;   // the grid above was built on the current positions
     hipEvent_t sync_ev = nullptr;   // waits of the droplet block (wait_stream)
     double* gm_host = nullptr;      // pinned: GMRES's small-problem head [0..5] and the list flags [8..11]
@@ -392,7 +393,12 @@ struct PartBuffers {
     int cand_cap = 0;
     int last_ncand = 0;         // the last search's count: the size of the next pair-kernel grid
     int* hit = nullptr;         // cap: droplet already counted as ih1 of a collision
-    int* flags = nullptr;       // device flags / counters (64 ints)
+    // device flags / counters (64 ints): [0..7] HI lists and coalescence, [40..42] the collision search, [48] relocation draws ran out, [50] droplets relocated by an overlap
+    // sweep, [51], [52] length of rlist (collision step, overlap sweep)
+    int* flags = nullptr;
+    unsigned long long* ext = nullptr;   // Extents: the step's displacement and radius, then overlap_setup's radius
+    int* rlist = nullptr;       // cap: the droplets of a removal list, in no order
+    bool step_cleared = false;  // the step's statistics, counters and flags were cleared with its history step
     long long* tested = nullptr;
     int* nirbin = nullptr;
     double* bins = nullptr;     // 7 * nset*nset*NBIN
@@ -459,8 +465,47 @@ inline hipError_t wait_stream(PartBuffers& pb, hipStream_t s)
 void part_free(PartBuffers& pb);
 // with HI on, also writes the HI solve's x0 and w in cell order (after part_history_fvp)
 int part_interp(PartBuffers& pb, const PartConst& pc, const void* uphys, hipStream_t s);
+// the history step; also clears what the step's searches write (ZeroSpans)
 int part_history_fvp(PartBuffers& pb, const PartConst& pc, hipStream_t s);
 int part_build_cells(PartBuffers& pb, const PartConst& pc, double hmin, hipStream_t s);
+// The grid of width hmin as the current one and that of width other as the spare, both built in
+// the same launches when neither is valid (as two part_build_cells calls would leave them, in
+// the order other, hmin).
+int part_build_two(PartBuffers& pb, const PartConst& pc, double hmin, double other, hipStream_t s);
+// Several device spans (4-byte multiples) cleared by one launch instead of one fill per span.
+struct ZeroSpans {
+    unsigned* p[10];
+    size_t words[10];
+    int n;
+};
+int part_step_spans(PartBuffers& pb, const PartConst& pc, ZeroSpans& z);
+__device__ __forceinline__ void zero_spans(const ZeroSpans& z, size_t at, size_t stride)
+{
+    for (int k = 0; k < z.n; ++k)
+        for (size_t i = at; i < z.words[k]; i += stride) z.p[k][i] = 0u;
+}
+// The largest displacement and droplet radius, as the bits of non-negative doubles (whose order
+// is the numeric order), in EXT_SLOTS slots of two that work-group b raises at slot b mod
+// EXT_SLOTS; a reader takes the largest of all slots.  A single address served a million
+// droplets' work-groups in 70 us (each XCD's atomics go to memory one after the other).
+constexpr int EXT_SLOTS = 32, EXT_STRIDE = 16, EXT_WORDS = EXT_SLOTS * EXT_STRIDE;   // a slot per 128 bytes
+
+// by one lane of a work-group; most find the slot as large already
+__device__ __forceinline__ void raise_extents(unsigned long long* ext, double far, double big)
+{
+    unsigned long long* e = ext + (blockIdx.x % EXT_SLOTS) * EXT_STRIDE;
+    const unsigned long long f = (unsigned long long)__double_as_longlong(far), b = (unsigned long long)__double_as_longlong(big);
+    if (far > 0.0 && f > *(volatile unsigned long long*)e) atomicMax(e, f);
+    if (big > 0.0 && b > *(volatile unsigned long long*)(e + 1)) atomicMax(e + 1, b);
+}
+// by all lanes of a wavefront; which: 0 the displacement, 1 the radius
+__device__ __forceinline__ double read_extent(const unsigned long long* ext, int which)
+{
+    double m = __longlong_as_double((long long)ext[(threadIdx.x % EXT_SLOTS) * EXT_STRIDE + which]);
+#pragma unroll
+    for (int o = EXT_SLOTS / 2; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    return m;
+}
 int part_hdi(PartBuffers& pb, const PartConst& pc, int maxiter, double tol, int* iters, double* res, hipStream_t s);
 // The start of a solve (neighbour lists, right-hand side, first Krylov vector) queued on s.
 int part_hdi_begin(PartBuffers& pb, const PartConst& pc, int maxiter, double tol, hipStream_t s);
@@ -495,14 +540,16 @@ int part_queue_counts(PartBuffers& pb, hipStream_t s);
 int exclusive_scan(const int* in, int* out, int n, int* tmp, hipStream_t s, bool clear_in = false);
 int part_take_counts(const PartBuffers& pb, const PartConst& pc, ddns_collision_counts* cc);
 int part_update_and_wrap(PartBuffers& pb, const PartConst& pc, bool relocate, hipStream_t s);
+// The droplets of rlist (flags[nlist] of them) relocated by one launch, no host round trip.
 // wrap: the drawn positions get the PERIODIC wrap (the step's wrap follows its relocation)
-int relocate_async(PartBuffers& pb, const PartConst& pc, hipStream_t s, bool wrap = false);
+int relocate_list(PartBuffers& pb, const PartConst& pc, int nlist, bool wrap, hipStream_t s);
 int part_overlap(PartBuffers& pb, const PartConst& pc, int* sweeps, int* relocated, hipStream_t s);
 // the step's overlap sweep: the first sweep queued without a host wait; the rest, if it
 // relocated droplets, after the caller has waited for the stream
 // next_width > 0: the grid of that width (the next step's first) is built too, on the
 // positions the sweep saw, and kept if the sweep moves nothing
-int part_overlap_queue(PartBuffers& pb, const PartConst& pc, hipStream_t s, double next_width = 0.0);
+// grown: coalescence has changed radii since the advance
+int part_overlap_queue(PartBuffers& pb, const PartConst& pc, hipStream_t s, double next_width, bool grown);
 int part_overlap_finish(PartBuffers& pb, const PartConst& pc, int* sweeps, int* relocated, hipStream_t s);
 int part_read_counts(const PartBuffers& pb, const PartConst& pc, ddns_collision_counts* cc, hipStream_t s);
 int part_read_bins(const PartBuffers& pb, const PartConst& pc, int* nirbin, double* const bins[7], hipStream_t s);

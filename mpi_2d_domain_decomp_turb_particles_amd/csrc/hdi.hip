@@ -829,7 +829,7 @@ static int queue_lists(PartBuffers& pb, const PartConst& pc, hipStream_t s)
         DDNS_HIP(hipMalloc(&pb.nei_idx, (size_t)pb.ell_width * pb.cap * sizeof(int)));
         DDNS_HIP(hipMalloc(&pb.nei_m, (size_t)6 * pb.ell_width * pb.cap * sizeof(T)));
     }
-    DDNS_HIP(hipMemsetAsync(pb.flags, 0, 8 * sizeof(int), s));
+    // the flags are clear: from the step's start, or from lists_outcome when the lists are filled again
     hipLaunchKernelGGL((k_nei<T>), dim3((n + NT_NEI - 1) / NT_NEI), dim3(NT_NEI), 0, s, (const double4*)pb.pk, pb.cell_start,
                        n, pb.G, pb.hc, pc.pi2, pc.hdi_trunc, pb.ell_width, pb.nei_cnt, pb.nei_idx, (T*)pb.nei_m,
                        pb.flags);
@@ -846,6 +846,8 @@ static int lists_outcome(PartBuffers& pb, const int* f)
     if (f[0] & 1) { set_error("inside NEI_LIST_PRECOMP: overlapping is not allowed"); return DDNS_ERR_OVERLAP; }
     if (f[0] & 2) { set_error("more than 100 HI neighbours for a droplet"); return DDNS_ERR_NEIGHBOUR_OVERFLOW; }
     if (f[4] <= pb.ell_width) return 0;
+    DDNS_HIP(hipMemset(pb.flags, 0, 8 * sizeof(int)));
+    DDNS_HIP(hipStreamSynchronize(nullptr));
     if (pb.nei_idx) { (void)hipFree(pb.nei_idx); (void)hipFree(pb.nei_m); pb.nei_idx = nullptr; pb.nei_m = nullptr; }
     pb.ell_width = std::min(DDNS_MAXNEI, (f[4] + ELL_STEP - 1) / ELL_STEP * ELL_STEP);
     DDNS_HIP(hipMalloc(&pb.nei_idx, (size_t)pb.ell_width * pb.cap * sizeof(int)));

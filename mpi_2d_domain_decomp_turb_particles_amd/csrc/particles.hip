@@ -62,27 +62,42 @@ __device__ __forceinline__ void scan_load(const int* in, long long i0, int n, in
     }
 }
 
+// One or two independent scans (grid y)
+struct ScanArgs {
+    const int* in[2];
+    int* out[2];
+    int* bsum[2];
+    int* zin[2];
+    int n[2];
+};
+
 template <int E>
-__global__ void __launch_bounds__(SCAN_T) k_scan_tiles(const int* __restrict__ in, int* __restrict__ bsum, int n)
+__global__ void __launch_bounds__(SCAN_T) k_scan_tiles(ScanArgs a)
 {
     __shared__ int sh[SCAN_W];
+    const int k = blockIdx.y, n = a.n[k];
+    if ((long long)blockIdx.x * SCAN_T * E >= n) return;
     int v[E];
-    scan_load<E>(in, ((long long)blockIdx.x * SCAN_T + threadIdx.x) * E, n, v);
+    scan_load<E>(a.in[k], ((long long)blockIdx.x * SCAN_T + threadIdx.x) * E, n, v);
     int tot = 0;
 #pragma unroll
     for (int q = 0; q < E; ++q) tot += v[q];
     tot = block_sum_int(tot, sh);
-    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+    if (threadIdx.x == 0) a.bsum[k][blockIdx.x] = tot;
 }
 
 // in may alias out: a thread reads its ints before it writes them.  zin (= in, not
 // aliasing out, or null): the input is cleared as it is read.
 template <int E>
-__global__ void __launch_bounds__(SCAN_T) k_scan_apply(const int* in, int* out, const int* __restrict__ bsum, int n,
-                                                       int* zin)
+__global__ void __launch_bounds__(SCAN_T) k_scan_apply(ScanArgs a)
 {
     __shared__ int sh[SCAN_W];
     __shared__ int wsum[SCAN_W];
+    const int k = blockIdx.y, n = a.n[k];
+    if (blockIdx.x > 0 && (long long)blockIdx.x * SCAN_T * E >= n) return;
+    const int* in = a.in[k];
+    const int* bsum = a.bsum[k];
+    int *out = a.out[k], *zin = a.zin[k];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     int pre = 0;
     for (int b = tid; b < (int)blockIdx.x; b += SCAN_T) pre += bsum[b];
@@ -127,15 +142,23 @@ __global__ void __launch_bounds__(SCAN_T) k_scan_apply(const int* in, int* out, 
         for (int q = 0; q < E; ++q)
             if (i0 + q < n) out[i0 + q] = r[q];
     }
-    if (blockIdx.x == gridDim.x - 1 && tid == SCAN_T - 1) out[n] = run;
+    // the last tile's last thread holds the total
+    if (tid == SCAN_T - 1 && ((long long)blockIdx.x + 1) * SCAN_T * E >= n) out[n] = run;
 }
 
-template <int E>
-static int scan_launch(const int* in, int* out, int n, int* tmp, int* zin, hipStream_t s)
+// k scans (1 or 2) in two launches
+static int scan_launch(const ScanArgs& a, int k, hipStream_t s)
 {
-    const unsigned nb = (unsigned)(((long long)n + (long long)E * SCAN_T - 1) / ((long long)E * SCAN_T));
-    hipLaunchKernelGGL(k_scan_tiles<E>, dim3(nb), dim3(SCAN_T), 0, s, in, tmp, n);
-    hipLaunchKernelGGL(k_scan_apply<E>, dim3(nb), dim3(SCAN_T), 0, s, in, out, (const int*)tmp, n, zin);
+    const long long n = std::max(a.n[0], k > 1 ? a.n[1] : 0);
+    const int E = n <= 16LL * SCAN_T * 1024 ? 16 : 32;
+    const unsigned nb = (unsigned)std::max<long long>(1, (n + (long long)E * SCAN_T - 1) / ((long long)E * SCAN_T));
+    if (E == 16) {
+        hipLaunchKernelGGL(k_scan_tiles<16>, dim3(nb, k), dim3(SCAN_T), 0, s, a);
+        hipLaunchKernelGGL(k_scan_apply<16>, dim3(nb, k), dim3(SCAN_T), 0, s, a);
+    } else {
+        hipLaunchKernelGGL(k_scan_tiles<32>, dim3(nb, k), dim3(SCAN_T), 0, s, a);
+        hipLaunchKernelGGL(k_scan_apply<32>, dim3(nb, k), dim3(SCAN_T), 0, s, a);
+    }
     DDNS_HIP(hipGetLastError());
     return 0;
 }
@@ -145,14 +168,13 @@ static int scan_launch(const int* in, int* out, int n, int* tmp, int* zin, hipSt
 // in[0..n-1] is left zero.
 int exclusive_scan(const int* in, int* out, int n, int* tmp, hipStream_t s, bool clear_in)
 {
-    int* zin = clear_in ? const_cast<int*>(in) : nullptr;
-    if (n <= 0) {
-        hipLaunchKernelGGL(k_scan_apply<4>, dim3(1), dim3(SCAN_T), 0, s, in, out, (const int*)tmp, 0, zin);
-        DDNS_HIP(hipGetLastError());
-        return 0;
-    }
-    if ((long long)n <= 16LL * SCAN_T * 1024) return scan_launch<16>(in, out, n, tmp, zin, s);
-    return scan_launch<32>(in, out, n, tmp, zin, s);
+    ScanArgs a{};
+    a.in[0] = in;
+    a.out[0] = out;
+    a.bsum[0] = tmp;
+    a.zin[0] = clear_in ? const_cast<int*>(in) : nullptr;
+    a.n[0] = std::max(0, n);
+    return scan_launch(a, 1, s);
 }
 
 // ints of scratch exclusive_scan needs for n elements
@@ -186,6 +208,7 @@ int part_alloc(PartBuffers& pb, int cap, int nset, int G)
     DDNS_HIP(hipMemset(pb.vp, 0, 3 * c * 8));
     DDNS_HIP(hipMalloc(&pb.cell_of, c * sizeof(int)));
     DDNS_HIP(hipMalloc(&pb.cell_rank, c * sizeof(int)));
+    DDNS_HIP(hipMalloc(&pb.rlist, c * sizeof(int)));
     DDNS_HIP(hipMalloc(&pb.sorted, c * sizeof(int)));
     DDNS_HIP(hipMalloc(&pb.pk, c * sizeof(double4)));
     DDNS_HIP(hipMalloc(&pb.mult, (c + 1) * sizeof(int)));
@@ -193,6 +216,8 @@ int part_alloc(PartBuffers& pb, int cap, int nset, int G)
     DDNS_HIP(hipMalloc(&pb.nei_cnt, (c + 1) * sizeof(int)));
     DDNS_HIP(hipMalloc(&pb.flags, 64 * sizeof(int)));
     DDNS_HIP(hipMemset(pb.flags, 0, 64 * sizeof(int)));
+    DDNS_HIP(hipMalloc(&pb.ext, 2 * EXT_WORDS * sizeof(unsigned long long)));
+    DDNS_HIP(hipMemset(pb.ext, 0, 2 * EXT_WORDS * sizeof(unsigned long long)));
     DDNS_HIP(hipMalloc(&pb.tested, 4 * sizeof(long long)));
     const size_t nb = (size_t)nset * nset * DDNS_NBIN;
     DDNS_HIP(hipMalloc(&pb.nirbin, nb * sizeof(int)));
@@ -217,7 +242,8 @@ void part_free(PartBuffers& pb)
                   pb.cell_count, pb.cell_start, pb.cell_of, pb.cell_rank, pb.sorted, pb.pk, pb.scan_tmp,
                   pb.nei_cnt, pb.nei_idx, pb.nei_m, pb.gm_Q, pb.gm_v, pb.gm_x0, pb.gm_b, pb.gm_w,
                   pb.gm_red, pb.gm_small, pb.mult, pb.cand, pb.hit, pb.flags, pb.tested, pb.nirbin, pb.bins, pb.counts,
-                  pb.pairs, pb.contact, pb.draws, pb.draw_off, pb.rng_state, pb.red, pb.stage};
+                  pb.pairs, pb.contact, pb.draws, pb.draw_off, pb.rng_state, pb.red, pb.stage, pb.cell_rank2,
+                  pb.rlist, pb.ext};
     for (void* p : ps) if (p) (void)hipFree(p);
     void* sp[] = {pb.spare.cell_count, pb.spare.cell_start, pb.spare.cell_of, pb.spare.sorted, pb.spare.pk};
     for (void* p : sp) if (p) (void)hipFree(p);
@@ -517,11 +543,13 @@ int part_interp(PartBuffers& pb, const PartConst& pc, const void* uphys, hipStre
 }
 
 // ------------------------------------------------------------------ histories
-// PART_HISTORY_FVP, partlib.f90:562-592
+// PART_HISTORY_FVP, partlib.f90:562-592, and the clearing of what this step's searches write
+// (a launch of its own and four fills before: a small run's step is bound by its launches)
 __global__ void k_hist_fvp(double* vel, const double* rad, double* fvp, int n, int cap, int newp, double Sv, int v0,
-                           int v1, int v2)
+                           int v1, int v2, ZeroSpans z)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    zero_spans(z, i, (size_t)gridDim.x * blockDim.x);
     if (i >= n) return;
     if (newp) {
         const double a = rad[i];
@@ -539,10 +567,15 @@ __global__ void k_hist_fvp(double* vel, const double* rad, double* fvp, int n, i
 
 int part_history_fvp(PartBuffers& pb, const PartConst& pc, hipStream_t s)
 {
+    pb.step_cleared = false;
     if (pc.n == 0) return 0;
-    hipLaunchKernelGGL(k_hist_fvp, dim3(nblk(pc.n)), dim3(PT), 0, s, pb.vel, pb.rad, pb.fvp, pc.n, pb.cap,
-                       pc.new_particle, pc.Sv_const, pb.vcol(0), pb.vcol(1), pb.vcol(2));
+    ZeroSpans z{};
+    const int st = part_step_spans(pb, pc, z);
+    if (st) return st;
+    hipLaunchKernelGGL(k_hist_fvp, dim3(std::max(64u, nblk(pc.n))), dim3(PT), 0, s, pb.vel, pb.rad, pb.fvp, pc.n, pb.cap,
+                       pc.new_particle, pc.Sv_const, pb.vcol(0), pb.vcol(1), pb.vcol(2), z);
     DDNS_HIP(hipGetLastError());
+    pb.step_cleared = true;
     pb.v0_stale = false;
     return 0;
 }
@@ -550,15 +583,19 @@ int part_history_fvp(PartBuffers& pb, const PartConst& pc, hipStream_t s)
 // ------------------------------------------------------------------ advance
 // PART_HISTORY_FDP (599-625) + PART_ADVANCE (629-726): implicit Adams-Moulton
 // velocity with Adams-Bashforth fluid history, Stokes or Schiller-Naumann drag,
-// gravity along +x, displacement dmove.
-__global__ void k_advance(double* vel, const double* rad, double* fvp, double* fdp, const double* vp,
+// gravity along +x, displacement dmove.  It also raises the step's largest displacement and
+// droplet radius (ext, cleared at the step's start), the reach of the collision search, which a
+// separate reduction over the displacements read again.
+__global__ void __launch_bounds__(PT) k_advance(double* vel, const double* rad, double* fvp, double* fdp, const double* vp,
                           const double* pert, double* dmove, int n, int cap, int newp, int hdi,
-                          int ndrag, double dt, double rnu, double Sv, double tau2, int4 vc, int4 dc)
+                          int ndrag, double dt, double rnu, double Sv, double tau2, int4 vc, int4 dc,
+                          unsigned long long* ext)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    double far = 0.0, big = 0.0;
+    if (i < n) {
     const size_t C = (size_t)cap;
-    double f0[3];
+    double f0[3], d2[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         f0[c] = hdi ? vp[c * C + i] + pert[3 * (size_t)i + c] : vp[c * C + i];
@@ -587,8 +624,32 @@ __global__ void k_advance(double* vel, const double* rad, double* fvp, double* f
         const double tempd = 55.0 * f0[c] - 59.0 * fdp[(dc.y + c) * C + i] + 37.0 * fdp[(dc.z + c) * C + i] -
                              9.0 * fdp[(dc.w + c) * C + i];
         const double vnew = (vel[c * C + i] + dt * unitv * wp_vel / taup * FSN - dtau * tempv + dtau * tempd) / (1.0 + 9.0 * dtau);
+        const double dm = dtc * (9.0 * vnew + 19.0 * fv0 - 5.0 * fv1 + fv2);
         vel[c * C + i] = vnew;
-        dmove[c * C + i] = dtc * (9.0 * vnew + 19.0 * fv0 - 5.0 * fv1 + fv2);
+        dmove[c * C + i] = dm;
+        d2[c] = dm * dm;
+    }
+    // rounded up: the bound may be a little larger than the displacement the search computes
+    far = sqrt(d2[0] + d2[1] + d2[2]) * (1.0 + 1e-14);
+    big = a;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        far = fmax(far, __shfl_xor(far, o, 64));
+        big = fmax(big, __shfl_xor(big, o, 64));
+    }
+    __shared__ double wm[2][PT / 64];
+    if ((threadIdx.x & 63) == 0) {
+        wm[0][threadIdx.x >> 6] = far;
+        wm[1][threadIdx.x >> 6] = big;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < PT / 64; ++w) {
+            far = fmax(far, wm[0][w]);
+            big = fmax(big, wm[1][w]);
+        }
+        raise_extents(ext, far, big);
     }
 }
 
@@ -599,7 +660,7 @@ int part_advance(PartBuffers& pb, const PartConst& pc, hipStream_t s)
     const int4 dc = make_int4(pb.dcol(0), pb.dcol(1), pb.dcol(2), pb.dcol(3));
     hipLaunchKernelGGL(k_advance, dim3(nblk(pc.n)), dim3(PT), 0, s, pb.vel, pb.rad, pb.fvp, pb.fdp, pb.vp, pb.pert,
                        pb.dmove, pc.n, pb.cap, pc.new_particle, pc.hdi, pc.ndrag, pc.dt, pc.rnu, pc.Sv_const, pc.tau2,
-                       vc, dc);
+                       vc, dc, pb.ext);
     DDNS_HIP(hipGetLastError());
     pb.d0_stale = false;
     return 0;
@@ -693,7 +754,7 @@ __global__ void k_draws(int* st, double* draws, const int* total, int cap, int* 
 // A droplet that appears m times in the sorted removal list consumes 3m draws at
 // offset off; the last triple is the position it keeps (RELOCATE, 1994-2006).
 __global__ void k_apply_reloc(double* pos, const int* mult, const int* off, const double* draws, int n, int cap, double pi2,
-                              long long draw_cap, int wrap)
+                              long long draw_cap)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -701,9 +762,7 @@ __global__ void k_apply_reloc(double* pos, const int* mult, const int* off, cons
     if (m <= 0) return;
     if (3 * ((long long)off[i] + m) > draw_cap) return;      // cut short by k_draws (capacity error)
     const double* d = draws + 3 * (size_t)(off[i] + m - 1);
-    double y[3] = {d[0] * pi2, d[1] * pi2 + 0.0 * pi2, d[2] * pi2 + 0.0 * pi2};
-    if (wrap)
-        for (int c = 0; c < 3; ++c) y[c] = wrap_periodic(y[c], pi2);
+    const double y[3] = {d[0] * pi2, d[1] * pi2 + 0.0 * pi2, d[2] * pi2 + 0.0 * pi2};
     pos[i] = y[0];
     pos[(size_t)cap + i] = y[1];
     pos[2 * (size_t)cap + i] = y[2];
@@ -742,20 +801,128 @@ int relocate_by_mult(PartBuffers& pb, const PartConst& pc, int* total_host, hipS
     hipLaunchKernelGGL(k_draws, dim3(1), dim3(1), 0, s, pb.rng_state, pb.draws, pb.draw_off + pc.n, pb.draw_cap,
                        pb.flags + 48);
     hipLaunchKernelGGL(k_apply_reloc, dim3(nblk(pc.n)), dim3(PT), 0, s, pb.pos, pb.mult, pb.draw_off, pb.draws,
-                       pc.n, pb.cap, pc.pi2, (long long)pb.draw_cap, 0);
+                       pc.n, pb.cap, pc.pi2, (long long)pb.draw_cap);
     DDNS_HIP(hipGetLastError());
     return 0;
 }
 
-// The relocation of the collision step (RELOCATE, partlib.f90:1984-2012) without a host
-// round trip: the draws are made for whatever the removal list holds, into a buffer of
-// three draws per droplet slot (each droplet relocated once; a step whose removal list
-// needs more sets the capacity flag flags[48], which the step reports as an error).
-// Droplets with no removal entry keep their positions.
-int relocate_async(PartBuffers& pb, const PartConst& pc, hipStream_t s, bool wrap)
+// The relocation of a step (RELOCATE, partlib.f90:1984-2012) by one work-group and without a
+// host round trip: the droplets that the search listed (in any order) are sorted by index,
+// which is the order of the reference's removal list, each takes 3 mult draws of the stream
+// and keeps the last three.  A step relocates a handful of droplets: a scan of all
+// multiplicities, the draws and the update as four launches took 40 us at 1M droplets.  A list
+// longer than the sort's room is walked in index order over all droplets instead.  At most
+// draw_cap draws are made: a list that needs more sets *err (a capacity error) and is cut short.
+constexpr int RL_T = 1024, RL_MAX = 4096;
+
+struct RelocArgs {
+    double* pos;
+    const int* mult;
+    const int* list;
+    const int* nlist;
+    int* off;               // cap + 1: scratch of the long list
+    double* draws;
+    int* rng;
+    int* total;             // list entries with their multiplicity
+    int* err;
+    int n, cap, draw_cap, wrap;
+    double pi2;
+};
+
+__device__ __forceinline__ void reloc_apply(const RelocArgs& a, int i, int off, int m)
 {
-    int st = exclusive_scan(pb.mult, pb.draw_off, pc.n, (int*)pb.scan_tmp, s);
-    if (st) return st;
+    if (3 * ((long long)off + m) > a.draw_cap) return;
+    const double* d = a.draws + 3 * (size_t)(off + m - 1);
+    double y[3] = {d[0] * a.pi2, d[1] * a.pi2 + 0.0 * a.pi2, d[2] * a.pi2 + 0.0 * a.pi2};
+    for (int c = 0; c < 3; ++c) a.pos[(size_t)c * a.cap + i] = a.wrap ? wrap_periodic(y[c], a.pi2) : y[c];
+}
+
+__device__ __forceinline__ void reloc_draws(const RelocArgs& a, int total, int* iv)
+{
+    if (threadIdx.x == 0) {
+        int* st = a.rng;
+        int idum = st[0], iy = st[1], idum2 = st[2];
+        for (int q = 0; q < 32; ++q) iv[q] = st[3 + q];
+        long long nd = 3LL * total;
+        if (nd > a.draw_cap) {
+            atomicOr(a.err, 1);
+            nd = a.draw_cap - a.draw_cap % 3;
+        }
+        for (long long q = 0; q < nd; ++q) a.draws[q] = dev_ranff2(&idum, iv, &iy, &idum2);
+        st[0] = idum; st[1] = iy; st[2] = idum2;
+        for (int q = 0; q < 32; ++q) st[3 + q] = iv[q];
+    }
+    __syncthreads();
+}
+
+__global__ void __launch_bounds__(RL_T) k_relocate(RelocArgs a)
+{
+    __shared__ int key[RL_MAX], off[RL_MAX], iv[32], wsum[RL_T / 64], run;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int m = *a.nlist;
+    if (m == 0) {
+        if (tid == 0) *a.total = 0;
+        return;
+    }
+    // exclusive sums of x over the work-group's threads, run carried from call to call
+    auto scan = [&](int x) {
+        int incl = x;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        if (lane == 63) wsum[wv] = incl;
+        __syncthreads();
+        int before = run;
+        for (int w = 0; w < wv; ++w) before += wsum[w];
+        __syncthreads();
+        if (tid == RL_T - 1) run = before + incl;
+        __syncthreads();
+        return before + incl - x;
+    };
+    if (tid == 0) run = 0;
+    if (m <= RL_MAX) {
+        int P = 1;
+        while (P < m) P <<= 1;
+        for (int i = tid; i < P; i += RL_T) key[i] = i < m ? a.list[i] : 0x7fffffff;
+        __syncthreads();
+        for (int k = 2; k <= P; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                for (int i = tid; i < P; i += RL_T) {
+                    const int l = i ^ j;
+                    if (l > i) {
+                        const int x = key[i], y = key[l];
+                        if ((x > y) == ((i & k) == 0)) { key[i] = y; key[l] = x; }
+                    }
+                }
+                __syncthreads();
+            }
+        for (int b = 0; b < m; b += RL_T) {
+            const int e = scan(b + tid < m ? a.mult[key[b + tid]] : 0);
+            if (b + tid < m) off[b + tid] = e;
+        }
+        const int total = run;
+        reloc_draws(a, total, iv);
+        for (int e = tid; e < m; e += RL_T) reloc_apply(a, key[e], off[e], a.mult[key[e]]);
+        if (tid == 0) *a.total = total;
+        return;
+    }
+    __syncthreads();
+    for (int b = 0; b < a.n; b += RL_T) {
+        const int i = b + tid;
+        const int e = scan(i < a.n ? a.mult[i] : 0);
+        if (i < a.n) a.off[i] = e;
+    }
+    const int total = run;
+    reloc_draws(a, total, iv);
+    for (int i = tid; i < a.n; i += RL_T)
+        if (a.mult[i] > 0) reloc_apply(a, i, a.off[i], a.mult[i]);
+    if (tid == 0) *a.total = total;
+}
+
+int relocate_list(PartBuffers& pb, const PartConst& pc, int nlist, bool wrap, hipStream_t s)
+{
     invalidate_cells(pb);                 // relocated droplets move
     const int need = 3 * std::max(pb.cap, 1 << 16);
     if (pb.draw_cap < need) {
@@ -763,10 +930,11 @@ int relocate_async(PartBuffers& pb, const PartConst& pc, hipStream_t s, bool wra
         pb.draw_cap = need;
         DDNS_HIP(hipMalloc(&pb.draws, (size_t)pb.draw_cap * sizeof(double)));
     }
-    hipLaunchKernelGGL(k_draws, dim3(1), dim3(1), 0, s, pb.rng_state, pb.draws, pb.draw_off + pc.n, pb.draw_cap,
-                       pb.flags + 48);
-    hipLaunchKernelGGL(k_apply_reloc, dim3(nblk(pc.n)), dim3(PT), 0, s, pb.pos, pb.mult, pb.draw_off, pb.draws,
-                       pc.n, pb.cap, pc.pi2, (long long)pb.draw_cap, wrap ? 1 : 0);
+    RelocArgs a{};
+    a.pos = pb.pos; a.mult = pb.mult; a.list = pb.rlist; a.nlist = pb.flags + nlist; a.off = pb.draw_off;
+    a.draws = pb.draws; a.rng = pb.rng_state; a.total = pb.flags + 50; a.err = pb.flags + 48;
+    a.n = pc.n; a.cap = pb.cap; a.draw_cap = pb.draw_cap; a.wrap = wrap ? 1 : 0; a.pi2 = pc.pi2;
+    hipLaunchKernelGGL(k_relocate, dim3(1), dim3(RL_T), 0, s, a);
     DDNS_HIP(hipGetLastError());
     return 0;
 }
@@ -782,7 +950,7 @@ int part_update_and_wrap(PartBuffers& pb, const PartConst& pc, bool relocate, hi
     pb.v0_stale = true;
     pb.d0_stale = true;
     if (relocate) {
-        int st = relocate_async(pb, pc, s, true);
+        int st = relocate_list(pb, pc, 51, true, s);
         if (st) return st;
     }
     return 0;
@@ -792,12 +960,22 @@ int part_update_and_wrap(PartBuffers& pb, const PartConst& pc, bool relocate, hi
 // A periodic grid of G^3 cells of width hc = 2pi/G >= the largest pair distance the
 // caller needs, so a 27-cell neighbourhood holds every candidate.  Counting sort by
 // cell, then each cell's slice is ordered by slot number (deterministic).
+// One or two grids over the same positions (grid y): every kernel of a build covers both.
+struct GridArgs {
+    int *cell_of[2], *rank[2], *cnt[2], *start[2], *sorted[2];
+    double4* pk[2];
+    int G[2], ncell[2];
+    double hc[2];
+};
+
 // cell of droplet i and its place among the droplets of that cell (the order in which
 // the atomics were served; k_cell_order makes the final order deterministic)
-__global__ void k_cell_key(const double* pos, int* cell_of, int* rank, int* cnt, int n, int cap, int G, double hc)
+__global__ void k_cell_key(const double* pos, GridArgs a, int n, int cap)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
     if (i >= n) return;
+    const int G = a.G[k];
+    const double hc = a.hc[k];
     int c3[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -806,31 +984,31 @@ __global__ void k_cell_key(const double* pos, int* cell_of, int* rank, int* cnt,
         c3[c] = q;
     }
     const int cell = cell_code(c3[0], c3[1], c3[2]);
-    cell_of[i] = cell;
-    rank[i] = atomicAdd(cnt + cell, 1);
+    a.cell_of[k][i] = cell;
+    a.rank[k][i] = atomicAdd(a.cnt[k] + cell, 1);
 }
 
 // Droplet i (read in slot order, so the reads coalesce) takes the next free place of
 // its cell and writes its index and its packed (x, y, z, radius) record there: the
 // pair searches then read each candidate cell as one contiguous run.
-__global__ void k_cell_fill(const int* __restrict__ cell_of, const int* __restrict__ rank, const int* __restrict__ start,
-                            int* __restrict__ sorted, const double* __restrict__ pos, const double* __restrict__ rad,
-                            double4* __restrict__ pk, int n, int cap)
+__global__ void k_cell_fill(GridArgs a, const double* __restrict__ pos, const double* __restrict__ rad, int n, int cap)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
     if (i >= n) return;
-    const int c = cell_of[i];
-    const int p = start[c] + rank[i];
-    sorted[p] = i;
-    pk[p] = make_double4(pos[i], pos[(size_t)cap + i], pos[2 * (size_t)cap + i], rad[i]);
+    const int p = a.start[k][a.cell_of[k][i]] + a.rank[k][i];
+    a.sorted[k][p] = i;
+    a.pk[k][p] = make_double4(pos[i], pos[(size_t)cap + i], pos[2 * (size_t)cap + i], rad[i]);
 }
 
 // the order inside a cell is by droplet index, so it does not depend on the order in
 // which the fill's atomics were served; the packed records move with their indices
-__global__ void k_cell_order(const int* __restrict__ start, int* __restrict__ sorted, double4* __restrict__ pk, int ncell)
+__global__ void k_cell_order(GridArgs a)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncell) return;
+    const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
+    if (c >= a.ncell[k]) return;
+    const int* start = a.start[k];
+    int* sorted = a.sorted[k];
+    double4* pk = a.pk[k];
     const int b = start[c], e = start[c + 1];
     for (int i = b + 1; i < e; ++i) {
         const int v = sorted[i];
@@ -877,26 +1055,88 @@ static int alloc_spare(PartBuffers& pb)
     return 0;
 }
 
+// cells per dimension of a grid of width hmin or more (0: too few)
+static int grid_cells(const PartConst& pc, double hmin)
+{
+    const int G = std::min(CELL_GMAX, (int)floor(pc.pi2 / hmin));
+    if (G < 3) set_error("domain too small for the pair search grid (need 3 cells of the interaction radius)");
+    return G < 3 ? 0 : G;
+}
+
+static int alloc_cells(PartBuffers& pb)
+{
+    if (pb.cell_count) return 0;
+    // sized once for the finest grid, so switching between the collision and the overlap
+    // grids never reallocates; the scratch of two scans at once
+    const long long nmax = (long long)CELL_GMAX * CELL_GMAX * CELL_GMAX + 1;
+    DDNS_HIP(hipMalloc(&pb.cell_count, nmax * sizeof(int)));
+    DDNS_HIP(hipMalloc(&pb.cell_start, nmax * sizeof(int)));
+    const size_t need = 2 * scan_tmp_ints(std::max(nmax, (long long)pb.cap + 1)) * sizeof(int);
+    if (need > pb.scan_tmp_bytes) {
+        (void)hipFree(pb.scan_tmp);
+        pb.scan_tmp = nullptr;
+        DDNS_HIP(hipMalloc(&pb.scan_tmp, need));
+        pb.scan_tmp_bytes = need;
+    }
+    return 0;
+}
+
+// The cell kernels over k grids: the current one, then the spare.
+static int build_grids(PartBuffers& pb, const PartConst& pc, int k, hipStream_t s)
+{
+    GridArgs a{};
+    ScanArgs sc{};
+    long long zero[2] = {0, 0};
+    int ncmax = 0;
+    const size_t half = pb.scan_tmp_bytes / sizeof(int) / 2;
+    for (int g = 0; g < k; ++g) {
+        PartBuffers::CellSet& o = pb.spare;
+        a.cell_of[g] = g ? o.cell_of : pb.cell_of;
+        a.cnt[g] = g ? o.cell_count : pb.cell_count;
+        a.start[g] = g ? o.cell_start : pb.cell_start;
+        a.sorted[g] = g ? o.sorted : pb.sorted;
+        a.pk[g] = g ? o.pk : pb.pk;
+        a.rank[g] = g ? pb.cell_rank2 : pb.cell_rank;
+        a.G[g] = g ? o.G : pb.G;
+        a.hc[g] = g ? o.hc : pb.hc;
+        a.ncell[g] = 1 << (3 * cell_bits(a.G[g]));              // Morton numbers of the G^3 cells (G <= 256)
+        ncmax = std::max(ncmax, a.ncell[g]);
+        // the counts are left zero by the scan of the last build into this buffer
+        long long& z = g ? o.count_zero : pb.cell_count_zero;
+        if (z < a.ncell[g] + 1) {
+            DDNS_HIP(hipMemsetAsync(a.cnt[g], 0, ((size_t)a.ncell[g] + 1) * sizeof(int), s));
+            z = a.ncell[g] + 1;
+        }
+        zero[g] = z;
+        z = 0;
+        sc.in[g] = a.cnt[g];
+        sc.out[g] = a.start[g];
+        sc.zin[g] = a.cnt[g];
+        sc.bsum[g] = (int*)pb.scan_tmp + g * half;
+        sc.n[g] = a.ncell[g];
+    }
+    if (pc.n > 0) hipLaunchKernelGGL(k_cell_key, dim3(nblk(pc.n), k), dim3(PT), 0, s, (const double*)pb.pos, a, pc.n, pb.cap);
+    const int st = scan_launch(sc, k, s);
+    if (st) return st;
+    pb.cell_count_zero = zero[0];
+    if (k > 1) pb.spare.count_zero = zero[1];
+    if (pc.n > 0) {
+        hipLaunchKernelGGL(k_cell_fill, dim3(nblk(pc.n), k), dim3(PT), 0, s, a, (const double*)pb.pos, (const double*)pb.rad,
+                           pc.n, pb.cap);
+        hipLaunchKernelGGL(k_cell_order, dim3(nblk(ncmax), k), dim3(PT), 0, s, a);
+    }
+    DDNS_HIP(hipGetLastError());
+    pb.cells_valid = true;
+    if (k > 1) pb.spare.valid = true;
+    return 0;
+}
+
 int part_build_cells(PartBuffers& pb, const PartConst& pc, double hmin, hipStream_t s)
 {
-    constexpr int GMAX = CELL_GMAX;
-    int G = (int)floor(pc.pi2 / hmin);
-    if (G > GMAX) G = GMAX;
-    if (G < 3) { set_error("domain too small for the pair search grid (need 3 cells of the interaction radius)"); return DDNS_ERR_DOMAIN; }
-    const long long ncell = 1LL << (3 * cell_bits(G));      // Morton numbers of the G^3 cells (G <= 256)
-    if (!pb.cell_count) {
-        // sized once for the finest grid, so switching between the collision and the
-        // overlap grids never reallocates
-        const long long nmax = (long long)GMAX * GMAX * GMAX + 1;
-        DDNS_HIP(hipMalloc(&pb.cell_count, nmax * sizeof(int)));
-        DDNS_HIP(hipMalloc(&pb.cell_start, nmax * sizeof(int)));
-        const size_t need = scan_tmp_ints(std::max(nmax, (long long)pb.cap + 1)) * sizeof(int);
-        if (need > pb.scan_tmp_bytes) {
-            (void)hipFree(pb.scan_tmp);
-            DDNS_HIP(hipMalloc(&pb.scan_tmp, need));
-            pb.scan_tmp_bytes = need;
-        }
-    }
+    const int G = grid_cells(pc, hmin);
+    if (!G) return DDNS_ERR_DOMAIN;
+    int st = alloc_cells(pb);
+    if (st) return st;
     if (pb.cells_valid && pb.G == G) return 0;                     // already built on these positions
     if (pb.spare.valid && pb.spare.G == G) {                      // kept from an earlier build
         swap_cells(pb);
@@ -904,34 +1144,33 @@ int part_build_cells(PartBuffers& pb, const PartConst& pc, double hmin, hipStrea
     }
     if (pb.cells_valid) {
         // keep the current grid (another width) for a later search: build into the spare
-        int st = alloc_spare(pb);
+        st = alloc_spare(pb);
         if (st) return st;
         swap_cells(pb);
     }
     pb.cells_valid = false;
     pb.G = G;
     pb.hc = pc.pi2 / G;
-    // the counts are left zero by the scan of the last build into this buffer
-    if (pb.cell_count_zero < ncell + 1) {
-        DDNS_HIP(hipMemsetAsync(pb.cell_count, 0, (ncell + 1) * sizeof(int), s));
-        pb.cell_count_zero = ncell + 1;
+    return build_grids(pb, pc, 1, s);
+}
+
+int part_build_two(PartBuffers& pb, const PartConst& pc, double hmin, double other, hipStream_t s)
+{
+    const int G = grid_cells(pc, hmin), H = grid_cells(pc, other);
+    if (!G || !H) return DDNS_ERR_DOMAIN;
+    if (G == H || pb.cells_valid || pb.spare.valid) {
+        const int st = part_build_cells(pb, pc, other, s);
+        return st ? st : part_build_cells(pb, pc, hmin, s);
     }
-    const long long zero = pb.cell_count_zero;
-    pb.cell_count_zero = 0;
-    if (pc.n > 0)
-        hipLaunchKernelGGL(k_cell_key, dim3(nblk(pc.n)), dim3(PT), 0, s, pb.pos, pb.cell_of, pb.cell_rank, pb.cell_count, pc.n,
-                           pb.cap, G, pb.hc);
-    int st = exclusive_scan(pb.cell_count, pb.cell_start, (int)ncell, (int*)pb.scan_tmp, s, true);
+    int st = alloc_cells(pb);
+    if (!st) st = alloc_spare(pb);
     if (st) return st;
-    pb.cell_count_zero = zero;
-    if (pc.n > 0) {
-        hipLaunchKernelGGL(k_cell_fill, dim3(nblk(pc.n)), dim3(PT), 0, s, pb.cell_of, pb.cell_rank, pb.cell_start,
-                           pb.sorted, pb.pos, pb.rad, pb.pk, pc.n, pb.cap);
-        hipLaunchKernelGGL(k_cell_order, dim3(nblk(ncell)), dim3(PT), 0, s, pb.cell_start, pb.sorted, pb.pk, (int)ncell);
-    }
-    DDNS_HIP(hipGetLastError());
-    pb.cells_valid = true;
-    return 0;
+    if (!pb.cell_rank2) DDNS_HIP(hipMalloc(&pb.cell_rank2, (size_t)pb.cap * sizeof(int)));
+    pb.G = G;
+    pb.hc = pc.pi2 / G;
+    pb.spare.G = H;
+    pb.spare.hc = pc.pi2 / H;
+    return build_grids(pb, pc, 2, s);
 }
 
 }  // namespace ddns

@@ -1,0 +1,32 @@
+"""Relocation within a step: the listed droplets are sorted by one work-group, and a list of more
+than 4096 droplets is walked over all droplets instead."""
+import numpy as np
+import pytest
+
+from helpers import random_droplets
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("pairs", [0, 1, 700, 2300, 5200])
+def test_step_relocates_as_the_oracle(ddns, oracle_mod, pairs):
+    """A step of droplets at rest in a fluid at rest, the first of them placed in overlapping
+    pairs: the draws of one stream go to the relocated droplets in index order, so positions and
+    counts are those of the oracle.  5200 pairs put more than 4096 droplets on the list."""
+    n = 20000
+    p = ddns.default_params(N=32, precision=0, npart=n, radius=[30.0], nonoverlap=1, dt=1e-4, rnu=0.02,
+                            gravity=1e-25, forcing=0, new_particle=0)
+    with oracle_mod.Oracle(p) as o, ddns.Solver(p) as s:
+        rad = o.scaling()["radius"][:1]
+        yp = random_droplets(n, 31, rad)
+        yp[3:6] = 0.0
+        order = np.random.default_rng(7).permutation(n)
+        a, b = order[:pairs], order[pairs:2 * pairs]
+        yp[:3, b] = np.mod(yp[:3, a] + 0.5 * rad[0], 2 * np.pi)
+        for x in (o, s):
+            x.set_droplets(yp)
+            x.step(1)
+        cg, co = s.collision_counts(), o.collision_counts()
+        print(pairs, co.ncoll, co.noverlap_sweeps, co.noverlap_relocated)
+        assert (cg.ncoll, cg.noverlap_sweeps, cg.noverlap_relocated) == (co.ncoll, co.noverlap_sweeps, co.noverlap_relocated)
+        assert np.allclose(s.get_droplets()["yp"][:3], o.get_droplets()["yp"][:3], rtol=0, atol=1e-12)
