@@ -398,7 +398,7 @@ __device__ __forceinline__ void stage_flush(const CollArgs& a, const CandStage& 
 }
 
 __device__ __forceinline__ void collide_search(const CollArgs& a, int t, int lane, int& tested, int& touching,
-                                               const CandStage& st, double dmax, double rbig)
+                                               const CandStage& st, RunList<CT>& runs, double dmax, double rbig)
 {
     const int ia = a.sorted[t];
     const size_t C = (size_t)a.cap;
@@ -429,21 +429,20 @@ __device__ __forceinline__ void collide_search(const CollArgs& a, int t, int lan
     // the walk covers the neighbour cells only: a reach beyond the cell width is reported,
     // and the search is repeated on wider cells
     if (reach + 1e-9 * g.hc > g.hc) atomicOr(a.far, 1);
-    for_each_candidate(a.cell_start, g.G, cc, a.pk, a.sorted, [&](int p, int kc, const double4& cb, int ib) {
+    for_each_candidate<1>(runs, a.cell_start, g.G, g.h, cc, a.pk, a.sorted,
+                       [&](int p, int w, double sx, double sy, double sz, const double4& cb, int ib) {
         if (p == t) return;
-        int wx, wy, wz;
-        neighbour_shift(kc, g.G, cc, &wx, &wy, &wz);
         ++tested;
         // the distance to the image the visiting rules would take (shift w * 2 pi): a
         // partner beyond the reach can neither be counted nor collide, so the rules are
         // replayed for the near ones only
         {
-            const double e0 = xa[0] - (cb.x + (double)wx * g.h), e1 = xa[1] - (cb.y + (double)wy * g.h),
-                         e2 = xa[2] - (cb.z + (double)wz * g.h);
+            const double e0 = xa[0] - (cb.x + sx), e1 = xa[1] - (cb.y + sy), e2 = xa[2] - (cb.z + sz);
             if (e0 * e0 + e1 * e1 + e2 * e2 > reach2) return;
         }
         double xb[3];
-        int di, dj, dk;
+        int di, dj, dk, wx, wy, wz;
+        shift_of(w, &wx, &wy, &wz);
         if (!ref_visit(g, ia, ib, xa[0], xa[1], xa[2], cb.x, cb.y, cb.z,
                        wx, wy, wz, &xb[0], &xb[1], &xb[2], &di, &dj, &dk))
             return;
@@ -467,7 +466,7 @@ __device__ __forceinline__ void collide_search(const CollArgs& a, int t, int lan
                 stage_flush(a, st, c, lane, __ballot(1));
                 c = 0;
             }
-            if (emit) st.buf[c + __popcll(m & ((1ull << lane) - 1))] = make_int2(t, (int)((unsigned)p | ((unsigned)kc << 27)));
+            if (emit) st.buf[c + __popcll(m & ((1ull << lane) - 1))] = make_int2(t, (int)((unsigned)p | ((unsigned)w << 27)));
             __builtin_amdgcn_wave_barrier();
             if (lane == __ffsll((long long)m) - 1) *st.cnt = c + k;
             __builtin_amdgcn_wave_barrier();
@@ -481,12 +480,13 @@ __global__ void __launch_bounds__(CT) k_collide(CollArgs a)
     const int lane = threadIdx.x & 63;
     __shared__ int2 stage_buf[CT / 64][STAGE];
     __shared__ int stage_cnt[CT / 64];
+    __shared__ RunList<CT> runs;
     const CandStage st{stage_buf[threadIdx.x >> 6], stage_cnt + (threadIdx.x >> 6)};
     if (lane == 0) *st.cnt = 0;
     __builtin_amdgcn_wave_barrier();
     int tested = 0, touching = 0;
     const double dmax = read_extent(a.ext, 0), rbig = read_extent(a.ext, 1);
-    if (t < a.n) collide_search(a, t, lane, tested, touching, st, dmax, rbig);
+    if (t < a.n) collide_search(a, t, lane, tested, touching, st, runs, dmax, rbig);
     // the whole wavefront is back together: hand on what its stage still holds
     {
         const int c = *st.cnt;
@@ -534,7 +534,7 @@ __global__ void __launch_bounds__(256) k_collide_pairs(CollArgs a)
     long long instat = 0;
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < ncand; r += gridDim.x * blockDim.x) {
         const int2 rec = a.cand[r];
-        const int t = rec.x, p = rec.y & ((1 << 27) - 1), kc = (int)((unsigned)rec.y >> 27);   // kc < 27: 5 bits
+        const int t = rec.x, p = rec.y & ((1 << 27) - 1), w = (int)((unsigned)rec.y >> 27);   // w < 27: 5 bits
         const int ia = a.sorted[t];
         const size_t C = (size_t)a.cap;
         const PairGeom& g = a.g;
@@ -547,14 +547,8 @@ __global__ void __launch_bounds__(256) k_collide_pairs(CollArgs a)
             const double d0 = a.dmove[ia], d1 = a.dmove[C + ia], d2 = a.dmove[2 * C + ia];
             dmove_a = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
         }
-        int cc[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            int q = (int)(xa[c] / g.hc);
-            cc[c] = q < 0 ? 0 : (q >= g.G ? g.G - 1 : q);
-        }
         int wx, wy, wz;
-        neighbour_shift(kc, g.G, cc, &wx, &wy, &wz);
+        shift_of(w, &wx, &wy, &wz);
         const int ib = a.sorted[p];
         const double4 cb = a.pk[p];
         double xb[3];
@@ -625,20 +619,20 @@ __global__ void __launch_bounds__(CT) k_overlap(OverArgs a)
         cc[c] = q < 0 ? 0 : (q >= g.G ? g.G - 1 : q);
     }
     int cnt = 0;
-    // a light kernel: the row-wise walk needs no LDS, which keeps its occupancy high;
     // only the cells within ra + rbig of the droplet can hold an overlapping partner,
     // and the visiting rules are replayed for the partners within that distance only
     const double reach = ra + rbig;
     const double reach2 = reach * reach * (1. + 1e-9);
-    for_each_candidate(a.cell_start, g.G, cc, a.pk, a.sorted, [&](int p, int kc, const double4& cb, int ib) {
+    __shared__ RunList<CT> runs;
+    for_each_candidate<1>(runs, a.cell_start, g.G, g.h, cc, a.pk, a.sorted,
+                       [&](int p, int w, double sx, double sy, double sz, const double4& cb, int ib) {
         if (p == t) return;
-        int wx, wy, wz;
-        neighbour_shift(kc, g.G, cc, &wx, &wy, &wz);
         {
-            const double e0 = xa - (cb.x + (double)wx * g.h), e1 = ya - (cb.y + (double)wy * g.h),
-                         e2 = za - (cb.z + (double)wz * g.h);
+            const double e0 = xa - (cb.x + sx), e1 = ya - (cb.y + sy), e2 = za - (cb.z + sz);
             if (e0 * e0 + e1 * e1 + e2 * e2 > reach2) return;
         }
+        int wx, wy, wz;
+        shift_of(w, &wx, &wy, &wz);
         double xb, yb, zb;
         int di, dj, dk;
         if (!ref_visit(g, ia, ib, xa, ya, za, cb.x, cb.y, cb.z, wx, wy, wz, &xb, &yb, &zb, &di, &dj, &dk)) return;
@@ -913,10 +907,13 @@ int part_overlap_queue(PartBuffers& pb, const PartConst& pc, hipStream_t s, doub
         st = overlap_setup(pb, pc, s);
         ext = pb.ext + EXT_WORDS;
     }
-    // the sweep's grid and the next step's, on the same positions, in the same launches (a
-    // relocation by this sweep invalidates both)
-    if (!st) st = next_width > 0.0 ? part_build_two(pb, pc, overlap_width(pc), next_width, s)
-                                   : part_build_cells(pb, pc, overlap_width(pc), s);
+    // the next step's grid, which serves the sweep too where it is wide enough and not too full;
+    // else the sweep's grid with it, on the same positions, in the same launches (a relocation by
+    // this sweep invalidates both)
+    const double width = overlap_width(pc);
+    const int G = (int)std::min(256.0, std::floor(pc.pi2 / next_width));
+    if (!st) st = next_width >= width && grid_serves(pc.n, G) ? part_build_cells(pb, pc, next_width, s)
+                                                              : part_build_two(pb, pc, width, next_width, s);
     if (!st) st = overlap_search(pb, pc, ext, s);
     if (st) return st;
     const bool kept = pb.cells_valid, spare_kept = pb.spare.valid;

@@ -949,7 +949,7 @@ static int droplet_rest(ddns_handle* h, float* ms)
     h->new_particle = 0;
     pc.new_particle = 0;
     DDNS_HIP(hipEventRecord(h->ev[12], s));
-    if (h->p.hdi_included && std::min(256, (int)std::floor(pc.pi2 / coll_cell_width(h))) > h->pb.G) {
+    if (h->p.hdi_included && !grid_serves(h->n, h->pb.G) && std::min(256, (int)std::floor(pc.pi2 / coll_cell_width(h))) > h->pb.G) {
         // finer grid for the collision search; the grid of the last overlap sweep has
         // this width and the same positions, and is swapped in when it is still valid
         st = part_build_cells(h->pb, pc, coll_cell_width(h), s);

@@ -31,21 +31,29 @@ constexpr int DDNS_PAIR_REC = 8;
 // reference's buffer(1:12, ij): index1, index2, va(3), vb(3), unit offset (3), Wr
 constexpr int DDNS_CONTACT_REC = 14;
 
-// Coarse-cell number of cell (x, y, z), 0 <= x, y, z < 256: the Morton (Z-curve)
-// interleave of the three indices, x in the lowest bit.  Droplets sorted by it form
-// compact 3-D blocks, so the lanes of a wavefront touch overlapping field stencils and
-// neighbouring cells.  The numbers of a G^3 grid lie below 8^cell_bits(G).
+// Coarse-cell number of cell (x, y, z) of a G^3 grid, G <= 256: the rows along x are whole, so the
+// candidates of a row's neighbouring cells are one run of the sorted droplets, and the rows
+// follow the Morton (Z-curve) interleave of y and z, so droplets close in the order are close in
+// space and the lanes of a wavefront touch overlapping field stencils and cells.
 __host__ __device__ __forceinline__ unsigned cell_spread(unsigned v)
 {
     v &= 0xffu;
-    v = (v | (v << 8)) & 0x0300f00fu;
-    v = (v | (v << 4)) & 0x030c30c3u;
-    v = (v | (v << 2)) & 0x09249249u;
+    v = (v | (v << 4)) & 0x0f0fu;
+    v = (v | (v << 2)) & 0x3333u;
+    v = (v | (v << 1)) & 0x5555u;
     return v;
 }
-__host__ __device__ __forceinline__ int cell_code(int x, int y, int z)
+__host__ __device__ __forceinline__ int cell_row(int y, int z)
 {
-    return (int)(cell_spread((unsigned)x) | (cell_spread((unsigned)y) << 1) | (cell_spread((unsigned)z) << 2));
+    return (int)(cell_spread((unsigned)y) | (cell_spread((unsigned)z) << 1));
+}
+__host__ __device__ __forceinline__ int cell_code(int x, int y, int z, int G) { return cell_row(y, z) * G + x; }
+// the numbers of a G^3 grid lie below this (at most 256^3)
+inline int cell_numbers(int G)
+{
+    int b = 0;
+    while ((1 << b) < G) ++b;
+    return G << (2 * b);
 }
 // Work-group b of a launch runs on XCD b % 8, and each of the 8 XCDs has its own L2.
 // This gives the work-groups of one XCD a contiguous range of the nb logical blocks,
@@ -80,91 +88,106 @@ __device__ __forceinline__ CellSpan reach_span(const double x[3], const int cc[3
     return s;
 }
 
-// The candidates of the 27 neighbour cells (or of the part of them that span selects)
-// in 9 rows: for each (y, z) offset the cells x-1, x, x+1 as one sequence.  One row's
-// three ranges are held at a time: the next row's ranges load while the current row runs,
-// and inside a row the next record loads while f works on the current one.  Holding all
-// 27 ranges (and unrolling the nine rows) took about 50 more registers, and a walk that
-// waits on about one record load per candidate gains more from the wavefronts those
-// registers allow per SIMD.  f(p, kc, rec, ib) gets the sorted position, the cell number
-// k = 9 (dx+1) + 3 (dy+1) + (dz+1) of neighbour_shift, the record pk[p] and, when sorted
-// is given, the droplet index sorted[p].
-template <typename F>
-__device__ __forceinline__ void for_each_candidate(const int* __restrict__ cell_start, int G, const int cc[3],
-                                                   const double4* __restrict__ pk, const int* __restrict__ sorted,
-                                                   F&& f, const CellSpan& span = CellSpan())
+// The periodic shift of a run of candidates along each axis, -1, 0 or +1, in 5 bits
+__device__ __forceinline__ int shift_code(int wx, int wy, int wz) { return 9 * (wx + 1) + 3 * (wy + 1) + wz + 1; }
+__device__ __forceinline__ void shift_of(int w, int* wx, int* wy, int* wz)
 {
-    auto wrap = [G](int q) { return q < 0 ? q + G : (q >= G ? q - G : q); };
-    // [s, e) of the cells x-1, x, x+1 of row r = 3 my + mz; empty where span leaves it out
-    auto load_row = [&](int r, int& s0, int& e0, int& s1, int& e1, int& s2, int& e2) {
-        const int my = r / 3, mz = r - 3 * my;
-        s0 = e0 = s1 = e1 = s2 = e2 = 0;
-        if (my - 1 < span.lo[1] || my - 1 > span.hi[1] || mz - 1 < span.lo[2] || mz - 1 > span.hi[2]) return;
-        const int qy = wrap(cc[1] + my - 1), qz = wrap(cc[2] + mz - 1);
-        if (span.lo[0] < 0) {
-            const int c = cell_code(wrap(cc[0] - 1), qy, qz);
-            s0 = cell_start[c]; e0 = cell_start[c + 1];
-        }
-        {
-            const int c = cell_code(cc[0], qy, qz);
-            s1 = cell_start[c]; e1 = cell_start[c + 1];
-        }
-        if (span.hi[0] > 0) {
-            const int c = cell_code(wrap(cc[0] + 1), qy, qz);
-            s2 = cell_start[c]; e2 = cell_start[c + 1];
-        }
-    };
-    int s0, e0, s1, e1, s2, e2;
-    load_row(0, s0, e0, s1, e1, s2, e2);
+    *wx = w / 9 - 1;
+    *wy = (w / 3) % 3 - 1;
+    *wz = w % 3 - 1;
+}
+
+// The candidates of the 27 neighbour cells (or of the part of them that span selects): for each
+// (y, z) offset the cells x-1, x, x+1 are one run (across the periodic face in x two, the second
+// in a pass of its own that only wavefronts at the face make).  The runs' ends load together,
+// the non-empty ones go to the lane's column of the LDS list, and one loop walks them, the next
+// record loading while f works on the current one: a wavefront takes as many turns as its
+// fullest lane has candidates, where a loop for each run took the sum of the runs' longest,
+// waiting for each run's ends.  At 1M droplets with half a droplet per cell the collision
+// search took 246 us that way and takes 222, the overlap search 65 and 53; at
+// 100 000 droplets 37 and 29, 10.8 and 7.0.  f(p, w, sx, sy, sz, rec, ib) gets the sorted
+// position, the shift code, the shift in lengths (h the box), the record pk[p] and, when sorted
+// is given, the droplet index sorted[p].  With L > 1, consecutive lanes of a wavefront share a
+// droplet, and lane j of them takes every L-th candidate from the j-th on.
+template <int NT>
+struct RunList {
+    int2 run[9][NT];
+};
+template <int L, int NT, typename F>
+__device__ __forceinline__ void for_each_candidate(RunList<NT>& list, const int* __restrict__ cell_start, int G, double h,
+                                                   const int cc[3], const double4* __restrict__ pk,
+                                                   const int* __restrict__ sorted, F&& f, const CellSpan& span = CellSpan())
+{
+    const int tid = threadIdx.x, sub = tid & (L - 1);
+    const int xl = cc[0] + span.lo[0], xh = cc[0] + span.hi[0];
+    const bool edge = xl < 0 || xh >= G;
+    const int passes = __any(edge) ? 2 : 1;
 #pragma unroll 1
-    for (int r = 0; r < 9; ++r) {
-        int n0 = 0, m0 = 0, n1 = 0, m1 = 0, n2 = 0, m2 = 0;
-        if (r + 1 < 9) load_row(r + 1, n0, m0, n1, m1, n2, m2);
-        int m = 0, p = s0, end = e0;
-        if (p >= end) { m = 1; p = s1; end = e1; }
-        if (p >= end) { m = 2; p = s2; end = e2; }
-        if (p < end) {
-            double4 next = pk[p];
-            int inext = sorted ? sorted[p] : 0;
-#pragma unroll 1
+    for (int pass = 0; pass < passes; ++pass) {
+        if (pass && !edge) break;
+        // the cells a..b of each row: those inside the box, then the one beyond its face (G >= 3)
+        const int wx = pass ? (xl < 0 ? -1 : 1) : 0;
+        const int a = pass ? (xl < 0 ? G - 1 : 0) : max(xl, 0), b = pass ? a : min(xh, G - 1);
+        int s[9], e[9], w[9];
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            const int dy = r / 3 - 1, dz = r % 3 - 1;
+            s[r] = e[r] = w[r] = 0;
+            if (dy < span.lo[1] || dy > span.hi[1] || dz < span.lo[2] || dz > span.hi[2]) continue;
+            const int qy = cc[1] + dy, qz = cc[2] + dz;
+            const int wy = qy < 0 ? -1 : (qy >= G ? 1 : 0), wz = qz < 0 ? -1 : (qz >= G ? 1 : 0);
+            const int* row = cell_start + cell_row(qy - wy * G, qz - wz * G) * G;
+            w[r] = shift_code(wx, wy, wz);
+            s[r] = row[a];
+            e[r] = row[b + 1];
+        }
+        int n = 0;
+#pragma unroll
+        for (int r = 0; r < 9; ++r)
+            if (e[r] > s[r]) list.run[n++][tid] = make_int2(s[r], ((e[r] - s[r]) << 5) | w[r]);
+        if (n == 0) continue;
+        int i = 0, p, end, wc, vx, vy, vz;
+        // the run i, entered at its candidate number skip; a shorter run passes the rest on
+        auto take = [&](int skip) {
             while (true) {
-                const int pc = p, kc = 9 * m + r;
-                const double4 rec = next;
-                const int ib = inext;
-                ++p;
-                while (p >= end && m < 2) {
-                    ++m;
-                    p = m == 1 ? s1 : s2;
-                    end = m == 1 ? e1 : e2;
-                }
-                const bool more = p < end;
-                if (more) {
-                    next = pk[p];
-                    if (sorted) inext = sorted[p];
-                }
-                f(pc, kc, rec, ib);
-                if (!more) break;
+                const int2 r = list.run[i][tid];
+                p = r.x + skip;
+                end = r.x + (r.y >> 5);
+                wc = r.y & 31;
+                if (L == 1 || p < end) return true;
+                if (++i == n) return false;
+                skip = p - end;
             }
+        };
+        if (!take(sub)) continue;
+        double4 next = pk[p];
+        int inext = sorted ? sorted[p] : 0;
+#pragma unroll 1
+        while (true) {
+            const int pc = p, w0 = wc;
+            const double4 rec = next;
+            const int ib = inext;
+            p += L;
+            bool more = p < end;
+            if (!more && ++i < n) more = take(p - end);
+            if (more) {
+                next = pk[p];
+                if (sorted) inext = sorted[p];
+            }
+            shift_of(w0, &vx, &vy, &vz);
+            f(pc, w0, (double)vx * h, (double)vy * h, (double)vz * h, rec, ib);
+            if (!more) break;
         }
-        s0 = n0; e0 = m0; s1 = n1; e1 = m1; s2 = n2; e2 = m2;
     }
 }
 
-// periodic shift (-1, 0, +1) of neighbour k along each axis for a lane in cell cc
-__device__ __forceinline__ void neighbour_shift(int k, int G, const int cc[3], int* wx, int* wy, int* wz)
-{
-    const int qx = cc[0] + k / 9 - 1, qy = cc[1] + (k / 3) % 3 - 1, qz = cc[2] + k % 3 - 1;
-    *wx = qx < 0 ? -1 : (qx >= G ? 1 : 0);
-    *wy = qy < 0 ? -1 : (qy >= G ? 1 : 0);
-    *wz = qz < 0 ? -1 : (qz >= G ? 1 : 0);
-}
-
-inline int cell_bits(int G)
-{
-    int b = 0;
-    while ((1 << b) < G) ++b;
-    return b;
-}
+// Whether the collision and overlap searches of n droplets use the cells of a G^3 grid that is
+// built in any case (the HI lists') instead of a finer grid of their own: the finer one saves
+// candidates, but costs a build, whose scattered reads and writes move whole cache lines.  A step
+// with one grid against two, by droplets per cell of the shared grid: 0.5 (128^3, 100 000) 0.59
+// against 0.60 ms, 1.4 (256^3, 1M) 2.62 against 2.73, 4.1 (128^3, 800 000) 3.14 against 3.29,
+// but 6 (64^3, 60 000, where a droplet's walk is a serial chain) 1.10 against 1.07.
+inline bool grid_serves(int n, int G) { return (double)n <= 4.0 * G * (double)G * G; }
 
 int hip_fail(hipError_t e, const char* what, const char* file, int line);
 struct PartBuffers;
@@ -546,8 +569,8 @@ int relocate_list(PartBuffers& pb, const PartConst& pc, int nlist, bool wrap, hi
 int part_overlap(PartBuffers& pb, const PartConst& pc, int* sweeps, int* relocated, hipStream_t s);
 // the step's overlap sweep: the first sweep queued without a host wait; the rest, if it
 // relocated droplets, after the caller has waited for the stream
-// next_width > 0: the grid of that width (the next step's first) is built too, on the
-// positions the sweep saw, and kept if the sweep moves nothing
+// next_width: the next step's first grid, built too, on the positions the sweep saw, and kept
+// if the sweep moves nothing
 // grown: coalescence has changed radii since the advance
 int part_overlap_queue(PartBuffers& pb, const PartConst& pc, hipStream_t s, double next_width, bool grown);
 int part_overlap_finish(PartBuffers& pb, const PartConst& pc, int* sweeps, int* relocated, hipStream_t s);

@@ -42,16 +42,26 @@ __device__ __forceinline__ double wave_sum(double x)
 
 // ------------------------------------------------------------------ neighbour lists
 // Row t (sorted position): every droplet p != t in the 27 cells around t with
-// |x_t - x_p| < trunc * r_p, in cell order, as partlib.f90:3280-3330 visits them.
-constexpr int NT_NEI = HT;
+// |x_t - x_p| < trunc * r_p (partlib.f90:3280-3330).  The walk only
+// decides, from the squared distance (the square root is taken where rounding could decide),
+// and leaves the accepted candidates in the list; a second, short loop forms their blocks.  In
+// the walk a wavefront of 64 rows met an accepted candidate on nearly every turn, and took the
+// blocks' divisions and six scattered stores there for one or two lanes each time (1M droplets
+// 274 us, now 202; 100 000: 42, now 27).  Four lanes share a row up to NEI_SHARED droplets, where
+// the rows alone leave the SIMDs short of wavefronts and each row's walk is a serial chain: the
+// 16 realisations of 9 000 to 60 000 droplets 105 -> 46 us a launch (two lanes: 64^3 with 60 000
+// droplets 0.76 ms a solve, four 0.73, eight 0.73), at 100 000 no difference.
+constexpr int NT_NEI = 128, NEI_SHARED = 131072;
 
-template <typename T>
+template <typename T, int L>
 __global__ void __launch_bounds__(NT_NEI) k_nei(const double4* __restrict__ pk, const int* __restrict__ cell_start,
                                                 int n, int G, double hc, double pi2, double trunc, int width,
                                                 int* __restrict__ cnt, int* __restrict__ idx, T* __restrict__ mm,
                                                 int* flags)
 {
-    const int t = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    __shared__ RunList<NT_NEI> runs;
+    const int t = (xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) / L;
+    const int sub = threadIdx.x & (L - 1), first = threadIdx.x & 63 & ~(L - 1);    // among the row's lanes; its first lane
     int k = 0;
     if (t < n) {
         const double4 me = pk[t];
@@ -65,40 +75,58 @@ __global__ void __launch_bounds__(NT_NEI) k_nei(const double4* __restrict__ pk, 
         }
         const size_t ld = (size_t)n;
         bool overlap = false;
-        for_each_candidate(cell_start, G, cc, pk, (const int*)nullptr, [&](int p, int kc, const double4& o, int) {
-            if (p == t) return;
-            int wx, wy, wz;
-            neighbour_shift(kc, G, cc, &wx, &wy, &wz);
-            const double d0 = xi - (o.x + (double)wx * pi2);
-            const double d1 = yi - (o.y + (double)wy * pi2);
-            const double d2 = zi - (o.z + (double)wz * pi2);
-            const double dnij = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-            const double rj = o.w;
-            if (dnij < ri + rj) overlap = true;                             // 3294-3299
-            if (!(dnij < trunc * rj)) return;                               // 3302-3305
-            if (k < width) {
-                double fact1 = rj / dnij;                                   // 3312-3324
-                const double fact2 = fact1 * fact1 * fact1;
-                fact1 = 0.75 * fact1;
-                const double gamma = (fact1 - 0.75 * fact2) / (dnij * dnij);
-                const double beta = fact1 + 0.25 * fact2;
-                idx[(size_t)k * ld + t] = p;
-                T* m = mm + (size_t)(6 * k) * ld + t;
-                m[0] = (T)(gamma * (d0 * d0) + beta);
-                m[ld] = (T)(gamma * d0 * d1);
-                m[2 * ld] = (T)(gamma * d0 * d2);
-                m[3 * ld] = (T)(gamma * (d1 * d1) + beta);
-                m[4 * ld] = (T)(gamma * d1 * d2);
-                m[5 * ld] = (T)(gamma * (d2 * d2) + beta);
-            }
-            ++k;
+        // sqrt(d2) < l, decided without the root where d2 is not within rounding of l^2
+        auto closer = [](double d2, double l) {
+            const double l2 = l * l;
+            if (fabs(d2 - l2) > 1e-12 * l2) return d2 < l2;
+            return sqrt(d2) < l;
+        };
+        for_each_candidate<L>(runs, cell_start, G, pi2, cc, pk, (const int*)nullptr,
+                           [&](int p, int w, double sx, double sy, double sz, const double4& o, int) {
+            const double d0 = xi - (o.x + sx), d1 = yi - (o.y + sy), d2 = zi - (o.z + sz);
+            const double dd = d0 * d0 + d1 * d1 + d2 * d2;
+            if (p != t && closer(dd, ri + o.w)) overlap = true;             // 3294-3299
+            const bool hit = p != t && closer(dd, trunc * o.w);             // 3302-3305
+            // the row's lanes append in the order of their candidates
+            const unsigned m = L == 1 ? (unsigned)hit : (unsigned)(__ballot(hit) >> first) & ((1u << L) - 1);
+            if (L > 1) k = __shfl(k, first, 64);     // the first lane has a candidate on every turn
+            const int j = k + __popc(m & ((1u << sub) - 1));
+            if (hit && j < width) idx[(size_t)j * ld + t] = (int)((unsigned)p | ((unsigned)w << 27));
+            k += __popc(m);
         });
+        if (L > 1) k = __shfl(k, first, 64);
         if (overlap) atomicOr(flags, 1);
         if (k > DDNS_MAXNEI) atomicOr(flags, 2);
         // a row with more neighbours than the lists hold keeps what fits: the products that
         // may run before the host has read the width flag stay inside the lists, and the
         // host fills them again, wider, before it uses any result
-        cnt[t] = k < width ? k : width;
+        const int kk = k < width ? k : width;
+        if (sub == 0) cnt[t] = kk;
+        if (L > 1) __threadfence_block();            // entries that other lanes of the row wrote
+        for (int j = sub; j < kk; j += L) {
+            const unsigned v = (unsigned)idx[(size_t)j * ld + t];
+            const int p = (int)(v & ((1u << 27) - 1));
+            int wx, wy, wz;
+            shift_of((int)(v >> 27), &wx, &wy, &wz);
+            const double4 o = pk[p];
+            const double d0 = xi - (o.x + (double)wx * pi2);
+            const double d1 = yi - (o.y + (double)wy * pi2);
+            const double d2 = zi - (o.z + (double)wz * pi2);
+            const double dnij = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+            double fact1 = o.w / dnij;                                      // 3312-3324
+            const double fact2 = fact1 * fact1 * fact1;
+            fact1 = 0.75 * fact1;
+            const double gamma = (fact1 - 0.75 * fact2) / (dnij * dnij);
+            const double beta = fact1 + 0.25 * fact2;
+            idx[(size_t)j * ld + t] = p;
+            T* m = mm + (size_t)(6 * j) * ld + t;
+            m[0] = (T)(gamma * (d0 * d0) + beta);
+            m[ld] = (T)(gamma * d0 * d1);
+            m[2 * ld] = (T)(gamma * d0 * d2);
+            m[3 * ld] = (T)(gamma * (d1 * d1) + beta);
+            m[4 * ld] = (T)(gamma * d1 * d2);
+            m[5 * ld] = (T)(gamma * (d2 * d2) + beta);
+        }
     }
     // the widest row of the wavefront, for the width check
     int km = k;
@@ -830,9 +858,13 @@ static int queue_lists(PartBuffers& pb, const PartConst& pc, hipStream_t s)
         DDNS_HIP(hipMalloc(&pb.nei_m, (size_t)6 * pb.ell_width * pb.cap * sizeof(T)));
     }
     // the flags are clear: from the step's start, or from lists_outcome when the lists are filled again
-    hipLaunchKernelGGL((k_nei<T>), dim3((n + NT_NEI - 1) / NT_NEI), dim3(NT_NEI), 0, s, (const double4*)pb.pk, pb.cell_start,
-                       n, pb.G, pb.hc, pc.pi2, pc.hdi_trunc, pb.ell_width, pb.nei_cnt, pb.nei_idx, (T*)pb.nei_m,
-                       pb.flags);
+    auto launch = [&](auto kernel, int lanes) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(((long long)n * lanes + NT_NEI - 1) / NT_NEI)), dim3(NT_NEI), 0, s,
+                           (const double4*)pb.pk, pb.cell_start, n, pb.G, pb.hc, pc.pi2, pc.hdi_trunc, pb.ell_width,
+                           pb.nei_cnt, pb.nei_idx, (T*)pb.nei_m, pb.flags);
+    };
+    if (n <= NEI_SHARED) launch(k_nei<T, 4>, 4);
+    else launch(k_nei<T, 1>, 1);
     DDNS_HIP(hipGetLastError());
     return 0;
 }

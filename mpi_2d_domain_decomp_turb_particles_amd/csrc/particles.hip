@@ -983,7 +983,7 @@ __global__ void k_cell_key(const double* pos, GridArgs a, int n, int cap)
         q = q < 0 ? 0 : (q >= G ? G - 1 : q);
         c3[c] = q;
     }
-    const int cell = cell_code(c3[0], c3[1], c3[2]);
+    const int cell = cell_code(c3[0], c3[1], c3[2], G);
     a.cell_of[k][i] = cell;
     a.rank[k][i] = atomicAdd(a.cnt[k] + cell, 1);
 }
@@ -1099,7 +1099,7 @@ static int build_grids(PartBuffers& pb, const PartConst& pc, int k, hipStream_t 
         a.rank[g] = g ? pb.cell_rank2 : pb.cell_rank;
         a.G[g] = g ? o.G : pb.G;
         a.hc[g] = g ? o.hc : pb.hc;
-        a.ncell[g] = 1 << (3 * cell_bits(a.G[g]));              // Morton numbers of the G^3 cells (G <= 256)
+        a.ncell[g] = cell_numbers(a.G[g]);
         ncmax = std::max(ncmax, a.ncell[g]);
         // the counts are left zero by the scan of the last build into this buffer
         long long& z = g ? o.count_zero : pb.cell_count_zero;
