@@ -232,9 +232,9 @@ __global__ void __launch_bounds__(HT) k_residual0(const double* __restrict__ b, 
 
 // The small problem cleared (ntot values), then norm_b = |b| and norm_rhs = |r0| from the
 // np partials of k_residual0 (fixed order), the tolerance, and the stop flag when the
-// initial residual is below 1e-5 (2866-2868)
+// initial residual is below 1e-5 (2866-2868); the head and the lists' flags to the host's copy
 __global__ void __launch_bounds__(HT) k_gm_start(double* sm, int ntot, double tol, const double* __restrict__ part,
-                                                 int np)
+                                                 int np, const int* __restrict__ flags, double* host)
 {
     __shared__ double sb[HT], sq[HT];
     for (int i = threadIdx.x; i < ntot; i += HT) sm[i] = 0.0;
@@ -254,11 +254,11 @@ __global__ void __launch_bounds__(HT) k_gm_start(double* sm, int ntot, double to
         __syncthreads();
     }
     if (threadIdx.x == 0) {                // after the barriers of the tree: the clearing is done
-        sm[0] = sqrt(sb[0]);
-        sm[1] = sqrt(sq[0]);
-        sm[3] = tol;
-        if (sm[1] < 1e-5) sm[4] = -1.0;
+        const double head[6] = {sqrt(sb[0]), sqrt(sq[0]), 0.0, tol, sqrt(sq[0]) < 1e-5 ? -1.0 : 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 6; ++k) sm[k] = host[k] = head[k];
     }
+    if (threadIdx.x < 8) ((int*)(host + 8))[threadIdx.x] = flags[threadIdx.x];
 }
 
 template <typename T>
@@ -552,34 +552,168 @@ __global__ void __launch_bounds__(RT) k_spmv_mdot(const int* __restrict__ cnt, c
     k_spmv_mdot_body<T, MODE, KC>(cnt, idx, mm, n, x, hx, qout, y, Q, ld, k, part, stop, blockIdx.x, gridDim.x);
 }
 
-// h = sum of part_in, v -= sum_j h[j] Q_j; with normpart, also the partials of |v|^2.
-// With gate (the second pass's update): gate[0 .. P) and gate[P .. 2P) hold the partials
-// of |w|^2 before the first pass and |v|^2 after it; when the first pass kept at least
-// 1/sqrt(2) of the norm (|v|^2 >= |w|^2 / 2, the DGKS criterion) the second pass's
-// corrections are below rounding and its update is skipped: v, hcol stay, and normpart
-// takes the partials of |v|^2 already summed.
-template <typename T>
-__device__ __forceinline__ void k_maxpy_body(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
-                                              long long ld, const double* __restrict__ part_in,
-                                              double* __restrict__ hcol, int add, double* __restrict__ normpart,
-                                              const double* __restrict__ stop, const double* __restrict__ gate_w,
-                                              const double* __restrict__ gate_v, int bx, int nbx)
+// Small least-squares update of HDI_GMRES (2904-2971), by one wavefront.
+// sm layout: [0] norm_b [1] norm_rhs [2] res [3] maxerr [4] done [5] iter
+//            H at 16 + (r-1) + M1*(c-1), Rn after it, Qn after it, then bn and y
+struct GmSmall {
+    int maxiter;
+    __host__ __device__ int M1() const { return maxiter + 1; }
+    __host__ __device__ size_t H0() const { return 16; }
+    __host__ __device__ size_t R0() const { return H0() + (size_t)M1() * maxiter; }
+    __host__ __device__ size_t Q0() const { return R0() + (size_t)M1() * M1(); }
+    __host__ __device__ size_t B0() const { return Q0() + (size_t)M1() * M1(); }
+    __host__ __device__ size_t Y0() const { return B0() + M1(); }
+    __host__ __device__ size_t total() const { return Y0() + M1(); }
+};
+
+constexpr int LT = 64;           // one wavefront; maxiter + 1 <= LT
+constexpr int LS_MAXITER = 50;   // the reference's value
+
+// The part of the small problem that iteration iter reads, in LDS with columns of iter + 1
+// entries: 16 head values, iter columns of H and of Rn, iter + 1 of Qn, and bn.
+__host__ __device__ constexpr int ls_doubles(int iter)
 {
-    if (*stop != 0.0) return;
+    return 16 + 2 * iter * (iter + 1) + (iter + 1) * (iter + 1) + iter + 1;
+}
+
+// its copy by threads t of nt
+__device__ __forceinline__ void ls_load(double* sm, const double* __restrict__ gsm, GmSmall L, int iter, int t, int nt)
+{
+    const int d = iter + 1, M1 = L.M1(), n1 = d * iter, n2 = 2 * n1, n3 = n2 + d * d, n4 = n3 + d;
+    for (int j = t; j < 16 + n4; j += nt) {
+        const int e = j - 16;
+        size_t a;
+        if (e < 0) a = j;
+        else if (e < n1) a = L.H0() + e % d + (size_t)M1 * (e / d);
+        else if (e < n2) a = L.R0() + (e - n1) % d + (size_t)M1 * ((e - n1) / d);
+        else if (e < n3) a = L.Q0() + (e - n2) % d + (size_t)M1 * ((e - n2) / d);
+        else a = L.B0() + (e - n3);
+        sm[j] = gsm[a];
+    }
+}
+
+// LDS accesses of one wavefront are served in order: only the compiler has to keep them so
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// x of lane l (the same l in every lane)
+__device__ __forceinline__ double of_lane(double x, int l)
+{
+    const long long b = __double_as_longlong(x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// One wavefront, sm as ls_load leaves it, hnext = H(iter + 1, iter).  Lane r owns row r + 1 of the
+// triangular factor, of the solution and of the residual; what the iteration changes goes back
+// to gsm, and the head to the host's copy as well (null: none).
+__device__ void ls_solve(double* sm, double* __restrict__ gsm, GmSmall L, int iter, double hnext, double* host)
+{
+    const int lane = threadIdx.x & 63, d = iter + 1, M1 = L.M1();
+    double* H = sm + 16;
+    double* Rn = H + d * iter;
+    double* Qn = Rn + d * iter;
+    double* bn = Qn + d * d;
+#define HH(r, c) H[((r) - 1) + d * ((c) - 1)]
+#define RN(r, c) Rn[((r) - 1) + d * ((c) - 1)]
+#define QN(r, c) Qn[((r) - 1) + d * ((c) - 1)]
+    const double norm_rhs = sm[1];
+    double* gH = gsm + L.H0() + (size_t)M1 * (iter - 1);
+    double* gR = gsm + L.R0() + (size_t)M1 * (iter - 1);
+    double* gQ = gsm + L.Q0();
+    if (lane == 0) {
+        HH(iter + 1, iter) = hnext;
+        gH[iter] = hnext;
+    }
+    wave_sync();
+    double b;                                   // bn(lane + 1)
+    if (iter == 1) {
+        const double nrm = sqrt(HH(1, 1) * HH(1, 1) + HH(2, 1) * HH(2, 1));
+        const double q11 = HH(1, 1) / nrm, q21 = HH(2, 1) / nrm;
+        b = q11 * norm_rhs;
+        if (lane == 0) {
+            gQ[0] = q11; gQ[1] = q21; gQ[M1] = q21; gQ[M1 + 1] = -q11;
+            RN(1, 1) = gR[0] = nrm;
+            gsm[L.B0()] = b;
+        }
+        wave_sync();
+    } else {
+        // new column of R: Qn(1:iter, 1:iter) H(1:iter, iter)
+        double r = 0.0;
+        if (lane < iter)
+            for (int c = 1; c <= iter; ++c) r = r + QN(lane + 1, c) * HH(c, iter);
+        const double aa = of_lane(r, iter - 1), bb = hnext;
+        const double dd = sqrt(aa * aa + bb * bb);
+        const double cc = aa / dd, ss = bb / dd;
+        if (lane == iter - 1) r = dd;
+        if (lane < iter) RN(lane + 1, iter) = gR[lane] = r;
+        // rows iter and iter + 1 of Qn after the rotation
+        const double qi = lane < iter ? QN(iter, lane + 1) : 0.0;
+        const double qa = lane < iter ? cc * qi : ss, qb = lane < iter ? -ss * qi : cc;
+        if (lane <= iter) {
+            gQ[(iter - 1) + (size_t)M1 * lane] = qa;
+            gQ[iter + (size_t)M1 * lane] = qb;
+        }
+        b = lane < iter ? bn[lane] : 0.0;
+        if (lane == iter - 2) b = QN(iter - 1, 1) * norm_rhs;
+        const double blast = of_lane(qa, 0) * norm_rhs;
+        if (lane == iter - 1) b = blast;
+        if (lane >= iter - 2 && lane < iter) gsm[L.B0() + lane] = b;
+        wave_sync();
+    }
+    // back substitution by columns: lane r accumulates row r + 1
+    double acc = 0.0, y = 0.0;
+    const double diag = lane < iter ? RN(lane + 1, lane + 1) : 1.0;
+    for (int c = iter; c >= 1; --c) {
+        const double rc = lane < c - 1 ? RN(lane + 1, c) : 0.0;
+        const double yc = of_lane((b - acc) / diag, c - 1);
+        if (lane == c - 1) y = yc;
+        if (lane < c - 1) acc = acc + yc * rc;
+    }
+    if (lane < iter) gsm[L.Y0() + lane] = y;
+    // residual H y - |r0| e1 (2958-2966)
+    double rv = 0.0;
+    for (int c = 1; c <= iter; ++c) rv = rv + (lane <= iter ? HH(lane + 1, c) : 0.0) * of_lane(y, c - 1);
+    if (lane == 0) rv = rv - norm_rhs;
+    double x_c = 0.0;
+    for (int r = 0; r <= iter; ++r) {
+        const double v = of_lane(rv, r);
+        x_c = x_c + v * v;
+    }
+    if (lane == 0) {
+        const double res = sqrt(x_c) / sm[0];
+        double maxerr = sm[3];
+        int done = 0;
+        if (res < maxerr) done = 1;
+        else {
+            if (iter == L.maxiter / 2) maxerr = maxerr * 10;
+            if (iter >= L.maxiter - 2) maxerr = maxerr * 10;
+        }
+        gsm[2] = res; gsm[3] = maxerr; gsm[4] = done; gsm[5] = iter;
+        if (host) { host[2] = res; host[3] = maxerr; host[4] = done; host[5] = iter; }
+    }
+#undef HH
+#undef RN
+#undef QN
+}
+
+// h = sum of part_in, v -= sum_j h[j] Q_j (hcol set or, with add, incremented); returns the
+// work-group's partial of |v|^2 in every thread
+template <typename T>
+__device__ __forceinline__ double update_body(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
+                                               long long ld, const double* __restrict__ part_in,
+                                               double* hcol, int add, int bx, int nbx)
+{
     constexpr int W = kvec<T>::W;
     __shared__ double hs[64];
     __shared__ double sh[RW][1];
     __shared__ double red[1];
-    __shared__ double g1[2];
     const int tid = threadIdx.x;
-    if (gate_w) {
-        const double nw = sum_one(gate_w, nbx, &g1[0]);
-        const double nv2 = sum_one(gate_v, nbx, &g1[1]);
-        if (nv2 >= 0.5 * nw) {
-            if (normpart && tid == 0) normpart[bx] = gate_v[bx];
-            return;
-        }
-    }
     sum_partials(part_in, nbx, k, hs, hcol, add, bx);
     double nacc[1] = {0.0};
     const long long nv = (n3 + W - 1) / W;
@@ -615,18 +749,72 @@ __device__ __forceinline__ void k_maxpy_body(T* __restrict__ v, const T* __restr
             }
         }
     }
-    if (!normpart) return;
     block_sums<1>(nacc, sh, red);
-    if (tid == 0) normpart[bx] = red[0];
+    return red[0];
 }
+
+// The first pass's update where it has a kernel of its own (k > 12)
 template <typename T>
 __global__ void __launch_bounds__(RT) k_maxpy(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
                                               long long ld, const double* __restrict__ part_in,
-                                              double* __restrict__ hcol, int add, double* __restrict__ normpart,
-                                              const double* __restrict__ stop, const double* __restrict__ gate_w,
-                                              const double* __restrict__ gate_v)
+                                              double* __restrict__ hcol, const double* __restrict__ stop)
 {
-    k_maxpy_body<T>(v, Q, k, n3, ld, part_in, hcol, add, normpart, stop, gate_w, gate_v, blockIdx.x, gridDim.x);
+    if (*stop != 0.0) return;
+    update_body<T>(v, Q, k, n3, ld, part_in, hcol, 0, blockIdx.x, gridDim.x);
+}
+
+// The end of iteration k: the second pass's update, then the least-squares update with
+// H(k + 1, k) = |v|.  gate_w and gate_v hold the partials of |w|^2 before the first pass and of
+// |v|^2 after it; when the first pass kept at least 1/sqrt(2) of the norm (|v|^2 >= |w|^2 / 2, the
+// DGKS criterion) the second pass's corrections are below rounding, its update is skipped (v and
+// hcol stay) and work-group 0 goes on by itself, its upper wavefronts having loaded the small
+// problem while the lower ones summed the gate.  Otherwise the last work-group to arrive (arrive
+// counts them and is left zero) sums the partials and goes on.  As two kernels the update and
+// the single wavefront of the least squares took 5.2 + 7.8 us at 100 000 droplets.
+// ls: ls_doubles(k) of LDS.
+template <typename T>
+__device__ __forceinline__ void k_finish_body(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
+                                               long long ld, const double* __restrict__ part_in,
+                                               double* hcol, double* __restrict__ normpart,
+                                               const double* __restrict__ stop, const double* __restrict__ gate_w,
+                                               const double* __restrict__ gate_v, double* gsm, GmSmall L, int* arrive,
+                                               double* host, double* ls, int bx, int nbx)
+{
+    __shared__ double g1[2];
+    __shared__ int last;
+    if (*stop != 0.0) return;
+    const int tid = threadIdx.x;
+    if (bx == 0 && tid >= RT / 2) ls_load(ls, gsm, L, k, tid - RT / 2, RT / 2);
+    const double nw = sum_one(gate_w, nbx, &g1[0]);
+    double nv2 = sum_one(gate_v, nbx, &g1[1]);
+    if (nv2 >= 0.5 * nw) {
+        if (bx != 0) return;
+    } else {
+        const double mine = update_body<T>(v, Q, k, n3, ld, part_in, hcol, 1, bx, nbx);
+        if (tid == 0) {
+            normpart[bx] = mine;
+            __threadfence();                       // the partial and hcol, before the arrival
+            last = atomicAdd(arrive, 1) == nbx - 1;
+        }
+        __syncthreads();
+        if (!last) return;
+        __threadfence();
+        if (tid == 0) *arrive = 0;
+        ls_load(ls, gsm, L, k, tid, RT);
+        nv2 = sum_one(normpart, nbx, &g1[0]);
+    }
+    if (tid < LT) ls_solve(ls, gsm, L, k, sqrt(nv2), host);
+}
+template <typename T>
+__global__ void __launch_bounds__(RT) k_finish(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
+                                               long long ld, const double* __restrict__ part_in,
+                                               double* hcol, double* normpart, const double* stop,
+                                               const double* __restrict__ gate_w, const double* __restrict__ gate_v,
+                                               double* gsm, GmSmall L, int* arrive, double* host)
+{
+    extern __shared__ double ls_lds[];
+    k_finish_body<T>(v, Q, k, n3, ld, part_in, hcol, normpart, stop, gate_w, gate_v, gsm, L, arrive, host, ls_lds,
+                     blockIdx.x, gridDim.x);
 }
 
 // pertvel = x0 + Q y (2951-2956), scattered back to the reference's droplet order.  The
@@ -651,198 +839,6 @@ __global__ void k_solution(const double* x0, const T* Q, long long ld, const dou
     double* dst = pert + 3 * (size_t)sorted[t];
 #pragma unroll
     for (int c = 0; c < 3; ++c) dst[c] = out[c];
-}
-
-// Small least-squares update of HDI_GMRES (2904-2971), one wavefront.
-// sm layout: [0] norm_b [1] norm_rhs [2] res [3] maxerr [4] done [5] iter
-//            H at 16 + (r-1) + M1*(c-1), Rn after it, Qn after it, bn, y, v1, v2, resv
-struct GmSmall {
-    int maxiter;
-    __host__ __device__ int M1() const { return maxiter + 1; }
-    __host__ __device__ size_t H0() const { return 16; }
-    __host__ __device__ size_t R0() const { return H0() + (size_t)M1() * maxiter; }
-    __host__ __device__ size_t Q0() const { return R0() + (size_t)M1() * M1(); }
-    __host__ __device__ size_t B0() const { return Q0() + (size_t)M1() * M1(); }
-    __host__ __device__ size_t Y0() const { return B0() + M1(); }
-    __host__ __device__ size_t V1() const { return Y0() + M1(); }
-    __host__ __device__ size_t V2() const { return V1() + M1(); }
-    __host__ __device__ size_t RV() const { return V2() + M1(); }
-    __host__ __device__ size_t total() const { return RV() + M1(); }
-};
-
-constexpr int LT = 64;         // k_ls: one wavefront; maxiter + 1 <= LT
-constexpr int LS_MAX = 8192;   // GmSmall::total() for maxiter <= 50, the reference's value
-
-__device__ void ls_solve(double* sm, GmSmall L, int iter);
-
-__device__ __forceinline__ void copy_range(double* dst, const double* src, size_t a, size_t b)
-{
-    for (size_t i = a + threadIdx.x; i < b; i += LT) dst[i] = src[i];
-}
-
-// The five ranges of the small problem that an iteration reads, copied to LDS with
-// the loads of up to 8 * LT values issued together: one memory round trip for the
-// usual iteration counts instead of one per range and pass.
-__device__ __forceinline__ void copy_in(double* sm, const double* __restrict__ gsm, GmSmall L, int iter)
-{
-    constexpr int KB = 8;
-    const size_t M1 = L.M1();
-    const size_t n0 = 16, n1 = M1 * iter, n2 = M1 * iter, n3 = M1 * (iter + 1), n4 = L.total() - L.B0();
-    const size_t tot = n0 + n1 + n2 + n3 + n4;
-    for (size_t b = 0; b < tot; b += (size_t)KB * LT) {
-        double r[KB];
-        size_t at[KB];
-#pragma unroll
-        for (int k = 0; k < KB; ++k) {
-            size_t j = b + (size_t)k * LT + threadIdx.x;
-            at[k] = ~(size_t)0;
-            if (j < tot) {
-                size_t a;
-                if (j < n0) a = j;
-                else if ((j -= n0) < n1) a = L.H0() + j;
-                else if ((j -= n1) < n2) a = L.R0() + j;
-                else if ((j -= n2) < n3) a = L.Q0() + j;
-                else a = L.B0() + (j - n3);
-                at[k] = a;
-                r[k] = gsm[a];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < KB; ++k)
-            if (at[k] != ~(size_t)0) sm[at[k]] = r[k];
-    }
-}
-
-__device__ __forceinline__ void k_ls_body(double* gsm, GmSmall L, int iter, const double* __restrict__ normpart,
-                                          int P, int bx, int nbx)
-{
-    // the part of the small problem this iteration touches is copied to LDS, solved
-    // there, and the changed part copied back
-    __shared__ double sm[LS_MAX];
-    const size_t M1 = L.M1();
-    // H(iter+1, iter) = |v| from the partials of the last projection kernel; their
-    // loads are issued together with those of the LDS copy
-    static_assert(RED_BLOCKS % LT == 0, "partials per lane");
-    double np[RED_BLOCKS / LT];
-#pragma unroll
-    for (int k = 0; k < RED_BLOCKS / LT; ++k) {
-        const int b = threadIdx.x + k * LT;
-        np[k] = b < P ? normpart[b] : 0.0;
-    }
-    const double done = gsm[4];
-    copy_in(sm, gsm, L, iter);
-    if (done != 0.0) return;     // converged in an earlier iteration of this batch
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < RED_BLOCKS / LT; ++k) acc += np[k];
-    acc = wave_sum(acc);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const size_t e = L.H0() + iter + M1 * (iter - 1);
-        sm[e] = gsm[e] = sqrt(acc);
-    }
-    __syncthreads();
-    ls_solve(sm, L, iter);
-    __syncthreads();
-    copy_range(gsm, sm, 0, 16);
-    copy_range(gsm, sm, L.R0(), L.R0() + M1 * iter);
-    copy_range(gsm, sm, L.Q0(), L.Q0() + M1 * (iter + 1));
-    copy_range(gsm, sm, L.B0(), L.total());
-}
-
-__global__ void __launch_bounds__(LT) k_ls(double* gsm, GmSmall L, int iter, const double* __restrict__ normpart,
-                                          int P)
-{
-    k_ls_body(gsm, L, iter, normpart, P, blockIdx.x, gridDim.x);
-}
-
-// All LT lanes call it.  Lane r owns row r + 1 of the triangular factor and of the
-// residual; the Givens rotation and the back substitution run over the lanes.
-__device__ void ls_solve(double* sm, GmSmall L, int iter)
-{
-    const int lane = threadIdx.x;
-    const int M1 = L.M1();
-    double* H = sm + L.H0();
-    double* Rn = sm + L.R0();
-    double* Qn = sm + L.Q0();
-    double* bn = sm + L.B0();
-    double* y = sm + L.Y0();
-    double* rv = sm + L.RV();
-#define HH(r, c) H[((r) - 1) + (size_t)M1 * ((c) - 1)]
-#define RN(r, c) Rn[((r) - 1) + (size_t)M1 * ((c) - 1)]
-#define QN(r, c) Qn[((r) - 1) + (size_t)M1 * ((c) - 1)]
-    const double norm_rhs = sm[1];
-    if (iter == 1) {
-        if (lane == 0) {
-            const double nrm = sqrt(HH(1, 1) * HH(1, 1) + HH(2, 1) * HH(2, 1));
-            const double q11 = HH(1, 1) / nrm, q21 = HH(2, 1) / nrm;
-            QN(1, 1) = q11; QN(2, 1) = q21;
-            QN(1, 2) = q21; QN(2, 2) = -q11;
-            RN(1, 1) = sqrt(HH(1, 1) * HH(1, 1) + HH(2, 1) * HH(2, 1));
-            bn[0] = q11 * norm_rhs;
-            y[0] = bn[0] / RN(1, 1);
-        }
-        __syncthreads();
-    } else {
-        // new column of R: Qn(1:iter, 1:iter) H(1:iter, iter)
-        if (lane < iter) {
-            double acc = 0.0;
-            for (int c = 1; c <= iter; ++c) acc = acc + QN(lane + 1, c) * HH(c, iter);
-            RN(lane + 1, iter) = acc;
-        }
-        __syncthreads();
-        const double aa = RN(iter, iter), bb = HH(iter + 1, iter);
-        const double dd = sqrt(aa * aa + bb * bb);
-        const double cc = aa / dd, ss = bb / dd;
-        const double qi = lane < iter ? QN(iter, lane + 1) : 0.0;
-        __syncthreads();
-        // rows iter and iter+1 of Qn after the rotation
-        if (lane < iter) { QN(iter, lane + 1) = cc * qi; QN(iter + 1, lane + 1) = -ss * qi; }
-        if (lane == iter) { QN(iter, iter + 1) = ss; QN(iter + 1, iter + 1) = cc; }
-        if (lane == 0) RN(iter, iter) = dd;
-        __syncthreads();
-        if (lane == 0) {
-            bn[iter - 2] = QN(iter - 1, 1) * norm_rhs;
-            bn[iter - 1] = QN(iter, 1) * norm_rhs;
-        }
-        __syncthreads();
-        // back substitution by columns: lane r accumulates row r + 1
-        double acc = 0.0;
-        for (int c = iter; c >= 1; --c) {
-            if (lane == c - 1) y[c - 1] = (bn[c - 1] - acc) / RN(c, c);
-            __syncthreads();
-            const double yc = y[c - 1];
-            if (lane < c - 1) acc = acc + yc * RN(lane + 1, c);
-        }
-        __syncthreads();
-    }
-    // residual H y - |r0| e1 (2958-2966)
-    if (lane <= iter) {
-        double acc = 0.0;
-        for (int c = 1; c <= iter; ++c) acc = acc + HH(lane + 1, c) * y[c - 1];
-        rv[lane] = acc;
-    }
-    __syncthreads();
-    if (lane == 0) {
-        rv[0] = rv[0] - norm_rhs;
-        double x_c = 0.0;
-        for (int r = 0; r <= iter; ++r) x_c = x_c + rv[r] * rv[r];
-        const double res = sqrt(x_c) / sm[0];
-        sm[2] = res;
-        sm[5] = iter;
-        double maxerr = sm[3];
-        int done = 0;
-        if (res < maxerr) done = 1;
-        else {
-            if (iter == L.maxiter / 2) maxerr = maxerr * 10;
-            if (iter >= L.maxiter - 2) maxerr = maxerr * 10;
-        }
-        sm[3] = maxerr;
-        sm[4] = done;
-    }
-#undef HH
-#undef RN
-#undef QN
 }
 
 // ------------------------------------------------------------------ driver
@@ -895,9 +891,10 @@ static int hdi_begin(PartBuffers& pb, const PartConst& pc, int maxiter, double t
 {
     const int n = pc.n;
     const long long n3 = 3LL * n;
-    if (maxiter + 1 > LT) { set_error("GMRES maxiter too large (at most 50)"); return DDNS_ERR_ARG; }
+    static_assert(LS_MAXITER + 1 <= LT && ls_doubles(LS_MAXITER) * sizeof(double) <= 63 * 1024, "least squares in one wavefront, in LDS");
+    if (maxiter > LS_MAXITER) { set_error("GMRES maxiter too large (at most 50)"); return DDNS_ERR_ARG; }
     GmSmall L{maxiter};
-    if (L.total() > (size_t)LS_MAX) { set_error("GMRES maxiter too large (at most 50)"); return DDNS_ERR_ARG; }
+    if (!pb.gm_host) DDNS_HIP(hipHostMalloc((void**)&pb.gm_host, 16 * sizeof(double), hipHostMallocDefault));
     // Krylov storage
     if (!pb.gm_small) {
         DDNS_HIP(hipMalloc(&pb.gm_small, 16384 * sizeof(double)));
@@ -921,17 +918,20 @@ static int hdi_begin(PartBuffers& pb, const PartConst& pc, int maxiter, double t
     hipLaunchKernelGGL((k_residual0<T>), dim3(nr0), dim3(HT), 0, s, pb.gm_b, ax0, Q, n3, pb.gm_red);
     // the tolerance, and the stop flag when the initial residual is below 1e-5
     // (2866-2868): then no iteration runs and pertvel keeps its warm-start value
-    hipLaunchKernelGGL(k_gm_start, dim3(1), dim3(HT), 0, s, sm, (int)L.total(), tol, (const double*)pb.gm_red, nr0);
+    hipLaunchKernelGGL(k_gm_start, dim3(1), dim3(HT), 0, s, sm, (int)L.total(), tol, (const double*)pb.gm_red, nr0,
+                       (const int*)pb.flags, pb.gm_host);
     hipLaunchKernelGGL((k_scale<T>), dim3(nb3), dim3(HT), 0, s, Q, sm + 1, n3);
     DDNS_HIP(hipGetLastError());
     return 0;
 }
 
-// work-groups of the projection kernels of a system of n droplets
+// work-groups of the projection kernels of a system of n droplets: as many as have about 700
+// rows each.  With twice the rows the 74 work-groups of 100 000 droplets left most CUs idle (a
+// solve 0.37 against 0.33 ms at 78 000 droplets in FP64, 0.73 against 0.58 at 60 000); with half
+// of them the merged launches of a batch grew from 4.6 to 5.2 ms a step.
 static int hdi_nred(int n)
 {
-    const long long n3 = 3LL * n;
-    return (int)std::min<long long>(RED_BLOCKS, (n3 + 4LL * RT - 1) / (4LL * RT));
+    return (int)std::min<long long>(RED_BLOCKS, (3LL * n + 2LL * RT - 1) / (2LL * RT));
 }
 
 template <typename T>
@@ -1019,30 +1019,27 @@ static int hdi_impl(PartBuffers& pb, const PartConst& pc, int maxiter, double to
                                        (const double*)part1, hcol, part2, stop);
                 else {
                     hipLaunchKernelGGL((k_maxpy<T>), dim3(nred), dim3(RT), 0, s, v, (const T*)Q, it, n3, ld,
-                                       (const double*)part1, hcol, 0, (double*)nullptr, stop, (const double*)nullptr,
-                                       (const double*)nullptr);
+                                       (const double*)part1, hcol, stop);
                     hipLaunchKernelGGL((k_mdot<T>), dim3(nred), dim3(RT), 0, s, (const T*)Q, (const T*)v, it, n3, ld, part2,
                                        stop);
                 }
-                // the second pass's update, skipped where the first kept 1/sqrt(2) of |v|
-                hipLaunchKernelGGL((k_maxpy<T>), dim3(nred), dim3(RT), 0, s, v, (const T*)Q, it, n3, ld, (const double*)part2,
-                                   hcol, 1, normpart, stop, (const double*)(part1 + (size_t)it * nred),
-                                   (const double*)(part2 + (size_t)it * nred));
-                hipLaunchKernelGGL(k_ls, dim3(1), dim3(LT), 0, s, sm, L, it, (const double*)normpart, (int)nred);
+                // the second pass's update, skipped where the first kept 1/sqrt(2) of |v|, and the
+                // least squares
+                hipLaunchKernelGGL((k_finish<T>), dim3(nred), dim3(RT), ls_doubles(it) * sizeof(double), s, v, (const T*)Q,
+                                   it, n3, ld, (const double*)part2, hcol, normpart, stop,
+                                   (const double*)(part1 + (size_t)it * nred), (const double*)(part2 + (size_t)it * nred),
+                                   sm, L, pb.flags + 56, pb.gm_host);
             }
             DDNS_HIP(hipGetLastError());
             iter = last;
-            // the first check also reads the neighbour lists' flags (pinned memory: the two
-            // copies are queued together and waited for once)
-            if (!pb.gm_host) DDNS_HIP(hipHostMalloc((void**)&pb.gm_host, 16 * sizeof(double), hipHostMallocDefault));
+            // the kernels leave the small problem's head, and the start the neighbour lists'
+            // flags, in host memory (two copies took the stream 10 us)
             int f[8];
-            int* fh = (int*)(pb.gm_host + 8);
-            if (first) DDNS_HIP(hipMemcpyAsync(fh, pb.flags, sizeof(f), hipMemcpyDeviceToHost, s));
-            DDNS_HIP(hipMemcpyAsync(pb.gm_host, sm, sizeof(st6), hipMemcpyDeviceToHost, s));
+            const int* fh = (const int*)(pb.gm_host + 8);
             if (!pb.sync_ev) DDNS_HIP(hipEventCreateWithFlags(&pb.sync_ev, hipEventDisableTiming));
             DDNS_HIP(hipEventRecord(pb.sync_ev, s));
             // the solution as far as this batch got (pertvel = x0 where no iteration ran),
-            // queued behind the copies: when the batch converged, the usual case, it runs
+            // queued behind the event: when the batch converged, the usual case, it runs
             // while the host reads the check and queues what follows; a later batch is
             // followed by its own
             hipLaunchKernelGGL((k_solution<T>), dim3(nbr), dim3(HT), 0, s, pb.gm_x0, (const T*)Q, ld, sm + L.Y0(),
@@ -1097,6 +1094,7 @@ struct GmDesc {
     const int* idx;
     const T* mm;
     const int* flags;          // the neighbour lists' flags (read at the first check)
+    int* arrive;               // counter of k_finish
     T* Q;                      // maxiter Krylov columns, then the two work vectors
     double* sm;                // the small problem (GmSmall layout)
     double* part1;             // first-pass projection partials
@@ -1172,27 +1170,25 @@ __global__ void __launch_bounds__(RT) kb_maxpy_mdot(const GmDesc<T>* __restrict_
     k_maxpy_mdot_body<T, KC>(q.v, g.Q, it, g.n3, g.ld, g.part1, q.hcol, g.part2, q.stop, blockIdx.x, g.nred);
 }
 
-// second = 0: the first pass's update (k > 12); 1: the second pass's DGKS-gated update
 template <typename T>
-__global__ void __launch_bounds__(RT) kb_maxpy(const GmDesc<T>* __restrict__ d, GmSmall L, int it, int second)
+__global__ void __launch_bounds__(RT) kb_maxpy(const GmDesc<T>* __restrict__ d, GmSmall L, int it)
 {
     const GmDesc<T>& g = d[blockIdx.y];
     if ((int)blockIdx.x >= g.nred) return;
     const GmIter<T> q = gm_iter(g, L, it);
-    if (second)
-        k_maxpy_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part2, q.hcol, 1, g.normpart, q.stop,
-                        g.part1 + (size_t)it * g.nred, g.part2 + (size_t)it * g.nred, blockIdx.x, g.nred);
-    else
-        k_maxpy_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part1, q.hcol, 0, nullptr, q.stop, nullptr, nullptr, blockIdx.x,
-                        g.nred);
+    if (*q.stop != 0.0) return;
+    update_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part1, q.hcol, 0, blockIdx.x, g.nred);
 }
 
 template <typename T>
-__global__ void __launch_bounds__(LT) kb_ls(const GmDesc<T>* __restrict__ d, GmSmall L, int it)
+__global__ void __launch_bounds__(RT) kb_finish(const GmDesc<T>* __restrict__ d, GmSmall L, int it)
 {
-    const GmDesc<T>& g = d[blockIdx.x];
-    if (g.nred == 0) return;
-    k_ls_body(g.sm, L, it, g.normpart, g.nred, 0, 1);
+    extern __shared__ double ls_lds[];
+    const GmDesc<T>& g = d[blockIdx.y];
+    if ((int)blockIdx.x >= g.nred) return;
+    const GmIter<T> q = gm_iter(g, L, it);
+    k_finish_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part2, q.hcol, g.normpart, q.stop, g.part1 + (size_t)it * g.nred,
+                     g.part2 + (size_t)it * g.nred, g.sm, L, g.arrive, nullptr, ls_lds, blockIdx.x, g.nred);
 }
 
 // each system's small-problem head sm[0..5] (and its lists' flags) into 16 doubles
@@ -1246,6 +1242,7 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
             continue;
         }
         g.cnt = pb.nei_cnt; g.idx = pb.nei_idx; g.mm = (const T*)pb.nei_m; g.flags = pb.flags;
+        g.arrive = pb.flags + 56;
         g.Q = (T*)pb.gm_Q; g.sm = pb.gm_small;
         g.part1 = pb.gm_red; g.part2 = g.part1 + (size_t)64 * RED_BLOCKS; g.normpart = g.part2 + (size_t)64 * RED_BLOCKS;
         g.n3 = 3LL * n; g.ld = (g.n3 + 63) / 64 * 64; g.n = n;
@@ -1279,11 +1276,10 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
             if (it <= 8) hipLaunchKernelGGL((kb_maxpy_mdot<T, 8>), g, dim3(RT), 0, s, td, L, it);
             else if (it <= 12) hipLaunchKernelGGL((kb_maxpy_mdot<T, 12>), g, dim3(RT), 0, s, td, L, it);
             else {
-                hipLaunchKernelGGL((kb_maxpy<T>), g, dim3(RT), 0, s, td, L, it, 0);
+                hipLaunchKernelGGL((kb_maxpy<T>), g, dim3(RT), 0, s, td, L, it);
                 hipLaunchKernelGGL((kb_mdot<T>), g, dim3(RT), 0, s, td, L, it, 1);
             }
-            hipLaunchKernelGGL((kb_maxpy<T>), g, dim3(RT), 0, s, td, L, it, 1);
-            hipLaunchKernelGGL((kb_ls<T>), dim3(R), dim3(LT), 0, s, td, L, it);
+            hipLaunchKernelGGL((kb_finish<T>), g, dim3(RT), ls_doubles(it) * sizeof(double), s, td, L, it);
         }
         DDNS_HIP(hipGetLastError());
         iter = last;
