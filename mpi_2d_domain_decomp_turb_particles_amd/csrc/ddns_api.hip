@@ -769,8 +769,7 @@ static int run_flow_steps(ddns_handle* h, int nsteps)
         auto body = [&]() {
             int st = 0;
             for (int k = 0; k < n && !st; ++k) {
-                st = flow_step(h->fb, h->fc, h->prec, FLOW_INV, s, nullptr);
-                if (!st) st = flow_step(h->fb, h->fc, h->prec, FLOW_FWD, s, nullptr);
+                st = flow_step(h->fb, h->fc, h->prec, FLOW_STEP, s, nullptr);
             }
             return st;
         };

@@ -309,7 +309,7 @@ int flow_prologue(const FlowBuffers& fb, const FlowConst& fc, int precision, hip
 // forward half in two pieces (forward y + pre, then z + sym) so that a wait can sit
 // between them.  capturing: the stream is being captured into a graph (the events
 // become graph nodes).
-enum FlowPart { FLOW_INV = 0, FLOW_FWD = 1, FLOW_FWD_Y = 2, FLOW_FWD_Z = 3 };
+enum FlowPart { FLOW_INV = 0, FLOW_FWD = 1, FLOW_FWD_Y = 2, FLOW_FWD_Z = 3, FLOW_STEP = 4 };
 int flow_step(const FlowBuffers& fb, const FlowConst& fc, int precision, int part, hipStream_t s,
               hipEvent_t* ev /* FLOW_EVENTS events or nullptr */, bool capturing = false);
 constexpr int FLOW_EVENTS = 9;

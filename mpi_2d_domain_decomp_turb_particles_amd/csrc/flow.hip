@@ -457,12 +457,14 @@ __global__ void __launch_bounds__((TC * (N / col_e<T, N>()))) k_y(KyArgs a)
 // ------------------------------------------------------------------ x stage
 // Half-length packing of a real line of N points as N/2 complex points.
 template <int N> constexpr int kx_lines() { return 2048 / N; }   // 4 complex points per thread
-#ifndef DDNS_KXF_PTS
-#define DDNS_KXF_PTS 2048
-#endif
-// lines of one k_x_fused work-group: DDNS_KXF_PTS / N (QP = DDNS_KXF_PTS / 512 complex
-// points per thread and field)
-template <int N> constexpr int kxf_lines() { return DDNS_KXF_PTS / N >= 1 ? DDNS_KXF_PTS / N : 1; }
+// lines of one k_x_fused work-group: 4 complex points per thread and field, and the least that
+// 16-byte accesses allow (1 in FP64, 2 in FP32) up to 64^3, where 4 left 16 or 128 work-groups
+// for 256 CUs, each with four times the serial work: 32^3 FP64 18.8 -> 13.1 us, FP32 16.1 -> 13.9;
+// 64^3 20.5 -> 15.1, 16.7 -> 13.6; at 128^3 the small tile is the slower one (FP32 28.9 -> 34.5)
+template <typename T, int N> constexpr int kxf_lines()
+{
+    return (N <= 64 ? 8192 / (int)sizeof(cpx<T>) : 2048) / N;
+}
 
 // C2R pre-processing of the tile (in place, pairs k and M-k of every line).
 template <typename T, int N, int TL, int LDR>
@@ -538,90 +540,6 @@ __device__ __forceinline__ void store_node_pair(double* p, double a0, double b0,
     ((double2*)p)[0] = make_double2(a0, b0);
     ((double2*)p)[1] = make_double2(c0, a1);
     ((double2*)p)[2] = make_double2(b1, c1);
-}
-
-// Fused x stage: six C2R (u, w), physical u for the droplets, u x w, three R2C.
-// The C2R transforms run two fields at a time and the R2C transforms three at a time
-// through the same FFT passes, so every pass has two or three butterflies per lane;
-// the next pair's loads are in flight while the current pair is transformed.
-template <typename T, int N>
-__global__ void __launch_bounds__(NT) k_x_fused(KxArgs a)
-{
-    using C = cpx<T>;
-    constexpr int M = N / 2;
-    constexpr int TL = kxf_lines<N>();
-    constexpr int LDR = TL + 1;
-    constexpr int TS = M * LDR;
-    constexpr int QP = TL * M / NT;
-    static_assert((TL * M) % NT == 0, "the lines must split evenly over the work-group");
-    __shared__ C lds[3 * TS];
-    __shared__ C tws[N], twhs[M];
-    const int tid = threadIdx.x;
-    const size_t line0 = (size_t)blockIdx.x * TL;
-    stage_twiddles<C, N, NT>(tws, (const C*)a.tw, tid);
-    stage_twiddles<C, M, NT>(twhs, (const C*)a.twh, tid);
-    const C* tw = tws;
-    const C* twh = twhs;
-    C ph[6][QP];
-    TileRegs<C, TL, M, NT> next0, next1;
-    // field f of this work-group's lines; every line is read before it is written
-    auto fetch = [&](TileRegs<C, TL, M, NT>& r, int f) {
-        if (f < 3) tile_fetch<C, TL, M, NT>(r, (const C*)a.B[f] + line0 * M, M, tid);
-        else tile_fetch<C, TL, M, NT>(r, (const C*)a.uphys + (3 * line0 + f - 3) * M, 3 * M, tid);
-    };
-    fetch(next0, 0);
-    fetch(next1, 1);
-#pragma unroll
-    for (int f = 0; f < 6; f += 2) {
-        tile_put<C, TL, M, LDR, NT, true>(lds, next0, tid);
-        tile_put<C, TL, M, LDR, NT, true>(lds + TS, next1, tid);
-        if (f < 4) {
-            fetch(next0, f + 2);
-            fetch(next1, f + 3);
-        }
-        __syncthreads();
-        c2r_pack<T, N, TL, LDR>(lds, tw, tid);
-        c2r_pack<T, N, TL, LDR>(lds + TS, tw, tid);
-        __syncthreads();
-        fft_tile<T, M, true, TL, LDR, NT, 2, TS>(lds, twh, tid);
-#pragma unroll
-        for (int q = 0; q < QP; ++q) {
-            const int e = tid + NT * q;
-            const int line = e / M, m = e % M;
-            ph[f][q] = lds[m * LDR + line];
-            ph[f + 1][q] = lds[TS + m * LDR + line];
-        }
-        __syncthreads();
-    }
-    // physical velocity for the droplet gather: [line][x][3], the two nodes of a complex
-    // value in three vector stores
-    {
-        T* up = (T*)a.uphys + line0 * (size_t)N * 3;
-#pragma unroll
-        for (int q = 0; q < QP; ++q) {
-            const int e = tid + NT * q;
-            const int line = e / M, m = e % M;
-            T* p = up + ((size_t)line * N + 2 * m) * 3;
-            store_node_pair(p, ph[0][q].x, ph[1][q].x, ph[2][q].x, ph[0][q].y, ph[1][q].y, ph[2][q].y);
-        }
-    }
-    // nonlinear term u x w (turb.f90:634-637) in natural component order, into the
-    // three tiles
-#pragma unroll
-    for (int q = 0; q < QP; ++q) {
-        const int e = tid + NT * q;
-        const int line = e / M, m = e % M;
-        const C ux = ph[0][q], uy = ph[1][q], uz = ph[2][q];
-        const C wx = ph[3][q], wy = ph[4][q], wz = ph[5][q];
-        lds[m * LDR + line] = mk<C>(uy.x * wz.x - uz.x * wy.x, uy.y * wz.y - uz.y * wy.y);
-        lds[TS + m * LDR + line] = mk<C>(uz.x * wx.x - ux.x * wz.x, uz.y * wx.y - ux.y * wz.y);
-        lds[2 * TS + m * LDR + line] = mk<C>(ux.x * wy.x - uy.x * wx.x, ux.y * wy.y - uy.y * wx.y);
-    }
-    __syncthreads();
-    fft_tile<T, M, false, TL, LDR, NT, 3, TS>(lds, twh, tid);
-    const T scale = (T)1 / (T)N;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) r2c_unpack_store<T, N, TL, LDR>(lds + c * TS, tw, (C*)a.B[c], line0, scale, tid);
 }
 
 // Stand-alone x transforms of one field (kernel-level parity of mpifft3DRC/CR).
@@ -751,6 +669,160 @@ __device__ __forceinline__ void sth_hermitian(double* t, int q)
     if (q == 0) { t[0] = 0.0; t[1] = 0.0; }
 }
 
+// supforSTH by the whole work-group: the draws by one wavefront, then one mode per thread (225
+// modes of white noise, 150 table entries per component).  The loops over the tables run once per
+// step on one work-group, so latency is all they cost (24 us, half of them the chain of draws).
+// It reads no field of the step: where a whole step is queued at once, a work-group of the x
+// stage does it beside the lines (a step at 64^3 FP32 64 -> 55 us, at 32^3 FP64 63 -> 44, at 128^3
+// FP32 107 -> 88).
+constexpr int OU_SCRATCH = 900 + 225;          // doubles of LDS
+__device__ __forceinline__ void ou_step(const PreArgs& a, int rr, double* scratch)
+{
+    const int tid = threadIdx.x;
+    double* low = a.low + (size_t)rr * LOW_STRIDE;
+    const bool own = a.forcing < 0;
+    int* st = a.sth_state + (size_t)rr * STH_STATE_STRIDE;
+    double (*fr)[150] = (double (*)[150])scratch, (*fo)[150] = fr + 3;
+    int* seq = (int*)(scratch + 900);
+    const double dt = a.dt, tf = own ? low[LOW_PAR + 3] : a.ou_tf, var = own ? low[LOW_PAR + 4] : a.ou_var;
+    const double pi2 = a.pi2;
+    if (tid < 64) ranff_draws(st, 450, seq);
+    __syncthreads();
+    if (tid < 225) {                                                 // flowlib.f90:405-419
+        const double AM = 1.0 / 2147483647, RNMX = 1.0 - 1.2e-7;
+        double cont1 = AM * (double)seq[2 * tid], rph = AM * (double)seq[2 * tid + 1];
+        cont1 = cont1 < RNMX ? cont1 : RNMX;
+        rph = rph < RNMX ? rph : RNMX;
+        if (cont1 < 1.e-6) cont1 = 1.e-6;
+        const double rmag = sqrt(-4.0 * var * dt * log(cont1) / tf);
+        const int mc = tid / 75, o = 2 * (tid % 75);
+        fr[mc][o] = rmag * cos(pi2 * rph);
+        fr[mc][o + 1] = rmag * sin(pi2 * rph);
+    }
+    __syncthreads();
+    if (tid < 36) sth_hermitian(fr[tid / 12], tid % 12);             // 424-440
+    __syncthreads();
+    double* b = a.sth_b + (size_t)rr * STH_B_STRIDE;
+    double* fa = low + 8;
+    if (tid < 150) {                                                 // 447-478
+        const double smallx = 1.0e-18, xkf = sqrt(8.0);
+        const int o = tid, i = o % 6, j = (o / 6) % 5, k = o / 30;
+        const double kx_ = (double)(i / 2);
+        const double ky_ = (double)(j <= 2 ? j : j - 5);
+        const double kz_ = (double)(k <= 2 ? k : k - 5);
+        const double radm = sqrt(kx_ * kx_ + ky_ * ky_ + kz_ * kz_);
+        double f0 = 0.0, f1 = 0.0, f2 = 0.0;
+        if (radm < xkf) {
+            const double b0 = b[o] * (1.0 - dt / tf) + fr[0][o];
+            const double b1 = b[150 + o] * (1.0 - dt / tf) + fr[1][o];
+            const double b2 = b[300 + o] * (1.0 - dt / tf) + fr[2][o];
+            b[o] = b0; b[150 + o] = b1; b[300 + o] = b2;
+            const double t1 = kx_ * b0, t2 = ky_ * b1, t3 = kz_ * b2;
+            double divb = (t1 + t2 + t3) / ((radm + smallx) * (radm + smallx));
+            if (radm == 0.) divb = 0.0;
+            f0 = b0 - kx_ * divb;
+            f1 = b1 - ky_ * divb;
+            f2 = b2 - kz_ * divb;
+        }
+        fo[0][o] = f0; fo[1][o] = f1; fo[2][o] = f2;
+    }
+    __syncthreads();
+    if (tid < 36) sth_hermitian(fo[tid / 12], tid % 12);             // 481-510
+    __syncthreads();
+    for (int e = tid; e < 450; e += NT) fa[e] = fo[e / 150][e % 150];
+}
+
+// Fused x stage: six C2R (u, w), physical u for the droplets, u x w, three R2C.
+// The C2R transforms run two fields at a time and the R2C transforms three at a time
+// through the same FFT passes, so every pass has two or three butterflies per lane;
+// the next pair's loads are in flight while the current pair is transformed.
+// OU: the first nou work-groups do the step's stochastic forcing (ou_step), one a realisation.
+template <typename T, int N, bool OU>
+__global__ void __launch_bounds__(NT) k_x_fused(KxArgs a, PreArgs pre, int nou)
+{
+    using C = cpx<T>;
+    constexpr int M = N / 2;
+    constexpr int TL = kxf_lines<T, N>();
+    constexpr int LDR = TL + 1;
+    constexpr int TS = M * LDR;
+    constexpr int QP = TL * M / NT;
+    static_assert((TL * M) % NT == 0, "the lines must split evenly over the work-group");
+    constexpr size_t LDS = 3 * TS * sizeof(C), NEED = OU && LDS < OU_SCRATCH * sizeof(double) ? OU_SCRATCH * sizeof(double) : LDS;
+    __shared__ __align__(16) char ldsb[NEED];
+    C* const lds = (C*)ldsb;
+    __shared__ C tws[N], twhs[M];
+    const int tid = threadIdx.x;
+    if (OU && (int)blockIdx.x < nou) {
+        ou_step(pre, blockIdx.x, (double*)ldsb);
+        return;
+    }
+    const size_t line0 = (size_t)(blockIdx.x - (OU ? nou : 0)) * TL;
+    stage_twiddles<C, N, NT>(tws, (const C*)a.tw, tid);
+    stage_twiddles<C, M, NT>(twhs, (const C*)a.twh, tid);
+    const C* tw = tws;
+    const C* twh = twhs;
+    C ph[6][QP];
+    TileRegs<C, TL, M, NT> next0, next1;
+    // field f of this work-group's lines; every line is read before it is written
+    auto fetch = [&](TileRegs<C, TL, M, NT>& r, int f) {
+        if (f < 3) tile_fetch<C, TL, M, NT>(r, (const C*)a.B[f] + line0 * M, M, tid);
+        else tile_fetch<C, TL, M, NT>(r, (const C*)a.uphys + (3 * line0 + f - 3) * M, 3 * M, tid);
+    };
+    fetch(next0, 0);
+    fetch(next1, 1);
+#pragma unroll
+    for (int f = 0; f < 6; f += 2) {
+        tile_put<C, TL, M, LDR, NT, true>(lds, next0, tid);
+        tile_put<C, TL, M, LDR, NT, true>(lds + TS, next1, tid);
+        if (f < 4) {
+            fetch(next0, f + 2);
+            fetch(next1, f + 3);
+        }
+        __syncthreads();
+        c2r_pack<T, N, TL, LDR>(lds, tw, tid);
+        c2r_pack<T, N, TL, LDR>(lds + TS, tw, tid);
+        __syncthreads();
+        fft_tile<T, M, true, TL, LDR, NT, 2, TS>(lds, twh, tid);
+#pragma unroll
+        for (int q = 0; q < QP; ++q) {
+            const int e = tid + NT * q;
+            const int line = e / M, m = e % M;
+            ph[f][q] = lds[m * LDR + line];
+            ph[f + 1][q] = lds[TS + m * LDR + line];
+        }
+        __syncthreads();
+    }
+    // physical velocity for the droplet gather: [line][x][3], the two nodes of a complex
+    // value in three vector stores
+    {
+        T* up = (T*)a.uphys + line0 * (size_t)N * 3;
+#pragma unroll
+        for (int q = 0; q < QP; ++q) {
+            const int e = tid + NT * q;
+            const int line = e / M, m = e % M;
+            T* p = up + ((size_t)line * N + 2 * m) * 3;
+            store_node_pair(p, ph[0][q].x, ph[1][q].x, ph[2][q].x, ph[0][q].y, ph[1][q].y, ph[2][q].y);
+        }
+    }
+    // nonlinear term u x w (turb.f90:634-637) in natural component order, into the
+    // three tiles
+#pragma unroll
+    for (int q = 0; q < QP; ++q) {
+        const int e = tid + NT * q;
+        const int line = e / M, m = e % M;
+        const C ux = ph[0][q], uy = ph[1][q], uz = ph[2][q];
+        const C wx = ph[3][q], wy = ph[4][q], wz = ph[5][q];
+        lds[m * LDR + line] = mk<C>(uy.x * wz.x - uz.x * wy.x, uy.y * wz.y - uz.y * wy.y);
+        lds[TS + m * LDR + line] = mk<C>(uz.x * wx.x - ux.x * wz.x, uz.y * wx.y - ux.y * wz.y);
+        lds[2 * TS + m * LDR + line] = mk<C>(ux.x * wy.x - uy.x * wx.x, ux.y * wy.y - uy.y * wx.y);
+    }
+    __syncthreads();
+    fft_tile<T, M, false, TL, LDR, NT, 3, TS>(lds, twh, tid);
+    const T scale = (T)1 / (T)N;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) r2c_unpack_store<T, N, TL, LDR>(lds + c * TS, tw, (C*)a.B[c], line0, scale, tid);
+}
+
 // supforDET's 225 low-mode sums (75 modes kx in 0..2, ky, kz in -2..2, times 3
 // components) of the forward z transform of N-hat, by direct DFT: one work-group per
 // sum, lanes over z, a fixed-order reduction; the result, scaled by 1/N like the
@@ -802,58 +874,8 @@ __global__ void __launch_bounds__(NT) k_pre(PreArgs a)
     const int forcing = real_forcing(a.forcing, low);
     const bool own = a.forcing < 0;
     if (forcing == 2) {
-        // supforSTH by the whole work-group: the draws by one wavefront, then one mode per
-        // thread (225 modes of white noise, 150 table entries per component).  The loops over
-        // the tables run once per step on one work-group, so latency is all they cost.
-        int* st = a.sth_state + (size_t)rr * STH_STATE_STRIDE;
-        __shared__ int seq[450];
-        __shared__ double fr[3][150], fo[3][150];
-        const double dt = a.dt, tf = own ? low[LOW_PAR + 3] : a.ou_tf, var = own ? low[LOW_PAR + 4] : a.ou_var;
-        const double pi2 = a.pi2;
-        if (tid < 64) ranff_draws(st, 450, seq);
-        __syncthreads();
-        if (tid < 225) {                                                 // flowlib.f90:405-419
-            const double AM = 1.0 / 2147483647, RNMX = 1.0 - 1.2e-7;
-            double cont1 = AM * (double)seq[2 * tid], rph = AM * (double)seq[2 * tid + 1];
-            cont1 = cont1 < RNMX ? cont1 : RNMX;
-            rph = rph < RNMX ? rph : RNMX;
-            if (cont1 < 1.e-6) cont1 = 1.e-6;
-            const double rmag = sqrt(-4.0 * var * dt * log(cont1) / tf);
-            const int mc = tid / 75, o = 2 * (tid % 75);
-            fr[mc][o] = rmag * cos(pi2 * rph);
-            fr[mc][o + 1] = rmag * sin(pi2 * rph);
-        }
-        __syncthreads();
-        if (tid < 36) sth_hermitian(fr[tid / 12], tid % 12);             // 424-440
-        __syncthreads();
-        double* b = a.sth_b + (size_t)rr * STH_B_STRIDE;
-        double* fa = low + 8;
-        if (tid < 150) {                                                 // 447-478
-            const double smallx = 1.0e-18, xkf = sqrt(8.0);
-            const int o = tid, i = o % 6, j = (o / 6) % 5, k = o / 30;
-            const double kx_ = (double)(i / 2);
-            const double ky_ = (double)(j <= 2 ? j : j - 5);
-            const double kz_ = (double)(k <= 2 ? k : k - 5);
-            const double radm = sqrt(kx_ * kx_ + ky_ * ky_ + kz_ * kz_);
-            double f0 = 0.0, f1 = 0.0, f2 = 0.0;
-            if (radm < xkf) {
-                const double b0 = b[o] * (1.0 - dt / tf) + fr[0][o];
-                const double b1 = b[150 + o] * (1.0 - dt / tf) + fr[1][o];
-                const double b2 = b[300 + o] * (1.0 - dt / tf) + fr[2][o];
-                b[o] = b0; b[150 + o] = b1; b[300 + o] = b2;
-                const double t1 = kx_ * b0, t2 = ky_ * b1, t3 = kz_ * b2;
-                double divb = (t1 + t2 + t3) / ((radm + smallx) * (radm + smallx));
-                if (radm == 0.) divb = 0.0;
-                f0 = b0 - kx_ * divb;
-                f1 = b1 - ky_ * divb;
-                f2 = b2 - kz_ * divb;
-            }
-            fo[0][o] = f0; fo[1][o] = f1; fo[2][o] = f2;
-        }
-        __syncthreads();
-        if (tid < 36) sth_hermitian(fo[tid / 12], tid % 12);             // 481-510
-        __syncthreads();
-        for (int e = tid; e < 450; e += NT) fa[e] = fo[e / 150][e % 150];
+        __shared__ double scratch[OU_SCRATCH];
+        ou_step(a, rr, scratch);
         return;
     }
     if (forcing != 1) return;
@@ -1237,13 +1259,28 @@ static PlainRows plain_rows(const FlowBuffers& fb)
 }
 
 template <typename T, int N>
-static int launch_x(const FlowBuffers& fb, hipStream_t s)
+static PreArgs pre_args(const FlowBuffers& fb, const FlowConst& fc)
+{
+    PreArgs a{};
+    for (int i = 0; i < 3; ++i) { a.B[i] = fb.A[i]; a.U[i] = fb.U[i]; a.O[i] = fb.O[i]; }
+    a.tw = fb.tw; a.low = fb.low; a.sth_state = fb.sth_state; a.sth_b = fb.sth_b;
+    a.dt = fc.dt; a.rnu = fc.rnu; a.force0 = fc.force0; a.force1 = fc.force1;
+    a.ou_tf = fc.ou_tf; a.ou_var = fc.ou_var; a.pi2 = fc.pi2; a.nek = fc.nek; a.forcing = fc.forcing;
+    a.rstride = fb.rstride;
+    return a;
+}
+
+// ou: the step's stochastic forcing as well, one more work-group for each realisation
+template <typename T, int N>
+static int launch_x(const FlowBuffers& fb, const FlowConst& fc, bool ou, hipStream_t s)
 {
     KxArgs a{};
     for (int i = 0; i < 3; ++i) a.B[i] = fb.B[i];
     a.uphys = fb.uphys; a.tw = fb.tw; a.twh = fb.twh;
-    const dim3 grid((unsigned)((size_t)fb.R * N * N / kxf_lines<N>()));
-    hipLaunchKernelGGL((k_x_fused<T, N>), grid, dim3(NT), 0, s, a);
+    const unsigned nb = (unsigned)((size_t)fb.R * N * N / kxf_lines<T, N>());
+    const PreArgs p = pre_args<T, N>(fb, fc);
+    if (ou) hipLaunchKernelGGL((k_x_fused<T, N, true>), dim3(nb + fb.R), dim3(NT), 0, s, a, p, fb.R);
+    else hipLaunchKernelGGL((k_x_fused<T, N, false>), dim3(nb), dim3(NT), 0, s, a, p, 0);
     DDNS_HIP(hipGetLastError());
     return 0;
 }
@@ -1252,12 +1289,7 @@ template <typename T, int N>
 static int launch_pre(const FlowBuffers& fb, const FlowConst& fc, hipStream_t s)
 {
     if (fc.forcing != 1 && fc.forcing != 2 && fc.forcing >= 0) return 0;
-    PreArgs a{};
-    for (int i = 0; i < 3; ++i) { a.B[i] = fb.A[i]; a.U[i] = fb.U[i]; a.O[i] = fb.O[i]; }
-    a.tw = fb.tw; a.low = fb.low; a.sth_state = fb.sth_state; a.sth_b = fb.sth_b;
-    a.dt = fc.dt; a.rnu = fc.rnu; a.force0 = fc.force0; a.force1 = fc.force1;
-    a.ou_tf = fc.ou_tf; a.ou_var = fc.ou_var; a.pi2 = fc.pi2; a.nek = fc.nek; a.forcing = fc.forcing;
-    a.rstride = fb.rstride;
+    const PreArgs a = pre_args<T, N>(fb, fc);
     if (fc.forcing == 1 || fc.forcing < 0) hipLaunchKernelGGL((k_pre_dft<T, N>), dim3(225, fb.R), dim3(NT), 0, s, a);
     hipLaunchKernelGGL((k_pre<T, N>), dim3(fb.R), dim3(NT), 0, s, a);
     DDNS_HIP(hipGetLastError());
@@ -1284,15 +1316,19 @@ static int step_impl(const FlowBuffers& fb, const FlowConst& fc, hipStream_t s, 
     // the first half, 3 forward y, 4 pre, 5 end of pre, 8 start of z, 6 end of z, 7 end.
     // evflags = hipEventRecordExternal while the stream is being captured into a graph:
     // the timing events then become event-record nodes of the graph
-    if (part == FLOW_INV) {
+    // FLOW_STEP: both halves; the stochastic forcing, which reads no field, then runs beside the x
+    // stage.  (A first half alone may be queued for a step that does not follow: it leaves the
+    // forcing's state alone.)
+    const bool ou = part == FLOW_STEP && fc.forcing == 2;
+    if (part == FLOW_INV || part == FLOW_STEP) {
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[0], s, evflags));
         int st = launch_y<T, N>(true, true, fb.A, plain_rows<T, N>(fb), 6, fb, fb.R * N, s, fc.nek);
         if (st) return st;
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[1], s, evflags));
-        st = launch_x<T, N>(fb, s);
+        st = launch_x<T, N>(fb, fc, ou, s);
         if (st) return st;
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[2], s, evflags));
-        return 0;
+        if (part == FLOW_INV) return 0;
     }
     int st = 0;
     if (part != FLOW_FWD_Z) {
@@ -1300,7 +1336,7 @@ static int step_impl(const FlowBuffers& fb, const FlowConst& fc, hipStream_t s, 
         st = launch_y<T, N>(false, false, fb.A, plain_rows<T, N>(fb), 3, fb, fb.R * N, s, fc.nek);
         if (st) return st;
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[4], s, evflags));
-        st = launch_pre<T, N>(fb, fc, s);
+        if (!ou) st = launch_pre<T, N>(fb, fc, s);
         if (st) return st;
         if (ev) DDNS_HIP(hipEventRecordWithFlags(ev[5], s, evflags));
         if (part == FLOW_FWD_Y) return 0;
