@@ -85,6 +85,15 @@ def sphere_fraction(N: int) -> float:
     return inside / (N * N * (N // 2))
 
 
+def column_fraction(N: int) -> float:
+    """Fraction of the (kx, ky) columns with a mode inside the dealiasing sphere."""
+    nek = int(N / 2 - 1.5)
+    k = np.arange(N)
+    k = np.where(k > N // 2, k - N, k)
+    k2 = np.arange(N // 2)[:, None] ** 2 + (k ** 2)[None, :]
+    return float((k2 <= nek * (nek + 1)).mean())
+
+
 def kernel_bytes(N: int, prec: int):
     """Compulsory HBM bytes per launch of each flow kernel (every input read once,
     every output written once).  C = one complex field N*N*(N/2), R = one real field."""
@@ -92,16 +101,15 @@ def kernel_bytes(N: int, prec: int):
     rs = cs // 2
     C = N * N * (N // 2) * cs
     R = N * N * N * rs
-    f = sphere_fraction(N)
+    f, g = sphere_fraction(N), column_fraction(N)
     return {
-        "y_inv": 12 * C,                    # 6 fields read + written
+        "y_inv": int(6 * g * C) + 6 * C,    # 6 fields, read inside the sphere's columns only
         "x_fused": 6 * C + 3 * C + 3 * R,   # read u, w; write u x w and the physical u
-        "y_fwd": 6 * C,
+        "y_fwd": 3 * C + int(3 * g * C),
         "pre": 0,
-        # below N = 512 one fused kernel reads N (3C) and writes the six inverse outputs
-        # (6C); it reads and writes u, o (12C) only inside the dealiasing sphere (fraction
-        # f).  From 512 the separate kernels move 24C + 12fC (36C when f = 1)
-        "z_stage": int(((9 if N < 512 else 24) + 12 * f) * C),
+        # one kernel at every N: reads N (3C) and writes the six inverse outputs (6C) in the
+        # sphere's columns, reads and writes u, o (12C) inside the sphere
+        "z_stage": int((9 * g + 12 * f) * C),
         "sym": 0,
     }
 

@@ -146,7 +146,7 @@ typedef struct ddns_timing {
     double total_ms;          /* whole call                                            */
     int    nsteps;
     int    pad;
-    /* flow kernels, summed over the call: inverse y stage, fused x stage, forward y
+    /* flow kernels (the call's last step, times nsteps; 0 without droplets): inverse y stage, fused x stage, forward y
        stage, low-mode pre-kernel, z stage (see ddns_profile_flow), kx = 0
        symmetrisation */
     double flow_kernel_ms[6];
@@ -256,10 +256,10 @@ int ddns_overlap_fix(ddns_handle* h);
  * physical velocity of the step's start; the flow does not see the droplets), the two
  * blocks overlapped on two streams.  Returns, with all work done, the first nonzero
  * status (a warning does not stop the loop).
- * The two halves of the flow step are captured into HIP graphs by the first step and
- * replayed from then on (DDNS_GRAPH=0 in the environment at ddns_create launches the
- * kernels one by one; the results are the same bits).  Without droplets the call then
- * waits for the device once, at its end, and ddns_timing holds the whole call's time as
+ * The flow step is captured into HIP graphs by the first step and replayed from then on:
+ * its two halves with droplets, one step and eight steps without (DDNS_GRAPH=0 in the
+ * environment at ddns_create launches the kernels one by one; the results are the same
+ * bits).  Without droplets the call then waits for the device once, at its end, and ddns_timing holds the whole call's time as
  * flow_ms with no per-kernel split; with droplets the droplet block waits each step on
  * device results (GMRES convergence, buffer sizes, relocations, overlap sweeps). */
 int ddns_step(ddns_handle* h, int nsteps);
@@ -288,12 +288,12 @@ int ddns_get_contact_records(ddns_handle* h, double* rec, int cap, int* n);
 /* Tile shapes chosen at ddns_create by timing the candidates (no counterpart in the
  * reference; the role its FFTW_MEASURE plans play, mpifft.f90:36-56):
  *   shapes[0] = kx columns per y-stage tile, shapes[1] = its default;
- *   shapes[2] = threads of the fused z-stage work-group, shapes[3] = its default;
+ *   shapes[2] = threads of the z-stage work-group (they go with its tile's width),
+ *   shapes[3] = its default;
  *   ms[0..2] = time of one inverse (6 fields) plus forward (3 fields) y stage at half,
- *   once and twice the default width; ms[3..5] = time of one fused z stage at once
- *   and twice the default threads (ms[5] is kept for a third size and is 0), 0 where a
- *   shape does not fit the tile constraints or was not timed (the z stage where the
- *   step runs it as separate kernels, from N = 512).
+ *   once and twice the default width; ms[3..5] = time of one z stage at once and
+ *   twice the default width (ms[5] is kept for a third size and is 0), 0 where a
+ *   shape does not fit the tile constraints or was not timed.
  * A shape changes how work is grouped, never a column's or a mode's arithmetic, so
  * results are the same bits.  Either pointer may be NULL; shapes takes 4 ints, ms 6
  * doubles. */
@@ -319,9 +319,8 @@ int ddns_collision_detect(ddns_handle* h, int n, const double* yp, const double*
 
 /* Kernel timing helper (no counterpart in the reference): run the flow step alone k
  * times and return the mean time (ms) of, in order: inverse y stage, fused x stage,
- * forward y stage, low-mode pre-kernel, z stage (one fused kernel below N = 512; from
- * N = 512 the three forward transforms, the update and the six inverse transforms),
- * kx = 0 symmetrisation, whole flow step.  nkernels <= 7 values are written.
+ * forward y stage, low-mode pre-kernel, z stage (one fused kernel), kx = 0
+ * symmetrisation, whole flow step.  nkernels <= 7 values are written.
  * The flow state (u-hat, history) advances by k steps; time, the step counter and the
  * droplets do not. */
 int ddns_profile_flow(ddns_handle* h, int k, double* ms_per_kernel, int nkernels);

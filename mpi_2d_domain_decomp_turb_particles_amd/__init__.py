@@ -240,7 +240,7 @@ class Solver:
 
     def tuning(self):
         """Tile shapes chosen at set-up: dict with the y-stage tile width and its default,
-        the fused z stage's threads and their default, and the timings of the candidates
+        the z stage's threads and their default, and the timings of the candidates
         (ms; 0 where a candidate was not timed)."""
         sh = np.zeros(4, dtype=np.int32)
         ms = np.zeros(6)

@@ -680,16 +680,17 @@ extern "C" int ddns_init_droplets(ddns_handle* h, int seed, int radii_kind, doub
 // 20 a_max, or the collision window 2 a_max plus both displacements of the step.  Two grid
 // spacings cover any step's displacement, and so does the statistics window at the usual
 // step sizes: where the droplets are dense the cells are only as wide as 20 a_max, with at
-// most about one (Morton-numbered) cell per four droplets so that the cell scan stays
+// most about four cells per droplet so that the cell scan stays
 // small; the search reports any droplet whose reach exceeds the cells (collide_regrid).
-// HI needs its truncation radius, usually much wider, so it gets its own, coarser grid.
+// HI needs its truncation radius, usually much wider, so it gets a coarser grid, which serves the
+// other searches too where it is not too full (grid_serves).
 static double coll_cell_width(const ddns_handle* h)
 {
     const double dx = h->pc.pi2 / h->N;
     const double wide = std::max(20.0 * h->pc.radmax, 2.0 * dx);
     if (h->coll_wide) return wide;
     static const long long per = [] {
-        const char* e = std::getenv("DDNS_COLL_CELLS");     // Morton cells allowed per droplet
+        const char* e = std::getenv("DDNS_COLL_CELLS");     // cells allowed per droplet
         const long long v = e ? std::atoll(e) : 4;
         return v > 0 ? v : 4;
     }();

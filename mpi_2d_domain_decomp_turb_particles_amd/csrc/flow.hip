@@ -251,9 +251,9 @@ __global__ void __launch_bounds__((kz_plain_threads<T, N>())) k_z(KzArgs a)
 //     forward transforms end with the modes where the update and the curl need them and the
 //     inverse ones start, so the stage has no pointwise pass over LDS and only the exchange
 //     buffer of one field in it (36 KB at 256^3 FP32, four tiles took 141 KB).
-//   - It is bound by HBM: at 256^3 FP32 it moves 9C x 0.78 + 12C x 0.51 (0.87 GB).
+//   - It is bound by HBM: at 256^3 FP32 it moves 9C x 0.77 + 12C x 0.51 (0.87 GB).
 //   - Beyond the dealiasing sphere nothing is moved: a column with kx^2 + ky^2 beyond it
-//     (21 % of them) is neither read from B nor written to A (the y stages leave it out too),
+//     (23 % of them) is neither read from B nor written to A (the y stages leave it out too),
 //     a tile of such columns ends at once, and the state's modes beyond the sphere are only
 //     written while they may still be nonzero (LOW_ZOUT).
 // The tile width (and with it the work-group's size) is timed at set-up; it changes no
@@ -385,7 +385,7 @@ __global__ void __launch_bounds__((kz_threads<T, N, TC>()), (kz_waves<T, N>())) 
 // Columns in registers as in the z stage; bound by memory.  The inverse stage takes a plane
 // from the intermediate layout to plain [y][kx] rows, where the x stage finds its lines; the
 // forward stage goes the other way.  In a step (a.low given) the rows beyond the circle
-// kx^2 + ky^2 of the dealiasing sphere (21 % of them) are left out: the inverse stage takes
+// kx^2 + ky^2 of the dealiasing sphere (23 % of them) are left out: the inverse stage takes
 // them as zero (unless the state was set since the last step, when the z transforms of that
 // state fill them), the forward stage does not store them.
 template <typename T, int N, bool INV, bool SYM, int TC>
