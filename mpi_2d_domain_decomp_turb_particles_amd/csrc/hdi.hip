@@ -869,13 +869,12 @@ static int queue_lists(PartBuffers& pb, const PartConst& pc, hipStream_t s)
 // neighbours), 1 when some row had more neighbours than the lists hold (they have been
 // widened; fill them again), else 0.
 template <typename T>
-static int lists_outcome(PartBuffers& pb, const int* f)
+static int lists_outcome(PartBuffers& pb, const int* f, hipStream_t s)
 {
     if (f[0] & 1) { set_error("inside NEI_LIST_PRECOMP: overlapping is not allowed"); return DDNS_ERR_OVERLAP; }
     if (f[0] & 2) { set_error("more than 100 HI neighbours for a droplet"); return DDNS_ERR_NEIGHBOUR_OVERFLOW; }
     if (f[4] <= pb.ell_width) return 0;
-    DDNS_HIP(hipMemset(pb.flags, 0, 8 * sizeof(int)));
-    DDNS_HIP(hipStreamSynchronize(nullptr));
+    DDNS_HIP(hipMemsetAsync(pb.flags, 0, 8 * sizeof(int), s));     // what fills them again follows on s
     if (pb.nei_idx) { (void)hipFree(pb.nei_idx); (void)hipFree(pb.nei_m); pb.nei_idx = nullptr; pb.nei_m = nullptr; }
     pb.ell_width = std::min(DDNS_MAXNEI, (f[4] + ELL_STEP - 1) / ELL_STEP * ELL_STEP);
     DDNS_HIP(hipMalloc(&pb.nei_idx, (size_t)pb.ell_width * pb.cap * sizeof(int)));
@@ -1049,7 +1048,7 @@ static int hdi_impl(PartBuffers& pb, const PartConst& pc, int maxiter, double to
             if (first) std::memcpy(f, fh, sizeof(f));
             if (first) {
                 first = false;
-                lists = lists_outcome<T>(pb, f);
+                lists = lists_outcome<T>(pb, f, s);
                 if (lists < 0) return lists;
                 if (lists > 0) break;            // fill the widened lists and solve again
             }
@@ -1305,7 +1304,7 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
                     th[r].nbr = 0;
                     retable = true;
                 }
-                const int lo = lists_outcome<T>(*pbs[r], f);
+                const int lo = lists_outcome<T>(*pbs[r], f, s);
                 if (lo < 0) {
                     status[r] = lo;
                     DDNS_HIP(hipMemcpyAsync(hb.table, th, (size_t)R * sizeof(GmDesc<T>), hipMemcpyHostToDevice, s));
