@@ -606,7 +606,7 @@ __device__ __forceinline__ unsigned ranff_mul(unsigned a, unsigned b)
 {
     const unsigned long long p = (unsigned long long)a * b;
     unsigned r = (unsigned)(p & 0x7fffffffu) + (unsigned)(p >> 31);
-    return r >= 0x7fffffffu ? r - 0x7fffffffu : r;      // a, b < 2^31 - 1, never 0: one fold is enough
+    return r >= 0x7fffffffu ? r - 0x7fffffffu : r;      // a <= 2^31 - 1, b < 2^31 - 1: one fold is enough
 }
 
 __device__ __forceinline__ void ranff_draws(int* st, int n, int* seq)
@@ -621,7 +621,7 @@ __device__ __forceinline__ void ranff_draws(int* st, int n, int* seq)
     }
     int idum = __builtin_amdgcn_readfirstlane(st[0]), iy = __builtin_amdgcn_readfirstlane(st[1]);
     int iv = lane < 32 ? st[2 + lane] : 0;
-    if (idum <= 0 || iy == 0) {
+    auto seed = [&]() {
         idum = (-idum > 1) ? -idum : 1;
         // 8 warm-up values, then the table from iv(32) down to iv(1): value 9 + q of the
         // stream is iv(32 - q)
@@ -629,9 +629,10 @@ __device__ __forceinline__ void ranff_draws(int* st, int n, int* seq)
         iv = __shfl((int)x, 39 - (lane & 31), 64);
         idum = __builtin_amdgcn_readlane((int)x, 39);
         iy = __builtin_amdgcn_readlane(iv, 0);
-    }
-    for (int n0 = 0; n0 < n; n0 += 64) {
-        const int m = min(64, n - n0);
+    };
+    if (idum <= 0 || iy == 0) seed();
+    // draws [n0, n0 + m), m <= 64
+    auto draws = [&](int n0, int m) {
         const int x = (int)ranff_mul((unsigned)idum, pw);
         int out = 0;
         for (int q = 0; q < m; ++q) {
@@ -642,6 +643,16 @@ __device__ __forceinline__ void ranff_draws(int* st, int n, int* seq)
         }
         idum = __builtin_amdgcn_readlane(x, m - 1);
         if (lane < m) seq[n0 + lane] = out;
+    };
+    if (idum % IM != 0 && !__any(lane < 32 && iv == 0)) {
+        for (int n0 = 0; n0 < n; n0 += 64) draws(n0, min(64, n - n0));
+    } else {
+        // A seed that IM divides gives zeros only, and a table that holds a zero can hand it to
+        // iy: the next draw then seeds the generator again.  From any other state no zero comes.
+        for (int q = 0; q < n; ++q) {
+            if (q > 0 && (idum <= 0 || iy == 0)) seed();
+            draws(q, 1);
+        }
     }
     if (lane == 0) { st[0] = idum; st[1] = iy; }
     if (lane < 32) st[2 + lane] = iv;
