@@ -259,9 +259,11 @@ int ddns_overlap_fix(ddns_handle* h);
  * The flow step is captured into HIP graphs by the first step and replayed from then on:
  * its two halves with droplets, one step and eight steps without (DDNS_GRAPH=0 in the
  * environment at ddns_create launches the kernels one by one; the results are the same
- * bits).  Without droplets the call then waits for the device once, at its end, and ddns_timing holds the whole call's time as
- * flow_ms with no per-kernel split; with droplets the droplet block waits each step on
- * device results (GMRES convergence, buffer sizes, relocations, overlap sweeps). */
+ * bits).  Without droplets the call then waits for the device once, at its end, and
+ * ddns_timing holds the whole call's time as flow_ms with no per-kernel split; with droplets
+ * the droplet block waits each step on device results (GMRES convergence, buffer sizes,
+ * relocations, overlap sweeps).  A wait polls the device for up to 2 ms and then waits as HIP
+ * does (hipDeviceScheduleBlockingSync lets the thread sleep). */
 int ddns_step(ddns_handle* h, int nsteps);
 
 /* Outcome of the last step's COLLISION_DET (and HI solve). */

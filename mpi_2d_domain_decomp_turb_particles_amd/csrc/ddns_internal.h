@@ -4,6 +4,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <chrono>
 #include <cstddef>
 #include <cstdint>
 #include <string>
@@ -465,17 +466,23 @@ int part_download(PartBuffers& pb, int n, double* yp, double* fvp, double* fdp, 
                   hipStream_t s);
 // one 3-vector per droplet (dst(3,n), component-major slots) from the host's a(3, n)
 int part_upload3(PartBuffers& pb, int n, double* dst, const double* a, hipStream_t s);
-// Waits for event e by polling it: after a blocking wait the host thread ran again tens
-// of microseconds after the GPU had finished, and the stream waited that long for the
-// launches that follow.
+// Waits for event e: by polling it for POLL_MS, then as the runtime waits.  After a blocking
+// wait the host thread ran again tens of microseconds after the GPU had finished, and the stream
+// waited that long for the launches that follow; past POLL_MS that is a few per cent of the
+// wait, and a program that has asked HIP for blocking waits (hipDeviceScheduleBlockingSync) gets
+// its core back: 64 flow steps at 256^3 take 45 ms and held it for all of them when this polled
+// to the end.
+constexpr double POLL_MS = 2.0;
 inline hipError_t spin_wait(hipEvent_t e)
 {
+    const auto t0 = std::chrono::steady_clock::now();
     for (;;) {
         const hipError_t r = hipEventQuery(e);
         if (r != hipErrorNotReady) return r;
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::duration<double, std::milli>(POLL_MS)) return hipEventSynchronize(e);
     }
 }
-// all work queued on s so far, waited for by polling (pb.sync_ev, made on first use)
+// all work queued on s so far, waited for by spin_wait (pb.sync_ev, made on first use)
 inline hipError_t wait_stream(PartBuffers& pb, hipStream_t s)
 {
     if (!pb.sync_ev) {
