@@ -30,3 +30,32 @@ def test_step_relocates_as_the_oracle(ddns, oracle_mod, pairs):
         print(pairs, co.ncoll, co.noverlap_sweeps, co.noverlap_relocated)
         assert (cg.ncoll, cg.noverlap_sweeps, cg.noverlap_relocated) == (co.ncoll, co.noverlap_sweeps, co.noverlap_relocated)
         assert np.allclose(s.get_droplets()["yp"][:3], o.get_droplets()["yp"][:3], rtol=0, atol=1e-12)
+
+
+def test_lists_beyond_the_sort_cost_little_more(ddns):
+    """A relocation of 4300 droplets among a million takes about the draws' time longer than one
+    of 4000 (both by one lane in order), though its list no longer fits the sort."""
+    n = 1000000
+    p = ddns.default_params(N=64, precision=1, npart=n, radius=[5.0], nonoverlap=1, dt=1e-4, rnu=0.02,
+                            gravity=1e-25, forcing=0, new_particle=0)
+    ms = {}
+    with ddns.Solver(p) as s:
+        s.init_flow(-1, 1)
+        s.init_droplets(seed=5)
+        base = s.get_droplets()["yp"].copy(order="F")
+        base[3:6] = 0.0
+        rng = np.random.default_rng(7)
+        for pairs in (4000, 4300):
+            t = []
+            for _ in range(4):
+                yp = base.copy(order="F")
+                order = rng.permutation(n)
+                a, b = order[:pairs], order[pairs:2 * pairs]
+                yp[:3, b] = np.mod(yp[:3, a] + 0.5 * base[6, 0], 2 * np.pi)
+                s.set_droplets(yp)
+                s.step(1)
+                assert s.collision_counts().noverlap_relocated >= pairs
+                t.append(s.timing().overlap_ms)
+            ms[pairs] = min(t)
+    print(ms, flush=True)
+    assert ms[4300] < 1.3 * ms[4000]
