@@ -67,3 +67,16 @@ def test_every_tile_width_gives_the_same_flow(ddns, oracle_mod, monkeypatch, pre
         ov = o.get_flow()[0]
     for shape in out:
         assert rel_l2(out[shape][0], ov) < (1e-11 if prec == 0 else 1e-5), shape
+
+
+def test_the_tuner_times_the_stages_of_a_step(ddns):
+    """The z stage is timed with the bytes that a step moves: what lies beyond the dealiasing
+    sphere, half of the state's modes, is left out."""
+    with ddns.Solver(ddns.default_params(N=256, precision=1, forcing=1, dt=1e-4, rnu=0.01)) as s:
+        t = s.tuning()
+        s.init_flow(ddns.SPEC_K4_GAUSS, 123, 4.0, 1.0)
+        s.step(2)
+        z = min(s.profile_flow(50)["z_stage"] for _ in range(2))
+    tuned = min(x for x in t["kz_ms"] if x > 0)
+    print(f"z stage: tuner {tuned:.4f} ms, step {z:.4f} ms", flush=True)
+    assert tuned < 1.2 * z
