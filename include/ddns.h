@@ -136,7 +136,8 @@ typedef struct ddns_collision_counts {
 /* Kernel-level timing of the last ddns_step call, from HIP events (milliseconds). */
 typedef struct ddns_timing {
     double flow_ms;           /* spectral step: FFT stages + fused update (with droplets:
-                                 the call's last step, times nsteps)                   */
+                                 from the steps that are timed, the first, the last and
+                                 every 16th, taken for all nsteps)                     */
     double interp_ms;         /* Lagrange gather                                       */
     double cells_ms;          /* cell binning (keys + sort)                            */
     double hdi_ms;            /* HI neighbour build + GMRES                            */
@@ -146,9 +147,9 @@ typedef struct ddns_timing {
     double total_ms;          /* whole call                                            */
     int    nsteps;
     int    pad;
-    /* flow kernels (the call's last step, times nsteps; 0 without droplets): inverse y stage, fused x stage, forward y
-       stage, low-mode pre-kernel, z stage (see ddns_profile_flow), kx = 0
-       symmetrisation */
+    /* flow kernels, summed over the call as flow_ms is (0 without droplets): inverse y
+       stage, fused x stage, forward y stage, low-mode pre-kernel, z stage (see
+       ddns_profile_flow), kx = 0 symmetrisation */
     double flow_kernel_ms[6];
 } ddns_timing;
 
