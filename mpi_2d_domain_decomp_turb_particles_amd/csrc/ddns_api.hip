@@ -1075,9 +1075,9 @@ static int droplet_rest(ddns_handle* h, float* ms)
     return status;
 }
 
-// A step that stops part-way leaves the inverse pipeline A partly transformed in place
-// (the inverse y stage overwrites its input) and may leave the next step's first half
-// queued.  Wait for both streams and have the next call rebuild A from u-hat.  The flow
+// A step that stops part-way leaves the inverse pipeline A as the start of no step (the
+// forward y stage overwrites its first three fields, the z stage all six) and may leave the
+// next step's first half queued.  Wait for both streams and have the next call rebuild A from u-hat.  The flow
 // state is then at the end of the failed step when its update had been queued, else at
 // its start; time and istep count the failed step either way.
 static int step_fail(ddns_handle* h, int st)
@@ -1348,7 +1348,8 @@ extern "C" int ddns_batch_create(const ddns_params* params, int nreal, ddns_batc
     *out = nullptr;
     const ddns_params& p0 = params[0];
     const int N = p0.nx;
-    if (N > 256) return bfail(nullptr, DDNS_ERR_ARG, "batched realisations need N <= 256 (the fused z stage)");
+    // one realisation of 512^3 fills the chip by itself: larger grids are not batched
+    if (N > 256) return bfail(nullptr, DDNS_ERR_ARG, "batched realisations need N <= 256");
     for (int r = 1; r < nreal; ++r) {
         const ddns_params& p = params[r];
         if (p.nx != N || p.ny != p0.ny || p.nz != p0.nz || p.precision != p0.precision || p.dt != p0.dt ||

@@ -22,13 +22,11 @@ template <> struct vec16<float2> {
     using V = float4;
     static constexpr int VW = 2;
     __device__ static void split(const V& v, float2* o) { o[0] = make_float2(v.x, v.y); o[1] = make_float2(v.z, v.w); }
-    __device__ static V join(const float2* c) { return make_float4(c[0].x, c[0].y, c[1].x, c[1].y); }
 };
 template <> struct vec16<double2> {
     using V = double2;
     static constexpr int VW = 1;
     __device__ static void split(const V& v, double2* o) { o[0] = v; }
-    __device__ static V join(const double2* c) { return c[0]; }
 };
 
 // the registers one lane holds for a tile in flight
@@ -73,23 +71,6 @@ __device__ __forceinline__ void tile_load(C* __restrict__ lds, const C* __restri
     TileRegs<C, R, W, NT> t;
     tile_fetch<C, R, W, NT>(t, src, rstride, tid);
     tile_put<C, R, W, LDR, NT, TRANS>(lds, t, tid);
-}
-
-template <typename C, int R, int W, int LDR, int NT>
-__device__ __forceinline__ void tile_store(C* __restrict__ dst, const C* __restrict__ lds, size_t rstride, int tid,
-                                           decltype(C{}.x) scale = 1)
-{
-    using VT = vec16<C>;
-    constexpr int VW = VT::VW, PER_ROW = W / VW, TOT = R * PER_ROW;
-    static_assert(W % VW == 0 && TOT % NT == 0, "tile must split evenly over the work-group");
-#pragma unroll
-    for (int q = 0; q < TOT / NT; ++q) {
-        const int e = tid + q * NT, r = e / PER_ROW, c = (e % PER_ROW) * VW;
-        C v[VW];
-#pragma unroll
-        for (int k = 0; k < VW; ++k) v[k] = cscale(lds[r * LDR + c + k], scale);
-        *(typename VT::V*)(dst + (size_t)r * rstride + c) = VT::join(v);
-    }
 }
 
 // ---------------------------------------------------------------- register DFTs
@@ -172,16 +153,14 @@ __device__ __forceinline__ void dft(C* v)
 }
 
 // ---------------------------------------------------------------- radix plans
+// of the x stage's half-length lines, N / 2 points
 template <int N> struct Plan;
-template <> struct Plan<4>    { static constexpr int P = 1, R0 = 4,  R1 = 1,  R2 = 1; };
-template <> struct Plan<8>    { static constexpr int P = 1, R0 = 8,  R1 = 1,  R2 = 1; };
 template <> struct Plan<16>   { static constexpr int P = 1, R0 = 16, R1 = 1,  R2 = 1; };
 template <> struct Plan<32>   { static constexpr int P = 2, R0 = 8,  R1 = 4,  R2 = 1; };
 template <> struct Plan<64>   { static constexpr int P = 2, R0 = 8,  R1 = 8,  R2 = 1; };
 template <> struct Plan<128>  { static constexpr int P = 2, R0 = 16, R1 = 8,  R2 = 1; };
 template <> struct Plan<256>  { static constexpr int P = 2, R0 = 16, R1 = 16, R2 = 1; };
 template <> struct Plan<512>  { static constexpr int P = 3, R0 = 8,  R1 = 8,  R2 = 8; };
-template <> struct Plan<1024> { static constexpr int P = 3, R0 = 16, R1 = 16, R2 = 4; };
 
 // One Stockham pass of stride NS (product of the radices already applied) over K
 // tiles at once (tile k at lds + k * TS): each work item runs one radix-R butterfly

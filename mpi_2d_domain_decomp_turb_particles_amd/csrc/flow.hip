@@ -78,7 +78,7 @@ __device__ __forceinline__ int xcd_tile(int L)
         return g * (8 * P) + (r % 8) * P + r / 8;
     }
 }
-// tile width of the plain z transforms (the diagnostics, the split z stage): rows of 128 bytes
+// tile width of the plain z transforms (the diagnostics, the stand-alone transforms): rows of 128 bytes
 template <typename T, int N> constexpr int kz_tc_plain() { return sizeof(T) == 4 || N == 32 ? 16 : 8; }
 template <typename T, int N> constexpr int kz_plain_threads() { return kz_tc_plain<T, N>() * (N / col_e<T, N>()); }
 __device__ __forceinline__ int wave_index(int i, int N) { return i <= N / 2 ? i : i - N; }
@@ -102,9 +102,10 @@ __device__ __forceinline__ bool mode_in_sphere(int kx, int ky, int kz, int N, in
 constexpr int LOW_STRIDE = 1024;
 constexpr int LOW_PAR = 1000;       // [0] forcing kind, [1..2] force(1:2), [3] OU time scale, [4] OU variance
 // [LOW_ZOUT] = 1 once a step has written the state's modes beyond the dealiasing sphere,
-// which every update sets to zero: the z stage then neither loads nor stores them (u-hat
-// and the AB2 history stay zero there).  Cleared by every upload of the state; set by the
-// step's k_sym, which runs after the z stage.
+// which every update sets to zero.  The z stage never loads them and stores the zeros only
+// while the flag is clear; the inverse y stage takes the columns beyond the sphere as zero once
+// it is set.  Cleared by every upload of the state; set by the step's k_sym, which runs after
+// the z stage.
 constexpr int LOW_ZOUT = LOW_PAR + 5;
 constexpr int STH_STATE_STRIDE = 64;
 constexpr int STH_B_STRIDE = 512;
@@ -1008,7 +1009,7 @@ __global__ void __launch_bounds__(256) k_init_modes(void* u0, void* u1, void* u2
     __syncthreads();
     for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < (size_t)N * N * M; t += (size_t)gridDim.x * 256) {
         int kx, ky, kz;
-    spec_mode<T>(N, t, kz, ky, kx);
+        spec_mode<T>(N, t, kz, ky, kx);
         const int kyw = wave_index(ky, N), kzw = wave_index(kz, N);
         const bool zero = ky == N / 2 || kz == N / 2 || (kx == 0 && ky == 0 && kz == 0);
         double2 g[3];
@@ -1497,7 +1498,7 @@ static int download_spectral(FlowBuffers& fb, const void* dev, int N, double* v,
 }
 
 // the state's modes beyond the dealiasing sphere may be nonzero again (an upload, a new
-// field): the next z stage loads and stores them all
+// field): the next inverse y stage reads every column, the next z stage stores the zeros
 static int mark_dense(const FlowBuffers& fb)
 {
     static const double zero = 0.0;
@@ -2007,7 +2008,7 @@ int flow_profile_copy(const FlowBuffers& fb, int N, int precision, int reps, dou
 // (cleared first), one untimed run and then the mean of three, and the fastest is kept:
 //   - the y-stage tile width: the inverse stage over six fields and the forward stage
 //     over three, as a step runs them;
-//   - the fused z stage's work-group size (where the step uses the fused z stage).
+//   - the z stage's tile width, by its work-group's threads.
 // The choices are cached per grid and precision for the life of the process.
 // DDNS_KY_TC / DDNS_KZ_NT in the environment force a shape (one that is not a candidate,
 // or does not fit, means the default) and skip the timing; DDNS_TUNE=0 keeps the defaults.
@@ -2026,7 +2027,7 @@ static bool ky_cand_fits(int k)
 template <typename T, int N>
 static bool kz_cand_fits(int k)
 {
-    return k == 0 || (k == 1 && kz_fits<T, N, kz_cand<T, N>(1)>());
+    return k == 0 || kz_fits<T, N, kz_cand<T, N>(1)>();
 }
 // threads of the fused z stage's work-group at candidate k (once or twice the default width)
 template <typename T, int N> constexpr int kz_nt_cand(int k) { return kz_threads<T, N, kz_tc<T, N>()>() << k; }
@@ -2068,7 +2069,7 @@ static int tune_impl(FlowBuffers& fb, const FlowConst& fc, hipStream_t s)
     }
     if (const char* f = std::getenv("DDNS_KZ_NT")) {
         const int want = std::atoi(f);
-        for (int k = 0; k < 3; ++k)
+        for (int k = 0; k < 2; ++k)
             if (want == kz_nt_cand<T, N>(k) && kz_cand_fits<T, N>(k)) fb.kz_nt = want;
         forced = true;
     }
@@ -2123,7 +2124,7 @@ static int tune_impl(FlowBuffers& fb, const FlowConst& fc, hipStream_t s)
     }
     {
         best = 0.f;
-        for (int k = 0; k < 3 && !st; ++k) {
+        for (int k = 0; k < 2 && !st; ++k) {
             if (!kz_cand_fits<T, N>(k)) continue;
             fb.kz_nt = kz_nt_cand<T, N>(k);
             fb.kz_ms[k] = time_runs([&]() { return launch_z<T, N>(KZ_FULL, fb, fc, s); }, 3, s, e0, e1, &st);

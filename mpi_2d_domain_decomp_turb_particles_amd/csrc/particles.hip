@@ -594,44 +594,44 @@ __global__ void __launch_bounds__(PT) k_advance(double* vel, const double* rad, 
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     double far = 0.0, big = 0.0;
     if (i < n) {
-    const size_t C = (size_t)cap;
-    double f0[3], d2[3];
+        const size_t C = (size_t)cap;
+        double f0[3], d2[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        f0[c] = hdi ? vp[c * C + i] + pert[3 * (size_t)i + c] : vp[c * C + i];
-        fdp[(dc.x + c) * C + i] = f0[c];
-        if (newp) { fdp[(dc.y + c) * C + i] = f0[c]; fdp[(dc.z + c) * C + i] = f0[c]; fdp[(dc.w + c) * C + i] = f0[c]; }
-    }
-    const double a = rad[i];
-    double FSN = 1.;
-    if (ndrag == 1) {
-        double d[3];
+        for (int c = 0; c < 3; ++c) {
+            f0[c] = hdi ? vp[c * C + i] + pert[3 * (size_t)i + c] : vp[c * C + i];
+            fdp[(dc.x + c) * C + i] = f0[c];
+            if (newp) { fdp[(dc.y + c) * C + i] = f0[c]; fdp[(dc.z + c) * C + i] = f0[c]; fdp[(dc.w + c) * C + i] = f0[c]; }
+        }
+        const double a = rad[i];
+        double FSN = 1.;
+        if (ndrag == 1) {
+            double d[3];
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
-            d[c] = hdi ? vel[c * C + i] - vp[c * C + i] - pert[3 * (size_t)i + c] : vel[c * C + i] - vp[c * C + i];
-        const double Vrel = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-        FSN = 1. + 0.15 * pow(Vrel * 2. * a / rnu, 0.687);
-    }
-    const double taup = tau2 * (a * a);
-    const double dtau = dt / (24.0 * taup) * FSN;
-    const double wp_vel = Sv * (a * a);
-    const double dtc = dt / 24.0;
+            for (int c = 0; c < 3; ++c)
+                d[c] = hdi ? vel[c * C + i] - vp[c * C + i] - pert[3 * (size_t)i + c] : vel[c * C + i] - vp[c * C + i];
+            const double Vrel = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+            FSN = 1. + 0.15 * pow(Vrel * 2. * a / rnu, 0.687);
+        }
+        const double taup = tau2 * (a * a);
+        const double dtau = dt / (24.0 * taup) * FSN;
+        const double wp_vel = Sv * (a * a);
+        const double dtc = dt / 24.0;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const double unitv = c == 0 ? 1.0 : 0.0;
-        const double fv0 = fvp[(vc.x + c) * C + i], fv1 = fvp[(vc.y + c) * C + i], fv2 = fvp[(vc.z + c) * C + i];
-        const double tempv = 19.0 * fv0 - 5.0 * fv1 + fv2;
-        const double tempd = 55.0 * f0[c] - 59.0 * fdp[(dc.y + c) * C + i] + 37.0 * fdp[(dc.z + c) * C + i] -
-                             9.0 * fdp[(dc.w + c) * C + i];
-        const double vnew = (vel[c * C + i] + dt * unitv * wp_vel / taup * FSN - dtau * tempv + dtau * tempd) / (1.0 + 9.0 * dtau);
-        const double dm = dtc * (9.0 * vnew + 19.0 * fv0 - 5.0 * fv1 + fv2);
-        vel[c * C + i] = vnew;
-        dmove[c * C + i] = dm;
-        d2[c] = dm * dm;
-    }
-    // rounded up: the bound may be a little larger than the displacement the search computes
-    far = sqrt(d2[0] + d2[1] + d2[2]) * (1.0 + 1e-14);
-    big = a;
+        for (int c = 0; c < 3; ++c) {
+            const double unitv = c == 0 ? 1.0 : 0.0;
+            const double fv0 = fvp[(vc.x + c) * C + i], fv1 = fvp[(vc.y + c) * C + i], fv2 = fvp[(vc.z + c) * C + i];
+            const double tempv = 19.0 * fv0 - 5.0 * fv1 + fv2;
+            const double tempd = 55.0 * f0[c] - 59.0 * fdp[(dc.y + c) * C + i] + 37.0 * fdp[(dc.z + c) * C + i] -
+                                 9.0 * fdp[(dc.w + c) * C + i];
+            const double vnew = (vel[c * C + i] + dt * unitv * wp_vel / taup * FSN - dtau * tempv + dtau * tempd) / (1.0 + 9.0 * dtau);
+            const double dm = dtc * (9.0 * vnew + 19.0 * fv0 - 5.0 * fv1 + fv2);
+            vel[c * C + i] = vnew;
+            dmove[c * C + i] = dm;
+            d2[c] = dm * dm;
+        }
+        // rounded up: the bound may be a little larger than the displacement the search computes
+        far = sqrt(d2[0] + d2[1] + d2[2]) * (1.0 + 1e-14);
+        big = a;
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
