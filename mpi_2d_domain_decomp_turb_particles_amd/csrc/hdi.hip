@@ -392,11 +392,11 @@ __global__ void __launch_bounds__(RT) k_mdot(const T* __restrict__ Q, const T* _
 }
 
 // First pass's update fused with the second pass's projections, for k <= KC columns:
-// h = sum of part_in (first pass), v -= sum_j h_j Q_j, partials of Q_j . v into part_out
+// h = sum of the P_in part_in (first pass), v -= sum_j h_j Q_j, partials of Q_j . v into part_out
 // and of v . v (the updated v) as its column k
 template <typename T, int KC>
 __device__ __forceinline__ void k_maxpy_mdot_body(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
-                                                   long long ld, const double* __restrict__ part_in,
+                                                   long long ld, const double* __restrict__ part_in, int P_in,
                                                    double* __restrict__ hcol, double* __restrict__ part_out,
                                                    const double* __restrict__ stop, int bx, int nbx)
 {
@@ -406,7 +406,7 @@ __device__ __forceinline__ void k_maxpy_mdot_body(T* __restrict__ v, const T* __
     __shared__ double sh[RW][KC + 1];
     __shared__ double red[KC + 1];
     const int tid = threadIdx.x;
-    sum_partials(part_in, nbx, k, hs, hcol, 0, bx);
+    sum_partials(part_in, P_in, k, hs, hcol, 0, bx);
     double acc[KC + 1];
 #pragma unroll
     for (int jj = 0; jj <= KC; ++jj) acc[jj] = 0.0;
@@ -458,11 +458,11 @@ __device__ __forceinline__ void k_maxpy_mdot_body(T* __restrict__ v, const T* __
 }
 template <typename T, int KC>
 __global__ void __launch_bounds__(RT) k_maxpy_mdot(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
-                                                   long long ld, const double* __restrict__ part_in,
+                                                   long long ld, const double* __restrict__ part_in, int P_in,
                                                    double* __restrict__ hcol, double* __restrict__ part_out,
                                                    const double* __restrict__ stop)
 {
-    k_maxpy_mdot_body<T, KC>(v, Q, k, n3, ld, part_in, hcol, part_out, stop, blockIdx.x, gridDim.x);
+    k_maxpy_mdot_body<T, KC>(v, Q, k, n3, ld, part_in, P_in, hcol, part_out, stop, blockIdx.x, gridDim.x);
 }
 
 // sum over b < P of part[b] (lane-strided in order, then the wavefront tree), the same
@@ -702,11 +702,11 @@ __device__ void ls_solve(double* sm, double* __restrict__ gsm, GmSmall L, int it
 #undef QN
 }
 
-// h = sum of part_in, v -= sum_j h[j] Q_j (hcol set or, with add, incremented); returns the
+// h = sum of the P_in part_in, v -= sum_j h[j] Q_j (hcol set or, with add, incremented); returns the
 // work-group's partial of |v|^2 in every thread
 template <typename T>
 __device__ __forceinline__ double update_body(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
-                                               long long ld, const double* __restrict__ part_in,
+                                               long long ld, const double* __restrict__ part_in, int P_in,
                                                double* hcol, int add, int bx, int nbx)
 {
     constexpr int W = kvec<T>::W;
@@ -714,7 +714,7 @@ __device__ __forceinline__ double update_body(T* __restrict__ v, const T* __rest
     __shared__ double sh[RW][1];
     __shared__ double red[1];
     const int tid = threadIdx.x;
-    sum_partials(part_in, nbx, k, hs, hcol, add, bx);
+    sum_partials(part_in, P_in, k, hs, hcol, add, bx);
     double nacc[1] = {0.0};
     const long long nv = (n3 + W - 1) / W;
     for (long long iv = (long long)bx * RT + tid; iv < nv; iv += (long long)nbx * RT) {
@@ -760,12 +760,12 @@ __global__ void __launch_bounds__(RT) k_maxpy(T* __restrict__ v, const T* __rest
                                               double* __restrict__ hcol, const double* __restrict__ stop)
 {
     if (*stop != 0.0) return;
-    update_body<T>(v, Q, k, n3, ld, part_in, hcol, 0, blockIdx.x, gridDim.x);
+    update_body<T>(v, Q, k, n3, ld, part_in, gridDim.x, hcol, 0, blockIdx.x, gridDim.x);
 }
 
 // The end of iteration k: the second pass's update, then the least-squares update with
-// H(k + 1, k) = |v|.  gate_w and gate_v hold the partials of |w|^2 before the first pass and of
-// |v|^2 after it; when the first pass kept at least 1/sqrt(2) of the norm (|v|^2 >= |w|^2 / 2, the
+// H(k + 1, k) = |v|.  gate_w and gate_v hold the P_w and nbx partials of |w|^2 before the first
+// pass and of |v|^2 after it; when the first pass kept at least 1/sqrt(2) of the norm (|v|^2 >= |w|^2 / 2, the
 // DGKS criterion) the second pass's corrections are below rounding, its update is skipped (v and
 // hcol stay) and work-group 0 goes on by itself, its upper wavefronts having loaded the small
 // problem while the lower ones summed the gate.  Otherwise the last work-group to arrive (arrive
@@ -777,20 +777,20 @@ __device__ __forceinline__ void k_finish_body(T* __restrict__ v, const T* __rest
                                                long long ld, const double* __restrict__ part_in,
                                                double* hcol, double* __restrict__ normpart,
                                                const double* __restrict__ stop, const double* __restrict__ gate_w,
-                                               const double* __restrict__ gate_v, double* gsm, GmSmall L, int* arrive,
-                                               double* host, double* ls, int bx, int nbx)
+                                               int P_w, const double* __restrict__ gate_v, double* gsm, GmSmall L,
+                                               int* arrive, double* host, double* ls, int bx, int nbx)
 {
     __shared__ double g1[2];
     __shared__ int last;
     if (*stop != 0.0) return;
     const int tid = threadIdx.x;
     if (bx == 0 && tid >= RT / 2) ls_load(ls, gsm, L, k, tid - RT / 2, RT / 2);
-    const double nw = sum_one(gate_w, nbx, &g1[0]);
+    const double nw = sum_one(gate_w, P_w, &g1[0]);
     double nv2 = sum_one(gate_v, nbx, &g1[1]);
     if (nv2 >= 0.5 * nw) {
         if (bx != 0) return;
     } else {
-        const double mine = update_body<T>(v, Q, k, n3, ld, part_in, hcol, 1, bx, nbx);
+        const double mine = update_body<T>(v, Q, k, n3, ld, part_in, nbx, hcol, 1, bx, nbx);
         if (tid == 0) {
             normpart[bx] = mine;
             __threadfence();                       // the partial and hcol, before the arrival
@@ -809,11 +809,12 @@ template <typename T>
 __global__ void __launch_bounds__(RT) k_finish(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
                                                long long ld, const double* __restrict__ part_in,
                                                double* hcol, double* normpart, const double* stop,
-                                               const double* __restrict__ gate_w, const double* __restrict__ gate_v,
-                                               double* gsm, GmSmall L, int* arrive, double* host)
+                                               const double* __restrict__ gate_w, int P_w,
+                                               const double* __restrict__ gate_v, double* gsm, GmSmall L, int* arrive,
+                                               double* host)
 {
     extern __shared__ double ls_lds[];
-    k_finish_body<T>(v, Q, k, n3, ld, part_in, hcol, normpart, stop, gate_w, gate_v, gsm, L, arrive, host, ls_lds,
+    k_finish_body<T>(v, Q, k, n3, ld, part_in, hcol, normpart, stop, gate_w, P_w, gate_v, gsm, L, arrive, host, ls_lds,
                      blockIdx.x, gridDim.x);
 }
 
@@ -933,6 +934,16 @@ static int hdi_nred(int n)
     return (int)std::min<long long>(RED_BLOCKS, (3LL * n + 2LL * RT - 1) / (2LL * RT));
 }
 
+// those of them that have a vector of 16 bytes for a thread: the work-groups of the kernels that
+// go by vectors.  In single precision that is half of them; the others added nothing to any sum,
+// but read all partials for it, in a batch of 48 systems 229 against 142 us a launch
+template <typename T>
+static int hdi_nvec(int n)
+{
+    constexpr long long per = (long long)kvec<T>::W * RT;
+    return (int)std::min<long long>(hdi_nred(n), (3LL * n + per - 1) / per);
+}
+
 template <typename T>
 static int hdi_impl(PartBuffers& pb, const PartConst& pc, int maxiter, double tol, int* iters_out, double* res_out,
                     hipStream_t s)
@@ -945,7 +956,7 @@ static int hdi_impl(PartBuffers& pb, const PartConst& pc, int maxiter, double to
     GmSmall L{maxiter};
     const long long ld = (n3 + 63) / 64 * 64;     // column stride of the Krylov vectors
     const unsigned nbr = (unsigned)((n + HT - 1) / HT);
-    const unsigned nred = (unsigned)hdi_nred(n);   // reduction grid
+    const unsigned nred = (unsigned)hdi_nred(n), nvec = (unsigned)hdi_nvec<T>(n);   // reduction grids
     // The neighbour lists are filled and the solve started without a host wait; the
     // first convergence check also reads the lists' flags, and when a row had more
     // neighbours than the lists hold they are widened and the solve starts over (its
@@ -1003,7 +1014,7 @@ static int hdi_impl(PartBuffers& pb, const PartConst& pc, int maxiter, double to
                     hipLaunchKernelGGL((k_spmv<T, 2>), dim3(nbr), dim3(HT), 0, s, nc, ni, nm, n, xin, hx, qo, v,
                                        (const double*)nullptr, (double*)nullptr, (const double*)nullptr, (double*)nullptr,
                                        stop);
-                    hipLaunchKernelGGL((k_mdot<T>), dim3(nred), dim3(RT), 0, s, (const T*)Q, (const T*)v, it, n3, ld, part1,
+                    hipLaunchKernelGGL((k_mdot<T>), dim3(nvec), dim3(RT), 0, s, (const T*)Q, (const T*)v, it, n3, ld, part1,
                                        stop);
                 }
                 // orthogonalise v against q_1..q_it: classical Gram-Schmidt, twice (the
@@ -1011,23 +1022,24 @@ static int hdi_impl(PartBuffers& pb, const PartConst& pc, int maxiter, double to
                 // second pass's update only where the DGKS criterion asks for it
                 double* hcol = Hd + (size_t)M1 * (it - 1);
                 if (it <= 8)
-                    hipLaunchKernelGGL((k_maxpy_mdot<T, 8>), dim3(nred), dim3(RT), 0, s, v, (const T*)Q, it, n3, ld,
-                                       (const double*)part1, hcol, part2, stop);
+                    hipLaunchKernelGGL((k_maxpy_mdot<T, 8>), dim3(nvec), dim3(RT), 0, s, v, (const T*)Q, it, n3, ld,
+                                       (const double*)part1, (int)nred, hcol, part2, stop);
                 else if (it <= 12)
-                    hipLaunchKernelGGL((k_maxpy_mdot<T, 12>), dim3(nred), dim3(RT), 0, s, v, (const T*)Q, it, n3, ld,
-                                       (const double*)part1, hcol, part2, stop);
+                    hipLaunchKernelGGL((k_maxpy_mdot<T, 12>), dim3(nvec), dim3(RT), 0, s, v, (const T*)Q, it, n3, ld,
+                                       (const double*)part1, (int)nred, hcol, part2, stop);
                 else {
-                    hipLaunchKernelGGL((k_maxpy<T>), dim3(nred), dim3(RT), 0, s, v, (const T*)Q, it, n3, ld,
+                    hipLaunchKernelGGL((k_maxpy<T>), dim3(nvec), dim3(RT), 0, s, v, (const T*)Q, it, n3, ld,
                                        (const double*)part1, hcol, stop);
-                    hipLaunchKernelGGL((k_mdot<T>), dim3(nred), dim3(RT), 0, s, (const T*)Q, (const T*)v, it, n3, ld, part2,
+                    hipLaunchKernelGGL((k_mdot<T>), dim3(nvec), dim3(RT), 0, s, (const T*)Q, (const T*)v, it, n3, ld, part2,
                                        stop);
                 }
                 // the second pass's update, skipped where the first kept 1/sqrt(2) of |v|, and the
                 // least squares
-                hipLaunchKernelGGL((k_finish<T>), dim3(nred), dim3(RT), ls_doubles(it) * sizeof(double), s, v, (const T*)Q,
+                const unsigned P1 = it <= 12 ? nred : nvec;        // partials of the first pass
+                hipLaunchKernelGGL((k_finish<T>), dim3(nvec), dim3(RT), ls_doubles(it) * sizeof(double), s, v, (const T*)Q,
                                    it, n3, ld, (const double*)part2, hcol, normpart, stop,
-                                   (const double*)(part1 + (size_t)it * nred), (const double*)(part2 + (size_t)it * nred),
-                                   sm, L, pb.flags + 56, pb.gm_host);
+                                   (const double*)(part1 + (size_t)it * P1), (int)P1,
+                                   (const double*)(part2 + (size_t)it * nvec), sm, L, pb.flags + 56, pb.gm_host);
             }
             DDNS_HIP(hipGetLastError());
             iter = last;
@@ -1100,7 +1112,7 @@ struct GmDesc {
     double* part2;             // second-pass projection partials
     double* normpart;          // |v|^2 partials
     long long n3, ld;
-    int n, nred, nbr;          // nred = 0: the system takes no part (any more)
+    int n, nred, nvec, nbr;    // 0: the system takes no part (any more)
 };
 
 template <typename T>
@@ -1155,28 +1167,28 @@ template <typename T>
 __global__ void __launch_bounds__(RT) kb_mdot(const GmDesc<T>* __restrict__ d, GmSmall L, int it, int second)
 {
     const GmDesc<T>& g = d[blockIdx.y];
-    if ((int)blockIdx.x >= g.nred) return;
+    if ((int)blockIdx.x >= g.nvec) return;
     const GmIter<T> q = gm_iter(g, L, it);
-    k_mdot_body<T>(g.Q, q.v, it, g.n3, g.ld, second ? g.part2 : g.part1, q.stop, blockIdx.x, g.nred);
+    k_mdot_body<T>(g.Q, q.v, it, g.n3, g.ld, second ? g.part2 : g.part1, q.stop, blockIdx.x, g.nvec);
 }
 
 template <typename T, int KC>
 __global__ void __launch_bounds__(RT) kb_maxpy_mdot(const GmDesc<T>* __restrict__ d, GmSmall L, int it)
 {
     const GmDesc<T>& g = d[blockIdx.y];
-    if ((int)blockIdx.x >= g.nred) return;
+    if ((int)blockIdx.x >= g.nvec) return;
     const GmIter<T> q = gm_iter(g, L, it);
-    k_maxpy_mdot_body<T, KC>(q.v, g.Q, it, g.n3, g.ld, g.part1, q.hcol, g.part2, q.stop, blockIdx.x, g.nred);
+    k_maxpy_mdot_body<T, KC>(q.v, g.Q, it, g.n3, g.ld, g.part1, g.nred, q.hcol, g.part2, q.stop, blockIdx.x, g.nvec);
 }
 
 template <typename T>
 __global__ void __launch_bounds__(RT) kb_maxpy(const GmDesc<T>* __restrict__ d, GmSmall L, int it)
 {
     const GmDesc<T>& g = d[blockIdx.y];
-    if ((int)blockIdx.x >= g.nred) return;
+    if ((int)blockIdx.x >= g.nvec) return;
     const GmIter<T> q = gm_iter(g, L, it);
     if (*q.stop != 0.0) return;
-    update_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part1, q.hcol, 0, blockIdx.x, g.nred);
+    update_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part1, g.nvec, q.hcol, 0, blockIdx.x, g.nvec);
 }
 
 template <typename T>
@@ -1184,10 +1196,11 @@ __global__ void __launch_bounds__(RT) kb_finish(const GmDesc<T>* __restrict__ d,
 {
     extern __shared__ double ls_lds[];
     const GmDesc<T>& g = d[blockIdx.y];
-    if ((int)blockIdx.x >= g.nred) return;
+    if ((int)blockIdx.x >= g.nvec) return;
     const GmIter<T> q = gm_iter(g, L, it);
-    k_finish_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part2, q.hcol, g.normpart, q.stop, g.part1 + (size_t)it * g.nred,
-                     g.part2 + (size_t)it * g.nred, g.sm, L, g.arrive, nullptr, ls_lds, blockIdx.x, g.nred);
+    const int P1 = it <= 12 ? g.nred : g.nvec;
+    k_finish_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part2, q.hcol, g.normpart, q.stop, g.part1 + (size_t)it * P1, P1,
+                     g.part2 + (size_t)it * g.nvec, g.sm, L, g.arrive, nullptr, ls_lds, blockIdx.x, g.nvec);
 }
 
 // each system's small-problem head sm[0..5] (and its lists' flags) into 16 doubles
@@ -1230,7 +1243,7 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
         hb.cap = R;
     }
     GmDesc<T>* th = (GmDesc<T>*)hb.table_host;
-    int nredmax = 0, nbrmax = 0, first = 3;
+    int nredmax = 0, nvecmax = 0, nbrmax = 0, first = 3;
     for (int r = 0; r < R; ++r) {
         PartBuffers& pb = *pbs[r];
         const int n = pcs[r]->n;
@@ -1245,9 +1258,10 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
         g.Q = (T*)pb.gm_Q; g.sm = pb.gm_small;
         g.part1 = pb.gm_red; g.part2 = g.part1 + (size_t)64 * RED_BLOCKS; g.normpart = g.part2 + (size_t)64 * RED_BLOCKS;
         g.n3 = 3LL * n; g.ld = (g.n3 + 63) / 64 * 64; g.n = n;
-        g.nred = hdi_nred(n); g.nbr = (n + HT - 1) / HT;
+        g.nred = hdi_nred(n); g.nvec = hdi_nvec<T>(n); g.nbr = (n + HT - 1) / HT;
         th[r] = g;
         nredmax = std::max(nredmax, g.nred);
+        nvecmax = std::max(nvecmax, g.nvec);
         nbrmax = std::max(nbrmax, g.nbr);
         first = std::max(first, pb.gm_last_iters);
     }
@@ -1263,22 +1277,22 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
         for (int r = 0; r < R; ++r) any = any || (!done[r] && !redo[r]);
         if (!any) break;
         const int last = std::min(maxiter, iter + (iter == 0 ? first : BATCH));
-        const dim3 g(nredmax, R);
+        const dim3 g(nredmax, R), gv(nvecmax, R);
         for (int it = iter + 1; it <= last; ++it) {
             if (it == 1) hipLaunchKernelGGL((kb_spmv_mdot<T, 1, 8>), g, dim3(RT), 0, s, td, L, it);
             else if (it <= 8) hipLaunchKernelGGL((kb_spmv_mdot<T, 2, 8>), g, dim3(RT), 0, s, td, L, it);
             else if (it <= 12) hipLaunchKernelGGL((kb_spmv_mdot<T, 2, 12>), g, dim3(RT), 0, s, td, L, it);
             else {
                 hipLaunchKernelGGL((kb_spmv2<T>), dim3(nbrmax, R), dim3(HT), 0, s, td, L, it);
-                hipLaunchKernelGGL((kb_mdot<T>), g, dim3(RT), 0, s, td, L, it, 0);
+                hipLaunchKernelGGL((kb_mdot<T>), gv, dim3(RT), 0, s, td, L, it, 0);
             }
-            if (it <= 8) hipLaunchKernelGGL((kb_maxpy_mdot<T, 8>), g, dim3(RT), 0, s, td, L, it);
-            else if (it <= 12) hipLaunchKernelGGL((kb_maxpy_mdot<T, 12>), g, dim3(RT), 0, s, td, L, it);
+            if (it <= 8) hipLaunchKernelGGL((kb_maxpy_mdot<T, 8>), gv, dim3(RT), 0, s, td, L, it);
+            else if (it <= 12) hipLaunchKernelGGL((kb_maxpy_mdot<T, 12>), gv, dim3(RT), 0, s, td, L, it);
             else {
-                hipLaunchKernelGGL((kb_maxpy<T>), g, dim3(RT), 0, s, td, L, it);
-                hipLaunchKernelGGL((kb_mdot<T>), g, dim3(RT), 0, s, td, L, it, 1);
+                hipLaunchKernelGGL((kb_maxpy<T>), gv, dim3(RT), 0, s, td, L, it);
+                hipLaunchKernelGGL((kb_mdot<T>), gv, dim3(RT), 0, s, td, L, it, 1);
             }
-            hipLaunchKernelGGL((kb_finish<T>), g, dim3(RT), ls_doubles(it) * sizeof(double), s, td, L, it);
+            hipLaunchKernelGGL((kb_finish<T>), gv, dim3(RT), ls_doubles(it) * sizeof(double), s, td, L, it);
         }
         DDNS_HIP(hipGetLastError());
         iter = last;
@@ -1300,8 +1314,7 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
                 std::memcpy(f, h + 8, sizeof(f));
                 // the system leaves the merged launches before its lists are reallocated
                 if (f[0] & 3 || f[4] > pbs[r]->ell_width) {
-                    th[r].nred = 0;
-                    th[r].nbr = 0;
+                    th[r].nred = th[r].nvec = th[r].nbr = 0;
                     retable = true;
                 }
                 const int lo = lists_outcome<T>(*pbs[r], f, s);
