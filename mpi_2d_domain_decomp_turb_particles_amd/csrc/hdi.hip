@@ -773,17 +773,18 @@ __global__ void __launch_bounds__(RT) k_maxpy(T* __restrict__ v, const T* __rest
 // the single wavefront of the least squares took 5.2 + 7.8 us at 100 000 droplets.
 // ls: ls_doubles(k) of LDS.
 template <typename T>
-__device__ __forceinline__ void k_finish_body(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
+__global__ void __launch_bounds__(RT) k_finish(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
                                                long long ld, const double* __restrict__ part_in,
-                                               double* hcol, double* __restrict__ normpart,
-                                               const double* __restrict__ stop, const double* __restrict__ gate_w,
-                                               int P_w, const double* __restrict__ gate_v, double* gsm, GmSmall L,
-                                               int* arrive, double* host, double* ls, int bx, int nbx)
+                                               double* hcol, double* normpart, const double* stop,
+                                               const double* __restrict__ gate_w, int P_w,
+                                               const double* __restrict__ gate_v, double* gsm, GmSmall L, int* arrive,
+                                               double* host)
 {
+    extern __shared__ double ls[];
     __shared__ double g1[2];
     __shared__ int last;
     if (*stop != 0.0) return;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, bx = blockIdx.x, nbx = gridDim.x;
     if (bx == 0 && tid >= RT / 2) ls_load(ls, gsm, L, k, tid - RT / 2, RT / 2);
     const double nw = sum_one(gate_w, P_w, &g1[0]);
     double nv2 = sum_one(gate_v, nbx, &g1[1]);
@@ -804,18 +805,6 @@ __device__ __forceinline__ void k_finish_body(T* __restrict__ v, const T* __rest
         nv2 = sum_one(normpart, nbx, &g1[0]);
     }
     if (tid < LT) ls_solve(ls, gsm, L, k, sqrt(nv2), host);
-}
-template <typename T>
-__global__ void __launch_bounds__(RT) k_finish(T* __restrict__ v, const T* __restrict__ Q, int k, long long n3,
-                                               long long ld, const double* __restrict__ part_in,
-                                               double* hcol, double* normpart, const double* stop,
-                                               const double* __restrict__ gate_w, int P_w,
-                                               const double* __restrict__ gate_v, double* gsm, GmSmall L, int* arrive,
-                                               double* host)
-{
-    extern __shared__ double ls_lds[];
-    k_finish_body<T>(v, Q, k, n3, ld, part_in, hcol, normpart, stop, gate_w, P_w, gate_v, gsm, L, arrive, host, ls_lds,
-                     blockIdx.x, gridDim.x);
 }
 
 // pertvel = x0 + Q y (2951-2956), scattered back to the reference's droplet order.  The
@@ -1105,7 +1094,6 @@ struct GmDesc {
     const int* idx;
     const T* mm;
     const int* flags;          // the neighbour lists' flags (read at the first check)
-    int* arrive;               // counter of k_finish
     T* Q;                      // maxiter Krylov columns, then the two work vectors
     double* sm;                // the small problem (GmSmall layout)
     double* part1;             // first-pass projection partials
@@ -1191,16 +1179,44 @@ __global__ void __launch_bounds__(RT) kb_maxpy(const GmDesc<T>* __restrict__ d, 
     update_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part1, g.nvec, q.hcol, 0, blockIdx.x, g.nvec);
 }
 
+// k_finish as two launches: the second pass's update, then the least squares of every system.  In
+// one launch each of the systems' work-groups, 2000 to 12 000 in all, wrote back and invalidated
+// its XCD's L2 for the arrival: 228 us a launch with 48 systems, 47 + 8 as two (a system alone has at most
+// 256, and saves the second launch).
 template <typename T>
-__global__ void __launch_bounds__(RT) kb_finish(const GmDesc<T>* __restrict__ d, GmSmall L, int it)
+__device__ __forceinline__ bool kb_gate(const GmDesc<T>& g, int it, double* g1, double* nv2)
 {
-    extern __shared__ double ls_lds[];
+    const int P1 = it <= 12 ? g.nred : g.nvec;
+    const double nw = sum_one(g.part1 + (size_t)it * P1, P1, &g1[0]);
+    *nv2 = sum_one(g.part2 + (size_t)it * g.nvec, g.nvec, &g1[1]);
+    return *nv2 >= 0.5 * nw;                     // the first pass suffices
+}
+
+template <typename T>
+__global__ void __launch_bounds__(RT) kb_second(const GmDesc<T>* __restrict__ d, GmSmall L, int it)
+{
+    __shared__ double g1[2];
     const GmDesc<T>& g = d[blockIdx.y];
     if ((int)blockIdx.x >= g.nvec) return;
     const GmIter<T> q = gm_iter(g, L, it);
-    const int P1 = it <= 12 ? g.nred : g.nvec;
-    k_finish_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part2, q.hcol, g.normpart, q.stop, g.part1 + (size_t)it * P1, P1,
-                     g.part2 + (size_t)it * g.nvec, g.sm, L, g.arrive, nullptr, ls_lds, blockIdx.x, g.nvec);
+    if (*q.stop != 0.0) return;
+    double nv2;
+    if (kb_gate(g, it, g1, &nv2)) return;
+    const double mine = update_body<T>(q.v, g.Q, it, g.n3, g.ld, g.part2, g.nvec, q.hcol, 1, blockIdx.x, g.nvec);
+    if (threadIdx.x == 0) g.normpart[blockIdx.x] = mine;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(HT) kb_ls(const GmDesc<T>* __restrict__ d, GmSmall L, int it)
+{
+    extern __shared__ double ls_lds[];
+    __shared__ double g1[2], g2;
+    const GmDesc<T>& g = d[blockIdx.x];
+    if (g.nred == 0 || g.sm[4] != 0.0) return;
+    ls_load(ls_lds, g.sm, L, it, threadIdx.x, HT);
+    double nv2;
+    if (!kb_gate(g, it, g1, &nv2)) nv2 = sum_one(g.normpart, g.nvec, &g2);
+    if (threadIdx.x < LT) ls_solve(ls_lds, g.sm, L, it, sqrt(nv2), nullptr);
 }
 
 // each system's small-problem head sm[0..5] (and its lists' flags) into 16 doubles
@@ -1254,7 +1270,6 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
             continue;
         }
         g.cnt = pb.nei_cnt; g.idx = pb.nei_idx; g.mm = (const T*)pb.nei_m; g.flags = pb.flags;
-        g.arrive = pb.flags + 56;
         g.Q = (T*)pb.gm_Q; g.sm = pb.gm_small;
         g.part1 = pb.gm_red; g.part2 = g.part1 + (size_t)64 * RED_BLOCKS; g.normpart = g.part2 + (size_t)64 * RED_BLOCKS;
         g.n3 = 3LL * n; g.ld = (g.n3 + 63) / 64 * 64; g.n = n;
@@ -1292,7 +1307,8 @@ static int hdi_batch_impl(HdiBatch& hb, PartBuffers* const* pbs, const PartConst
                 hipLaunchKernelGGL((kb_maxpy<T>), gv, dim3(RT), 0, s, td, L, it);
                 hipLaunchKernelGGL((kb_mdot<T>), gv, dim3(RT), 0, s, td, L, it, 1);
             }
-            hipLaunchKernelGGL((kb_finish<T>), gv, dim3(RT), ls_doubles(it) * sizeof(double), s, td, L, it);
+            hipLaunchKernelGGL((kb_second<T>), gv, dim3(RT), 0, s, td, L, it);
+            hipLaunchKernelGGL((kb_ls<T>), dim3(R), dim3(HT), ls_doubles(it) * sizeof(double), s, td, L, it);
         }
         DDNS_HIP(hipGetLastError());
         iter = last;
