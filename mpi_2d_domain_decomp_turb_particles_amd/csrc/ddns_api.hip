@@ -432,6 +432,7 @@ static void destroy_impl(ddns_handle* h)
         if (h->fb.dg_part) (void)hipFree(h->fb.dg_part);
         if (h->fb.spec_part) (void)hipFree(h->fb.spec_part);
         if (h->fb.stage) (void)hipFree(h->fb.stage);
+        if (h->fb.bounce.host) (void)hipHostFree(h->fb.bounce.host);
     }
     part_free(h->pb);
     for (int i = 0; i < 16; ++i) if (h->ev[i]) (void)hipEventDestroy(h->ev[i]);

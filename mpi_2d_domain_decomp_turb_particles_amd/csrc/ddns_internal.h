@@ -252,6 +252,26 @@ template <typename T> __device__ __forceinline__ void spec_mode(int N, size_t t,
     ky = (int)(row / ((size_t)N * nb));
     kx = kb * W + (int)(t % W);
 }
+// Outputs of at most BOUNCE_BYTES in all are formed side by side on the device, copied to pinned
+// memory at once and from there to the caller's arrays by the host.  A copy straight to pageable
+// memory waits for its kernel and takes 20 to 65 us however small it is, and an output has three to
+// six of them: 1000 droplets 178 us, now 64, 5000 250 and 130, the velocity at 32^3 FP32 82 and 66,
+// the state there 236 and 140 (through host loops 245, 222, 54 and 217).  The host's second pass
+// over the values eats the gain up with size: 6 MB of droplets take 410 us for 505.
+constexpr size_t BOUNCE_BYTES = 8u << 20;
+struct Bounce {
+    double* host = nullptr;                     // pinned, grown to the largest such output
+    size_t bytes = 0;
+};
+inline int bounce_room(Bounce& b, size_t bytes)
+{
+    if (b.bytes >= bytes) return 0;
+    if (b.host) DDNS_HIP(hipHostFree(b.host));
+    b = Bounce{};
+    DDNS_HIP(hipHostMalloc((void**)&b.host, bytes, hipHostMallocDefault));
+    b.bytes = bytes;
+    return 0;
+}
 struct FlowBuffers {
     void* U[3] = {nullptr, nullptr, nullptr};  // state u-hat
     void* O[3] = {nullptr, nullptr, nullptr};  // AB2 history
@@ -268,6 +288,7 @@ struct FlowBuffers {
     double* spec_part = nullptr;                // E(k): SPEC_BLOCKS partial rows of SPEC_NEK_MAX shells, then the result
     void* stage = nullptr;                      // state transfers: a part of a field in the reference's layout
     size_t stage_bytes = 0;                     // (allocated on first use, kept with the handle)
+    Bounce bounce;                              // small outputs on their way to the caller's arrays
     int ky_tc = 0;                              // y-stage tile width chosen by flow_tune (0: the default)
     float ky_ms[3] = {0, 0, 0};                 // the tuner's time per y stage pair of each candidate (0: not valid)
     int kz_nt = 0;                              // threads of the fused z stage chosen by flow_tune (0: the default)
@@ -438,7 +459,9 @@ struct PartBuffers {
     int* draw_off = nullptr;    // cap + 1
     int* rng_state = nullptr;   // ranff2 state: idum, iy, idum2, iv[32]
     double* red = nullptr;      // generic reduction scratch
-    double* stage = nullptr;    // 12*cap: one droplet array in the reference's layout, made on the first transfer
+    double* stage = nullptr;    // droplet arrays in the reference's layout, made on the first transfer: one
+                                // array of 12*cap, or several of a small output (Bounce)
+    Bounce bounce;
 };
 
 struct PartConst {

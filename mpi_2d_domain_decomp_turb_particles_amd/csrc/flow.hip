@@ -1154,6 +1154,7 @@ void flow_free(FlowBuffers& fb)
     if (fb.dg_part) (void)hipFree(fb.dg_part);
     if (fb.spec_part) (void)hipFree(fb.spec_part);
     if (fb.stage) (void)hipFree(fb.stage);
+    if (fb.bounce.host) (void)hipHostFree(fb.bounce.host);
     fb = FlowBuffers{};
 }
 
@@ -1523,6 +1524,36 @@ int flow_upload_state(FlowBuffers& fb, int N, int precision, const double* const
 
 int flow_download_state(FlowBuffers& fb, int N, int precision, double* const dst[6], hipStream_t s)
 {
+    const size_t each = (size_t)N * (N + 2) * (N + 2);
+    size_t nf = 0;
+    for (int f = 0; f < 6; ++f) nf += dst[f] != nullptr;
+    if (nf > 0 && nf * each * sizeof(double) <= BOUNCE_BYTES) {
+        double* st = nullptr;
+        int rc = bounce_room(fb.bounce, nf * each * sizeof(double));
+        if (!rc) rc = stage_buffer(fb, nf * each * sizeof(double), &st);
+        if (rc) return rc;
+        size_t at = 0;
+        for (int f = 0; f < 6; ++f) {
+            if (!dst[f]) continue;
+            void* dev = f < 3 ? fb.U[f] : fb.O[f - 3];
+            const dim3 g((N + 2 + 31) / 32, (N / 2 + 1 + 31) / 32, N);
+            if (precision == DDNS_FP64)
+                hipLaunchKernelGGL((k_layout<double, true>), g, dim3(256), 0, s, (cpx<double>*)dev, st + at, N, 0);
+            else
+                hipLaunchKernelGGL((k_layout<float, true>), g, dim3(256), 0, s, (cpx<float>*)dev, st + at, N, 0);
+            at += each;
+        }
+        DDNS_HIP(hipGetLastError());
+        DDNS_HIP(hipMemcpyAsync(fb.bounce.host, st, at * sizeof(double), hipMemcpyDeviceToHost, s));
+        DDNS_HIP(hipStreamSynchronize(s));
+        at = 0;
+        for (int f = 0; f < 6; ++f) {
+            if (!dst[f]) continue;
+            std::memcpy(dst[f], fb.bounce.host + at, each * sizeof(double));
+            at += each;
+        }
+        return 0;
+    }
     for (int f = 0; f < 6; ++f) {
         if (!dst[f]) continue;
         const void* dev = f < 3 ? fb.U[f] : fb.O[f - 3];
@@ -1549,17 +1580,22 @@ static int download_phys_t(FlowBuffers& fb, int N, double* ux, double* uy, doubl
     const size_t n3 = (size_t)N * N * N;
     const size_t chunk = std::min(n3, STAGE_BYTES / (3 * sizeof(double)) / 256 * 256);
     double* st = nullptr;
-    const int rc = stage_buffer(fb, 3 * chunk * sizeof(double), &st);
+    const bool small = 3 * n3 * sizeof(double) <= BOUNCE_BYTES;          // then one chunk
+    int rc = stage_buffer(fb, 3 * chunk * sizeof(double), &st);
+    if (!rc && small) rc = bounce_room(fb.bounce, 3 * n3 * sizeof(double));
     if (rc) return rc;
     double* d[3] = {ux, uy, uz};
     for (size_t i = 0; i < n3; i += chunk) {
         const size_t m = std::min(chunk, n3 - i);
         hipLaunchKernelGGL((k_phys_planes<T>), dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, (const T*)fb.uphys, st, i, m);
         DDNS_HIP(hipGetLastError());
+        if (small) DDNS_HIP(hipMemcpyAsync(fb.bounce.host, st, 3 * m * sizeof(double), hipMemcpyDeviceToHost, s));
         for (int c = 0; c < 3; ++c)
-            if (d[c]) DDNS_HIP(hipMemcpyAsync(d[c] + i, st + c * m, m * sizeof(double), hipMemcpyDeviceToHost, s));
+            if (d[c] && !small) DDNS_HIP(hipMemcpyAsync(d[c] + i, st + c * m, m * sizeof(double), hipMemcpyDeviceToHost, s));
     }
     DDNS_HIP(hipStreamSynchronize(s));
+    for (int c = 0; c < 3; ++c)
+        if (d[c] && small) std::memcpy(d[c], fb.bounce.host + c * n3, n3 * sizeof(double));
     return 0;
 }
 

@@ -12,6 +12,8 @@
 // removal list and of the relocation draws) is evaluated on slot numbers.
 #include "ddns_internal.h"
 
+#include <cstring>
+
 #include <algorithm>
 #include <cmath>
 
@@ -250,6 +252,7 @@ void part_free(PartBuffers& pb)
     if (pb.sync_ev) (void)hipEventDestroy(pb.sync_ev);
     if (pb.gm_host) (void)hipHostFree(pb.gm_host);
     if (pb.found_host) (void)hipHostFree(pb.found_host);
+    if (pb.bounce.host) (void)hipHostFree(pb.bounce.host);
     if (pb.counts_host) (void)hipHostFree(pb.counts_host);
     pb = PartBuffers{};
 }
@@ -275,7 +278,8 @@ __global__ void __launch_bounds__(PT) k_columns(Columns a, int K, double* __rest
 
 static int stage_rows(PartBuffers& pb)
 {
-    if (!pb.stage) DDNS_HIP(hipMalloc(&pb.stage, 12 * (size_t)pb.cap * sizeof(double)));
+    const size_t all = std::min(35 * (size_t)pb.cap * sizeof(double), BOUNCE_BYTES);   // yp, fvp, fdp, vp, dmove
+    if (!pb.stage) DDNS_HIP(hipMalloc(&pb.stage, std::max(12 * (size_t)pb.cap * sizeof(double), all)));
     return 0;
 }
 
@@ -366,11 +370,35 @@ int part_download(PartBuffers& pb, int n, double* yp, double* fvp, double* fdp, 
         for (int q = 0; q < 3; ++q) a.col[3 * t + q] = pb.fvp + (size_t)(pb.vcol(t == 0 && pb.v0_stale ? 1 : t) + q) * c;
     for (int t = 0; t < 4; ++t)
         for (int q = 0; q < 3; ++q) b.col[3 * t + q] = pb.fdp + (size_t)(pb.dcol(t == 0 && pb.d0_stale ? 1 : t) + q) * c;
-    st = columns_out(pb, yp_columns(pb), 8, yp, n, s);
-    if (!st) st = columns_out(pb, a, 9, fvp, n, s);
-    if (!st) st = columns_out(pb, b, 12, fdp, n, s);
-    if (!st) st = columns_out(pb, vec_columns(pb.vp, pb.cap), 3, vp, n, s);
-    if (!st) st = columns_out(pb, vec_columns(pb.dmove, pb.cap), 3, dmove, n, s);
+    const Columns cols[5] = {yp_columns(pb), a, b, vec_columns(pb.vp, pb.cap), vec_columns(pb.dmove, pb.cap)};
+    const int K[5] = {8, 9, 12, 3, 3};
+    double* const host[5] = {yp, fvp, fdp, vp, dmove};
+    size_t per = 0;                                 // values of a droplet that go through the staging buffer
+    for (int k = 0; k < 5; ++k) per += host[k] ? K[k] : 0;
+    const size_t m = (size_t)std::max(0, n), pv = pertvel ? 3 * m : 0, bytes = (per * m + pv) * sizeof(double);
+    if (bytes > 0 && bytes <= BOUNCE_BYTES) {
+        st = bounce_room(pb.bounce, bytes);
+        if (st) return st;
+        double* at = pb.stage;
+        for (int k = 0; k < 5; ++k) {
+            if (!host[k]) continue;
+            hipLaunchKernelGGL(k_columns<true>, dim3(nblk((long long)n * K[k])), dim3(PT), 0, s, cols[k], K[k], at, n);
+            at += K[k] * m;
+        }
+        DDNS_HIP(hipGetLastError());
+        if (per) DDNS_HIP(hipMemcpyAsync(pb.bounce.host, pb.stage, per * m * sizeof(double), hipMemcpyDeviceToHost, s));
+        if (pv) DDNS_HIP(hipMemcpyAsync(pb.bounce.host + per * m, pb.pert, pv * sizeof(double), hipMemcpyDeviceToHost, s));
+        DDNS_HIP(hipStreamSynchronize(s));
+        const double* from = pb.bounce.host;
+        for (int k = 0; k < 5; ++k) {
+            if (!host[k]) continue;
+            std::memcpy(host[k], from, K[k] * m * sizeof(double));
+            from += K[k] * m;
+        }
+        if (pv) std::memcpy(pertvel, from, pv * sizeof(double));
+        return 0;
+    }
+    for (int k = 0; k < 5 && !st; ++k) st = columns_out(pb, cols[k], K[k], host[k], n, s);
     if (st) return st;
     if (pertvel && n > 0) DDNS_HIP(hipMemcpyAsync(pertvel, pb.pert, 3 * (size_t)n * sizeof(double), hipMemcpyDeviceToHost, s));
     DDNS_HIP(hipStreamSynchronize(s));

@@ -1,5 +1,7 @@
 """State transfers: the layouts are formed on the device, in pieces where an array is larger
 than the staging buffer."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -52,3 +54,26 @@ def test_droplet_round_trip(ddns, n):
         s.set_droplets(yp[:, :n // 2])
         d = s.get_droplets()
         assert np.array_equal(d["yp"], yp[:, :n // 2]) and not any(d[k].any() for k in a)
+
+
+@pytest.mark.parametrize("n", [3, 27000, 40000])
+def test_some_of_the_droplet_arrays(ddns, n):
+    """Each array alone, pairs of them and all give the same values: outputs of up to 8 MB go to the
+    caller through one copy, larger ones array by array."""
+    rng = np.random.default_rng(n)
+    p = ddns.default_params(N=32, precision=0, npart=n, nset=1, radius=[5.0], dt=1e-6)
+    size = dict(yp=8, fvp=9, fdp=12, pertvel=3, vp=3, dmove=3)
+    with ddns.Solver(p) as s:
+        s.init_flow(ddns.SPEC_K4_GAUSS, 3, 4.0, 0.1)
+        s.init_droplets(seed=5)
+        s.step(2)
+        d = s.get_droplets()
+        s.set_droplets(d["yp"], d["fvp"], d["fdp"], np.asfortranarray(rng.random((3, n))))
+        every = {k: np.ravel(a, order="F") for k, a in s.get_droplets().items()}
+        assert all(every[k].size == size[k] * n and every[k].any() for k in size)
+        for chosen in ([k] for k in size):
+            chosen = chosen + list(size)[::3]
+            out = {k: np.full(size[k] * n, np.nan) for k in chosen}
+            ptr = [out[k].ctypes.data_as(ctypes.POINTER(ctypes.c_double)) if k in out else None for k in size]
+            assert s.lib.ddns_get_droplets(s.h, None, *ptr) == 0
+            assert all(np.array_equal(out[k], every[k]) for k in out)
