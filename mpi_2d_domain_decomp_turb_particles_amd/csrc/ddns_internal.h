@@ -252,13 +252,16 @@ template <typename T> __device__ __forceinline__ void spec_mode(int N, size_t t,
     ky = (int)(row / ((size_t)N * nb));
     kx = kb * W + (int)(t % W);
 }
-// Outputs of at most BOUNCE_BYTES in all are formed side by side on the device, copied to pinned
-// memory at once and from there to the caller's arrays by the host.  A copy straight to pageable
-// memory waits for its kernel and takes 20 to 65 us however small it is, and an output has three to
-// six of them: 1000 droplets 178 us, now 64, 5000 250 and 130, the velocity at 32^3 FP32 82 and 66,
-// the state there 236 and 140 (through host loops 245, 222, 54 and 217).  The host's second pass
-// over the values eats the gain up with size: 6 MB of droplets take 410 us for 505.
-constexpr size_t BOUNCE_BYTES = 8u << 20;
+// Small outputs are formed side by side on the device, copied to pinned memory at once and from
+// there to the caller's arrays by the host.  A copy straight to pageable memory waits for its
+// kernel and takes 20 to 65 us however small it is, and an output has three to six of them: 1000
+// droplets 178 us, now 64, 5000 250 and 130, the velocity at 32^3 FP32 82 and 66, the state there
+// 236 and 140 (through host loops 245, 222, 54 and 217).  The host's second pass over the values
+// eats the gain up with size, and a handle's first small output allocates the memory (0.1 to
+// 0.4 ms).  Droplets: up to 2 MB, where a copy per array becomes as fast as the host loops were
+// (with 8 MB the first pass of a new batch of 16 is 70 -> 81 ms).  Fields: up to 8 MB, so that the
+// velocity at 64^3 FP32 is among them (475 and 430 us; 16 MB: no faster).
+constexpr size_t BOUNCE_ROWS = 2u << 20, BOUNCE_FIELDS = 8u << 20;
 struct Bounce {
     double* host = nullptr;                     // pinned, grown to the largest such output
     size_t bytes = 0;

@@ -1527,7 +1527,7 @@ int flow_download_state(FlowBuffers& fb, int N, int precision, double* const dst
     const size_t each = (size_t)N * (N + 2) * (N + 2);
     size_t nf = 0;
     for (int f = 0; f < 6; ++f) nf += dst[f] != nullptr;
-    if (nf > 0 && nf * each * sizeof(double) <= BOUNCE_BYTES) {
+    if (nf > 0 && nf * each * sizeof(double) <= BOUNCE_FIELDS) {
         double* st = nullptr;
         int rc = bounce_room(fb.bounce, nf * each * sizeof(double));
         if (!rc) rc = stage_buffer(fb, nf * each * sizeof(double), &st);
@@ -1580,7 +1580,7 @@ static int download_phys_t(FlowBuffers& fb, int N, double* ux, double* uy, doubl
     const size_t n3 = (size_t)N * N * N;
     const size_t chunk = std::min(n3, STAGE_BYTES / (3 * sizeof(double)) / 256 * 256);
     double* st = nullptr;
-    const bool small = 3 * n3 * sizeof(double) <= BOUNCE_BYTES;          // then one chunk
+    const bool small = 3 * n3 * sizeof(double) <= BOUNCE_FIELDS;          // then one chunk
     int rc = stage_buffer(fb, 3 * chunk * sizeof(double), &st);
     if (!rc && small) rc = bounce_room(fb.bounce, 3 * n3 * sizeof(double));
     if (rc) return rc;

@@ -278,7 +278,7 @@ __global__ void __launch_bounds__(PT) k_columns(Columns a, int K, double* __rest
 
 static int stage_rows(PartBuffers& pb)
 {
-    const size_t all = std::min(35 * (size_t)pb.cap * sizeof(double), BOUNCE_BYTES);   // yp, fvp, fdp, vp, dmove
+    const size_t all = std::min(35 * (size_t)pb.cap * sizeof(double), BOUNCE_ROWS);   // yp, fvp, fdp, vp, dmove
     if (!pb.stage) DDNS_HIP(hipMalloc(&pb.stage, std::max(12 * (size_t)pb.cap * sizeof(double), all)));
     return 0;
 }
@@ -376,7 +376,7 @@ int part_download(PartBuffers& pb, int n, double* yp, double* fvp, double* fdp, 
     size_t per = 0;                                 // values of a droplet that go through the staging buffer
     for (int k = 0; k < 5; ++k) per += host[k] ? K[k] : 0;
     const size_t m = (size_t)std::max(0, n), pv = pertvel ? 3 * m : 0, bytes = (per * m + pv) * sizeof(double);
-    if (bytes > 0 && bytes <= BOUNCE_BYTES) {
+    if (bytes > 0 && bytes <= BOUNCE_ROWS) {
         st = bounce_room(pb.bounce, bytes);
         if (st) return st;
         double* at = pb.stage;

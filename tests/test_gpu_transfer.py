@@ -56,9 +56,9 @@ def test_droplet_round_trip(ddns, n):
         assert np.array_equal(d["yp"], yp[:, :n // 2]) and not any(d[k].any() for k in a)
 
 
-@pytest.mark.parametrize("n", [3, 27000, 40000])
+@pytest.mark.parametrize("n", [3, 6800, 27000, 40000])
 def test_some_of_the_droplet_arrays(ddns, n):
-    """Each array alone, pairs of them and all give the same values: outputs of up to 8 MB go to the
+    """Each array alone, pairs of them and all give the same values: outputs of up to 2 MB go to the
     caller through one copy, larger ones array by array."""
     rng = np.random.default_rng(n)
     p = ddns.default_params(N=32, precision=0, npart=n, nset=1, radius=[5.0], dt=1e-6)
