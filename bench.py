@@ -456,7 +456,7 @@ def main(argv=None):
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(dom, N, dd.FP32_MIXED),
                      "algorithmic_bytes": kb[dom],
-                     "timing": "frac: mean launch time in the first, the last and every 16th of the timed steps "
+                     "timing": "frac: mean launch time in the last and every 16th of the timed steps "
                                "(HIP events on the flow stream, with the droplet block running beside it); "
                                "frac_alone: the flow step alone",
                      "achieved_alone": achieved_alone, "frac_alone": achieved_alone / HBM_PEAK_GBS},

@@ -136,8 +136,9 @@ typedef struct ddns_collision_counts {
 /* Kernel-level timing of the last ddns_step call, from HIP events (milliseconds). */
 typedef struct ddns_timing {
     double flow_ms;           /* spectral step: FFT stages + fused update (with droplets:
-                                 from the steps that are timed, the first, the last and
-                                 every 16th, taken for all nsteps)                     */
+                                 from the steps that are timed, the last and every
+                                 16th, taken for all nsteps, and the inverse
+                                 transforms of a new state)                            */
     double interp_ms;         /* Lagrange gather                                       */
     double cells_ms;          /* cell binning (keys + sort)                            */
     double hdi_ms;            /* HI neighbour build + GMRES                            */

@@ -77,11 +77,12 @@ struct ddns_handle {
     // environment at ddns_create)
     hipGraphExec_t gflow[4][3] = {};
     // Whether the step in progress, and the one after it, record their kernels' times: the
-    // first and the last of a call do and every TIMED_EVERY-th between (timed_step), and the
+    // last of a call does and of a longer one every TIMED_EVERY-th (timed_step), and the
     // others are taken to be like them.  Nine event nodes in every step kept the flow stream
     // busier than its kernels did: with 10 000 droplets at 64^3 a step took 0.157 instead of
-    // 0.139 ms, at 128^3 with HI 0.568 instead of 0.551, at 256^3 2.67 instead of 2.65.  (The
-    // last step alone, taken for all, gave 15 to 29 us for the z stage at 64^3, 16 on average.)
+    // 0.139 ms, at 128^3 with HI 0.568 instead of 0.551, at 256^3 2.67 instead of 2.65; in the
+    // first of two steps, 128^3 with 130 000 droplets, 0.288 instead of 0.272.  (The last step
+    // alone, taken for all of a long call, gave 15 to 29 us for the z stage at 64^3, 16 on average.)
     bool timed = true, timed_next = true;
     // a set whose step's flow is queued and whose times are not in the sums of the call yet:
     // they are taken when the set is needed again (take_flow_times), so no step waits for them
@@ -801,7 +802,7 @@ static int run_flow_steps(ddns_handle* h, int nsteps)
 }
 
 constexpr int TIMED_EVERY = 16;
-static bool timed_step(int k, int nsteps) { return k == 0 || k + 1 == nsteps || k % TIMED_EVERY == TIMED_EVERY / 2; }
+static bool timed_step(int k, int nsteps) { return k + 1 == nsteps || k % TIMED_EVERY == TIMED_EVERY / 2; }
 
 // Adds the times of the timed step that last used event set q to the sums of the call.  The
 // first half that needs the set again is queued behind a whole step that follows those times
